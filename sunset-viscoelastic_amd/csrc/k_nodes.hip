@@ -17,10 +17,6 @@
 
 #include <hipcub/hipcub.hpp>
 
-#include <climits>
-#include <cstdint>
-#include <thread>
-
 #include "sv_internal.h"
 
 #define SS 2.0
@@ -455,299 +451,5 @@ int sv_dev_build_sell(sv_ctx *c) {
   SV_HIP(c, hipGetLastError());
   SV_HIP(c, hipStreamSynchronize(c->stream));
   c->sell_dirty = false;
-  return 0;
-}
-
-// ---- time-loop layout (Morton order) --------------------------------------
-namespace {
-
-// Loop-order SELL packing: block (s, y) fills links [16y, 16y+16) of the 64
-// nodes of slice s.  The CSR rows are read 16 links at a time (one cache
-// line of each array per row), transposed through LDS, and written as the
-// slice's link-major columns (64 consecutive slots per link).  Links past a
-// node's count, and slots past npfb, get the padding entry: the node's own
-// slot (0 past npfb) with zero weights.
-constexpr int PK_K = 16;           // links per block
-constexpr int PK_T = 256;          // threads per block
-constexpr int PK_LD = PK_K + 1;    // LDS row stride of the tiles
-__global__ __launch_bounds__(PK_T) void k_loop_pack(
-    int npfb, const int64_t *off, const int *perm, const int *iperm, const int64_t *row_ptr,
-    const int *cnt, const int *col_raw, const int *irel, const int *vrel, const double *wx,
-    const double *wy, const double *wl, const double *wh, int64_t nnz_max, int *lcol,
-    double *lwx, double *lwy, double *lwl, double *lwh, uint8_t *lflip) {
-  __shared__ double tx[SV_WAVE * PK_LD], ty[SV_WAVE * PK_LD], tl[SV_WAVE * PK_LD],
-      th[SV_WAVE * PK_LD];
-  __shared__ int tc[SV_WAVE * PK_LD];
-  __shared__ uint8_t tf[SV_WAVE * PK_LD];
-  __shared__ int rnode[SV_WAVE], rcnt[SV_WAVE];
-  __shared__ int64_t rbase[SV_WAVE];
-  const int s = blockIdx.x;
-  const int t = threadIdx.x;
-  const int64_t o = off[s];
-  const int W = (int)((off[s + 1] - o) / SV_WAVE);
-  const int k0 = blockIdx.y * PK_K;
-  if (k0 >= W) return;
-  if (t < SV_WAVE) {
-    const int slot = s * SV_WAVE + t;
-    const int i = slot < npfb ? perm[slot] : -1;
-    rnode[t] = i;
-    rcnt[t] = i >= 0 ? cnt[i] : 0;
-    rbase[t] = i >= 0 ? row_ptr[i] : 0;
-  }
-  __syncthreads();
-  // gather: 16 consecutive threads read 16 consecutive links of one row
-  for (int p = t; p < SV_WAVE * PK_K; p += PK_T) {
-    const int r = p / PK_K, kk = p % PK_K, k = k0 + kk;
-    const int slot = s * SV_WAVE + r;
-    const int e = r * PK_LD + kk;
-    if (rnode[r] >= 0 && k < rcnt[r]) {
-      const int64_t sidx = rbase[r] + k;
-      const int raw = col_raw[sidx];
-      tc[e] = iperm[irel[raw]];
-      tx[e] = wx[sidx];
-      ty[e] = wy[sidx];
-      tl[e] = wl[sidx];
-      th[e] = wh[sidx];
-      const int vr = (lflip && raw >= npfb) ? vrel[raw] : 0;
-      tf[e] = (uint8_t)(vr >= 2 ? vr - 1 : 0);
-    } else {
-      tc[e] = slot < npfb ? slot : 0;
-      tx[e] = 0.0;
-      ty[e] = 0.0;
-      tl[e] = 0.0;
-      th[e] = 0.0;
-      tf[e] = 0;
-    }
-  }
-  __syncthreads();
-  // scatter: 64 consecutive threads write one link's column of the slice
-  for (int p = t; p < SV_WAVE * PK_K; p += PK_T) {
-    const int kk = p / SV_WAVE, l = p % SV_WAVE, k = k0 + kk;
-    if (k >= W) break;
-    const int64_t d = o + (int64_t)k * SV_WAVE + l;
-    if (d >= nnz_max) break;
-    const int e = l * PK_LD + kk;
-    lcol[d] = tc[e];
-    lwx[d] = tx[e];
-    lwy[d] = ty[e];
-    lwl[d] = tl[e];
-    lwh[d] = th[e];
-    if (lflip) lflip[d] = tf[e];
-  }
-}
-
-template <typename T>
-__global__ void k_permute(int n, const int *perm, const T *src, T *dst) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) dst[k] = src[perm[k]];
-}
-
-// interleave the low 16 bits of a and b (Morton key)
-uint32_t morton2(uint32_t a, uint32_t b) {
-  auto spread = [](uint32_t v) {
-    v &= 0xffff;
-    v = (v | (v << 8)) & 0x00ff00ff;
-    v = (v | (v << 4)) & 0x0f0f0f0f;
-    v = (v | (v << 2)) & 0x33333333;
-    v = (v | (v << 1)) & 0x55555555;
-    return v;
-  };
-  return spread(a) | (spread(b) << 1);
-}
-
-}  // namespace
-
-
-// Per-block halos of the loop layout (see sv_loopl): host pass over the SELL
-// columns, O(nnz log K) at setup.
-static int build_halos(sv_ctx *c) {
-  sv_loopl &L = c->L;
-  const int n = c->npfb, ns = L.nslices;
-  const int nb = (n + SV_BLOCK - 1) / SV_BLOCK;
-  std::vector<int64_t> off(ns + 1);
-  std::vector<int> col(L.nnz), cnt(n);
-  SV_HIP(c, hipMemcpy(off.data(), L.off, sizeof(int64_t) * (ns + 1), hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(col.data(), L.col, sizeof(int) * L.nnz, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(cnt.data(), L.cnt, sizeof(int) * n, hipMemcpyDeviceToHost));
-  if (L.lflip) {
-    // a mirror link and a plain link to the same parent are different halo
-    // records (the mirror one carries the sign flips)
-    std::vector<uint8_t> fl(L.nnz);
-    SV_HIP(c, hipMemcpy(fl.data(), L.lflip, L.nnz, hipMemcpyDeviceToHost));
-    for (int64_t e = 0; e < L.nnz; e++) col[e] |= (int)fl[e] << SV_FLIP_SHIFT;
-  }
-  // blocks are independent: each one's halo (sorted unique link targets) and
-  // its links' block-local indices, on up to 16 host threads over
-  // contiguous block ranges; the halos are concatenated in block order after
-  std::vector<std::vector<int>> hb(nb);
-  std::vector<uint16_t> lcol(L.nnz, 0);
-  constexpr int SPB = SV_BLOCK / SV_WAVE;   // slices per block
-  // one block: its halo (the sorted unique link targets) and each link's
-  // rank in it.  Targets within a narrow range (the usual case in Morton
-  // order) are ranked with a dense marker array in one pass; a wide range
-  // (a Morton seam, or flipped mirror keys) takes a sort and binary searches.
-  // Both give the same halo and ranks.
-  auto one_block = [&](int b, std::vector<int> &h, std::vector<int> &mark) {
-    h.clear();
-    int lo = INT32_MAX, hi = INT32_MIN;
-    for (int s = b * SPB; s < std::min(ns, (b + 1) * SPB); s++)
-      for (int l = 0; l < SV_WAVE && s * SV_WAVE + l < n; l++) {
-        const int slot = s * SV_WAVE + l;
-        for (int k = 0; k < cnt[slot]; k++) {
-          const int v = col[off[s] + (int64_t)k * SV_WAVE + l];
-          h.push_back(v);
-          lo = std::min(lo, v);
-          hi = std::max(hi, v);
-        }
-      }
-    if (h.empty()) return;
-    const int64_t range = (int64_t)hi - lo + 1;
-    const bool dense = range <= 4 * (int64_t)h.size() + 4096;
-    if (dense) {
-      mark.assign((size_t)range, -1);
-      for (int v : h) mark[v - lo] = 0;
-      h.clear();
-      for (int64_t q = 0; q < range; q++)
-        if (mark[q] == 0) {
-          mark[q] = (int)h.size();
-          h.push_back(lo + (int)q);
-        }
-    } else {
-      std::sort(h.begin(), h.end());
-      h.erase(std::unique(h.begin(), h.end()), h.end());
-    }
-    if (h.size() > 65535) return;   // too large for 16-bit indices: no halo sweeps
-    for (int s = b * SPB; s < std::min(ns, (b + 1) * SPB); s++)
-      for (int l = 0; l < SV_WAVE && s * SV_WAVE + l < n; l++) {
-        const int slot = s * SV_WAVE + l;
-        for (int k = 0; k < cnt[slot]; k++) {
-          const int64_t e = off[s] + (int64_t)k * SV_WAVE + l;
-          lcol[e] = dense ? (uint16_t)mark[col[e] - lo]
-                          : (uint16_t)(std::lower_bound(h.begin(), h.end(), col[e]) - h.begin());
-        }
-      }
-  };
-  const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-  const int nt = (int)std::min<unsigned>(std::min(hw, 16u), (unsigned)std::max(nb, 1));
-  {
-    std::vector<std::thread> pool;
-    for (int t = 0; t < nt; t++)
-      pool.emplace_back([&, t] {
-        std::vector<int> mark;
-        for (int b = (int)((int64_t)nb * t / nt); b < (int)((int64_t)nb * (t + 1) / nt); b++)
-          one_block(b, hb[b], mark);
-      });
-    for (auto &th : pool) th.join();
-  }
-  std::vector<int64_t> hoff(nb + 1, 0);
-  int hmax = 0;
-  bool fits = true;
-  for (int b = 0; b < nb; b++) {
-    hmax = std::max(hmax, (int)hb[b].size());
-    if (hb[b].size() > 65535) fits = false;
-    hoff[b + 1] = hoff[b] + (int64_t)hb[b].size();
-  }
-  std::vector<int> hidx((size_t)hoff[nb]);
-  for (int b = 0; b < nb; b++) std::copy(hb[b].begin(), hb[b].end(), hidx.begin() + hoff[b]);
-  L.hmax = hmax;
-  // the LC sweep keeps 72 bytes per halo record in LDS
-  L.halo = c->halo_sweeps && fits && (size_t)hmax * 72 <= SV_HALO_LDS_MAX;
-  if (!L.halo) return 0;
-  if (sv_alloc(c, (void **)&L.hoff, sizeof(int64_t) * (nb + 1)) ||
-      sv_alloc(c, (void **)&L.hidx, sizeof(int) * (hidx.size() + 1)) ||
-      sv_alloc(c, (void **)&L.lcol, sizeof(uint16_t) * (L.nnz + 1)))
-    return SV_E_NOMEM;
-  SV_HIP(c, hipMemcpy(L.hoff, hoff.data(), sizeof(int64_t) * (nb + 1), hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(L.hidx, hidx.data(), sizeof(int) * hidx.size(), hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(L.lcol, lcol.data(), sizeof(uint16_t) * L.nnz, hipMemcpyHostToDevice));
-  return 0;
-}
-
-int sv_dev_build_loop(sv_ctx *c) {
-  const int n = c->npfb;
-  sv_loopl &L = c->L;
-  // permutation
-  std::vector<double> x(n), y(n);
-  SV_HIP(c, hipMemcpy(x.data(), c->x, sizeof(double) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(y.data(), c->y, sizeof(double) * n, hipMemcpyDeviceToHost));
-  L.hperm.resize(n);
-  for (int i = 0; i < n; i++) L.hperm[i] = i;
-  if (c->loop_order) {
-    const double sx = 65535.0 / (c->xmax - c->xmin), sy = 65535.0 / (c->ymax - c->ymin);
-    std::vector<uint32_t> key(n);
-    for (int i = 0; i < n; i++) {
-      const double fx = std::min(std::max((x[i] - c->xmin) * sx, 0.0), 65535.0);
-      const double fy = std::min(std::max((y[i] - c->ymin) * sy, 0.0), 65535.0);
-      key[i] = morton2((uint32_t)fx, (uint32_t)fy);
-    }
-    // stable LSD radix sort of the 32-bit keys, two 16-bit digits: the same
-    // permutation as a stable comparison sort
-    std::vector<int> tmp(n);
-    std::vector<int> cnt16(65537);
-    for (int shift = 0; shift < 32; shift += 16) {
-      std::fill(cnt16.begin(), cnt16.end(), 0);
-      for (int i = 0; i < n; i++) cnt16[((key[L.hperm[i]] >> shift) & 0xffff) + 1]++;
-      for (int d = 1; d <= 65536; d++) cnt16[d] += cnt16[d - 1];
-      for (int i = 0; i < n; i++) tmp[cnt16[(key[L.hperm[i]] >> shift) & 0xffff]++] = L.hperm[i];
-      L.hperm.swap(tmp);
-    }
-  }
-  std::vector<int> iperm(c->np);
-  for (int k = 0; k < n; k++) iperm[L.hperm[k]] = k;
-  for (int j = n; j < c->np; j++) iperm[j] = -1;   // ghosts are folded before lookup
-  std::vector<int> cnt(n);
-  SV_HIP(c, hipMemcpy(cnt.data(), c->cnt, sizeof(int) * n, hipMemcpyDeviceToHost));
-  const int ns = (n + SV_WAVE - 1) / SV_WAVE;
-  std::vector<int64_t> off(ns + 1);
-  off[0] = 0;
-  int wmax = 0;
-  for (int s = 0; s < ns; s++) {
-    int m = 0;
-    for (int l = 0; l < SV_WAVE && s * SV_WAVE + l < n; l++) m = std::max(m, cnt[L.hperm[s * SV_WAVE + l]]);
-    wmax = std::max(wmax, m);
-    off[s + 1] = off[s] + (int64_t)m * SV_WAVE;
-  }
-  // (re)allocate
-  void *old[] = {L.off, L.col, L.wx, L.wy, L.wl, L.wh, L.cnt, L.cnt_small, L.gsx, L.gsy,
-                 L.lsum, L.hsum, L.vol, L.s, L.perm, L.iperm, L.hoff, L.hidx, L.lcol,
-                 L.bidx, L.brec, L.lflip};
-  for (void *b : old)
-    if (b) sv_free(c, b);
-  std::vector<int> hp = std::move(L.hperm);
-  L = sv_loopl{};
-  L.nslices = ns;
-  L.nnz = off[ns];
-  L.hperm = std::move(hp);
-  const size_t E = (size_t)L.nnz + 1, D = sizeof(double), I = sizeof(int);
-  if (sv_alloc(c, (void **)&L.off, sizeof(int64_t) * (ns + 1)) ||
-      sv_alloc(c, (void **)&L.col, I * E) || sv_alloc(c, (void **)&L.wx, D * E) ||
-      sv_alloc(c, (void **)&L.wy, D * E) || sv_alloc(c, (void **)&L.wl, D * E) ||
-      sv_alloc(c, (void **)&L.wh, D * E) || sv_alloc(c, (void **)&L.cnt, I * n) ||
-      sv_alloc(c, (void **)&L.cnt_small, I * n) || sv_alloc(c, (void **)&L.gsx, D * n) ||
-      sv_alloc(c, (void **)&L.gsy, D * n) || sv_alloc(c, (void **)&L.lsum, D * n) ||
-      sv_alloc(c, (void **)&L.hsum, D * n) || sv_alloc(c, (void **)&L.vol, D * n) ||
-      sv_alloc(c, (void **)&L.s, D * n) || sv_alloc(c, (void **)&L.perm, I * n) ||
-      sv_alloc(c, (void **)&L.iperm, I * c->np))
-    return SV_E_NOMEM;
-  SV_HIP(c, hipMemcpy(L.off, off.data(), sizeof(int64_t) * (ns + 1), hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(L.perm, L.hperm.data(), I * n, hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(L.iperm, iperm.data(), I * c->np, hipMemcpyHostToDevice));
-  dim3 grid(ns, (wmax + PK_K - 1) / PK_K);
-  if (c->has_mirror && sv_alloc(c, (void **)&L.lflip, (size_t)L.nnz + 1)) return SV_E_NOMEM;
-  k_loop_pack<<<grid, PK_T, 0, c->stream>>>(n, L.off, L.perm, L.iperm, c->row_ptr, c->cnt,
-                                               c->col_raw, c->irel, c->vrel, c->wx, c->wy,
-                                               c->wl, c->wh, L.nnz, L.col, L.wx, L.wy, L.wl,
-                                               L.wh, L.lflip);
-  SV_HIP(c, hipGetLastError());
-  const int B = 256, nb = (n + B - 1) / B;
-  k_permute<int><<<nb, B, 0, c->stream>>>(n, L.perm, c->cnt, L.cnt);
-  k_permute<int><<<nb, B, 0, c->stream>>>(n, L.perm, c->cnt_small, L.cnt_small);
-  const double *src[6] = {c->gsx, c->gsy, c->lsum, c->hsum, c->vol, c->s};
-  double *dst[6] = {L.gsx, L.gsy, L.lsum, L.hsum, L.vol, L.s};
-  for (int k = 0; k < 6; k++) k_permute<double><<<nb, B, 0, c->stream>>>(n, L.perm, src[k], dst[k]);
-  SV_HIP(c, hipGetLastError());
-  SV_HIP(c, hipStreamSynchronize(c->stream));
-  if (int rc = build_halos(c)) return rc;
-  L.valid = true;
   return 0;
 }

@@ -1003,7 +1003,7 @@ int sv_get_stencil_stats(sv_ctx *c, double *stats) {
   stats[5] = 0.0;                  // halo records per node staged by the sweeps
   if (c->L.valid && c->L.halo) {
     int64_t tot = 0;
-    const int nb = (c->npfb + SV_BLOCK - 1) / SV_BLOCK;
+    const int nb = (c->npfb + c->L.hb - 1) / c->L.hb;
     SV_HIP(c, hipMemcpy(&tot, c->L.hoff + nb, sizeof(int64_t), hipMemcpyDeviceToHost));
     stats[5] = (double)tot / c->npfb;
   }

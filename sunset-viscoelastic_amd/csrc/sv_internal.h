@@ -119,6 +119,9 @@ void sv_adj_free(sv_ctx *c);
 // LDS budget of a block's staged halo records (bytes); above it the sweeps
 // gather from global memory instead
 #define SV_HALO_LDS_MAX (60 * 1024)
+// LDS bytes of a staged halo record (log-conformation form; the direct form's
+// are smaller)
+#define SV_HALO_REC 72
 struct sv_segk {
   int base;      // first node (concatenated numbering), a multiple of SV_BLOCK
   int npfb;      // real nodes
@@ -129,9 +132,9 @@ struct sv_segk {
 };
 
 // Time-loop layout: the arrays the RK sweeps read, with the real nodes in
-// "loop order" -- a Morton (Z-order) sort of the positions, so a block of 256
-// consecutive loop slots is a compact patch of the domain and the neighbour
-// records it gathers are shared across its nodes in the caches.  perm[k] is
+// "loop order" -- recursive splits of the positions (k_loop.hip), so a block
+// of 256 consecutive loop slots is a compact rectangle of the domain and the
+// neighbour records it gathers are shared across its nodes.  perm[k] is
 // the caller's node in loop slot k, iperm its inverse.  SELL-64 over loop
 // slots; columns are loop slots of the (ghost-folded) neighbours.  Per-node
 // arrays are in loop order; the drop-in operators keep the caller's order.
@@ -147,12 +150,14 @@ struct sv_loopl {
   double *s = nullptr;
   int *perm = nullptr, *iperm = nullptr;
   std::vector<int> hperm;
-  // Per-block neighbour halos: the distinct neighbour slots of the SV_BLOCK
+  // Per-block neighbour halos: the distinct neighbour slots of the hb
   // slots of block b are hidx[hoff[b] .. hoff[b+1]) (ascending); lcol[e] is
   // the position of col[e] in its block's halo.  The sweeps stage a block's
   // halo records in LDS once and read every link from there.
   bool halo = false;
+  int hb = SV_BLOCK;        // slots per halo block
   int hmax = 0;             // largest halo of a block
+  std::vector<int> hcnt;    // halo sizes
   int64_t *hoff = nullptr;  // [nblocks + 1]
   int *hidx = nullptr;
   uint16_t *lcol = nullptr; // [nnz]
