@@ -190,10 +190,10 @@ int sv_get_timing(sv_ctx *ctx, const char *what, double *ms);
  *       reports the mode of the last call, "weights_mixed_tune_<mode>" the
  *       sample times.
  *   "loop_order" (default 1, before sv_set_initial): 1 runs the time loop in
- *       Morton order of the nodes, 0 in the caller's order.
+ *       an order of compact blocks of nodes, 0 in the caller's order.
  *   "halo_sweeps" (default 1, before sv_set_initial): the RK sweeps copy each
- *       256-node block's neighbour records into LDS once and read the links
- *       from there (when the largest block halo fits 60 KB); 0 gathers every
+ *       node block's neighbour records into LDS once and read the links
+ *       from there (when the largest block halo fits); 0 gathers every
  *       link from global memory.
  *   "ensemble_groups" (ensemble contexts): with members of several LABFM
  *       orders, the stage and filter sweeps run either as one launch over all

@@ -626,15 +626,13 @@ static int build_transpose(sv_ctx *c, sv_adj *A) {
   const int n = c->npfb, ns = LP.nslices;
   std::vector<int> cnt(n), cs(n), scol(LP.nnz);
   std::vector<int64_t> off(ns);
-  std::vector<double> wx(LP.nnz), wy(LP.nnz), wl(LP.nnz), wh(LP.nnz);
+  std::vector<double> w3(3 * LP.nnz), wh(LP.nnz);
   SV_HIP(c, hipMemcpy(cnt.data(), LP.cnt, sizeof(int) * n, hipMemcpyDeviceToHost));
   SV_HIP(c, hipMemcpy(cs.data(), LP.cnt_small, sizeof(int) * n, hipMemcpyDeviceToHost));
   SV_HIP(c, hipMemcpy(off.data(), LP.off, sizeof(int64_t) * ns, hipMemcpyDeviceToHost));
   const size_t L = sizeof(double) * LP.nnz;
   SV_HIP(c, hipMemcpy(scol.data(), LP.col, sizeof(int) * LP.nnz, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(wx.data(), LP.wx, L, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(wy.data(), LP.wy, L, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(wl.data(), LP.wl, L, hipMemcpyDeviceToHost));
+  SV_HIP(c, hipMemcpy(w3.data(), LP.w3, 3 * L, hipMemcpyDeviceToHost));
   SV_HIP(c, hipMemcpy(wh.data(), LP.wh, L, hipMemcpyDeviceToHost));
   std::vector<int> tc(n, 0);
   for (int i = 0; i < n; i++)
@@ -667,10 +665,10 @@ static int build_transpose(sv_ctx *c, sv_adj *A) {
       const int64_t d = toff[j >> 6] + (int64_t)(fill[j]++) * SV_WAVE + (j & 63);
       tcol[d] = i;
       const bool small = k < cs[i];
-      tx[d] = small ? wx[e] : 0.0;
-      ty[d] = small ? wy[e] : 0.0;
-      tl[d] = small ? wl[e] : 0.0;
-      th[d] = wh[e];
+      tx[d] = small ? w3[sv_w3(e, 0)] : 0.0;
+      ty[d] = small ? w3[sv_w3(e, 1)] : 0.0;
+      tl[d] = small ? w3[sv_w3(e, 2)] : 0.0;
+      th[d] = wh[sv_pair(e)];
     }
   if (sv_alloc(c, (void **)&A->toff, sizeof(int64_t) * (nsl + 1)) ||
       sv_alloc(c, (void **)&A->tcnt, sizeof(int) * n) ||

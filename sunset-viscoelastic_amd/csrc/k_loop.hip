@@ -38,7 +38,7 @@ __global__ __launch_bounds__(PK_T) void k_loop_pack(
     int npfb, const int64_t *off, const int *perm, const int *iperm, const int64_t *row_ptr,
     const int *cnt, const int *col_raw, const int *irel, const int *vrel, const double *wx,
     const double *wy, const double *wl, const double *wh, int64_t nnz_max, int *lcol,
-    double *lwx, double *lwy, double *lwl, double *lwh, uint8_t *lflip) {
+    double *lw3, double *lwh, uint8_t *lflip) {
   __shared__ double tx[SV_WAVE * PK_LD], ty[SV_WAVE * PK_LD], tl[SV_WAVE * PK_LD],
       th[SV_WAVE * PK_LD];
   __shared__ int tc[SV_WAVE * PK_LD];
@@ -92,10 +92,10 @@ __global__ __launch_bounds__(PK_T) void k_loop_pack(
     if (d >= nnz_max) break;
     const int e = l * PK_LD + kk;
     lcol[d] = tc[e];
-    lwx[d] = tx[e];
-    lwy[d] = ty[e];
-    lwl[d] = tl[e];
-    lwh[d] = th[e];
+    lw3[sv_w3(d, 0)] = tx[e];
+    lw3[sv_w3(d, 1)] = ty[e];
+    lw3[sv_w3(d, 2)] = tl[e];
+    lwh[sv_pair(d)] = th[e];
     if (lflip) lflip[d] = tf[e];
   }
 }
@@ -176,13 +176,27 @@ __global__ void k_kd_split(int nseg, const int *start, const int *left, const in
 }
 
 // ---- SELL offsets -------------------------------------------------------------
-// entries of slice s: 64 times its longest list
+// entries of slice s: 64 times its longest list, made even
 __global__ void k_slice_width(int n, const int *cnt, int64_t *w) {
   const int s = blockIdx.x, slot = s * SV_WAVE + (int)threadIdx.x;
   int m = slot < n ? cnt[slot] : 0;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o));
-  if (threadIdx.x == 0) w[s] = (int64_t)m * SV_WAVE;
+  if (threadIdx.x == 0) w[s] = (int64_t)((m + 1) & ~1) * SV_WAVE;
+}
+
+// fewest and most links of the slice's nodes, small and full lists
+__global__ void k_slice_range(const int *cnt_small, const int *cnt, int4 *out) {
+  const int s = blockIdx.x, slot = s * SV_WAVE + (int)threadIdx.x;
+  int4 r{cnt_small[slot], cnt_small[slot], cnt[slot], cnt[slot]};
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    r.x = min(r.x, __shfl_xor(r.x, o));
+    r.y = max(r.y, __shfl_xor(r.y, o));
+    r.z = min(r.z, __shfl_xor(r.z, o));
+    r.w = max(r.w, __shfl_xor(r.w, o));
+  }
+  if (threadIdx.x == 0) out[s] = r;
 }
 
 // ---- halos ----------------------------------------------------------------------
@@ -271,12 +285,20 @@ __global__ __launch_bounds__(HTHREADS) void k_halo(int hb, int nslot, const int6
     if (s * SV_WAVE >= nslot) break;
     const int64_t o = off[s];
     const int K = slot < nslot ? cnt[slot] : 0;
-    for (int k = wave; k < K; k += HTHREADS / SV_WAVE) {
+    int W = K;   // the slice's padded length: padding entries get rank 0
+#pragma unroll
+    for (int o2 = 32; o2 >= 1; o2 >>= 1) W = max(W, __shfl_xor(W, o2));
+    W = (W + 1) & ~1;
+    for (int k = wave; k < W; k += HTHREADS / SV_WAVE) {
       const int64_t e = o + (int64_t)k * SV_WAVE + lane;
+      if (k >= K) {
+        lcol[sv_pair(e)] = 0;
+        continue;
+      }
       const int key = flip ? col[e] | (int)flip[e] << SV_FLIP_SHIFT : col[e];
       int h = halo_hash(key);
       while (tab[h] != key) h = (h + 1) & (HT - 1);
-      lcol[e] = rank[h];
+      lcol[sv_pair(e)] = rank[h];
     }
   }
 }
@@ -314,8 +336,15 @@ int kd_left(int size) {
   return SV_BLOCK * (((slices + SPB - 1) / SPB) / 2);
 }
 
-// perm[k] = node in loop slot k
-int kd_order(sv_ctx *c, int *perm) {
+// key of slot k: its block, then its node's links, most first
+__global__ void k_len_key(int n, int hb, const int *ids, const int *cnt, uint64_t *key) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) key[k] = (uint64_t)(k / hb) << 16 | (uint64_t)(65535 - min(cnt[ids[k]], 65535));
+}
+
+// perm[k] = node in loop slot k; by_len: the nodes of each block sorted by
+// their number of links
+int kd_order(sv_ctx *c, int *perm, int by_len) {
   const int n = c->npfb, B = 256;
   // the tree's shape depends on n alone: starts, left sizes and first child
   // of every level, concatenated
@@ -344,7 +373,6 @@ int kd_order(sv_ctx *c, int *perm) {
   const int levels = (int)first.size() - 2;   // the last level splits nothing
   k_iota<<<(n + B - 1) / B, B, 0, c->stream>>>(n, perm);
   SV_HIP(c, hipGetLastError());
-  if (levels == 0) return 0;
   DevTmp<int> plan, alt;
   DevTmp<uint64_t> key;
   DevTmp<KdBox> boxes;
@@ -383,6 +411,14 @@ int kd_order(sv_ctx *c, int *perm) {
                                                         vb.Current(), out);
     SV_HIP(c, hipGetLastError());
   }
+  if (by_len) {
+    int bits = 16;
+    while ((n - 1) / by_len >> (bits - 16)) bits++;
+    k_len_key<<<(n + B - 1) / B, B, 0, c->stream>>>(n, by_len, vb.Current(), c->cnt, kb.Current());
+    SV_HIP(c, hipGetLastError());
+    SV_HIP(c, hipcub::DeviceRadixSort::SortPairs((void *)tmp, tb, kb, vb, n, 0, bits,
+                                                 c->stream));
+  }
   if (vb.Current() != perm)
     SV_HIP(c, hipMemcpyAsync(perm, vb.Current(), sizeof(int) * n, hipMemcpyDeviceToDevice,
                              c->stream));
@@ -390,26 +426,26 @@ int kd_order(sv_ctx *c, int *perm) {
   return 0;
 }
 
-}  // namespace
-
-// Per-block halos of the layout in c->L (a context's own, or an ensemble's
-// concatenated one): hb slots per block, nslot slots in all.  L.halo stays
-// false when a block's halo exceeds the LDS budget of the sweeps.
-static int build_halos(sv_ctx *c, int hb, int nslot) {
+// Halos of hb slots per block, nslot slots in all.  L.halo stays false when a
+// block's halo exceeds the LDS budget of the sweeps.
+int build_halos(sv_ctx *c, int hb, int nslot) {
   sv_loopl &L = c->L;
-  const int nb = (nslot + hb - 1) / hb;
+  // whole node blocks, as the sweeps' grids cover them: the halo blocks past
+  // the last slot are empty
+  const int nb = (nslot + SV_BLOCK - 1) / SV_BLOCK * (SV_BLOCK / hb);
   DevTmp<int> hcnt, list;
   SV_HIP(c, hcnt.alloc((size_t)nb + 1));
   SV_HIP(c, list.alloc((size_t)nb * HC));
-  uint16_t *lcol = nullptr;
-  int64_t *hoff = nullptr;
-  if (sv_alloc(c, (void **)&lcol, sizeof(uint16_t) * (L.nnz + 1)) ||
-      sv_alloc(c, (void **)&hoff, sizeof(int64_t) * ((size_t)nb + 1)))
-    return SV_E_NOMEM;
-  L.lcol = lcol;
-  L.hoff = hoff;
+  if (!L.lcol) {
+    const int nsl = (nslot + SV_BLOCK - 1) / SV_BLOCK * (SV_BLOCK / SV_WAVE);
+    if (sv_alloc(c, (void **)&L.lcol, sizeof(uint16_t) * (L.nnz + 1)) ||
+        sv_alloc(c, (void **)&L.krange, sizeof(int4) * (size_t)nsl))
+      return SV_E_NOMEM;
+    k_slice_range<<<nsl, SV_WAVE, 0, c->stream>>>(L.cnt_small, L.cnt, L.krange);
+    SV_HIP(c, hipGetLastError());
+  }
   k_halo<<<nb, HTHREADS, 0, c->stream>>>(hb, nslot, L.off, L.cnt, L.col, L.lflip, hcnt, list,
-                                         lcol);
+                                         L.lcol);
   SV_HIP(c, hipGetLastError());
   L.hcnt.resize(nb);
   SV_HIP(c, hipMemcpyAsync(L.hcnt.data(), hcnt.p, sizeof(int) * nb, hipMemcpyDeviceToHost,
@@ -421,43 +457,81 @@ static int build_halos(sv_ctx *c, int hb, int nslot) {
     L.hmax = std::max(L.hmax, v);
     tot += v;
   }
-  // the LC sweep keeps SV_HALO_REC bytes per halo record in LDS
-  L.halo = (size_t)L.hmax * SV_HALO_REC <= SV_HALO_LDS_MAX;
+  L.halo = L.hmax <= SV_HALO_MAX && (size_t)L.hmax * SV_HALO_REC <= SV_HALO_LDS_MAX;
   if (!L.halo) return 0;
   L.hb = hb;
   SV_HIP(c, hipMemsetAsync(hcnt.p + nb, 0, sizeof(int), c->stream));
   hipcub::TransformInputIterator<int64_t, ToI64, const int *> in(hcnt.p, ToI64());
-  if (int rc = scan_i64(c, in, hoff, nb + 1)) return rc;
-  if (sv_alloc(c, (void **)&L.hidx, sizeof(int) * ((size_t)tot + 1))) return SV_E_NOMEM;
-  k_halo_compact<<<nb, HTHREADS, 0, c->stream>>>(hoff, list, L.hidx);
+  if (sv_alloc(c, (void **)&L.hoff, sizeof(int64_t) * ((size_t)nb + 1)) ||
+      sv_alloc(c, (void **)&L.hidx, sizeof(int) * ((size_t)tot + 1)))
+    return SV_E_NOMEM;
+  if (int rc = scan_i64(c, in, L.hoff, nb + 1)) return rc;
+  k_halo_compact<<<nb, HTHREADS, 0, c->stream>>>(L.hoff, list, L.hidx);
   SV_HIP(c, hipGetLastError());
   SV_HIP(c, hipStreamSynchronize(c->stream));
   return 0;
 }
 
-int sv_dev_build_loop(sv_ctx *c) {
+}  // namespace
+
+// Workgroup size of the sweeps and whether their weights stream past the
+// caches, from the node count and the links.  One RK3 step, us, for workgroups
+// of 64 / 128 with cached loads, 128 / 256 with non-temporal ones:
+//   128^2 order 6 LC   73 /  79,   91 /  128   (few waves: one per workgroup)
+//   200^2 order 6 LC   99 / 103,  115 /  142
+//   260^2 order 6 LC  140 / 140,  150 /  171
+//   301x283 order 8 DI 189 / 180, 192 /  206
+//   360^2 order 6 LC  283 / 237,  233 /  232
+//   512^2 order 6 LC  588 / 552,  457 /  498   (1024 blocks of 256 leave CUs idle)
+//   700^2 order 6 LC    - /1014,  851 /  857
+//   1024^2 order 6 LC   - /2082, 1916 / 1882   (fewer halo records per node)
+// Cached loads win while a stage's weights and link targets (26 bytes a link)
+// stay in the 256 MB Infinity Cache between stages.
+struct Blocks {
+  int hb;
+  bool nt;
+};
+static Blocks choose_blocks(int nslot, int64_t links) {
+  if (nslot <= 32768) return {64, false};
+  if (26 * links <= (int64_t)256 << 20) return {128, false};
+  return {nslot <= 500000 ? 128 : 256, true};
+}
+
+int sv_dev_build_halos(sv_ctx *c, int nslot) {
+  const Blocks b = choose_blocks(nslot, c->L.nnz);
+  c->L.nt = b.nt;
+  if (int rc = build_halos(c, b.hb, nslot)) return rc;
+  return c->L.halo || b.hb == SV_WAVE ? 0 : build_halos(c, SV_WAVE, nslot);
+}
+
+static int build_layout(sv_ctx *c, int hb) {
   const int n = c->npfb;
   sv_loopl &L = c->L;
   // (re)allocate
-  void *old[] = {L.off, L.col, L.wx, L.wy, L.wl, L.wh, L.cnt, L.cnt_small, L.gsx, L.gsy,
+  void *old[] = {L.off, L.col, L.w3, L.wh, L.cnt, L.cnt_small, L.gsx, L.gsy,
                  L.lsum, L.hsum, L.vol, L.s, L.perm, L.iperm, L.hoff, L.hidx, L.lcol,
-                 L.bidx, L.brec, L.lflip};
+                 L.bidx, L.brec, L.lflip, L.krange};
   for (void *b : old)
     if (b) sv_free(c, b);
   L = sv_loopl{};
   const int ns = (n + SV_WAVE - 1) / SV_WAVE;
   L.nslices = ns;
   const size_t D = sizeof(double), I = sizeof(int);
-  if (sv_alloc(c, (void **)&L.off, sizeof(int64_t) * (ns + 1)) ||
-      sv_alloc(c, (void **)&L.cnt, I * n) || sv_alloc(c, (void **)&L.cnt_small, I * n) ||
+  // whole blocks of counts and slice offsets: no links past the last node
+  const int nslot = (n + SV_BLOCK - 1) / SV_BLOCK * SV_BLOCK;
+  if (sv_alloc(c, (void **)&L.off, sizeof(int64_t) * (nslot / SV_WAVE + 1)) ||
+      sv_alloc(c, (void **)&L.cnt, I * nslot) || sv_alloc(c, (void **)&L.cnt_small, I * nslot) ||
       sv_alloc(c, (void **)&L.gsx, D * n) || sv_alloc(c, (void **)&L.gsy, D * n) ||
       sv_alloc(c, (void **)&L.lsum, D * n) || sv_alloc(c, (void **)&L.hsum, D * n) ||
       sv_alloc(c, (void **)&L.vol, D * n) || sv_alloc(c, (void **)&L.s, D * n) ||
       sv_alloc(c, (void **)&L.perm, I * n) || sv_alloc(c, (void **)&L.iperm, I * c->np))
     return SV_E_NOMEM;
+  SV_HIP(c, hipMemsetAsync(L.off, 0, sizeof(int64_t) * (nslot / SV_WAVE + 1), c->stream));
+  SV_HIP(c, hipMemsetAsync(L.cnt, 0, I * nslot, c->stream));
+  SV_HIP(c, hipMemsetAsync(L.cnt_small, 0, I * nslot, c->stream));
   const int B = 256, nb = (n + B - 1) / B;
   if (c->loop_order) {
-    if (int rc = kd_order(c, L.perm)) return rc;
+    if (int rc = kd_order(c, L.perm, hb == SV_WAVE ? 0 : hb)) return rc;
   } else {
     k_iota<<<nb, B, 0, c->stream>>>(n, L.perm);
     SV_HIP(c, hipGetLastError());
@@ -481,22 +555,31 @@ int sv_dev_build_loop(sv_ctx *c) {
   }
   SV_HIP(c, hipMemcpy(&L.nnz, L.off + ns, sizeof(int64_t), hipMemcpyDeviceToHost));
   const size_t E = (size_t)L.nnz + 1;
-  if (sv_alloc(c, (void **)&L.col, I * E) || sv_alloc(c, (void **)&L.wx, D * E) ||
-      sv_alloc(c, (void **)&L.wy, D * E) || sv_alloc(c, (void **)&L.wl, D * E) ||
+  if (sv_alloc(c, (void **)&L.col, I * E) || sv_alloc(c, (void **)&L.w3, 3 * D * E) ||
       sv_alloc(c, (void **)&L.wh, D * E))
     return SV_E_NOMEM;
   if (c->has_mirror && sv_alloc(c, (void **)&L.lflip, E)) return SV_E_NOMEM;
   if (c->maxK > 0) {
-    dim3 grid(ns, (c->maxK + PK_K - 1) / PK_K);
+    dim3 grid(ns, (c->maxK + 1 + PK_K - 1) / PK_K);
     k_loop_pack<<<grid, PK_T, 0, c->stream>>>(n, L.off, L.perm, L.iperm, c->row_ptr, c->cnt,
                                               c->col_raw, c->irel, c->vrel, c->wx, c->wy, c->wl,
-                                              c->wh, L.nnz, L.col, L.wx, L.wy, L.wl, L.wh,
-                                              L.lflip);
+                                              c->wh, L.nnz, L.col, L.w3, L.wh, L.lflip);
     SV_HIP(c, hipGetLastError());
   }
   if (c->halo_sweeps)
-    if (int rc = build_halos(c, SV_BLOCK, n)) return rc;
+    if (int rc = build_halos(c, hb, n)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));
   L.valid = true;
+  return 0;
+}
+
+int sv_dev_build_loop(sv_ctx *c) {
+  const Blocks b = choose_blocks(c->npfb, c->nnz);
+  if (int rc = build_layout(c, b.hb)) return rc;
+  if (!c->L.halo && c->halo_sweeps && b.hb != SV_WAVE) {
+    c->L.valid = false;   // halos too large: the smallest blocks
+    if (int rc = build_layout(c, SV_WAVE)) return rc;
+  }
+  c->L.nt = b.nt && c->L.hb != SV_WAVE;
   return 0;
 }

@@ -24,12 +24,13 @@
 // Memory layout of the state (records, see sv_internal.h): what a neighbour
 // gather needs of node j sits in one packed 80-byte record (LC) or 48-byte
 // record (DI), so a link costs at most two cache lines instead of one line
-// per field, and records of Morton-adjacent nodes share lines.
+// per field, and records of adjacent nodes share lines.
 #include "sv_internal.h"
 
 namespace {
 
 constexpr int BS = SV_BLOCK;   // threads per block of the node kernels
+constexpr int SPB = BS / SV_WAVE;   // slices (and partial results) per block
 
 // Gather-loop tuning (compile time): links processed per iteration, and
 // whether the streamed stencil arrays (columns, weights; read once per sweep)
@@ -41,11 +42,17 @@ constexpr int BS = SV_BLOCK;   // threads per block of the node kernels
 #ifndef SV_STREAM_NT
 #define SV_STREAM_NT 1
 #endif
-// links per batch in the halo-staged sweeps (global streams prefetched one
-// batch ahead)
-#ifndef SV_HALO_UNROLL
-#define SV_HALO_UNROLL 2
-#endif
+// Pairs of links per batch in the halo-staged sweeps (the global streams are
+// prefetched one batch ahead), by threads per workgroup: a small node set has
+// one wave per SIMD at most and needs many requests per wave (128^2 order 6,
+// stage: 1 pair 24 us, 2 15.6, 3 14.2); a large one has twelve waves per CU and
+// is slower with more (1024^2: 1 pair 421 us, 2 436).
+template <int NB>
+struct HaloU {
+  static constexpr int U = NB == 64 ? 3 : NB == 128 ? 2 : 1;   // stage sweeps
+  static constexpr int UF = NB == 64 ? 4 : 2;                  // the filter
+};
+typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 template <typename T>
 __device__ __forceinline__ T ld_stream(const T *p) {
@@ -63,15 +70,44 @@ struct NodeRef {
   bool act;
 };
 
+// bid: workgroup of NB consecutive slots (NB divides SV_BLOCK)
+template <int NB = BS>
 __device__ __forceinline__ NodeRef node_ref(const int *blk_seg, const sv_segk *seg, int bid) {
   NodeRef r;
-  r.sg = blk_seg[bid];
+  r.sg = blk_seg[bid / (BS / NB)];
   const sv_segk &S = seg[r.sg];
-  const int li = (bid - S.blk0) * BS + (int)threadIdx.x;
-  r.act = li < S.npfb;
-  r.i = S.base + li;
+  r.i = bid * NB + (int)threadIdx.x;
+  r.act = r.i - S.base < S.npfb;
   r.ii = r.act ? r.i : S.base;
   return r;
+}
+
+// Logical workgroup of NB slots: the XCD-aware index, through a launch group's
+// block list (256-slot blocks) when the launch covers a subset
+template <int NB>
+__device__ __forceinline__ int logical_wg(const int *blist) {
+  constexpr int SUB = BS / NB;
+  const int b = sv_xcd_block();
+  return blist ? blist[b / SUB] * SUB + b % SUB : b;
+}
+
+// Reductions over a wavefront in a fixed order (every lane ends with the
+// result).  The partial results of the node kernels are per 64-slot slice, so
+// they do not depend on the workgroup size a sweep runs with.
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+  return v;
+}
+__device__ __forceinline__ double wave_min(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+  return v;
 }
 
 // ---- conformation algebra (conf_transforms.F90) -------------------------
@@ -194,7 +230,7 @@ __device__ __forceinline__ void store_g(double *G, int i, const Rec9 &r) {
   p[2] = double2{r.cxy, r.cyy};
   if (FORM == SV_FORM_LC) {
     p[3] = double2{r.pxx, r.pxy};
-    G[(size_t)i * S + SV_G_PYY] = r.pyy;
+    p[4] = double2{r.pyy, 0.0};   // the pad too: whole lines reach memory
   }
 }
 
@@ -218,7 +254,7 @@ struct StageArgs {
   const int64_t *off;
   const int *kcnt;
   const int *col;
-  const double *wx, *wy, *wl;
+  const double *w3;
   const double *gsx, *gsy, *lsum;
   const double *G;      // gathered records (stage input)
   const double *reg_in; // register 1 input (stage 1: the state)
@@ -229,17 +265,17 @@ struct StageArgs {
   double *rhs_out;      // STAGE 0: six arrays of npfb
   const double *fx;
   const sv_ctrl *ctrl;  // [nseg]
-  double *partial;      // stage 4: per-block max error
+  double *partial;      // stage 4: max error per slice
   int rk1;              // STAGE 0: reference stage counter is 1
   // DI only, nullable: the stage's own gather record [ntot][SV_US] and its
   // derivative values [ntot][16] (rx ry ux uy lu vx vy lv, cxx_x cxx_y, cxy_x
   // cxy_y, cyy_x cyy_y, 0 0), the tape the adjoint sweep reads
   double *tapeG, *tapeD;
+  const int4 *krange;   // links per slice (sv_loopl)
   // per-block halos (k_stage_h)
   const int64_t *hoff;
   const int *hidx;
   const uint16_t *lcol;
-  int hcap;             // records the dynamic LDS holds
   // boundary nodes (nullable): per loop slot the record index or -1, records
   const int *bidx;
   const double *brec;
@@ -567,7 +603,6 @@ __device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef 
 // STAGE 1..4: RK stages; STAGE 0: write the right-hand side into rhs_out.
 template <int FORM, int STAGE, bool MDIFF, bool BND>
 __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
-  __shared__ double red[BS / SV_WAVE];
   const int bid = sv_logical_block(a.blist);
   const NodeRef nr = node_ref(a.blk_seg, a.seg, bid);
   const int ii = nr.ii;
@@ -611,7 +646,8 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
       if (k + u < K) {
         const int64_t e = b + (int64_t)(k + u) * SV_WAVE;
         r[u] = load_g<FORM>(a.G, jn[u]);
-        wxk[u] = ld_stream(a.wx + e); wyk[u] = ld_stream(a.wy + e); wlk[u] = ld_stream(a.wl + e);
+        wxk[u] = ld_stream(a.w3 + sv_w3(e, 0)); wyk[u] = ld_stream(a.w3 + sv_w3(e, 1));
+        wlk[u] = ld_stream(a.w3 + sv_w3(e, 2));
       }
     }
 #pragma unroll
@@ -629,137 +665,245 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
     emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S);
   }
   if (STAGE == 4) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) emax_loc = fmax(emax_loc, __shfl_xor(emax_loc, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = emax_loc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double m = red[0];
-      for (int w = 1; w < BS / SV_WAVE; w++) m = fmax(m, red[w]);
-      a.partial[bid] = m;
-    }
+    emax_loc = wave_max(emax_loc);
+    if ((threadIdx.x & 63) == 0) a.partial[nr.i >> 6] = emax_loc;
   }
 }
 
 // ---- halo-staged sweeps ---------------------------------------------------
-// A block first copies the gather records of its halo (the distinct neighbours
-// of its 256 nodes, ~2.6 per node on a Morton-ordered lattice) into LDS, then
-// every link reads its record from LDS by a 16-bit block-local index.  The
-// L1 then serves only the streamed arrays (indices, weights) and the halo copy,
-// instead of one scattered record per link.
-// LDS record layout: 8 doubles (ro u v cxx cxy cyy pxx pxy) + pyy in a
-// separate array for LC (72 bytes per record); 6 doubles for DI.
+// A workgroup of NB threads (one per slot of its halo block) first copies the
+// gather records of its halo (the distinct neighbours of its nodes: 2.3 per
+// node at 256 slots, 3.0 at 128, 4.0 at 64 on an order-6 lattice) into LDS,
+// then every link reads its record from LDS by a 16-bit block-local index.
+// What bounds it, by size (LC order 6, one RK stage with its launch):
+//   1M nodes    HBM: 2.47 GB in 421-439 us, 5.7 TB/s (a plain read of that
+//               size reaches 6.95 TB/s non-temporally, a copy 6.2)
+//   68k nodes   31 us (40 with 256-slot workgroups and one request pair in
+//               flight): one or two waves per SIMD, memory latency and the
+//               random LDS reads (50 clocks a link of a wave for 72 bytes a
+//               lane, 36 without bank conflicts)
+//   16k nodes   14 us (34): the chain launch -> layout -> keys -> records ->
+//               LDS -> links -> pointwise part of one wave per CU
+// LDS records are the gather records as they are: 10 doubles (80 B, the last
+// one a pad) for LC, 6 for DI (48 B), read 16 bytes at a time.  Both strides
+// are odd multiples of 16 bytes, so the records' starts spread over all LDS
+// banks (64-byte records all start on one of four bank groups).
 template <int FORM>
 struct HaloL {
-  static constexpr int RS = FORM == SV_FORM_LC ? 8 : 6;   // doubles in the main record
-  static constexpr int BYTES = FORM == SV_FORM_LC ? 72 : 48;
+  static constexpr int RS = FORM == SV_FORM_LC ? SV_GS_LC : SV_GS_DI;
+  static constexpr int BYTES = 8 * RS;
+};
+static_assert(HaloL<SV_FORM_LC>::BYTES == SV_HALO_REC, "the halo budget counts LC records");
+
+// Records a thread stages at once: a usual halo (~600 records per 256 slots,
+// ~270 per 64) in one round of requests, since a round costs two dependent
+// trips to memory (key, record).
+template <int NB>
+struct HaloC {
+  static constexpr int C = NB == SV_WAVE ? 5 : NB == 128 ? 4 : 3;
 };
 
-template <int FORM>
-__device__ __forceinline__ void halo_stage(const double *G, const int *hidx, int64_t h0, int nh,
-                                           double *hl, double *hz) {
-  constexpr int RS = HaloL<FORM>::RS;
-  for (int h = threadIdx.x; h < nh; h += BS) {
-    const int key = hidx[h0 + h];
-    Rec9 r = load_g<FORM>(G, key & SV_FLIP_MASK);
-    const int fl = key >> SV_FLIP_SHIFT;
-    if (fl) {   // mirror ghost (reapply_mirror_bcs, mirror_boundaries.F90:285-340)
-      if (fl != 2) r.u = -r.u;
-      if (fl != 1) r.v = -r.v;
-      if (fl != 3) { r.cxy = -r.cxy; r.pxy = -r.pxy; }
-    }
-    double2 *d = reinterpret_cast<double2 *>(hl + (size_t)h * RS);
-    d[0] = double2{r.ro, r.u};
-    d[1] = double2{r.v, r.cxx};
-    d[2] = double2{r.cxy, r.cyy};
-    if (FORM == SV_FORM_LC) {
-      d[3] = double2{r.pxx, r.pxy};
-      hz[h] = r.pyy;
-    }
+// The halo keys of this thread's records h, h + NB, ... of a round; past the
+// end the last key (a valid record, not stored)
+template <int NB>
+struct HaloKeys {
+  int key[HaloC<NB>::C];
+  __device__ __forceinline__ void get(const int *hx, int h, int nh) {
+#pragma unroll
+    for (int c = 0; c < HaloC<NB>::C; c++) key[c] = hx[min(h + c * NB, nh - 1)];
+  }
+};
+
+// The block's halo to LDS: load(key) reads a record, put(h, key, record)
+// stores it as record h.  keys holds the first round's keys.
+template <int NB, class Load, class Put>
+__device__ __forceinline__ void halo_stage(const int *hx, int nh, HaloKeys<NB> &keys, Load load,
+                                           Put put) {
+  constexpr int C = HaloC<NB>::C;
+  auto round = [&](int h) {
+    decltype(load(0)) r[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) r[c] = load(keys.key[c] & SV_FLIP_MASK);
+#pragma unroll
+    for (int c = 0; c < C; c++)
+      if (h + c * NB < nh) put(h + c * NB, keys.key[c] >> SV_FLIP_SHIFT, r[c]);
+  };
+  // the first round apart: its requests wait for the keys only, not for the
+  // links requested after them
+  if (nh > 0) round(threadIdx.x);
+  for (int h = threadIdx.x + C * NB; h < nh; h += C * NB) {
+    keys.get(hx, h, nh);
+    round(h);
   }
 }
 
 template <int FORM>
-__device__ __forceinline__ Rec9 halo_rec(const double *hl, const double *hz, int h) {
-  constexpr int RS = HaloL<FORM>::RS;
-  const double2 *d = reinterpret_cast<const double2 *>(hl + (size_t)h * RS);
-  Rec9 r;
-  const double2 a = d[0], b = d[1], c = d[2];
-  r.ro = a.x; r.u = a.y; r.v = b.x; r.cxx = b.y; r.cxy = c.x; r.cyy = c.y;
-  if (FORM == SV_FORM_LC) {
-    const double2 e = d[3];
-    r.pxx = e.x; r.pxy = e.y; r.pyy = hz[h];
-  } else {
-    r.pxx = r.pxy = r.pyy = 0.0;
-  }
-  return r;
+__device__ __forceinline__ Rec9 halo_rec(const double *hl, int h) {
+  return load_g<FORM>(hl, h);
 }
 
-template <int FORM, int STAGE, bool MDIFF, bool BND>
-__global__ __launch_bounds__(BS) void k_stage_h(StageArgs a) {
+// One streamed array of a wavefront's slice (W groups of 64 values of 4 or 16
+// bytes per pair of links), read through a buffer descriptor of exactly the
+// slice's pairs: a batch costs one address addition (the pairs within it are
+// immediate offsets), and entries past them read as 0 by the hardware's range
+// check, which covers the vector and immediate offsets used here (it leaves
+// out the scalar one, kept 0), so the requests need no guards.
+template <typename T, int W, bool NT>
+struct Stream {
+  __amdgpu_buffer_rsrc_t r;
+  // n: links of the slice's longest list
+  __device__ __forceinline__ Stream(const void *base, int n)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0,
+                                            (n + 1) / 2 * W * SV_WAVE * (int)sizeof(T),
+                                            0x00020000)) {}
+  // group c of the u-th pair from position p (entry_at)
+  __device__ __forceinline__ T at(int p, int u, int c) const {
+    const int vo = p * W * (int)sizeof(T) + (int)(threadIdx.x & (SV_WAVE - 1)) * (int)sizeof(T) +
+                   (u * W + c) * SV_WAVE * (int)sizeof(T);
+    constexpr int aux = NT ? 2 : 0;   // nt
+    if constexpr (sizeof(T) == 16)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, vo, 0, aux));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, vo, 0, aux));
+  }
+};
+
+// Position of link pair k / 2 in its slice (64 per pair), kept opaque so that
+// the pairs after it stay immediate offsets (the loop's strength reduction
+// would otherwise carry one address per pair)
+__device__ __forceinline__ int entry_at(int k) {
+  int p = k / 2 * SV_WAVE;
+  asm volatile("" : "+v"(p));
+  return p;
+}
+
+// The links of one wavefront's slice, walked in batches of U pairs with the
+// next batch's global streams in flight while a batch is consumed (two register
+// sets, no copies between them), and each link's LDS record requested before
+// the link before it is summed.  Batches that reach past the shortest list of
+// the slice send the requests of lanes past their own list out of range (no
+// memory traffic for the padding; they read record 0) and guard the sums.
+//   load(set, u, p)  requests the u-th pair from position p into entry u
+//   fetch(set, l)    the LDS record of link l of the set's 2U
+//   link(r, set, l)  adds it, with its record r
+constexpr int OUT_OF_RANGE = 1 << 22;   // past every list, in pairs times 64
+template <int U, class Rec, class Load, class Fetch, class Link>
+__device__ __forceinline__ void walk_links(int K, int KF, int KM, Load load, Fetch fetch,
+                                           Link link) {
+  constexpr int V = 2 * U;   // links of a batch
+  auto fill = [&](int s, int k0) {
+    const int p = entry_at(k0);
+#pragma unroll
+    for (int u = 0; u < U; u++) load(s, u, p);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto fill_guarded = [&](int s, int k0) {
+    const int p = entry_at(k0);
+#pragma unroll
+    for (int u = 0; u < U; u++) load(s, u, k0 + 2 * u < K ? p : OUT_OF_RANGE);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int k = 0;
+  Rec r = fetch(0, 0);
+  for (; k + 3 * V <= KF; k += 2 * V) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      fill(1 - s, k + (1 + s) * V);
+#pragma unroll
+      for (int l = 0; l < V; l++) {
+        const Rec n = l + 1 < V ? fetch(s, l + 1) : fetch(1 - s, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        link(r, s, l);
+        r = n;
+      }
+    }
+  }
+  for (; k < KM; k += 2 * V) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      fill_guarded(1 - s, k + (1 + s) * V);
+#pragma unroll
+      for (int l = 0; l < V; l++) {
+        const Rec n = l + 1 < V ? fetch(s, l + 1) : fetch(1 - s, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (k + s * V + l < K) link(r, s, l);
+        r = n;
+      }
+    }
+  }
+}
+
+template <int FORM, int STAGE, bool MDIFF, bool BND, int NB, bool NT>
+__global__ __launch_bounds__(NB) void k_stage_h(StageArgs a) {
   extern __shared__ double hl[];
-  __shared__ double red[BS / SV_WAVE];
-  double *hz = hl + (size_t)a.hcap * HaloL<FORM>::RS;
-  const int bid = sv_logical_block(a.blist);
-  const NodeRef nr = node_ref(a.blk_seg, a.seg, bid);
-  const int ii = nr.ii;
+  const int bid = logical_wg<NB>(a.blist);
+  // the layout's arrays cover whole blocks (no links past the last node), so
+  // nothing of the streams waits for the segment
+  const int slice = __builtin_amdgcn_readfirstlane((bid * NB + (int)threadIdx.x) >> 6);
+  const int K = a.kcnt[bid * NB + (int)threadIdx.x];
+  const int KF = a.krange[slice].x, KM = a.krange[slice].y;
+  const int64_t o = a.off[slice];
+  const int64_t h0 = a.hoff[bid];
+  const int nh = (int)(a.hoff[bid + 1] - h0);
+  const NodeRef nr = node_ref<NB>(a.blk_seg, a.seg, bid);
   const bool act = nr.act;
-  const int64_t b = a.off[ii >> 6] + (ii & 63);
-  const int K = act ? a.kcnt[ii] : 0;
   double rx = 0, ry = 0, ux = 0, uy = 0, vx = 0, vy = 0, lu = 0, lv = 0;
   double axx = 0, ayx = 0, axy = 0, ayy = 0, bxy = 0, byy = 0;
   double cxx_l = 0, cxy_l = 0, cyy_l = 0;
   double q1x = 0, q1y = 0, q2x = 0, q2y = 0, q3x = 0, q3y = 0;
-  // The global streams (block-local column, three weights) of the next batch
-  // of links are loaded before the current batch is consumed, so each lane
-  // keeps SV_HALO_UNROLL links (26 bytes each) in flight; records come from LDS.
-  // The first batch is requested before the halo is staged.
-  constexpr int U = SV_HALO_UNROLL;
-  int jn[U];
-  double wxn[U], wyn[U], wln[U];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (k0 + u < K) {
-        const int64_t e = b + (int64_t)(k0 + u) * SV_WAVE;
-        jn[u] = (int)ld_stream(a.lcol + e);
-        wxn[u] = ld_stream(a.wx + e); wyn[u] = ld_stream(a.wy + e); wln[u] = ld_stream(a.wl + e);
-      }
+  constexpr int U = HaloU<NB>::U;
+  const Stream<uint32_t, 1, NT> sc(a.lcol + o, KM);
+  const Stream<dbl2, 3, NT> sw(a.w3 + 3 * o, KM);
+  uint32_t jc[2][U];
+  dbl2 wg[2][2 * U], wl[2][U];   // d/dx and d/dy of a link; Laplacian of a pair
+  auto load = [&](int s, int u, int p) {
+    jc[s][u] = sc.at(p, u, 0);
+    wg[s][2 * u] = sw.at(p, u, 0); wg[s][2 * u + 1] = sw.at(p, u, 1); wl[s][u] = sw.at(p, u, 2);
+  };
+  auto fetch = [&](int s, int l) {
+    return halo_rec<FORM>(hl, (int)(l & 1 ? jc[s][l / 2] >> 16 : jc[s][l / 2] & 0xffff));
+  };
+  auto link = [&](const Rec9 &q, int s, int l) {
+    const double wx_ = wg[s][l].x, wy_ = wg[s][l].y;
+    const double wl_ = l & 1 ? wl[s][l / 2].y : wl[s][l / 2].x;
+    rx += q.ro * wx_; ry += q.ro * wy_;
+    ux += q.u * wx_; uy += q.u * wy_; lu += q.u * wl_;
+    vx += q.v * wx_; vy += q.v * wy_; lv += q.v * wl_;
+    if (FORM == SV_FORM_LC) {
+      axx += q.cxx * wx_;
+      axy += q.cxy * wx_; ayy += q.cxy * wy_;
+      byy += q.cyy * wy_;
+      q1x += q.pxx * wx_; q1y += q.pxx * wy_;
+      q2x += q.pxy * wx_; q2y += q.pxy * wy_;
+      q3x += q.pyy * wx_; q3y += q.pyy * wy_;
+    } else {
+      axx += q.cxx * wx_; ayx += q.cxx * wy_;
+      axy += q.cxy * wx_; ayy += q.cxy * wy_;
+      bxy += q.cyy * wx_; byy += q.cyy * wy_;
+      if (MDIFF) { cxx_l += q.cxx * wl_; cxy_l += q.cxy * wl_; cyy_l += q.cyy * wl_; }
     }
   };
-  fetch(0);
-  const int64_t h0 = a.hoff[bid];
-  halo_stage<FORM>(a.G, a.hidx, h0, (int)(a.hoff[bid + 1] - h0), hl, hz);
-  __syncthreads();
-  for (int k = 0; k < K; k += U) {
-    int jc[U];
-    double wxc[U], wyc[U], wlc[U];
+  // the halo's keys first, then the first batch of links, in flight while the
+  // halo is staged
+  const int *hx = a.hidx + h0;
+  HaloKeys<NB> keys;
+  if (nh > 0) keys.get(hx, threadIdx.x, nh);
+  __builtin_amdgcn_sched_barrier(0);
+  const int p0 = entry_at(0);
 #pragma unroll
-    for (int u = 0; u < U; u++) { jc[u] = jn[u]; wxc[u] = wxn[u]; wyc[u] = wyn[u]; wlc[u] = wln[u]; }
-    fetch(k + U);
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (k + u < K) {
-        const Rec9 q = halo_rec<FORM>(hl, hz, jc[u]);
-        const double wx_ = wxc[u], wy_ = wyc[u], wl_ = wlc[u];
-        rx += q.ro * wx_; ry += q.ro * wy_;
-        ux += q.u * wx_; uy += q.u * wy_; lu += q.u * wl_;
-        vx += q.v * wx_; vy += q.v * wy_; lv += q.v * wl_;
-        if (FORM == SV_FORM_LC) {
-          axx += q.cxx * wx_;
-          axy += q.cxy * wx_; ayy += q.cxy * wy_;
-          byy += q.cyy * wy_;
-          q1x += q.pxx * wx_; q1y += q.pxx * wy_;
-          q2x += q.pxy * wx_; q2y += q.pxy * wy_;
-          q3x += q.pyy * wx_; q3y += q.pyy * wy_;
-        } else {
-          axx += q.cxx * wx_; ayx += q.cxx * wy_;
-          axy += q.cxy * wx_; ayy += q.cxy * wy_;
-          bxy += q.cyy * wx_; byy += q.cyy * wy_;
-          if (MDIFF) { cxx_l += q.cxx * wl_; cxy_l += q.cxy * wl_; cyy_l += q.cyy * wl_; }
+  for (int u = 0; u < U; u++) load(0, u, 2 * u < K ? p0 : OUT_OF_RANGE);
+  halo_stage<NB>(
+      hx, nh, keys, [&](int j) { return load_g<FORM>(a.G, j); },
+      [&](int h, int fl, Rec9 r) {
+        if (fl) {   // mirror ghost (reapply_mirror_bcs, mirror_boundaries.F90:285-340)
+          if (fl != 2) r.u = -r.u;
+          if (fl != 1) r.v = -r.v;
+          if (fl != 3) { r.cxy = -r.cxy; r.pxy = -r.pxy; }
         }
-      }
-  }
+        store_g<FORM>(hl, h, r);
+      });
+  __syncthreads();
+  walk_links<U, Rec9>(K, KF, KM, load, fetch, link);
   double emax_loc = 0.0;
   if (act) {
     const Sums S{rx, ry, ux, uy, vx, vy, lu, lv, axx, ayx, axy, ayy, bxy, byy, cxx_l, cxy_l,
@@ -767,15 +911,8 @@ __global__ __launch_bounds__(BS) void k_stage_h(StageArgs a) {
     emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S);
   }
   if (STAGE == 4) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) emax_loc = fmax(emax_loc, __shfl_xor(emax_loc, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = emax_loc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double m = red[0];
-      for (int w = 1; w < BS / SV_WAVE; w++) m = fmax(m, red[w]);
-      a.partial[bid] = m;
-    }
+    emax_loc = wave_max(emax_loc);
+    if ((threadIdx.x & 63) == 0) a.partial[nr.i >> 6] = emax_loc;
   }
 }
 
@@ -788,17 +925,16 @@ struct FilterArgs {
   const double *wh, *hsum, *vol;
   const double *U;   // gathered state records
   double *Uf;        // filtered state records
-  double *Gout;      // psi (LC) and c of the filtered state
-  double *partial;
+  double *partial;       // sum of (ro_f - rho_char)*vol per slice
+  const int4 *krange;    // links per slice (sv_loopl)
   const int64_t *hoff;   // per-block halos (k_filter_h)
   const int *hidx;
-  const uint16_t *lcol;   // per-block sum of (ro_f - rho_char)*vol
+  const uint16_t *lcol;
   const int *blist;       // launch group's logical blocks (nullable: all blocks)
 };
 
-// Pointwise part of the filter for one node: filtered record, its gather
-// record (psi and c = exp(psi) for LC), and the mass-correction term.
-template <int FORM>
+// Pointwise part of the filter for one node: the filtered record and its
+// mass-correction term.
 __device__ __forceinline__ double filter_point(const FilterArgs &a, const NodeRef &nr,
                                                const double t[6]) {
   const int i = nr.i;
@@ -808,20 +944,10 @@ __device__ __forceinline__ double filter_point(const FilterArgs &a, const NodeRe
 #pragma unroll
   for (int q = 0; q < 6; q++) g[q] = f[q] + (t[q] - f[q] * hs);
   store_u(a.Uf, i, g);
-  constexpr int S = (FORM == SV_FORM_LC) ? SV_GS_LC : SV_GS_DI;
-  double *G = a.Gout + (size_t)i * S;
-  double c1 = g[3], c2 = g[4], c3 = g[5];
-  if (FORM == SV_FORM_LC) {
-    G[SV_G_PXX] = g[3]; G[SV_G_PXY] = g[4]; G[SV_G_PYY] = g[5];
-    c_from_psi(g[3], g[4], g[5], c1, c2, c3);
-  }
-  G[SV_G_CXX] = c1; G[SV_G_CXY] = c2; G[SV_G_CYY] = c3;
   return (g[0] - a.seg[nr.sg].pk.rho_char) * a.vol[i];
 }
 
-template <int FORM>
 __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
-  __shared__ double red[BS];
   const int bid = sv_logical_block(a.blist);
   const NodeRef nr = node_ref(a.blk_seg, a.seg, bid);
   const int ii = nr.ii;
@@ -840,7 +966,7 @@ __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
     for (int u = 0; u < U; u++) {
       if (k + u < K) {
         load_u(a.U, jn[u], f[u]);
-        w[u] = ld_stream(a.wh + b + (int64_t)(k + u) * SV_WAVE);
+        w[u] = ld_stream(a.wh + sv_pair(b + (int64_t)(k + u) * SV_WAVE));
       }
     }
 #pragma unroll
@@ -855,88 +981,77 @@ __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
         for (int q = 0; q < 6; q++) t[q] += f[u][q] * w[u];
       }
   }
-  const double m = act ? filter_point<FORM>(a, nr, t) : 0.0;
-  red[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) a.partial[bid] = red[0];
+  const double m = wave_sum(act ? filter_point(a, nr, t) : 0.0);
+  if ((threadIdx.x & 63) == 0) a.partial[nr.i >> 6] = m;
 }
 
 // Halo-staged form of k_filter (see k_stage_h): the block's neighbour state
 // records (6 doubles) go to LDS once, links read them by block-local index.
-template <int FORM>
-__global__ __launch_bounds__(BS) void k_filter_h(FilterArgs a) {
+template <int NB, bool NT>
+__global__ __launch_bounds__(NB) void k_filter_h(FilterArgs a) {
   extern __shared__ double hl[];
-  __shared__ double red[BS];
-  const int bid = sv_logical_block(a.blist);
-  const NodeRef nr = node_ref(a.blk_seg, a.seg, bid);
-  const int ii = nr.ii;
-  const bool act = nr.act;
-  const int64_t b = a.off[ii >> 6] + (ii & 63);
-  const int K = act ? a.kcnt[ii] : 0;
-  double t[6] = {0, 0, 0, 0, 0, 0};
-  constexpr int U = SV_HALO_UNROLL;
-  int jn[U];
-  double wn[U];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (k0 + u < K) {
-        const int64_t e = b + (int64_t)(k0 + u) * SV_WAVE;
-        jn[u] = (int)ld_stream(a.lcol + e);
-        wn[u] = ld_stream(a.wh + e);
-      }
-  };
-  fetch(0);   // the first batch is in flight while the halo is staged
+  const int bid = logical_wg<NB>(a.blist);
+  const int slice = __builtin_amdgcn_readfirstlane((bid * NB + (int)threadIdx.x) >> 6);
+  const int K = a.kcnt[bid * NB + (int)threadIdx.x];   // as k_stage_h
+  const int KF = a.krange[slice].z, KM = a.krange[slice].w;
+  const int64_t o = a.off[slice];
   const int64_t h0 = a.hoff[bid];
   const int nh = (int)(a.hoff[bid + 1] - h0);
-  for (int h = threadIdx.x; h < nh; h += BS) {
-    double f[6];
-    const int key = a.hidx[h0 + h];
-    load_u(a.U, key & SV_FLIP_MASK, f);
-    const int fl = key >> SV_FLIP_SHIFT;
-    if (fl) {   // mirror ghost: rho u, rho v and the xy component
-      if (fl != 2) f[1] = -f[1];
-      if (fl != 1) f[2] = -f[2];
-      if (fl != 3) f[4] = -f[4];
-    }
-    double2 *d = reinterpret_cast<double2 *>(hl + (size_t)h * 6);
-    d[0] = double2{f[0], f[1]};
-    d[1] = double2{f[2], f[3]};
-    d[2] = double2{f[4], f[5]};
-  }
-  __syncthreads();
-  for (int k = 0; k < K; k += U) {
-    int jc[U];
-    double wc[U];
+  const NodeRef nr = node_ref<NB>(a.blk_seg, a.seg, bid);
+  const bool act = nr.act;
+  double t[6] = {0, 0, 0, 0, 0, 0};
+  constexpr int U = HaloU<NB>::UF;
+  const Stream<uint32_t, 1, NT> sc(a.lcol + o, KM);
+  const Stream<dbl2, 1, NT> sw(a.wh + o, KM);
+  uint32_t jc[2][U];
+  dbl2 w[2][U];
+  auto load = [&](int s, int u, int p) {
+    jc[s][u] = sc.at(p, u, 0);
+    w[s][u] = sw.at(p, u, 0);
+  };
+  struct Rec6 {
+    double2 d0, d1, d2;
+  };
+  auto fetch = [&](int s, int l) {
+    const int j = (int)(l & 1 ? jc[s][l / 2] >> 16 : jc[s][l / 2] & 0xffff);
+    const double2 *d = reinterpret_cast<const double2 *>(hl + j * 6);
+    return Rec6{d[0], d[1], d[2]};
+  };
+  auto link = [&](const Rec6 &q, int s, int l) {
+    const double w_ = l & 1 ? w[s][l / 2].y : w[s][l / 2].x;
+    t[0] += q.d0.x * w_; t[1] += q.d0.y * w_; t[2] += q.d1.x * w_;
+    t[3] += q.d1.y * w_; t[4] += q.d2.x * w_; t[5] += q.d2.y * w_;
+  };
+  const int *hx = a.hidx + h0;   // keys, first links, halo: as k_stage_h
+  HaloKeys<NB> keys;
+  if (nh > 0) keys.get(hx, threadIdx.x, nh);
+  __builtin_amdgcn_sched_barrier(0);
+  const int p0 = entry_at(0);
 #pragma unroll
-    for (int u = 0; u < U; u++) { jc[u] = jn[u]; wc[u] = wn[u]; }
-    fetch(k + U);
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (k + u < K) {
-        const double2 *d = reinterpret_cast<const double2 *>(hl + (size_t)jc[u] * 6);
-        const double2 d0 = d[0], d1 = d[1], d2 = d[2];
-        const double w = wc[u];
-        t[0] += d0.x * w; t[1] += d0.y * w; t[2] += d1.x * w;
-        t[3] += d1.y * w; t[4] += d2.x * w; t[5] += d2.y * w;
-      }
-  }
-  const double m = act ? filter_point<FORM>(a, nr, t) : 0.0;
-  red[threadIdx.x] = m;
+  for (int u = 0; u < U; u++) load(0, u, 2 * u < K ? p0 : OUT_OF_RANGE);
+  halo_stage<NB>(
+      hx, nh, keys,
+      [&](int j) {
+        const double2 *q = reinterpret_cast<const double2 *>(a.U + (size_t)j * SV_US);
+        return Rec6{q[0], q[1], q[2]};
+      },
+      [&](int h, int fl, Rec6 r) {
+        if (fl) {   // mirror ghost: rho u, rho v and the xy component
+          if (fl != 2) r.d0.y = -r.d0.y;
+          if (fl != 1) r.d1.x = -r.d1.x;
+          if (fl != 3) r.d2.x = -r.d2.x;
+        }
+        double2 *d = reinterpret_cast<double2 *>(hl + h * 6);
+        d[0] = r.d0; d[1] = r.d1; d[2] = r.d2;
+      });
   __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) a.partial[bid] = red[0];
+  walk_links<U, Rec6>(K, KF, KM, load, fetch, link);
+  const double m = wave_sum(act ? filter_point(a, nr, t) : 0.0);
+  if ((threadIdx.x & 63) == 0) a.partial[nr.i >> 6] = m;
 }
 
 // mass correction value, emax and the end-of-step counters; one block per
-// segment over that segment's per-block partials
+// segment over that segment's per-slice partials
 __global__ __launch_bounds__(1024) void k_reduce(const sv_segk *seg, const double *pmass,
                                                  const double *perr, sv_ctrl *ctrl_all) {
   __shared__ double s1[1024], s2[1024];
@@ -944,9 +1059,15 @@ __global__ __launch_bounds__(1024) void k_reduce(const sv_segk *seg, const doubl
   sv_ctrl *ctrl = ctrl_all + blockIdx.x;
   const double volsum = S.volsum;
   double a = 0.0, m = 0.0;
+  // a thread takes the four slices of a block at a time
+  static_assert(SPB == 4, "two double2 per block");
+  const double2 *pm = reinterpret_cast<const double2 *>(pmass) + 2 * (size_t)S.blk0;
+  const double2 *pe = reinterpret_cast<const double2 *>(perr) + 2 * (size_t)S.blk0;
+#pragma unroll 4
   for (int k = threadIdx.x; k < S.nblk; k += 1024) {
-    a += pmass[S.blk0 + k];
-    m = fmax(m, perr[S.blk0 + k]);
+    const double2 m0 = pm[2 * k], m1 = pm[2 * k + 1], e0 = pe[2 * k], e1 = pe[2 * k + 1];
+    a += (m0.x + m0.y) + (m1.x + m1.y);
+    m = fmax(fmax(fmax(m, e0.x), fmax(e0.y, e1.x)), e1.y);
   }
   s1[threadIdx.x] = a;
   s2[threadIdx.x] = m;
@@ -979,7 +1100,6 @@ __global__ __launch_bounds__(1024) void k_reduce(const sv_segk *seg, const doubl
 }
 
 struct ApplyArgs {
-  int gs;
   const int *blk_seg;
   const sv_segk *seg;
   const double *Uf;
@@ -987,17 +1107,19 @@ struct ApplyArgs {
   double *G;
   const double *s;
   const sv_ctrl *ctrl;   // ctrl[sg].dro is subtracted; nullptr for no correction
-  double *pcfl, *pvisc;  // per-block minima for set_tstep
+  double *pcfl, *pvisc;  // minima for set_tstep per slice
   const int *bidx;       // boundary nodes (nullable), as StageArgs
   const double *brec;
 };
 
-// rho -= drho (rhs_lc.F90:887-889); u = rou/rho (step.F90:514-529); set_tstep
-// partial minima (step.F90:579-602)
+// rho -= drho (rhs_lc.F90:887-889); the gather record: u = rou/rho
+// (step.F90:514-529), psi and c = exp(psi) (LC); set_tstep partial minima
+// (step.F90:579-602).  The record is written here as a whole (the filter
+// writing psi and c and this kernel ro, u, v made two partial writes of
+// every line).
+template <int FORM>
 __global__ __launch_bounds__(BS) void k_apply_state(ApplyArgs a) {
-  __shared__ double r1[BS], r2[BS];
-  const int bid = sv_xcd_block();
-  const NodeRef nr = node_ref(a.blk_seg, a.seg, bid);
+  const NodeRef nr = node_ref(a.blk_seg, a.seg, sv_xcd_block());
   const int i = nr.i;
   double mc = 1.0e10, mv = 1.0e10;
   if (nr.act) {
@@ -1019,26 +1141,24 @@ __global__ __launch_bounds__(BS) void k_apply_state(ApplyArgs a) {
     store_u(a.U, i, f);
     const double ooro = 1.0 / f[0];
     const double u = f[1] * ooro, v = f[2] * ooro;
-    double *G = a.G + (size_t)i * a.gs;
-    reinterpret_cast<double2 *>(G)[0] = double2{f[0], u};
-    G[SV_G_V] = v;
+    Rec9 g;
+    g.ro = f[0]; g.u = u; g.v = v;
+    if (FORM == SV_FORM_LC) {
+      g.pxx = f[3]; g.pxy = f[4]; g.pyy = f[5];
+      c_from_psi(f[3], f[4], f[5], g.cxx, g.cxy, g.cyy);
+    } else {
+      g.cxx = f[3]; g.cxy = f[4]; g.cyy = f[5];
+    }
+    store_g<FORM>(a.G, i, g);
     const double um = sqrt(u * u + v * v + 0.0);
     const double si = a.s[i];
     // slightly smaller on outflows (step.F90:591-595)
     mc = bk == 2 ? 0.8 * si / (um + P.cs) : si / (um + P.cs);
     mv = si * si * f[0] / P.visc_total;
   }
-  r1[threadIdx.x] = mc;
-  r2[threadIdx.x] = mv;
-  __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      r1[threadIdx.x] = fmin(r1[threadIdx.x], r1[threadIdx.x + s]);
-      r2[threadIdx.x] = fmin(r2[threadIdx.x], r2[threadIdx.x + s]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) { a.pcfl[bid] = r1[0]; a.pvisc[bid] = r2[0]; }
+  mc = wave_min(mc);
+  mv = wave_min(mv);
+  if ((threadIdx.x & 63) == 0) { a.pcfl[i >> 6] = mc; a.pvisc[i >> 6] = mv; }
 }
 
 // set_tstep (step.F90:569-622) + set_tstep_PID (:624-682) + the start of
@@ -1051,9 +1171,13 @@ __global__ __launch_bounds__(1024) void k_dt(const sv_segk *seg, const double *p
   sv_ctrl *c = ctrl_all + blockIdx.x;
   const double L_char = S.pk.L_char;
   double a = 1.0e10, m = 1.0e10;
+  const double2 *p = reinterpret_cast<const double2 *>(pcfl) + 2 * (size_t)S.blk0;
+  const double2 *q = reinterpret_cast<const double2 *>(pvisc) + 2 * (size_t)S.blk0;
+#pragma unroll 4
   for (int k = threadIdx.x; k < S.nblk; k += 1024) {
-    a = fmin(a, pcfl[S.blk0 + k]);
-    m = fmin(m, pvisc[S.blk0 + k]);
+    const double2 p0 = p[2 * k], p1 = p[2 * k + 1], q0 = q[2 * k], q1 = q[2 * k + 1];
+    a = fmin(fmin(fmin(a, p0.x), fmin(p0.y, p1.x)), p1.y);
+    m = fmin(fmin(fmin(m, q0.x), fmin(q0.y, q1.x)), q1.y);
   }
   s1[threadIdx.x] = a;
   s2[threadIdx.x] = m;
@@ -1097,25 +1221,6 @@ __global__ __launch_bounds__(1024) void k_dt(const sv_segk *seg, const double *p
   c->time0 = c->time;
 }
 
-// initial gather records: psi (LC) and c of the state (ro, u, v by k_apply_state)
-template <int FORM>
-__global__ __launch_bounds__(BS) void k_init_gather(const int *blk_seg, const sv_segk *seg,
-                                                     const double *U, double *G) {
-  const NodeRef nr = node_ref(blk_seg, seg, (int)blockIdx.x);
-  if (!nr.act) return;
-  const int i = nr.i;
-  double f[6];
-  load_u(U, i, f);
-  constexpr int S = (FORM == SV_FORM_LC) ? SV_GS_LC : SV_GS_DI;
-  double *g = G + (size_t)i * S;
-  double c1 = f[3], c2 = f[4], c3 = f[5];
-  if (FORM == SV_FORM_LC) {
-    g[SV_G_PXX] = f[3]; g[SV_G_PXY] = f[4]; g[SV_G_PYY] = f[5];
-    c_from_psi(f[3], f[4], f[5], c1, c2, c3);
-  }
-  g[SV_G_CXX] = c1; g[SV_G_CXY] = c2; g[SV_G_CYY] = c3;
-}
-
 StageArgs stage_args(sv_ctx *c, int stage, const double *Gin, double *Gout) {
   StageArgs a{};
   a.rhs_stride = c->npfb;
@@ -1124,7 +1229,7 @@ StageArgs stage_args(sv_ctx *c, int stage, const double *Gin, double *Gout) {
   a.off = c->L.off;
   a.kcnt = c->L.cnt_small;
   a.col = c->L.col;
-  a.wx = c->L.wx; a.wy = c->L.wy; a.wl = c->L.wl;
+  a.w3 = c->L.w3;
   a.gsx = c->L.gsx; a.gsy = c->L.gsy; a.lsum = c->L.lsum;
   a.G = Gin;
   a.reg_in = (stage == 1) ? c->U : c->reg;
@@ -1134,43 +1239,44 @@ StageArgs stage_args(sv_ctx *c, int stage, const double *Gin, double *Gout) {
   a.Gout = Gout;
   a.fx = c->any_forcing ? c->fx : nullptr;
   a.ctrl = c->ctrl;
+  a.krange = c->L.krange;
   a.hoff = c->L.hoff;
   a.hidx = c->L.hidx;
   a.lcol = c->L.lcol;
-  a.hcap = c->L.hmax;
   a.partial = c->partial;
   a.bidx = c->L.bidx;
   a.brec = c->L.brec;
   return a;
 }
 
+// nb: 256-slot blocks of the launch
+template <int FORM, int STAGE, bool MDIFF, bool BND>
+void launch_sweep(sv_ctx *c, const StageArgs &a, int nb, int hmax) {
+  if (!c->L.halo) {
+    k_stage<FORM, STAGE, MDIFF, BND><<<nb, BS, 0, c->stream>>>(a);
+    return;
+  }
+  const size_t shm = (size_t)hmax * HaloL<FORM>::BYTES;
+  const int hb = c->L.hb, grid = nb * (BS / hb);
+  if (hb == 64)
+    k_stage_h<FORM, STAGE, MDIFF, BND, 64, false><<<grid, 64, shm, c->stream>>>(a);
+  else if (hb == 128 && !c->L.nt)
+    k_stage_h<FORM, STAGE, MDIFF, BND, 128, false><<<grid, 128, shm, c->stream>>>(a);
+  else if (hb == 128)
+    k_stage_h<FORM, STAGE, MDIFF, BND, 128, true><<<grid, 128, shm, c->stream>>>(a);
+  else
+    k_stage_h<FORM, STAGE, MDIFF, BND, 256, true><<<grid, 256, shm, c->stream>>>(a);
+}
+
 template <int FORM, int STAGE>
 void launch_stage_grid(sv_ctx *c, const StageArgs &a, int nb, int hmax) {
-  const bool md = FORM == SV_FORM_DI && c->any_mdiff;
-  if constexpr (FORM == SV_FORM_LC) {
-    const bool bnd = a.bidx != nullptr;
-    if (c->L.halo) {
-      const size_t shm = (size_t)hmax * HaloL<FORM>::BYTES;
-      if (bnd) k_stage_h<FORM, STAGE, false, true><<<nb, BS, shm, c->stream>>>(a);
-      else k_stage_h<FORM, STAGE, false, false><<<nb, BS, shm, c->stream>>>(a);
-    } else {
-      if (bnd) k_stage<FORM, STAGE, false, true><<<nb, BS, 0, c->stream>>>(a);
-      else k_stage<FORM, STAGE, false, false><<<nb, BS, 0, c->stream>>>(a);
-    }
+  const bool bnd = a.bidx != nullptr;
+  if (FORM == SV_FORM_DI && c->any_mdiff) {
+    if (bnd) launch_sweep<FORM, STAGE, FORM == SV_FORM_DI, true>(c, a, nb, hmax);
+    else launch_sweep<FORM, STAGE, FORM == SV_FORM_DI, false>(c, a, nb, hmax);
   } else {
-    const bool bnd = a.bidx != nullptr;
-    if (c->L.halo) {
-      const size_t shm = (size_t)hmax * HaloL<FORM>::BYTES;
-      if (md && bnd) k_stage_h<FORM, STAGE, true, true><<<nb, BS, shm, c->stream>>>(a);
-      else if (md) k_stage_h<FORM, STAGE, true, false><<<nb, BS, shm, c->stream>>>(a);
-      else if (bnd) k_stage_h<FORM, STAGE, false, true><<<nb, BS, shm, c->stream>>>(a);
-      else k_stage_h<FORM, STAGE, false, false><<<nb, BS, shm, c->stream>>>(a);
-    } else {
-      if (md && bnd) k_stage<FORM, STAGE, true, true><<<nb, BS, 0, c->stream>>>(a);
-      else if (md) k_stage<FORM, STAGE, true, false><<<nb, BS, 0, c->stream>>>(a);
-      else if (bnd) k_stage<FORM, STAGE, false, true><<<nb, BS, 0, c->stream>>>(a);
-      else k_stage<FORM, STAGE, false, false><<<nb, BS, 0, c->stream>>>(a);
-    }
+    if (bnd) launch_sweep<FORM, STAGE, false, true>(c, a, nb, hmax);
+    else launch_sweep<FORM, STAGE, false, false>(c, a, nb, hmax);
   }
 }
 
@@ -1182,7 +1288,6 @@ void launch_stage(sv_ctx *c, const StageArgs &a, int nb) {
     for (const sv_ctx::lgroup &g : c->lgroups) {
       StageArgs b = a;
       b.blist = g.blist;
-      b.hcap = g.hmax;
       launch_stage_grid<FORM, STAGE>(c, b, g.nblk, g.hmax);
     }
     return;
@@ -1190,29 +1295,37 @@ void launch_stage(sv_ctx *c, const StageArgs &a, int nb) {
   launch_stage_grid<FORM, STAGE>(c, a, nb, c->L.hmax);
 }
 
-template <int FORM>
+void launch_filter_grid(sv_ctx *c, const FilterArgs &f, int nb, int hmax) {
+  const size_t shm = sizeof(double) * 6 * (size_t)hmax;
+  const int hb = c->L.hb, grid = nb * (BS / hb);
+  if (hb == 64) k_filter_h<64, false><<<grid, 64, shm, c->stream>>>(f);
+  else if (hb == 128 && !c->L.nt) k_filter_h<128, false><<<grid, 128, shm, c->stream>>>(f);
+  else if (hb == 128) k_filter_h<128, true><<<grid, 128, shm, c->stream>>>(f);
+  else k_filter_h<256, true><<<grid, 256, shm, c->stream>>>(f);
+}
+
 void launch_filter(sv_ctx *c, const FilterArgs &f, int nb) {
   if (!c->L.halo) {
-    k_filter<FORM><<<nb, BS, 0, c->stream>>>(f);
+    k_filter<<<nb, BS, 0, c->stream>>>(f);
     return;
   }
   if (c->lgroup_mode == 1 && !c->lgroups.empty()) {
     for (const sv_ctx::lgroup &g : c->lgroups) {
       FilterArgs b = f;
       b.blist = g.blist;
-      k_filter_h<FORM><<<g.nblk, BS, sizeof(double) * 6 * (size_t)g.hmax, c->stream>>>(b);
+      launch_filter_grid(c, b, g.nblk, g.hmax);
     }
     return;
   }
-  k_filter_h<FORM><<<nb, BS, sizeof(double) * 6 * (size_t)c->L.hmax, c->stream>>>(f);
+  launch_filter_grid(c, f, nb, c->L.hmax);
 }
 
 // ev (nullable): SV_NKERNELS+1 events recorded between the launches of one step
 template <int FORM>
 int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
   const int nb = c->nblk;
-  double *pm = c->partial, *pe = c->partial + nb, *pc = c->partial + 2 * nb,
-         *pv = c->partial + 3 * nb;
+  const size_t np = (size_t)nb * SPB;   // partial results of one kind
+  double *pm = c->partial, *pe = pm + np, *pc = pm + 2 * np, *pv = pm + 3 * np;
   int ke = 0;
   auto mark = [&]() {
     if (ev) (void)hipEventRecord(ev[ke++], c->stream);
@@ -1244,17 +1357,16 @@ int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
   f.vol = c->L.vol;
   f.U = c->U;
   f.Uf = c->Uf;
-  f.Gout = c->GA;
   f.partial = pm;
+  f.krange = c->L.krange;
   f.hoff = c->L.hoff;
   f.hidx = c->L.hidx;
   f.lcol = c->L.lcol;
-  launch_filter<FORM>(c, f, nb);
+  launch_filter(c, f, nb);
   mark();
   k_reduce<<<c->nseg, 1024, 0, c->stream>>>(c->segk, pm, pe, c->ctrl);
   mark();
   ApplyArgs ap{};
-  ap.gs = c->gs;
   ap.blk_seg = c->blk_seg;
   ap.seg = c->segk;
   ap.Uf = c->Uf;
@@ -1266,7 +1378,7 @@ int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
   ap.pvisc = pv;
   ap.bidx = c->L.bidx;
   ap.brec = c->L.brec;
-  k_apply_state<<<nb, BS, 0, c->stream>>>(ap);
+  k_apply_state<FORM><<<nb, BS, 0, c->stream>>>(ap);
   mark();
   SV_HIP(c, hipGetLastError());
   return 0;
@@ -1274,11 +1386,11 @@ int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
 
 }  // namespace
 
-int sv_dev_init_partials(sv_ctx *c) {
-  // u, v and the set_tstep partial minima of the current state (no correction)
+int sv_dev_init_state(sv_ctx *c) {
+  // gather records and the set_tstep partial minima of the current state (no
+  // correction)
   const int nb = c->nblk;
   ApplyArgs ap{};
-  ap.gs = c->gs;
   ap.blk_seg = c->blk_seg;
   ap.seg = c->segk;
   ap.Uf = c->U;
@@ -1286,24 +1398,15 @@ int sv_dev_init_partials(sv_ctx *c) {
   ap.G = c->GA;
   ap.s = c->L.s;
   ap.ctrl = nullptr;
-  ap.pcfl = c->partial + 2 * nb;
-  ap.pvisc = c->partial + 3 * nb;
+  ap.pcfl = c->partial + 2 * (size_t)nb * SPB;
+  ap.pvisc = c->partial + 3 * (size_t)nb * SPB;
   ap.bidx = c->L.bidx;
   ap.brec = c->L.brec;
-  k_apply_state<<<nb, BS, 0, c->stream>>>(ap);
+  if (c->cfg.form == SV_FORM_LC) k_apply_state<SV_FORM_LC><<<nb, BS, 0, c->stream>>>(ap);
+  else k_apply_state<SV_FORM_DI><<<nb, BS, 0, c->stream>>>(ap);
   SV_HIP(c, hipGetLastError());
   SV_HIP(c, hipStreamSynchronize(c->stream));
   return 0;
-}
-
-int sv_dev_init_state(sv_ctx *c) {
-  const int nb = c->nblk;
-  if (c->cfg.form == SV_FORM_LC)
-    k_init_gather<SV_FORM_LC><<<nb, BS, 0, c->stream>>>(c->blk_seg, c->segk, c->U, c->GA);
-  else
-    k_init_gather<SV_FORM_DI><<<nb, BS, 0, c->stream>>>(c->blk_seg, c->segk, c->U, c->GA);
-  SV_HIP(c, hipGetLastError());
-  return sv_dev_init_partials(c);
 }
 
 int sv_dev_step(sv_ctx *c, hipEvent_t *ev) {

@@ -599,7 +599,7 @@ static int ensure_state_buffers(sv_ctx *c) {
     return SV_E_NOMEM;
   SV_HIP(c, hipMemset(c->GA, 0, ng));
   SV_HIP(c, hipMemset(c->GB, 0, ng));
-  c->npartial = 4 * c->nblk;
+  c->npartial = 4 * c->nblk * (SV_BLOCK / SV_WAVE);   // four kinds, one per slice
   if (sv_alloc(c, (void **)&c->partial, sizeof(double) * (c->npartial + 8)) ||
       sv_alloc(c, (void **)&c->ctrl, sizeof(sv_ctrl)) ||
       sv_alloc(c, (void **)&c->fx, sizeof(double) * c->ntot) ||
@@ -684,7 +684,7 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
   if (int rc = sv_ensure_loop(c)) return rc;
   SV_CHECK(c, !c->has_mirror || c->L.halo,
            "symmetric/no-slip mirror ghosts need the LDS halo sweeps (halo_sweeps = 1 and "
-           "block halos within %d bytes)", SV_HALO_LDS_MAX);
+           "block halos within %d records)", SV_HALO_MAX);
   if (int rc = ensure_state_buffers(c)) return rc;
   const int n = c->npfb;
   std::vector<double> a(n), b(n), d(n), e(n), f(n), g(n);
@@ -1003,7 +1003,7 @@ int sv_get_stencil_stats(sv_ctx *c, double *stats) {
   stats[5] = 0.0;                  // halo records per node staged by the sweeps
   if (c->L.valid && c->L.halo) {
     int64_t tot = 0;
-    const int nb = (c->npfb + c->L.hb - 1) / c->L.hb;
+    const int nb = c->nblk * (SV_BLOCK / c->L.hb);
     SV_HIP(c, hipMemcpy(&tot, c->L.hoff + nb, sizeof(int64_t), hipMemcpyDeviceToHost));
     stats[5] = (double)tot / c->npfb;
   }

@@ -10,7 +10,7 @@
 // member's block range, and each member keeps its own control block (dt, PID
 // history, itime, inflow ramp) and physics constants.  Boundary records are
 // concatenated with their FD-row slots rebased; mirror ghosts keep their
-// sign-flip codes in the rebased halo keys.  The members' own contexts stay
+// sign-flip codes; the halos are built over the concatenated layout.  The members' own contexts stay
 // valid and unchanged: the ensemble holds copies taken at creation.
 #include <string.h>
 
@@ -111,22 +111,21 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
   const size_t N = (size_t)E->ntot, D = sizeof(double), I = sizeof(int);
   sv_loopl &EL = E->L;
   void **bufs[] = {(void **)&EL.off, (void **)&EL.cnt, (void **)&EL.cnt_small,
-                   (void **)&EL.col, (void **)&EL.wx, (void **)&EL.wy, (void **)&EL.wl,
-                   (void **)&EL.wh, (void **)&EL.gsx, (void **)&EL.gsy, (void **)&EL.lsum,
+                   (void **)&EL.col, (void **)&EL.w3, (void **)&EL.wh, (void **)&EL.gsx, (void **)&EL.gsy, (void **)&EL.lsum,
                    (void **)&EL.hsum, (void **)&EL.vol, (void **)&EL.s, (void **)&E->fx,
                    (void **)&E->U, (void **)&E->Uf, (void **)&E->reg, (void **)&E->eacc,
                    (void **)&E->GA, (void **)&E->GB, (void **)&E->partial, (void **)&E->ctrl,
                    (void **)&E->segk, (void **)&E->blk_seg};
   const size_t sizes[] = {sizeof(int64_t) * (EL.nslices + 1), I * N, I * N,
-                          I * (size_t)sell, D * (size_t)sell, D * (size_t)sell,
-                          D * (size_t)sell, D * (size_t)sell, D * N, D * N, D * N, D * N, D * N,
+                          I * (size_t)sell, 3 * D * (size_t)sell, D * (size_t)sell, D * N, D * N, D * N, D * N, D * N,
                           D * N, D * N, D * SV_US * N, D * SV_US * N, D * SV_US * N,
                           D * SV_US * N, D * E->gs * N, D * E->gs * N,
-                          D * (4 * (size_t)blocks + 8), sizeof(sv_ctrl) * nmembers,
+                          D * (4 * (size_t)blocks * (SV_BLOCK / SV_WAVE) + 8),
+                          sizeof(sv_ctrl) * nmembers,
                           sizeof(sv_segk) * nmembers, I * (size_t)blocks};
   for (size_t k = 0; k < sizeof(sizes) / sizeof(sizes[0]); k++)
     if (sv_alloc(E, bufs[k], sizes[k])) return fail(SV_E_NOMEM);
-  E->npartial = 4 * blocks;
+  E->npartial = 4 * blocks * (SV_BLOCK / SV_WAVE);
   if (hipMemsetAsync(EL.off, 0, sizes[0], E->stream) != hipSuccess ||
       hipMemsetAsync(EL.cnt, 0, I * N, E->stream) != hipSuccess ||
       hipMemsetAsync(EL.cnt_small, 0, I * N, E->stream) != hipSuccess ||
@@ -136,38 +135,19 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
       hipMemsetAsync(E->GA, 0, D * E->gs * N, E->stream) != hipSuccess ||
       hipMemsetAsync(E->GB, 0, D * E->gs * N, E->stream) != hipSuccess)
     return fail(SV_E_HIP);
-  // per-block halos: used when every member has them (see sv_loopl)
+  // per-block halos: used when every member has them, and built over the
+  // concatenated layout once that is in place
   bool halo = true;
-  int hmax = 0;
-  std::vector<int64_t> hbase(nmembers + 1, 0);
-  for (int m = 0; m < nmembers; m++) {
-    const sv_loopl &CL = members[m]->L;
-    halo = halo && CL.halo;
-    if (!halo) {
-      // mirror flips live in the halo keys
-      if (E->has_mirror)
-        return fail_msg(SV_E_ARG, "a member has mirror ghosts, so every member needs "
-                                  "per-block neighbour halos (a member has none: its halo "
-                                  "exceeds the LDS budget or halo_sweeps is off)");
-      break;
-    }
-    hmax = std::max(hmax, CL.hmax);
-    const int nbm = E->hseg[m].nblk;
-    int64_t last = 0;
-    if (hipMemcpy(&last, CL.hoff + nbm, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess)
+  for (int m = 0; m < nmembers; m++) halo = halo && members[m]->L.halo;
+  // mirror flips live in the halo keys
+  if (!halo && E->has_mirror)
+    return fail_msg(SV_E_ARG, "a member has mirror ghosts, so every member needs "
+                              "per-block neighbour halos (a member has none: its halo "
+                              "exceeds the LDS budget or halo_sweeps is off)");
+  if (E->has_mirror) {
+    if (sv_alloc(E, (void **)&EL.lflip, (size_t)sell + 1)) return fail(SV_E_NOMEM);
+    if (hipMemsetAsync(EL.lflip, 0, (size_t)sell + 1, E->stream) != hipSuccess)
       return fail(SV_E_HIP);
-    hbase[m + 1] = hbase[m] + last;
-  }
-  if (halo) {
-    if (sv_alloc(E, (void **)&EL.hoff, sizeof(int64_t) * ((size_t)blocks + 1)) ||
-        sv_alloc(E, (void **)&EL.hidx, I * ((size_t)hbase[nmembers] + 1)) ||
-        sv_alloc(E, (void **)&EL.lcol, sizeof(uint16_t) * ((size_t)sell + 1)))
-      return fail(SV_E_NOMEM);
-    const int64_t tot = hbase[nmembers];
-    if (hipMemcpy(EL.hoff + blocks, &tot, sizeof(int64_t), hipMemcpyHostToDevice) != hipSuccess)
-      return fail(SV_E_HIP);
-    EL.halo = true;
-    EL.hmax = hmax;
   }
   std::vector<int> bseg(blocks);
   std::vector<int> ebidx;
@@ -188,10 +168,8 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
     if (!rc) rc = sv_dev_offset_i64(E, EL.off + b / SV_WAVE, CL.nslices, sb);
     if (!rc) rc = copy_d2d(E, EL.col + sb, CL.col, I * (size_t)CL.nnz);
     if (!rc) rc = sv_dev_offset_int(E, EL.col + sb, CL.nnz, S.base);
-    const double *wsrc[4] = {CL.wx, CL.wy, CL.wl, CL.wh};
-    double *wdst[4] = {EL.wx, EL.wy, EL.wl, EL.wh};
-    for (int k = 0; k < 4 && !rc; k++)
-      rc = copy_d2d(E, wdst[k] + sb, wsrc[k], D * (size_t)CL.nnz);
+    if (!rc) rc = copy_d2d(E, EL.w3 + 3 * sb, CL.w3, 3 * D * (size_t)CL.nnz);
+    if (!rc) rc = copy_d2d(E, EL.wh + sb, CL.wh, D * (size_t)CL.nnz);
     if (!rc) rc = copy_d2d(E, EL.cnt + b, CL.cnt, I * n);
     if (!rc) rc = copy_d2d(E, EL.cnt_small + b, CL.cnt_small, I * n);
     const double *nsrc[7] = {CL.gsx, CL.gsy, CL.lsum, CL.hsum, CL.vol, CL.s, c->fx};
@@ -213,14 +191,7 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
         for (int k = 4; k < 8; k++) br[(size_t)SV_BREC * jb + k] += (double)S.base;
       ebrec.insert(ebrec.end(), br.begin(), br.end());
     }
-    if (!rc && halo) {
-      const int64_t hb = hbase[m], hn = hbase[m + 1] - hbase[m];
-      rc = copy_d2d(E, EL.hoff + S.blk0, CL.hoff, sizeof(int64_t) * (size_t)S.nblk);
-      if (!rc) rc = sv_dev_offset_i64(E, EL.hoff + S.blk0, S.nblk, hb);
-      if (!rc) rc = copy_d2d(E, EL.hidx + hb, CL.hidx, I * (size_t)hn);
-      if (!rc) rc = sv_dev_offset_int(E, EL.hidx + hb, hn, S.base);
-      if (!rc) rc = copy_d2d(E, EL.lcol + sb, CL.lcol, sizeof(uint16_t) * (size_t)CL.nnz);
-    }
+    if (!rc && CL.lflip) rc = copy_d2d(E, EL.lflip + sb, CL.lflip, (size_t)CL.nnz);
     if (rc) return fail(rc);
   }
   if (E->nb > 0) {
@@ -238,14 +209,16 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
                      E->stream) != hipSuccess ||
       hipStreamSynchronize(E->stream) != hipSuccess)
     return fail(SV_E_HIP);
+  if (halo)
+    if (int rc = sv_dev_build_halos(E, E->ntot)) return fail(rc);
   E->sell_dirty = false;
   EL.valid = true;
   E->have_phys = true;
   E->have_state = true;
-  if (int rc = sv_dev_init_partials(E)) return fail(rc);
+  if (int rc = sv_dev_init_state(E)) return fail(rc);
   // launch groups: the blocks of the members of each LABFM order, with the
   // largest halo among them; the autotuner keeps one launch or one per group
-  if (halo) {
+  if (EL.halo) {
     std::vector<int> orders;
     for (int m = 0; m < nmembers; m++) {
       const int o = members[m]->cfg.morder;
@@ -260,7 +233,9 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
           if (members[m]->cfg.morder != o) continue;
           const sv_segk &S = E->hseg[m];
           for (int k = 0; k < S.nblk; k++) bl.push_back(S.blk0 + k);
-          g.hmax = std::max(g.hmax, members[m]->L.hmax);
+          const int sub = SV_BLOCK / EL.hb;   // halo blocks per node block
+          for (int k = S.blk0 * sub; k < (S.blk0 + S.nblk) * sub; k++)
+            g.hmax = std::max(g.hmax, EL.hcnt[k]);
         }
         g.nblk = (int)bl.size();
         if (sv_alloc(E, (void **)&g.blist, I * bl.size()) ||

@@ -92,7 +92,8 @@ struct sv_physk {
 //   [ro, u, v, cxx, cxy, cyy, psixx, psixy, psiyy]  (LC: 10 doubles =  80 B)
 //   [ro, u, v, cxx, cxy, cyy]                        (DI:  6 doubles =  48 B)
 // packed (16-byte aligned, no padding to a cache line): a sweep's gathers of
-// Morton-neighbouring records then read whole lines of useful fields.
+// neighbouring records then read whole lines of useful fields.  Written whole,
+// pad included, so that lines reach memory complete.
 // State / register / error records: [ro, rou, rov, f1, f2, f3], 6 doubles
 // (48 B, packed), f = psi (LC) or c (DI).
 #define SV_GS_LC 10
@@ -116,12 +117,13 @@ void sv_adj_free(sv_ctx *c);
 // SV_BLOCK nodes, so every block of the node kernels lies in one member and
 // per-block partial reductions are per-member partial reductions.
 #define SV_BLOCK 256
-// LDS budget of a block's staged halo records (bytes); above it the sweeps
-// gather from global memory instead
-#define SV_HALO_LDS_MAX (60 * 1024)
+// LDS budget of a block's staged halo records (bytes)
+#define SV_HALO_LDS_MAX (64 * 1024)
 // LDS bytes of a staged halo record (log-conformation form; the direct form's
 // are smaller)
-#define SV_HALO_REC 72
+#define SV_HALO_REC 80
+// Halo records a block may have for the halo sweeps to be used at all
+#define SV_HALO_MAX 853
 struct sv_segk {
   int base;      // first node (concatenated numbering), a multiple of SV_BLOCK
   int npfb;      // real nodes
@@ -144,18 +146,26 @@ struct sv_loopl {
   int64_t nnz = 0;
   int64_t *off = nullptr;
   int *col = nullptr;
-  double *wx = nullptr, *wy = nullptr, *wl = nullptr, *wh = nullptr;
+  // weights of the sweeps by pairs of links (slices hold an even number), so
+  // that a lane reads 16 bytes at a time and a wavefront one sequential
+  // stream: w3 the stages' three per entry (sv_w3), wh the filter's (sv_pair)
+  double *w3 = nullptr, *wh = nullptr;
   int *cnt = nullptr, *cnt_small = nullptr;
+  // per slice, over its 64 slots: fewest and most links of the small lists (x,
+  // y) and of the full ones (z, w); with the halos
+  int4 *krange = nullptr;
   double *gsx = nullptr, *gsy = nullptr, *lsum = nullptr, *hsum = nullptr, *vol = nullptr;
   double *s = nullptr;
   int *perm = nullptr, *iperm = nullptr;
   std::vector<int> hperm;
   // Per-block neighbour halos: the distinct neighbour slots of the hb
-  // slots of block b are hidx[hoff[b] .. hoff[b+1]) (ascending); lcol[e] is
-  // the position of col[e] in its block's halo.  The sweeps stage a block's
+  // slots of block b are hidx[hoff[b] .. hoff[b+1]) (ascending); lcol[sv_pair(e)]
+  // is the position of col[e] in its block's halo.  The sweeps stage a block's
   // halo records in LDS once and read every link from there.
   bool halo = false;
-  int hb = SV_BLOCK;        // slots per halo block
+  int hb = SV_BLOCK;        // slots per halo block = threads per workgroup of
+                            // the sweeps: 64, 128 or 256
+  bool nt = false;          // weights loaded non-temporally
   int hmax = 0;             // largest halo of a block
   std::vector<int> hcnt;    // halo sizes
   int64_t *hoff = nullptr;  // [nblocks + 1]
@@ -169,6 +179,21 @@ struct sv_loopl {
   // only when the node set has symmetric / no-slip mirror ghosts
   uint8_t *lflip = nullptr;
 };
+
+// index of entry e (link k of its slice, lane l) in an array ordered by pairs of
+// links: the 64 lanes' entries of links 2p and 2p + 1 side by side
+__host__ __device__ __forceinline__ int64_t sv_pair(int64_t e) {
+  const int64_t l = e & (SV_WAVE - 1), b = (e / SV_WAVE) & 1;
+  return (e & ~(int64_t)(2 * SV_WAVE - 1)) + 2 * l + b;
+}
+// index in w3 of weight c (0 d/dx, 1 d/dy, 2 Laplacian) of entry e: per pair of
+// links the lanes' two gradient weights of the first, of the second, then the
+// lanes' Laplacian weights of both
+__host__ __device__ __forceinline__ int64_t sv_w3(int64_t e, int c) {
+  const int64_t l = e & (SV_WAVE - 1), b = (e / SV_WAVE) & 1;
+  const int64_t p = 3 * (e & ~(int64_t)(2 * SV_WAVE - 1)) + 2 * l;
+  return c < 2 ? p + 2 * SV_WAVE * b + c : p + 4 * SV_WAVE + b;
+}
 
 // Mirror ghosts (mirror_boundaries.F90:263-352): a link to a ghost of vrelation
 // 2 (x mirror) reads its parent's record with u and the conformation's xy
@@ -261,7 +286,7 @@ struct sv_ctx {
   bool is_ensemble = false;
   sv_adj *adj = nullptr;
   sv_loopl L;
-  int loop_order = 1;       // 1: Morton order for the time loop, 0: the caller's order
+  int loop_order = 1;       // 1: compact blocks for the time loop, 0: the caller's order
   int halo_sweeps = 1;      // 1: stage neighbour halos in LDS when they fit
   int adj_lanes = 0;        // lanes per node of the adjoint's transposed gathers
                             // (1, 4; 0: by node count), read by sv_adj_setup
@@ -345,6 +370,9 @@ int sv_dev_adapt(sv_ctx *c, int *reductions_host);
 int sv_dev_build_sell(sv_ctx *c);
 // time-loop layout from the final weights (after sums and filter coefficients)
 int sv_dev_build_loop(sv_ctx *c);
+// the halos of the layout in c->L over nslot slots (a context's own, or an
+// ensemble's concatenated one)
+int sv_dev_build_halos(sv_ctx *c, int nslot);
 int sv_ensure_loop(sv_ctx *c);
 // ---- kernels: weights (k_weights.hip) ----
 int sv_dev_weights(sv_ctx *c, const int *order_map_host);
@@ -379,6 +407,7 @@ int sv_dev_to_caller_order(sv_ctx *c, int nf, const double *in, double *out);
 // runtime, else an SV_E_ARG failure naming `what`
 int sv_check_device_ptr(sv_ctx *c, const void *p, const char *what);
 // ---- kernels: time stepping (k_step.hip) ----
+// gather records and set_tstep minima of the state in U (no correction)
 int sv_dev_init_state(sv_ctx *c);
 // one step; ev (nullable) gets SV_NKERNELS+1 events recorded between launches
 #define SV_NKERNELS 8
@@ -389,8 +418,6 @@ int sv_dev_rhs(sv_ctx *c, int iRKstep, double *out6, double *tapeG = nullptr,
 // ([ntot][SV_US]) and the derivative values to tape[2k+1] ([ntot][SV_TAPE_D])
 #define SV_TAPE_D 16
 int sv_dev_step_tape(sv_ctx *c, double *const tape[8]);
-// per-block partial minima of set_tstep for the current state (no correction)
-int sv_dev_init_partials(sv_ctx *c);
 // ensembles: time one launch against per-group launches, keep the faster
 int sv_dev_tune_groups(sv_ctx *c, int reps);
 // dst[k] += add for k < n (index rebasing when members are concatenated)
