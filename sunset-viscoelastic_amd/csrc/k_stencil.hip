@@ -13,39 +13,98 @@
 
 namespace {
 
+// Fields of one launch: the links' columns and weights are read once for all of
+// them.
+constexpr int AP_NF = 4;
 struct ApplyArgs {
   int npfb;
   const int64_t *off;
+  const int *width;         // links per slice, padding included
   const int *kcnt;          // links per node for this operator
   const int *col;
   const double *w0, *w1;
   const double *s0, *s1;    // weight sums
-  const double *phi;
-  double *o0, *o1;
+  const double *phi[AP_NF];
+  double *o0[AP_NF], *o1[AP_NF];
 };
 
+// One lane per node, one wavefront per workgroup, links in batches of AP_U:
+// every column and weight of a batch, then every gathered value, are requested
+// before the first sum.  A batch past a node's own list reads the slice's
+// padding (or its last link again) and leaves it out of the sums.
+// 511x513 order 6, three fields: gradients 315 us in three launches of one field
+// each, 152 so, Laplacians 200 and 122, filters 195 and 115 (the scattered reads
+// of phi, up to 64 lines a wave, are what is left).
+constexpr int AP_U = 4;
+template <int OP, int NF>
+__global__ __launch_bounds__(SV_WAVE) void k_apply(ApplyArgs a) {
+  constexpr bool GRAD = OP == SV_OP_GRAD;
+  const int s = sv_xcd_block();
+  const int i = s * SV_WAVE + (int)threadIdx.x;
+  const bool act = i < a.npfb;
+  const int64_t b = a.off[s] + threadIdx.x;
+  const int K = act ? a.kcnt[i] : 0, W = a.width[s];
+  double t0[NF], t1[NF];
+#pragma unroll
+  for (int f = 0; f < NF; f++) t0[f] = t1[f] = 0.0;
+  for (int k = 0; k < W; k += AP_U) {
+    int j[AP_U];
+    double w0[AP_U], w1[AP_U];
+#pragma unroll
+    for (int u = 0; u < AP_U; u++) {
+      const int64_t e = b + (int64_t)min(k + u, W - 1) * SV_WAVE;
+      j[u] = a.col[e];
+      w0[u] = a.w0[e];
+      if (GRAD) w1[u] = a.w1[e];
+    }
+    double p[AP_U][NF];
+#pragma unroll
+    for (int u = 0; u < AP_U; u++)
+#pragma unroll
+      for (int f = 0; f < NF; f++) p[u][f] = a.phi[f][j[u]];
+#pragma unroll
+    for (int u = 0; u < AP_U; u++)
+      if (k + u < K) {
+#pragma unroll
+        for (int f = 0; f < NF; f++) {
+          t0[f] = t0[f] + p[u][f] * w0[u];
+          if (GRAD) t1[f] = t1[f] + p[u][f] * w1[u];
+        }
+      }
+  }
+  if (!act) return;
+  const double s0 = a.s0[i], s1 = GRAD ? a.s1[i] : 0.0;
+#pragma unroll
+  for (int f = 0; f < NF; f++) {
+    const double pi = a.phi[f][i];
+    if (OP == SV_OP_FILTER) a.o0[f][i] = pi + (t0[f] - pi * s0);
+    else a.o0[f][i] = t0[f] - pi * s0;
+    if (GRAD) a.o1[f][i] = t1[f] - pi * s1;
+  }
+}
+
 template <int OP>
-__global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
-  const int i = sv_xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= a.npfb) return;
-  const int64_t b = a.off[i >> 6] + (i & 63);
-  const int K = a.kcnt[i];
-  double t0 = 0.0, t1 = 0.0;
-  for (int k = 0; k < K; k++) {
-    const int64_t e = b + (int64_t)k * SV_WAVE;
-    const double pj = a.phi[a.col[e]];
-    t0 = t0 + pj * a.w0[e];
-    if (OP == SV_OP_GRAD) t1 = t1 + pj * a.w1[e];
+void launch_apply(const ApplyArgs &a, int nf, int ns, hipStream_t st) {
+  switch (nf) {
+  case 1: k_apply<OP, 1><<<ns, SV_WAVE, 0, st>>>(a); break;
+  case 2: k_apply<OP, 2><<<ns, SV_WAVE, 0, st>>>(a); break;
+  case 3: k_apply<OP, 3><<<ns, SV_WAVE, 0, st>>>(a); break;
+  default: k_apply<OP, 4><<<ns, SV_WAVE, 0, st>>>(a); break;
   }
-  const double pi = a.phi[i];
-  if (OP == SV_OP_GRAD) {
-    a.o0[i] = t0 - pi * a.s0[i];
-    a.o1[i] = t1 - pi * a.s1[i];
-  } else if (OP == SV_OP_FILTER) {
-    a.o0[i] = pi + (t0 - pi * a.s0[i]);
-  } else {
-    a.o0[i] = t0 - pi * a.s0[i];
-  }
+}
+
+// Whether the fields of one call may share a launch: no output overlaps
+// another field's input or output (a call may chain fields, one's output the
+// next one's input, as the launches of the fields follow each other)
+bool fields_apart(int n, int nf, const double *const *phi, double *const *out, size_t nout) {
+  auto overlap = [](const double *p, size_t np, const double *q, size_t nq) {
+    return p < q + nq && q < p + np;
+  };
+  for (int f = 0; f < nf; f++)
+    for (int g = 0; g < nf; g++)
+      if (f != g && (overlap(out[f], nout, phi[g], n) || overlap(out[f], nout, out[g], nout)))
+        return false;
+  return true;
 }
 
 }  // namespace
@@ -87,15 +146,13 @@ int sv_dev_mass_correct(sv_ctx *c, double *ro, hipStream_t st) {
   return 0;
 }
 
-int sv_dev_apply(sv_ctx *c, int op, const double *phi, double *out, bool raw_cols,
-                 hipStream_t st) {
+int sv_dev_apply(sv_ctx *c, int op, int nfields, const double *const *phi, double *const *out,
+                 bool raw_cols, hipStream_t st) {
   ApplyArgs a{};
   a.npfb = c->npfb;
   a.off = c->sell_off;
+  a.width = c->sell_w;
   a.col = raw_cols ? c->scol_raw : c->scol;
-  a.phi = phi;
-  a.o0 = out;
-  a.o1 = out + c->npfb;
   switch (op) {
   case SV_OP_GRAD: a.kcnt = c->cnt_small; a.w0 = c->swx; a.w1 = c->swy; a.s0 = c->gsx; a.s1 = c->gsy; break;
   case SV_OP_LAP:
@@ -106,16 +163,30 @@ int sv_dev_apply(sv_ctx *c, int op, const double *phi, double *out, bool raw_col
   case SV_OP_FILTER_TERM: a.kcnt = c->cnt; a.w0 = c->swh; a.s0 = c->hsum; break;
   default: return sv_fail(c, SV_E_ARG, "unknown operator %d", op);
   }
-  const int B = 256, nb = (c->npfb + B - 1) / B;
-  switch (op) {
-  case SV_OP_GRAD: k_apply<SV_OP_GRAD><<<nb, B, 0, st>>>(a); break;
-  case SV_OP_FILTER: k_apply<SV_OP_FILTER><<<nb, B, 0, st>>>(a); break;
-  default: k_apply<SV_OP_LAP><<<nb, B, 0, st>>>(a); break;
+  const size_t nout = (op == SV_OP_GRAD ? 2 : 1) * (size_t)c->npfb;
+  const size_t nin = raw_cols ? c->np : c->npfb;
+  for (int f0 = 0; f0 < nfields;) {
+    int nf = nfields - f0 < AP_NF ? nfields - f0 : AP_NF;
+    if (!fields_apart(nin, nf, phi + f0, out + f0, nout)) nf = 1;
+    for (int f = 0; f < nf; f++) {
+      a.phi[f] = phi[f0 + f];
+      a.o0[f] = out[f0 + f];
+      a.o1[f] = out[f0 + f] + c->npfb;
+    }
+    switch (op) {
+    case SV_OP_GRAD: launch_apply<SV_OP_GRAD>(a, nf, c->nslices, st); break;
+    case SV_OP_FILTER: launch_apply<SV_OP_FILTER>(a, nf, c->nslices, st); break;
+    default: launch_apply<SV_OP_LAP>(a, nf, c->nslices, st); break;
+    }
+    SV_HIP(c, hipGetLastError());
+    // calc_laplacian_transverse_only_on_bound: the Laplacian on the internal
+    // nodes (derivatives.F90:315-325), the boundary nodes overwritten with the
+    // tangential part (:327-337)
+    if (op == SV_OP_LAP_TRANSVERSE)
+      for (int f = 0; f < nf; f++)
+        if (int rc = sv_dev_boundary_tt_apply(c, phi[f0 + f], out[f0 + f], raw_cols, st))
+          return rc;
+    f0 += nf;
   }
-  SV_HIP(c, hipGetLastError());
-  // calc_laplacian_transverse_only_on_bound: the Laplacian on the internal
-  // nodes (derivatives.F90:315-325), the boundary nodes overwritten with the
-  // tangential part (:327-337)
-  if (op == SV_OP_LAP_TRANSVERSE) return sv_dev_boundary_tt_apply(c, phi, out, raw_cols, st);
   return 0;
 }

@@ -509,7 +509,9 @@ int sv_apply(sv_ctx *c, int32_t op, double *phi, double *out) {
   if (int rc = ensure_sell(c)) return rc;
   if (int rc = ensure_tmp(c)) return rc;
   SV_HIP(c, hipMemcpy(c->tmp_phi, phi, sizeof(double) * c->np, hipMemcpyHostToDevice));
-  if (int rc = sv_dev_apply(c, op, c->tmp_phi, c->tmp_out, true, c->stream)) return rc;
+  const double *in[1] = {c->tmp_phi};
+  double *res[1] = {c->tmp_out};
+  if (int rc = sv_dev_apply(c, op, 1, in, res, true, c->stream)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));
   const size_t nout = (op == SV_OP_GRAD ? 2 : 1) * (size_t)c->npfb;
   SV_HIP(c, hipMemcpy(op == SV_OP_FILTER ? phi : out, c->tmp_out, sizeof(double) * nout,
@@ -551,9 +553,7 @@ int sv_apply_dev(sv_ctx *c, int32_t op, int32_t nfields, const double *const *ph
   // stream, which orders the launches with the caller's work there (a
   // framework's default stream is the null stream)
   hipStream_t st = (hipStream_t)stream;
-  for (int f = 0; f < nfields; f++)
-    if (int rc = sv_dev_apply(c, op, phi[f], out[f], false, st)) return rc;
-  return 0;
+  return sv_dev_apply(c, op, nfields, phi, out, false, st);
 }
 
 static void derive_phys(sv_ctx *c) {
@@ -844,14 +844,16 @@ int sv_filter_variables(sv_ctx *c, double *ro, double *rou, double *rov, double 
   SV_HIP(c, in.alloc(6 * (size_t)np));
   SV_HIP(c, out.alloc(6 * (size_t)n));
   double *f[6] = {ro, rou, rov, xx, xy, yy};
+  const double *fin[6];
+  double *fout[6];
   for (int k = 0; k < 6; k++) {
     SV_HIP(c, hipMemcpyAsync(in.p + (size_t)k * np, f[k], sizeof(double) * np,
                              hipMemcpyHostToDevice, c->stream));
-    // calc_filtered_var on the caller's ghost values (raw ghost columns)
-    if (int rc = sv_dev_apply(c, SV_OP_FILTER, in.p + (size_t)k * np, out.p + (size_t)k * n,
-                              true, c->stream))
-      return rc;
+    fin[k] = in.p + (size_t)k * np;
+    fout[k] = out.p + (size_t)k * n;
   }
+  // calc_filtered_var on the caller's ghost values (raw ghost columns)
+  if (int rc = sv_dev_apply(c, SV_OP_FILTER, 6, fin, fout, true, c->stream)) return rc;
   if (int rc = sv_dev_mass_correct(c, out.p, c->stream)) return rc;
   for (int k = 0; k < 6; k++)
     SV_HIP(c, hipMemcpyAsync(f[k], out.p + (size_t)k * n, sizeof(double) * n,

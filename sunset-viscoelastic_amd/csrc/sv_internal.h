@@ -390,8 +390,10 @@ int sv_dev_boundary_tt_sums(sv_ctx *c);
 int sv_dev_boundary_tt_apply(sv_ctx *c, const double *phi, double *out, bool raw_cols,
                              hipStream_t st);
 // ---- kernels: stencil operators (k_stencil.hip) ----
-int sv_dev_apply(sv_ctx *c, int op, const double *phi, double *out, bool raw_cols,
-                 hipStream_t st);
+// the operator on nfields fields, in their order (host arrays of device
+// pointers)
+int sv_dev_apply(sv_ctx *c, int op, int nfields, const double *const *phi, double *const *out,
+                 bool raw_cols, hipStream_t st);
 // ro (npfb, caller order) -= the volume-weighted mean deviation from 1
 int sv_dev_mass_correct(sv_ctx *c, double *ro, hipStream_t st);
 // caller-order device arrays (six of npfb, null entries read as 0 / skipped)
