@@ -993,114 +993,138 @@ __global__ __launch_bounds__(320, 1) void k_weights_big(SysArgs S_) {
   }
 }
 
-// The setup sums below run one thread per node over its CSR row, adding in
-// the reference's sequential order.  A block's rows are one contiguous range
-// of the CSR arrays (row_ptr is a prefix sum), which is staged through LDS in
-// coalesced chunks; each thread then adds the part of its row that lies in the
-// chunk.  Entries past cnt[i] (rows pruned after the lists were built) lie in
-// the range and are skipped by the per-row bounds.
-constexpr int SUM_B = 256;     // nodes (threads) per block
-constexpr int SUM_CH = 1024;   // CSR entries per staged chunk
+// The setup sums below take a group of consecutive rows per block: one
+// contiguous range of the CSR arrays (row_ptr is a prefix sum) of at most
+// SUM_E entries, staged in LDS by all threads; then one thread per row and
+// array adds its row in the reference's sequential order.  Entries past cnt[i]
+// (rows pruned after the lists were built) lie in the range and are skipped.
+// (With 256 rows per block streamed through 1024-entry chunks only the ~14
+// rows of a chunk had work: 240 us for the sums and 925 us for the filter
+// coefficients of 262k order-6 nodes; 212, at 5 TB/s, and 335 so;
+// 1581 -> 194 us on the 126k-node cylinder channel.)
+constexpr int SUM_B = 256;      // threads per block
+constexpr int SUM_E = 1024;     // CSR entries per block: sums, four arrays
+constexpr int FIL_E = 2048;     // filter coefficients, two arrays
+constexpr int SUM_R = 64;       // most rows per block
+
+// rows per block for lists of at most maxk links (SUM_E / maxk, at least 1;
+// longer lists than that are walked in pieces)
+inline int sum_rows(int maxk, int entries) {
+  return std::max(1, std::min(SUM_R, entries / std::max(maxk, 1)));
+}
 
 // calc_labf_sums (labf.F90:396-451): row sums of the four weight arrays, then
 // the gradient and Laplacian weights scaled by L_char (written back from the
-// staged chunk, so every CSR entry of the range is read and written once)
-__global__ __launch_bounds__(SUM_B) void k_sums(int npfb, const int64_t *row_ptr, const int *cnt,
-                                                double L, double *wx, double *wy, double *wl,
-                                                const double *wh, double *gsx, double *gsy,
-                                                double *lsum, double *hsum) {
-  __shared__ double cx[SUM_CH], cy[SUM_CH], cl[SUM_CH], ch[SUM_CH];
-  const int i0 = blockIdx.x * SUM_B;
-  const int i1 = min(i0 + SUM_B, npfb);
-  const int i = i0 + (int)threadIdx.x;
+// staged entries, so every CSR entry is read and written once)
+__global__ __launch_bounds__(SUM_B) void k_sums(int npfb, int rows, const int64_t *row_ptr,
+                                                const int *cnt, double L, double *wx, double *wy,
+                                                double *wl, const double *wh, double *gsx,
+                                                double *gsy, double *lsum, double *hsum) {
+  __shared__ double buf[4][SUM_E];
+  const int i0 = blockIdx.x * rows, i1 = min(i0 + rows, npfb);
   const int64_t R0 = row_ptr[i0], R1 = row_ptr[i1];
-  int64_t b = 0;
-  int K = 0;
-  if (i < npfb) { b = row_ptr[i]; K = cnt[i]; }
-  double sh = 0.0, sx = 0.0, sy = 0.0, sl = 0.0;
-  for (int64_t cs = R0; cs < R1; cs += SUM_CH) {
-    const int n = (int)min((int64_t)SUM_CH, R1 - cs);
-    for (int e = threadIdx.x; e < n; e += SUM_B) {
-      cx[e] = wx[cs + e]; cy[e] = wy[cs + e]; cl[e] = wl[cs + e]; ch[e] = wh[cs + e];
-    }
-    __syncthreads();
-    const int lo = (int)(max(b, cs) - cs);
-    const int hi = (int)(min(b + K, cs + n) - cs);
-    for (int e = lo; e < hi; e++) {
-      sh += ch[e];
-      sx += cx[e];
-      sy += cy[e];
-      sl += cl[e];
-    }
-    for (int e = threadIdx.x; e < n; e += SUM_B) {
-      wx[cs + e] = cx[e] / L;
-      wy[cs + e] = cy[e] / L;
-      wl[cs + e] = cl[e] / L / L;
-    }
-    __syncthreads();
-  }
-  if (i >= npfb) return;
-  hsum[i] = sh;
-  gsx[i] = sx / L;
-  gsy[i] = sy / L;
-  lsum[i] = sl / L / L;
-}
-
-// filter_coefficients (labf.F90:1723-1811).  Two passes over the block's
-// staged range: the first sums (test function) x w_hyp along each row, which
-// fixes the row's coefficient; the second scales the row by it, sums the
-// scaled weights and writes the chunk back.
-__global__ __launch_bounds__(SUM_B) void k_filter_coeffs(int npfb, const int64_t *row_ptr,
-                                                         const int *cnt, const int *col,
-                                                         const double *x, const double *y,
-                                                         const double *h, const double *s,
-                                                         const int *nt, int nb, double *wh,
-                                                         double *hsum) {
-  __shared__ double cw[SUM_CH];
-  __shared__ int cc[SUM_CH];
-  const int i0 = blockIdx.x * SUM_B;
-  const int i1 = min(i0 + SUM_B, npfb);
-  const int i = i0 + (int)threadIdx.x;
-  const int64_t R0 = row_ptr[i0], R1 = row_ptr[i1];
-  const bool act = i < npfb;
+  // wave q sums array q (x, y, Laplacian, filter), lane r row i0 + r
+  const int q = threadIdx.x / SV_WAVE, i = i0 + (int)(threadIdx.x % SV_WAVE);
+  const bool act = i < i1;
   int64_t b = 0;
   int K = 0;
   if (act) { b = row_ptr[i]; K = cnt[i]; }
-  const int t = (act && nb > 0) ? nt[i] : 999;
-  // boundary nodes filter along the boundary only: radial test function,
-  // length scale s (:1770-1792); the others the product test function with
-  // length scale 2 h sqrt(pi / K) (:1738-1755)
-  const bool radial = t >= 0 && t <= 2;
-  double tmp = 0.0, xi = 0.0, yi = 0.0;
-  if (act) {
-    xi = x[i];
-    yi = y[i];
-    if (radial) {
-      tmp = (2.0 / 3.0) * SV_PI / s[i];
-    } else {
-      const double lscal = 2.0 * h[i] * sqrt(SV_PI / (double)K);
-      tmp = (2.0 / 3.0) * SV_PI / lscal;
+  double sum = 0.0;
+  for (int64_t cs = R0; cs < R1; cs += SUM_E) {   // once, unless a list is longer than SUM_E
+    const int n = (int)min((int64_t)SUM_E, R1 - cs);
+    for (int e = threadIdx.x; e < n; e += SUM_B) {
+      const double x = wx[cs + e], y = wy[cs + e], l = wl[cs + e];
+      buf[0][e] = x; buf[1][e] = y; buf[2][e] = l; buf[3][e] = wh[cs + e];
+      wx[cs + e] = x / L;
+      wy[cs + e] = y / L;
+      wl[cs + e] = l / L / L;
     }
-  }
-  double ls = 0.0;
-  for (int64_t cs = R0; cs < R1; cs += SUM_CH) {
-    const int n = (int)min((int64_t)SUM_CH, R1 - cs);
-    for (int e = threadIdx.x; e < n; e += SUM_B) { cw[e] = wh[cs + e]; cc[e] = col[cs + e]; }
     __syncthreads();
     const int lo = (int)(max(b, cs) - cs);
     const int hi = (int)(min(b + K, cs + n) - cs);
-    for (int e = lo; e < hi; e++) {
-      const int j = cc[e];
-      const double dx = x[j] - xi, dy = y[j] - yi;
-      const double f = radial ? 1.0 - cos(tmp * sqrt(dx * dx + dy * dy))
-                              : 1.0 - cos(tmp * dx) * cos(tmp * dy);
-      ls = ls + f * cw[e];
-    }
+    for (int e = lo; e < hi; e++) sum += buf[q][e];
     __syncthreads();
   }
-  double fc = 0.0;
+  if (!act) return;
+  if (q == 0) gsx[i] = sum / L;
+  else if (q == 1) gsy[i] = sum / L;
+  else if (q == 2) lsum[i] = sum / L / L;
+  else hsum[i] = sum;
+}
+
+// filter_coefficients (labf.F90:1723-1811).  Every entry's (test function) x
+// w_hyp is evaluated by its own thread (two cosines, the bulk of the work),
+// the rows' sums of them fix the rows' coefficients, every entry is scaled by
+// its row's and written back, and the rows' scaled weights are summed.
+__global__ __launch_bounds__(SUM_B) void k_filter_coeffs(int npfb, int rows,
+                                                         const int64_t *row_ptr, const int *cnt,
+                                                         const int *col, const double *x,
+                                                         const double *y, const double *h,
+                                                         const double *s, const int *nt, int nb,
+                                                         double *wh, double *hsum) {
+  __shared__ double tf[FIL_E], tw[FIL_E];   // test function, weight
+  __shared__ int64_t rp[SUM_R + 1];
+  __shared__ double rx[SUM_R], ry[SUM_R], rtmp[SUM_R], rfc[SUM_R];
+  __shared__ int rK[SUM_R], rrad[SUM_R];
+  const int i0 = blockIdx.x * rows, i1 = min(i0 + rows, npfb), nr = i1 - i0;
+  const int tx = threadIdx.x, i = i0 + tx;
+  const bool act = tx < nr;
+  int t = 999;
+  if (tx <= nr) rp[tx] = row_ptr[i];
   if (act) {
+    const int K = cnt[i];
+    if (nb > 0) t = nt[i];
+    // boundary nodes filter along the boundary only: radial test function,
+    // length scale s (:1770-1792); the others the product test function with
+    // length scale 2 h sqrt(pi / K) (:1738-1755)
+    const bool radial = t >= 0 && t <= 2;
     if (radial) {
+      rtmp[tx] = (2.0 / 3.0) * SV_PI / s[i];
+    } else {
+      const double lscal = 2.0 * h[i] * sqrt(SV_PI / (double)K);
+      rtmp[tx] = (2.0 / 3.0) * SV_PI / lscal;
+    }
+    rx[tx] = x[i];
+    ry[tx] = y[i];
+    rK[tx] = K;
+    rrad[tx] = radial;
+  }
+  __syncthreads();
+  const int64_t R0 = rp[0], R1 = rp[nr];
+  // the row of entry e: rp[r] <= e < rp[r + 1]
+  auto row_of = [&](int64_t e) {
+    int lo = 0, hi = nr;
+    while (hi - lo > 1) {
+      const int m = (lo + hi) >> 1;
+      if (rp[m] <= e) lo = m;
+      else hi = m;
+    }
+    return lo;
+  };
+  const int64_t b = act ? rp[tx] : 0;
+  const int K = act ? rK[tx] : 0;
+  double ls = 0.0;
+  for (int64_t cs = R0; cs < R1; cs += FIL_E) {   // once, unless a list is longer than FIL_E
+    const int n = (int)min((int64_t)FIL_E, R1 - cs);
+    for (int e = tx; e < n; e += SUM_B) {
+      const int r = row_of(cs + e);
+      if (cs + e - rp[r] >= rK[r]) continue;
+      const int j = col[cs + e];
+      const double dx = x[j] - rx[r], dy = y[j] - ry[r], tmp = rtmp[r];
+      const double f = rrad[r] ? 1.0 - cos(tmp * sqrt(dx * dx + dy * dy))
+                               : 1.0 - cos(tmp * dx) * cos(tmp * dy);
+      tf[e] = f;
+      tw[e] = wh[cs + e];
+    }
+    __syncthreads();
+    const int lo = (int)(max(b, cs) - cs);
+    const int hi = (int)(min(b + K, cs + n) - cs);
+    for (int e = lo; e < hi; e++) ls = ls + tf[e] * tw[e];
+    __syncthreads();
+  }
+  if (act) {
+    double fc;
+    if (rrad[tx]) {
       fc = (1.0 / 3.0) / ls;
       fc = fc * 0.5;
     } else {
@@ -1114,21 +1138,27 @@ __global__ __launch_bounds__(SUM_B) void k_filter_coeffs(int npfb, const int64_t
         if (t == -4) fc = fc * oosqrt2;
       }
     }
+    rfc[tx] = fc;
   }
+  __syncthreads();
+  const double fc = act ? rfc[tx] : 0.0;
+  const bool once = R1 - R0 <= FIL_E;   // the weights are still in tw
   double hs = 0.0;
-  for (int64_t cs = R0; cs < R1; cs += SUM_CH) {
-    const int n = (int)min((int64_t)SUM_CH, R1 - cs);
-    for (int e = threadIdx.x; e < n; e += SUM_B) cw[e] = wh[cs + e];
+  for (int64_t cs = R0; cs < R1; cs += FIL_E) {
+    const int n = (int)min((int64_t)FIL_E, R1 - cs);
+    for (int e = tx; e < n; e += SUM_B) {
+      const int r = row_of(cs + e);
+      if (cs + e - rp[r] >= rK[r]) continue;
+      if (!once) tw[e] = wh[cs + e];
+      wh[cs + e] = tw[e] * rfc[r];
+    }
     __syncthreads();
     const int lo = (int)(max(b, cs) - cs);
     const int hi = (int)(min(b + K, cs + n) - cs);
     for (int e = lo; e < hi; e++) {
-      const double w = cw[e] * fc;
-      cw[e] = w;
+      const double w = tw[e] * fc;
       hs = hs + w;
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < n; e += SUM_B) wh[cs + e] = cw[e];
     __syncthreads();
   }
   if (act) hsum[i] = hs;
@@ -1516,9 +1546,10 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
 }
 
 int sv_dev_sums(sv_ctx *c) {
-  const int n = c->npfb, B = SUM_B;
-  k_sums<<<(n + B - 1) / B, B, 0, c->stream>>>(n, c->row_ptr, c->cnt, c->L_char, c->wx, c->wy,
-                                               c->wl, c->wh, c->gsx, c->gsy, c->lsum, c->hsum);
+  const int n = c->npfb, R = sum_rows(c->maxK, SUM_E);
+  k_sums<<<(n + R - 1) / R, SUM_B, 0, c->stream>>>(n, R, c->row_ptr, c->cnt, c->L_char, c->wx,
+                                                   c->wy, c->wl, c->wh, c->gsx, c->gsy, c->lsum,
+                                                   c->hsum);
   SV_HIP(c, hipGetLastError());
   if (int rc = sv_dev_boundary_tt_sums(c)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));
@@ -1529,10 +1560,10 @@ int sv_dev_sums(sv_ctx *c) {
 }
 
 int sv_dev_filter_coeffs(sv_ctx *c) {
-  const int n = c->npfb, B = SUM_B;
-  k_filter_coeffs<<<(n + B - 1) / B, B, 0, c->stream>>>(n, c->row_ptr, c->cnt, c->col_raw, c->x,
-                                                        c->y, c->h, c->s, c->node_type, c->nb,
-                                                        c->wh, c->hsum);
+  const int n = c->npfb, R = sum_rows(c->maxK, FIL_E);
+  k_filter_coeffs<<<(n + R - 1) / R, SUM_B, 0, c->stream>>>(n, R, c->row_ptr, c->cnt, c->col_raw,
+                                                            c->x, c->y, c->h, c->s, c->node_type,
+                                                            c->nb, c->wh, c->hsum);
   SV_HIP(c, hipGetLastError());
   SV_HIP(c, hipStreamSynchronize(c->stream));
   c->have_filter = true;
