@@ -170,7 +170,7 @@ int sv_get_weights(sv_ctx *ctx, int32_t nplink, double *ij_w_grad, double *ij_w_
  * "weights_tune_m<order>_<variant>" the autotuning sample time of a variant. */
 int sv_get_timing(sv_ctx *ctx, const char *what, double *ms);
 /* Tuning switches:
- *   "weights_autotune" (default 1): for an order with >= 16384 systems, the
+ *   "weights_autotune" (default 1): for an order with >= 409600 systems, the
  *       first sv_calc_labf_weights times the four launch variants (one block
  *       per system or a persistent grid fed from a work queue, times assembly
  *       tiles of 16 or 32 neighbours) on a strided 4096-system sample and uses

@@ -26,6 +26,8 @@
 // stencil), and then share the factorisation (4 right-hand sides).
 #include <algorithm>
 
+#include <hipcub/hipcub.hpp>
+
 #include "sv_internal.h"
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
@@ -1004,7 +1006,8 @@ __global__ __launch_bounds__(320, 1) void k_weights_big(SysArgs S_) {
 // 1581 -> 194 us on the 126k-node cylinder channel.)
 constexpr int SUM_B = 256;      // threads per block
 constexpr int SUM_E = 1024;     // CSR entries per block: sums, four arrays
-constexpr int FIL_E = 2048;     // filter coefficients, two arrays
+constexpr int FIL_E = 2048;     // filter coefficients, two arrays; no list is longer: the
+                                // neighbour search sorts at most 1365 candidates in LDS
 constexpr int SUM_R = 64;       // most rows per block
 
 // rows per block for lists of at most maxk links (SUM_E / maxk, at least 1;
@@ -1101,27 +1104,21 @@ __global__ __launch_bounds__(SUM_B) void k_filter_coeffs(int npfb, int rows,
     }
     return lo;
   };
-  const int64_t b = act ? rp[tx] : 0;
-  const int K = act ? rK[tx] : 0;
-  double ls = 0.0;
-  for (int64_t cs = R0; cs < R1; cs += FIL_E) {   // once, unless a list is longer than FIL_E
-    const int n = (int)min((int64_t)FIL_E, R1 - cs);
-    for (int e = tx; e < n; e += SUM_B) {
-      const int r = row_of(cs + e);
-      if (cs + e - rp[r] >= rK[r]) continue;
-      const int j = col[cs + e];
-      const double dx = x[j] - rx[r], dy = y[j] - ry[r], tmp = rtmp[r];
-      const double f = rrad[r] ? 1.0 - cos(tmp * sqrt(dx * dx + dy * dy))
-                               : 1.0 - cos(tmp * dx) * cos(tmp * dy);
-      tf[e] = f;
-      tw[e] = wh[cs + e];
-    }
-    __syncthreads();
-    const int lo = (int)(max(b, cs) - cs);
-    const int hi = (int)(min(b + K, cs + n) - cs);
-    for (int e = lo; e < hi; e++) ls = ls + tf[e] * tw[e];
-    __syncthreads();
+  const int n = (int)(R1 - R0);   // <= rows * (most links of a list) <= FIL_E
+  for (int e = tx; e < n; e += SUM_B) {
+    const int r = row_of(R0 + e);
+    if (R0 + e - rp[r] >= rK[r]) continue;
+    const int j = col[R0 + e];
+    const double dx = x[j] - rx[r], dy = y[j] - ry[r], tmp = rtmp[r];
+    const double f = rrad[r] ? 1.0 - cos(tmp * sqrt(dx * dx + dy * dy))
+                             : 1.0 - cos(tmp * dx) * cos(tmp * dy);
+    tf[e] = f;
+    tw[e] = wh[R0 + e];
   }
+  __syncthreads();
+  const int lo = act ? (int)(rp[tx] - R0) : 0, hi = act ? lo + rK[tx] : 0;
+  double ls = 0.0;
+  for (int e = lo; e < hi; e++) ls = ls + tf[e] * tw[e];
   if (act) {
     double fc;
     if (rrad[tx]) {
@@ -1141,31 +1138,98 @@ __global__ __launch_bounds__(SUM_B) void k_filter_coeffs(int npfb, int rows,
     rfc[tx] = fc;
   }
   __syncthreads();
-  const double fc = act ? rfc[tx] : 0.0;
-  const bool once = R1 - R0 <= FIL_E;   // the weights are still in tw
-  double hs = 0.0;
-  for (int64_t cs = R0; cs < R1; cs += FIL_E) {
-    const int n = (int)min((int64_t)FIL_E, R1 - cs);
-    for (int e = tx; e < n; e += SUM_B) {
-      const int r = row_of(cs + e);
-      if (cs + e - rp[r] >= rK[r]) continue;
-      if (!once) tw[e] = wh[cs + e];
-      wh[cs + e] = tw[e] * rfc[r];
-    }
-    __syncthreads();
-    const int lo = (int)(max(b, cs) - cs);
-    const int hi = (int)(min(b + K, cs + n) - cs);
-    for (int e = lo; e < hi; e++) {
-      const double w = tw[e] * fc;
-      hs = hs + w;
-    }
-    __syncthreads();
+  for (int e = tx; e < n; e += SUM_B) {
+    const int r = row_of(R0 + e);
+    if (R0 + e - rp[r] >= rK[r]) continue;
+    wh[R0 + e] = tw[e] * rfc[r];
   }
-  if (act) hsum[i] = hs;
+  if (!act) return;
+  const double fc = rfc[tx];
+  double hs = 0.0;
+  for (int e = lo; e < hi; e++) {
+    const double w = tw[e] * fc;
+    hs = hs + w;
+  }
+  hsum[i] = hs;
 }
 
 #define SV_TUNE_SAMPLE 4096
 #define SV_TUNE_VARIANTS 4
+// The autotuner runs from this many systems of an order on: its fourteen
+// sample launches cost as much as ~75,000 systems (3.0 of the 8 ms of solving
+// 126k order-8 systems), and every launch shape gives the same weights.
+#define SV_TUNE_MIN (100 * SV_TUNE_SAMPLE)
+
+// ---- the systems of a call, listed on the device -------------------------
+// The systems of node i: both operators in one where the two coincide, or a
+// derivative and a filter system, or the filter's alone (FD rows 1 and 2,
+// whose derivative weights calc_boundary_weights makes), or none (boundary
+// nodes, which are not on internal_list: labf.F90:82, :268).
+struct NodeSys {
+  int n, m[2], K[2], kind[2];
+};
+struct SysList {
+  int n, morder, forder, nb, maxk;
+  const int *order_map;   // or null
+  const int *cnt, *cnt_small, *node_type;
+  const double *h, *hs;
+};
+__device__ __forceinline__ NodeSys node_systems(const SysList &a, int i) {
+  NodeSys s;
+  const int md = a.order_map ? a.order_map[i] : a.morder;
+  const int mf = a.order_map ? a.order_map[i] : a.forder;
+  const int t = a.nb > 0 ? a.node_type[i] : 999;
+  const int K = a.cnt[i], Ks = a.cnt_small[i];
+  if (t >= 0 && t <= 2) {
+    s.n = 0;
+  } else if (t == -1 || t == -2) {
+    s.n = 1; s.m[0] = mf; s.K[0] = K; s.kind[0] = SYS_F;
+  } else if (md == mf && a.h[i] == a.hs[i] && K == Ks) {
+    s.n = 1; s.m[0] = md; s.K[0] = K; s.kind[0] = SYS_D | SYS_F;
+  } else {
+    s.n = 2;
+    s.m[0] = md; s.K[0] = Ks; s.kind[0] = SYS_D;
+    s.m[1] = mf; s.K[1] = K; s.kind[1] = SYS_F;
+  }
+  return s;
+}
+
+__global__ void k_sys_count(SysList a, int *num) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= a.n) num[i] = i < a.n ? node_systems(a, i).n : 0;
+}
+
+// key: by order, then by decreasing stencil length (equal ones by node: the
+// sort is stable)
+__global__ void k_sys_emit(SysList a, const int *first, uint32_t *key, uint32_t *val) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const NodeSys s = node_systems(a, i);
+  for (int q = 0; q < s.n; q++) {
+    key[first[i] + q] = (uint32_t)((s.m[q] / 2 - 2) * (a.maxk + 1) + (a.maxk - s.K[q]));
+    val[first[i] + q] = (uint32_t)i << 2 | (uint32_t)s.kind[q];
+  }
+}
+
+// nodes and kinds of the sorted list, and where each order's systems begin
+__global__ void k_sys_split(int n, int maxk, const uint32_t *key, const uint32_t *val, int *node,
+                            int *kind, int *begin) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  node[s] = (int)(val[s] >> 2);
+  kind[s] = (int)(val[s] & 3u);
+  const int o = (int)(key[s] / (uint32_t)(maxk + 1));
+  if (s == 0 || (int)(key[s - 1] / (uint32_t)(maxk + 1)) != o) begin[o] = s;
+}
+
+// every stride-th system
+__global__ void k_sys_sample(int n, int stride, const int *node, const int *kind, int *sn,
+                             int *sk) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  sn[q] = node[q * stride];
+  sk[q] = kind[q * stride];
+}
 
 // systems per wavefront of order m (Pack<m>::G)
 int pack_of(int m) { return m == 8 ? Pack<8>::G : m == 6 ? Pack<6>::G : Pack<4>::G; }
@@ -1269,60 +1333,62 @@ int launch_mixed(sv_ctx *c, SysArgs a, int count, int mmax, int mode) {
 // Build the system lists (one per order), launch, and check for zero pivots.
 int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   const int n = c->npfb;
-  std::vector<int> cnt(n), cs(n);
-  std::vector<double> h(n), hs(n);
-  const std::vector<int> &nt = c->hnt;
-  SV_HIP(c, hipMemcpy(cnt.data(), c->cnt, sizeof(int) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(cs.data(), c->cnt_small, sizeof(int) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(h.data(), c->h, sizeof(double) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(hs.data(), c->hs, sizeof(double) * n, hipMemcpyDeviceToHost));
-  // systems grouped by order: entries (order, K, node, kind)
-  struct Sys { int m, K, node, kind; };
-  std::vector<Sys> sys;
-  sys.reserve(2 * (size_t)n);
   for (int i = 0; i < n; i++) {
     const int md = order_map_host ? order_map_host[i] : c->cfg.morder;
     const int mf = order_map_host ? order_map_host[i] : c->cfg.forder;
     for (int m : {md, mf})
       if (!sv_order_supported(m))
         return sv_fail(c, SV_E_ARG, "LABFM order %d not supported on the device (4, 6, 8, 10)", m);
-    // boundary nodes are not on internal_list (labf.F90:82, :268): their
-    // operators come from calc_boundary_weights, which also replaces the
-    // derivative weights of FD rows 1 and 2 (only their filter system is kept)
-    if (c->nb > 0 && nt[i] >= 0 && nt[i] <= 2) continue;
-    if (c->nb > 0 && (nt[i] == -1 || nt[i] == -2)) {
-      sys.push_back({mf, cnt[i], i, SYS_F});
-      continue;
-    }
-    if (md == mf && h[i] == hs[i] && cnt[i] == cs[i]) {
-      sys.push_back({md, cnt[i], i, SYS_D | SYS_F});
-    } else {
-      sys.push_back({md, cs[i], i, SYS_D});
-      sys.push_back({mf, cnt[i], i, SYS_F});
-    }
+    if (!order_map_host) break;
   }
-  // by order, then by decreasing stencil length, stable: a counting sort over
-  // the (order, length) keys gives the order of a stable comparison sort
-  {
-    int kmax = 0;
-    for (const Sys &e : sys) kmax = std::max(kmax, e.K);
-    const int nk = kmax + 1;
-    auto key = [&](const Sys &e) { return (e.m / 2 - 2) * nk + (kmax - e.K); };
-    std::vector<int64_t> start((size_t)4 * nk + 1, 0);
-    for (const Sys &e : sys) start[key(e) + 1]++;
-    for (size_t q = 1; q < start.size(); q++) start[q] += start[q - 1];
-    std::vector<Sys> sorted(sys.size());
-    for (const Sys &e : sys) sorted[start[key(e)]++] = e;
-    sys.swap(sorted);
+  // the systems on the device, by order and then by decreasing stencil length
+  DevTmp<int> dn, dk, dq, dmap, num, first;
+  DevTmp<uint32_t> keys, vals;
+  DevTmp<char> tmp;
+  const size_t N2 = 2 * (size_t)n;
+  SV_HIP(c, dn.alloc(N2 + 1));
+  SV_HIP(c, dk.alloc(N2 + 1));
+  SV_HIP(c, dq.alloc(8));
+  SV_HIP(c, num.alloc((size_t)n + 1));
+  SV_HIP(c, first.alloc((size_t)n + 1));
+  SV_HIP(c, keys.alloc(2 * N2));
+  SV_HIP(c, vals.alloc(2 * N2));
+  SysList sl_{n, c->cfg.morder, c->cfg.forder, c->nb, c->maxK, nullptr, c->cnt, c->cnt_small,
+              c->node_type, c->h, c->hs};
+  if (order_map_host) {
+    SV_HIP(c, dmap.alloc(n));
+    SV_HIP(c, hipMemcpyAsync(dmap.p, order_map_host, sizeof(int) * n, hipMemcpyHostToDevice,
+                             c->stream));
+    sl_.order_map = dmap.p;
   }
-  std::vector<int> hn(sys.size()), hk(sys.size());
-  for (size_t s = 0; s < sys.size(); s++) { hn[s] = sys[s].node; hk[s] = sys[s].kind; }
-  DevTmp<int> dn, dk, dq;
-  SV_HIP(c, dn.alloc(sys.size() + 1));
-  SV_HIP(c, dk.alloc(sys.size() + 1));
-  SV_HIP(c, dq.alloc(4));
-  SV_HIP(c, hipMemcpy(dn, hn.data(), sizeof(int) * sys.size(), hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(dk, hk.data(), sizeof(int) * sys.size(), hipMemcpyHostToDevice));
+  hipcub::DoubleBuffer<uint32_t> kb(keys.p, keys.p + N2), vb(vals.p, vals.p + N2);
+  int bits = 1;
+  while (4ll * (c->maxK + 1) > (1ll << bits)) bits++;
+  size_t tb1 = 0, tb2 = 0;
+  SV_HIP(c, hipcub::DeviceScan::ExclusiveSum(nullptr, tb1, num.p, first.p, n + 1, c->stream));
+  SV_HIP(c, hipcub::DeviceRadixSort::SortPairs(nullptr, tb2, kb, vb, (int)N2, 0, bits, c->stream));
+  size_t tb = std::max(tb1, tb2);
+  SV_HIP(c, tmp.alloc(tb > 0 ? tb : 16));
+  const int TB = 256;
+  SV_HIP(c, hipMemsetAsync(dq.p, 0xff, sizeof(int) * 8, c->stream));
+  k_sys_count<<<(n + TB) / TB, TB, 0, c->stream>>>(sl_, num);
+  SV_HIP(c, hipGetLastError());
+  SV_HIP(c, hipcub::DeviceScan::ExclusiveSum((void *)tmp, tb, num.p, first.p, n + 1, c->stream));
+  int nsys = 0;
+  SV_HIP(c, hipMemcpyAsync(&nsys, first.p + n, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  SV_HIP(c, hipStreamSynchronize(c->stream));
+  int begin[4] = {-1, -1, -1, -1};   // of orders 4, 6, 8, 10
+  if (nsys > 0) {
+    k_sys_emit<<<(n + TB - 1) / TB, TB, 0, c->stream>>>(sl_, first, kb.Current(), vb.Current());
+    SV_HIP(c, hipGetLastError());
+    SV_HIP(c, hipcub::DeviceRadixSort::SortPairs((void *)tmp, tb, kb, vb, nsys, 0, bits,
+                                                 c->stream));
+    k_sys_split<<<(nsys + TB - 1) / TB, TB, 0, c->stream>>>(nsys, c->maxK, kb.Current(),
+                                                            vb.Current(), dn, dk, dq.p + 4);
+    SV_HIP(c, hipGetLastError());
+    SV_HIP(c, hipMemcpyAsync(begin, dq.p + 4, sizeof(begin), hipMemcpyDeviceToHost, c->stream));
+    SV_HIP(c, hipStreamSynchronize(c->stream));
+  }
   const size_t L = (size_t)c->nnz + 1;
   if (!c->wx) {
     if (sv_alloc(c, (void **)&c->wx, sizeof(double) * L) ||
@@ -1342,7 +1408,7 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   SV_HIP(c, hipMemsetAsync(c->wl, 0, sizeof(double) * L, c->stream));
   SV_HIP(c, hipMemsetAsync(c->wh, 0, sizeof(double) * L, c->stream));
   SV_HIP(c, hipMemsetAsync(c->singular, 0, sizeof(int) * 4, c->stream));
-  SysArgs a{dn, dk, (int)sys.size(), c->x, c->y, c->h, c->hs, c->node_type, c->row_ptr,
+  SysArgs a{dn, dk, nsys, c->x, c->y, c->h, c->hs, c->node_type, c->row_ptr,
             c->col_raw, c->cnt, c->cnt_small, c->h2, c->wx, c->wy, c->wl, c->wh, c->vol,
             c->singular, dq, nullptr, nullptr, 0};
   EventTmp e0, e1, t0, t1;
@@ -1374,14 +1440,14 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   struct Slice { int m, first, count; };
   std::vector<Slice> slices;
   bool has_big = false;
-  for (int m : {4, 6, 8, 10}) {
-    int f = 0;
-    while (f < (int)sys.size() && sys[f].m != m) f++;
-    int cnt = 0;
-    while (f + cnt < (int)sys.size() && sys[f + cnt].m == m) cnt++;
-    if (cnt) slices.push_back({m, f, cnt});
-    if (cnt && m > 8) has_big = true;
-  }
+  for (int o = 0; o < 4; o++)
+    if (begin[o] >= 0) {
+      int end = nsys;
+      for (int p = o + 1; p < 4; p++)
+        if (begin[p] >= 0) { end = begin[p]; break; }
+      slices.push_back({4 + 2 * o, begin[o], end - begin[o]});
+      if (o == 3) has_big = true;
+    }
   const int S = SV_TUNE_SAMPLE;
   // 1. per order: the launch variant (grid kind x assembly tile), timed on a
   //    strided sample of that order's systems (sorted by stencil length, so
@@ -1390,18 +1456,14 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   for (const Slice &sl : slices) {
     if (sl.m > 8) continue;   // one launch shape
     const int mi = sl.m / 2 - 2;
-    if (!c->weights_autotune || sl.count < 4 * S || c->wtune[mi] >= 0) continue;
+    if (!c->weights_autotune || sl.count < SV_TUNE_MIN || c->wtune[mi] >= 0) continue;
     const int stride = sl.count / S;
-    std::vector<int> sn(S), sk(S);
-    for (int q = 0; q < S; q++) {
-      sn[q] = hn[sl.first + q * stride];
-      sk[q] = hk[sl.first + q * stride];
-    }
     DevTmp<int> tn, tk;
     SV_HIP(c, tn.alloc(S));
     SV_HIP(c, tk.alloc(S));
-    SV_HIP(c, hipMemcpy(tn, sn.data(), sizeof(int) * S, hipMemcpyHostToDevice));
-    SV_HIP(c, hipMemcpy(tk, sk.data(), sizeof(int) * S, hipMemcpyHostToDevice));
+    k_sys_sample<<<(S + TB - 1) / TB, TB, 0, c->stream>>>(S, stride, dn.p + sl.first,
+                                                          dk.p + sl.first, tn, tk);
+    SV_HIP(c, hipGetLastError());
     SysArgs ts = a;
     ts.sys_node = tn;
     ts.sys_kind = tk;
@@ -1417,38 +1479,51 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   auto order_variant = [&](int m) {
     if (m > 8) return 0;
     const int mi = m / 2 - 2;
-    return (c->weights_autotune && c->wtune[mi] >= 0) ? c->wtune[mi] : c->weights_fixed;
+    if (!c->weights_autotune) return c->weights_fixed;
+    // untuned (few systems): one block per system; 32-neighbour tiles except at
+    // order 8 (a 4096-system sample 0.234 ms, 0.205 with 16)
+    return c->wtune[mi] >= 0 ? c->wtune[mi] : m == 8 ? 0 : 2;
   };
   // 2. several orders: one persistent launch over all of them (queue order 8
   //    first) against the per-order launches, on a strided sample of that queue
   int mode = c->weights_autotune ? 0 : c->weights_mixed;
-  std::vector<int> qn, qk, qm;   // the mixed queue
+  std::vector<int> qm;           // the mixed queue: orders, longest lists first
+  DevTmp<int> mn, mk;            // its nodes and kinds
+  // the queue: the orders' slices, highest order first
+  auto make_queue = [&]() -> int {
+    SV_HIP(c, mn.alloc(nsys));
+    SV_HIP(c, mk.alloc(nsys));
+    int at = 0;
+    for (auto it = slices.rbegin(); it != slices.rend(); ++it) {
+      const size_t b = sizeof(int) * it->count;
+      SV_HIP(c, hipMemcpyAsync(mn.p + at, dn.p + it->first, b, hipMemcpyDeviceToDevice, c->stream));
+      SV_HIP(c, hipMemcpyAsync(mk.p + at, dk.p + it->first, b, hipMemcpyDeviceToDevice, c->stream));
+      at += it->count;
+    }
+    return 0;
+  };
   if (has_big) {
     mode = 0;   // the mixed launch covers orders 4-8
   } else if (slices.size() >= 2) {
-    for (auto it = slices.rbegin(); it != slices.rend(); ++it)
-      for (int q = it->first; q < it->first + it->count; q++) {
-        qn.push_back(hn[q]);
-        qk.push_back(hk[q]);
-        qm.push_back(it->m);
-      }
-    const int total = (int)qn.size();
-    if (c->weights_autotune && total >= 4 * S && c->wmixed < 0) {
+    const int total = nsys;
+    const bool tune = c->weights_autotune && total >= SV_TUNE_MIN && c->wmixed < 0;
+    if (tune || (c->weights_autotune ? c->wmixed > 0 : mode > 0)) {
+      if (int rc = make_queue()) return rc;
+      for (auto it = slices.rbegin(); it != slices.rend(); ++it)
+        qm.insert(qm.end(), it->count, it->m);
+    }
+    if (tune) {
       const int stride = total / S;
-      std::vector<int> sn(S), sk(S), sm(S);
-      for (int q = 0; q < S; q++) {
-        sn[q] = qn[q * stride];
-        sk[q] = qk[q * stride];
-        sm[q] = qm[q * stride];
-      }
+      std::vector<int> sm(S);
+      for (int q = 0; q < S; q++) sm[q] = qm[q * stride];
       const std::vector<int> su = units_of(sm);
       DevTmp<int> tn, tk, tm, tu;
       SV_HIP(c, tn.alloc(S));
       SV_HIP(c, tk.alloc(S));
       SV_HIP(c, tm.alloc(S));
       SV_HIP(c, tu.alloc(su.size()));
-      SV_HIP(c, hipMemcpy(tn, sn.data(), sizeof(int) * S, hipMemcpyHostToDevice));
-      SV_HIP(c, hipMemcpy(tk, sk.data(), sizeof(int) * S, hipMemcpyHostToDevice));
+      k_sys_sample<<<(S + TB - 1) / TB, TB, 0, c->stream>>>(S, stride, mn, mk, tn, tk);
+      SV_HIP(c, hipGetLastError());
       SV_HIP(c, hipMemcpy(tm, sm.data(), sizeof(int) * S, hipMemcpyHostToDevice));
       SV_HIP(c, hipMemcpy(tu, su.data(), sizeof(int) * su.size(), hipMemcpyHostToDevice));
       SysArgs ts = a;
@@ -1501,15 +1576,11 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
       if (sl.m <= 8) c->wvariant[sl.m / 2 - 2] = variant;
     }
   } else {
-    const int total = (int)qn.size();
+    const int total = nsys;
     const std::vector<int> qu = units_of(qm);
-    DevTmp<int> mn, mk, mm, mu;
-    SV_HIP(c, mn.alloc(total));
-    SV_HIP(c, mk.alloc(total));
+    DevTmp<int> mm, mu;
     SV_HIP(c, mm.alloc(total));
     SV_HIP(c, mu.alloc(qu.size()));
-    SV_HIP(c, hipMemcpy(mn, qn.data(), sizeof(int) * total, hipMemcpyHostToDevice));
-    SV_HIP(c, hipMemcpy(mk, qk.data(), sizeof(int) * total, hipMemcpyHostToDevice));
     SV_HIP(c, hipMemcpy(mm, qm.data(), sizeof(int) * total, hipMemcpyHostToDevice));
     SV_HIP(c, hipMemcpy(mu, qu.data(), sizeof(int) * qu.size(), hipMemcpyHostToDevice));
     SysArgs am = a;
@@ -1533,7 +1604,7 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   (void)ms;
   c->t_weights_tune = tune_ms;
   c->t_weights = solve_ms;
-  c->n_systems = (int)sys.size();
+  c->n_systems = nsys;
   int nsing = 0;
   SV_HIP(c, hipMemcpy(&nsing, c->singular, sizeof(int), hipMemcpyDeviceToHost));
   c->have_weights = true;

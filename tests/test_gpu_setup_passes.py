@@ -1,0 +1,102 @@
+"""The set-up passes at the edges of their work splits: row sums and filter
+coefficients of lists that fill a block's staged range with many rows, with few
+and with less than one; the lists of weight systems of an order map that mixes
+every order; the initial records and the volume sum made on the device."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import sunset_amd
+from sunset_amd.nodes import jittered_lattice, wall_channel
+
+pytestmark = pytest.mark.gpu
+
+
+def _nodes(kind):
+    if kind == "short":           # ~40 links: dozens of rows a block, a ragged last block
+        return jittered_lattice(31, 27, seed=2, h_over_s=1.8), 4
+    if kind == "long":            # ~1040 links: one row is more than a staged range
+        ns = jittered_lattice(41, 40, seed=2, h_over_s=9.1)
+        return dataclasses.replace(ns, smax=4 * ns.smax), 4   # the search cells follow smax
+    return wall_channel(16, 16, order=6, seed=1), 6
+
+
+@pytest.mark.parametrize("kind", ["short", "long", "walls"])
+def test_sums_and_filter_rows(kind):
+    """The sequential sums over the links in list order: bit for bit, but for
+    the filter's second sum, whose products are not rounded before they are
+    added: within K roundings of the terms' sizes."""
+    ns, order = _nodes(kind)
+    s = sunset_amd.Solver(morder=order)
+    s.set_nodes(ns)
+    s.find_neighbours(copy=False)
+    s.calc_weights()
+    s.calc_boundary_weights()
+    K = max(40, int(4 * np.pi * (ns.h / ns.s).max() ** 2 * 1.4))
+    s.calc_sums()
+    b = s.weights(K)
+    s.filter_coefficients()
+    c = s.weights(K)
+    seq = lambda w: np.cumsum(w, axis=1)[:, -1]      # padding entries are zeros, at the end
+    free = np.ones(s.npfb, bool)
+    if kind == "walls":            # boundary rows' sums follow other rules
+        free[:] = False
+        free[ns.nb * 5:] = True
+    # links: the node itself (weight 0) and these
+    assert (b["w_hyp"] != 0).sum(1).max() >= (1024 if kind == "long" else 20)
+    for d in range(2):
+        assert np.array_equal(seq(b["w_grad"][:, :, d])[free], b["gsum"][free, d])
+    assert np.array_equal(seq(b["w_lap"])[free], b["lsum"][free])
+    assert np.array_equal(seq(b["w_hyp"])[free], b["hsum"][free])
+    bound = K * np.finfo(float).eps * np.abs(c["w_hyp"]).sum(1)
+    assert (np.abs(seq(c["w_hyp"]) - c["hsum"]) <= bound).all()
+    # one factor a row
+    nz = b["w_hyp"] != 0
+    fac = np.where(nz, c["w_hyp"] / np.where(nz, b["w_hyp"], 1.0), np.nan)
+    assert np.nanmax(np.nanmax(fac, 1) / np.nanmin(fac, 1) - 1.0) < 8 * np.finfo(float).eps
+    s.close()
+
+
+def test_weight_systems_of_mixed_orders():
+    """Every node's weights under an order map of all orders are, bit for bit,
+    those under a map of its own order alone: a system's result does not
+    depend on the list it was solved from."""
+    ns = jittered_lattice(23, 19, seed=5, h_over_s=2.9)
+    n = ns.npfb
+    K = 110
+    mix = np.random.default_rng(1).choice([4, 6, 8], n).astype(np.int32)
+    out = {}
+    for key in (4, 6, 8, "mix"):
+        s = sunset_amd.Solver(morder=8)
+        s.set_nodes(ns)
+        s.find_neighbours(copy=False)
+        s.calc_weights(mix if key == "mix" else np.full(n, key, np.int32))
+        s.calc_sums()
+        out[key] = s.weights(K)
+        s.close()
+    for o in (4, 6, 8):
+        sel = mix == o
+        for w in ("w_grad", "w_lap", "w_hyp"):
+            assert np.array_equal(out["mix"][w][sel], out[o][w][sel]), (o, w)
+
+
+def test_initial_records_round_trip():
+    """set_initial / get_state with no step in between, on node counts at and
+    around a wavefront and a workgroup; a new set_phys keeps the state."""
+    for nx, ny in ((16, 16), (17, 15), (23, 19)):
+        ns = jittered_lattice(nx, ny, seed=4, h_over_s=1.8)
+        n = ns.npfb
+        rng = np.random.default_rng(0)
+        ic = {k: rng.uniform(0.9, 1.1, n) for k in ("ro", "u", "v", "cxx", "cyy")}
+        ic["cxy"] = rng.uniform(-0.1, 0.1, n)
+        for form in ("di", "lc"):
+            s = sunset_amd.Solver(morder=4, form=form).setup(ns)
+            s.set_phys(Re=10.0, Wi=1.0, beta=0.5, Ma=0.1)
+            s.set_initial(ic, dt=1e-6)
+            tol = 4 * np.finfo(float).eps     # u: a product and a quotient
+            s.set_phys(Re=10.0, Wi=1.0, beta=0.5, Ma=0.1, kol_amp=0.1, kol_k=2.0)
+            g = s.fields()
+            for k in ic if form == "di" else ("ro", "u", "v"):
+                assert np.abs(g[k] - ic[k]).max() <= tol, (form, k)
+            s.close()
