@@ -463,6 +463,7 @@ int sv_dev_boundary_weights(sv_ctx *c) {
   SV_HIP(c, hipGetLastError());
   SV_HIP(c, hipStreamSynchronize(c->stream));
   c->have_bweights = true;
+  c->have_volsum = false;
   c->sell_dirty = true;
   c->L.valid = false;
   return 0;

@@ -1608,6 +1608,7 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   int nsing = 0;
   SV_HIP(c, hipMemcpy(&nsing, c->singular, sizeof(int), hipMemcpyDeviceToHost));
   c->have_weights = true;
+  c->have_volsum = false;
   c->have_sums = false;
   c->have_filter = false;
   c->sell_dirty = true;

@@ -169,7 +169,7 @@ int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, cons
   if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
   c->graph_valid = false;
   c->have_lists = c->have_weights = c->have_sums = c->have_filter = false;
-  c->have_state = false;
+  c->have_state = c->have_volsum = false;
   c->blist = nullptr; c->rnx = c->rny = nullptr; c->ooR = nullptr;
   c->wtt = c->wtt_sum = nullptr; c->wtt_ld = 0;
   c->fields_buf = nullptr;
@@ -612,18 +612,14 @@ static int ensure_state_buffers(sv_ctx *c) {
 }
 
 // The single segment of a plain context: physics constants, volume sum and the
-// per-node Kolmogorov forcing (setup only).
+// per-node Kolmogorov forcing.
 static int upload_segment(sv_ctx *c) {
   const int n = c->npfb;
-  std::vector<double> y(n), vol(n), fx(n);
-  SV_HIP(c, hipMemcpy(y.data(), c->y, sizeof(double) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(vol.data(), c->vol, sizeof(double) * n, hipMemcpyDeviceToHost));
-  double tv = 0.0;
-  for (int i = 0; i < n; i++) tv += vol[i];
-  c->volsum = tv;
-  const std::vector<int> &P = c->L.hperm;   // loop order
-  for (int k = 0; k < n; k++) fx[k] = c->pk.kol_amp * sin(c->pk.kol_k * y[P[k]]);
-  SV_HIP(c, hipMemcpy(c->fx, fx.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  if (!c->have_volsum)
+    if (int rc = sv_dev_volume_sum(c, &c->volsum)) return rc;
+  c->have_volsum = true;
+  const double tv = c->volsum;
+  if (int rc = sv_dev_forcing(c)) return rc;
   c->hseg.assign(1, sv_segk{});
   sv_segk &S = c->hseg[0];
   S.base = 0; S.npfb = n; S.blk0 = 0; S.nblk = c->nblk; S.volsum = tv; S.pk = c->pk;
@@ -650,30 +646,6 @@ int sv_set_phys(sv_ctx *c, const sv_phys *p) {
   return 0;
 }
 
-// log_conf_psi_from_c on the host (setup only), conf_transforms.F90:177-215
-static void psi_from_c(double a, double b, double d, double *pxx, double *pxy, double *pyy) {
-  double l1, l2, R[4];
-  if (fabs(b) <= 1.0e-16) {
-    l1 = a; l2 = d; R[0] = 1; R[1] = 0; R[2] = 0; R[3] = 1;
-  } else {
-    const double tr = a + d, det = a * d - b * b;
-    double t = 0.25 * tr * tr - det;
-    if (t <= 1.0e-16) t = 0.0;
-    t = sqrt(t);
-    l1 = 0.5 * tr + t;
-    l2 = 0.5 * tr - t;
-    double r11 = l1 - d, r21 = b;
-    const double nrm = sqrt(r11 * r11 + r21 * r21);
-    r11 /= nrm; r21 /= nrm;
-    R[0] = r11; R[1] = r21; R[2] = -r21; R[3] = r11;
-  }
-  const double e1 = log(l1), e2 = log(l2);
-  const double i11 = e1 * R[0], i12 = e1 * R[1], i21 = e2 * R[2], i22 = e2 * R[3];
-  *pxx = R[0] * i11 + R[2] * i21;
-  *pxy = R[1] * i11 + R[3] * i21;
-  *pyy = R[1] * i12 + R[3] * i22;
-}
-
 int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v,
                    const double *cxx, const double *cxy, const double *cyy) {
   SV_CHECK(c, c && ro && u && v && cxx && cxy && cyy, "null argument");
@@ -687,28 +659,22 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
            "block halos within %d records)", SV_HALO_MAX);
   if (int rc = ensure_state_buffers(c)) return rc;
   const int n = c->npfb;
-  std::vector<double> a(n), b(n), d(n), e(n), f(n), g(n);
+  const bool lc = c->cfg.form == SV_FORM_LC;
   for (int i = 0; i < n; i++) {
     SV_CHECK(c, ro[i] > 0, "node %d: density must be positive", i);
-    a[i] = ro[i];
-    b[i] = ro[i] * u[i];
-    d[i] = ro[i] * v[i];
-    if (c->cfg.form == SV_FORM_LC) {
+    if (lc)
       SV_CHECK(c, cxx[i] * cyy[i] - cxy[i] * cxy[i] > 0 && cxx[i] > 0,
                "node %d: conformation tensor not positive definite", i);
-      psi_from_c(cxx[i], cxy[i], cyy[i], &e[i], &f[i], &g[i]);
-    } else {
-      e[i] = cxx[i]; f[i] = cxy[i]; g[i] = cyy[i];
-    }
   }
-  std::vector<double> rec((size_t)SV_US * n, 0.0);
-  const std::vector<int> &P = c->L.hperm;   // record k holds the caller's node P[k]
-  for (int k = 0; k < n; k++) {
-    double *r = rec.data() + (size_t)SV_US * k;
-    const int i = P[k];
-    r[0] = a[i]; r[1] = b[i]; r[2] = d[i]; r[3] = e[i]; r[4] = f[i]; r[5] = g[i];
-  }
-  SV_HIP(c, hipMemcpy(c->U, rec.data(), sizeof(double) * rec.size(), hipMemcpyHostToDevice));
+  // the six arrays to the device as they are, the records made there
+  if (!c->fields_buf && sv_alloc(c, (void **)&c->fields_buf, sizeof(double) * 12 * (size_t)n))
+    return SV_E_NOMEM;
+  const double *src[6] = {ro, u, v, cxx, cxy, cyy};
+  for (int q = 0; q < 6; q++)
+    SV_HIP(c, hipMemcpyAsync(c->fields_buf + (size_t)q * n, src[q], sizeof(double) * n,
+                             hipMemcpyHostToDevice, c->stream));
+  if (int rc = sv_dev_init_records(c, c->fields_buf)) return rc;
+  const std::vector<int> &P = c->L.hperm;   // loop slot k holds the caller's node P[k]
   if (c->nb > 0) {
     // boundary records and the loop slot -> record map; u_inflow_local starts
     // at U_char, on inflow nodes at the initial u (setup_flow.F90:48-51, :130-137)

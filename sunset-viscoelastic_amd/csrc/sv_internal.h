@@ -277,7 +277,9 @@ struct sv_ctx {
   int gs = SV_GS_LC;
   double *fx = nullptr;    // per-node Kolmogorov forcing
   double *partial = nullptr; int npartial = 0;
-  double volsum = 0.0;     // sum of node volumes (the mass-correction denominator)
+  // sum of node volumes (the mass-correction denominator), of the current ones
+  double volsum = 0.0;
+  bool have_volsum = false;
   sv_ctrl *ctrl = nullptr;  // [nseg]
   // segments: ntot = padded node count of the state arrays, nblk = blocks
   int nseg = 1, ntot = 0, nblk = 0;
@@ -408,6 +410,12 @@ int sv_dev_to_caller_order(sv_ctx *c, int nf, const double *in, double *out);
 // 0 if p is device memory of the context's device in this library's HIP
 // runtime, else an SV_E_ARG failure naming `what`
 int sv_check_device_ptr(sv_ctx *c, const void *p, const char *what);
+// ---- kernels: initial state (k_init.hip) ----
+// state records in U from six caller-order device arrays (ro, u, v, c),
+// fields[6][npfb]
+int sv_dev_init_records(sv_ctx *c, const double *fields);
+int sv_dev_forcing(sv_ctx *c);                       // fx from the physics constants
+int sv_dev_volume_sum(sv_ctx *c, double *sum);       // of the real nodes
 // ---- kernels: time stepping (k_step.hip) ----
 // gather records and set_tstep minima of the state in U (no correction)
 int sv_dev_init_state(sv_ctx *c);
