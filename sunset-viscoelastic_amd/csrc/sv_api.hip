@@ -597,8 +597,8 @@ static int ensure_state_buffers(sv_ctx *c) {
       sv_alloc(c, (void **)&c->reg, nu) || sv_alloc(c, (void **)&c->eacc, nu) ||
       sv_alloc(c, (void **)&c->GA, ng) || sv_alloc(c, (void **)&c->GB, ng))
     return SV_E_NOMEM;
-  SV_HIP(c, hipMemset(c->GA, 0, ng));
-  SV_HIP(c, hipMemset(c->GB, 0, ng));
+  SV_HIP(c, hipMemsetAsync(c->GA, 0, ng, c->stream));
+  SV_HIP(c, hipMemsetAsync(c->GB, 0, ng, c->stream));
   c->npartial = 4 * c->nblk * (SV_BLOCK / SV_WAVE);   // four kinds, one per slice
   if (sv_alloc(c, (void **)&c->partial, sizeof(double) * (c->npartial + 8)) ||
       sv_alloc(c, (void **)&c->ctrl, sizeof(sv_ctrl)) ||
@@ -606,8 +606,8 @@ static int ensure_state_buffers(sv_ctx *c) {
       sv_alloc(c, (void **)&c->segk, sizeof(sv_segk)) ||
       sv_alloc(c, (void **)&c->blk_seg, sizeof(int) * c->nblk))
     return SV_E_NOMEM;
-  SV_HIP(c, hipMemset(c->fx, 0, sizeof(double) * c->ntot));
-  SV_HIP(c, hipMemset(c->blk_seg, 0, sizeof(int) * c->nblk));
+  SV_HIP(c, hipMemsetAsync(c->fx, 0, sizeof(double) * c->ntot, c->stream));
+  SV_HIP(c, hipMemsetAsync(c->blk_seg, 0, sizeof(int) * c->nblk, c->stream));
   return 0;
 }
 
