@@ -487,19 +487,30 @@ int build_halos(sv_ctx *c, int hb, int nslot) {
 //   1024^2 order 6 LC   - /2082, 1916 / 1882   (fewer halo records per node)
 // Cached loads win while a stage's weights and link targets (26 bytes a link)
 // stay in the 256 MB Infinity Cache between stages.
+// Up to 32768 nodes several wavefronts walk a slice's links, each for its own
+// fields: with one, a CU has one or two waves, which wait for one request after
+// another.  A step in us, one and several:
+//   64^2 order 4 DI     44 / 41     150^2 order 6 LC    85 / 74
+//   64^2 order 6 LC     62 / 54     165^2 order 8 DI    89 / 81
+//   127^2 order 6 LC    74 / 65     180^2 order 6 LC    90 / 85
+//   128^2 order 6 DI    63 / 57
+// (Four waves with a quarter of the links each are faster still, 57 at 127^2,
+// but then the order of the sums depends on the node count.)
 struct Blocks {
   int hb;
   bool nt;
+  bool split;
 };
 static Blocks choose_blocks(int nslot, int64_t links) {
-  if (nslot <= 32768) return {64, false};
-  if (26 * links <= (int64_t)256 << 20) return {128, false};
-  return {nslot <= 500000 ? 128 : 256, true};
+  if (nslot <= 32768) return {64, false, true};
+  if (26 * links <= (int64_t)256 << 20) return {128, false, false};
+  return {nslot <= 500000 ? 128 : 256, true, false};
 }
 
 int sv_dev_build_halos(sv_ctx *c, int nslot) {
   const Blocks b = choose_blocks(nslot, c->L.nnz);
   c->L.nt = b.nt;
+  c->L.split = b.split;
   if (int rc = build_halos(c, b.hb, nslot)) return rc;
   return c->L.halo || b.hb == SV_WAVE ? 0 : build_halos(c, SV_WAVE, nslot);
 }
@@ -581,5 +592,6 @@ int sv_dev_build_loop(sv_ctx *c) {
     if (int rc = build_layout(c, SV_WAVE)) return rc;
   }
   c->L.nt = b.nt && c->L.hb != SV_WAVE;
+  c->L.split = b.split;
   return 0;
 }

@@ -25,7 +25,10 @@
 // gather needs of node j sits in one packed 80-byte record (LC) or 48-byte
 // record (DI), so a link costs at most two cache lines instead of one line
 // per field, and records of adjacent nodes share lines.
+#include <algorithm>
+
 #include "sv_internal.h"
+#include "sweep.h"
 
 namespace {
 
@@ -52,8 +55,6 @@ struct HaloU {
   static constexpr int U = NB == 64 ? 3 : NB == 128 ? 2 : 1;   // stage sweeps
   static constexpr int UF = NB == 64 ? 4 : 2;                  // the filter
 };
-typedef double dbl2 __attribute__((ext_vector_type(2)));
-
 template <typename T>
 __device__ __forceinline__ T ld_stream(const T *p) {
 #if SV_STREAM_NT
@@ -70,13 +71,14 @@ struct NodeRef {
   bool act;
 };
 
-// bid: workgroup of NB consecutive slots (NB divides SV_BLOCK)
+// bid: workgroup of NB consecutive slots (NB divides SV_BLOCK); waves past
+// them (a list shared by several) repeat its slots
 template <int NB = BS>
 __device__ __forceinline__ NodeRef node_ref(const int *blk_seg, const sv_segk *seg, int bid) {
   NodeRef r;
   r.sg = blk_seg[bid / (BS / NB)];
   const sv_segk &S = seg[r.sg];
-  r.i = bid * NB + (int)threadIdx.x;
+  r.i = bid * NB + (int)threadIdx.x % NB;
   r.act = r.i - S.base < S.npfb;
   r.ii = r.act ? r.i : S.base;
   return r;
@@ -419,12 +421,29 @@ struct Sums {
   double rx, ry, ux, uy, vx, vy, lu, lv, axx, ayx, axy, ayy, bxy, byy, cxx_l, cxy_l, cyy_l, q1x, q1y, q2x, q2y, q3x, q3y;
 };
 
+// A node's own values in a stage: its gather record, the sums of its weights,
+// the RK register and the error accumulators.
+struct Own {
+  Rec9 s;
+  double sx, sy, sl, r1[6], eo[6];
+};
+
+template <int FORM, int STAGE>
+__device__ __forceinline__ Own load_own(const StageArgs &a, int i) {
+  Own o;
+  o.s = load_g<FORM>(a.G, i);
+  o.sx = a.gsx[i]; o.sy = a.gsy[i]; o.sl = a.lsum[i];
+  if (STAGE > 0) load_u(a.reg_in, i, o.r1);
+  if (STAGE > 1) load_u(a.e, i, o.eo);
+  return o;
+}
+
 // Pointwise part of a stage for one node: the right-hand side from the
 // gathered sums and the own record, then the RK update.  Returns the node's
 // error norm contribution (stage 4).
 template <int FORM, int STAGE, bool MDIFF, bool BND>
-__device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef &nr,
-                                              const Sums &S) {
+__device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef &nr, const Sums &S,
+                                              const Own &own) {
   const int i = nr.i;
   double rx = S.rx, ry = S.ry, ux = S.ux, uy = S.uy, vx = S.vx, vy = S.vy, lu = S.lu, lv = S.lv;
   double axx = S.axx, ayx = S.ayx, axy = S.axy, ayy = S.ayy, bxy = S.bxy, byy = S.byy, cxx_l = S.cxx_l, cxy_l = S.cxy_l;
@@ -433,8 +452,8 @@ __device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef 
   (void)q1x; (void)q1y; (void)q2x; (void)q2y; (void)q3x; (void)q3y;
   double emax_loc = 0.0;
   {
-    const double sx = a.gsx[i], sy = a.gsy[i], sl = a.lsum[i];
-    const Rec9 s = load_g<FORM>(a.G, i);
+    const double sx = own.sx, sy = own.sy, sl = own.sl;
+    const Rec9 s = own.s;
     const double ro = s.ro, u = s.u, v = s.v, cxx = s.cxx, cxy = s.cxy, cyy = s.cyy;
     rx = rx - ro * sx; ry = ry - ro * sy;
     ux = ux - u * sx; uy = uy - u * sy; lu = lu - u * sl;
@@ -555,14 +574,12 @@ __device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef 
       for (int f = 0; f < 6; f++) a.rhs_out[(size_t)f * a.rhs_stride + i] = rhs[f];
     } else if (STAGE <= 3) {
       const double ra = C->RKa[STAGE - 1], rb = C->RKb[STAGE - 1], rm = C->RKbmbh[STAGE - 1];
-      double r1[6], eo[6], Un[6], ro_[6];
-      load_u(a.reg_in, i, r1);
-      if (STAGE > 1) load_u(a.e, i, eo);
+      double eo[6], Un[6], ro_[6];
 #pragma unroll
       for (int f = 0; f < 6; f++) {
-        Un[f] = r1[f] + ra * rhs[f];
-        ro_[f] = r1[f] + rb * rhs[f];
-        eo[f] = (STAGE == 1 ? 0.0 : eo[f]) + rm * rhs[f];
+        Un[f] = own.r1[f] + ra * rhs[f];
+        ro_[f] = own.r1[f] + rb * rhs[f];
+        eo[f] = (STAGE == 1 ? 0.0 : own.eo[f]) + rm * rhs[f];
       }
       store_u(a.reg_out, i, ro_);
       store_u(a.e, i, eo);
@@ -583,14 +600,12 @@ __device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef 
       store_g<FORM>(a.Gout, i, g);
     } else {
       const double rb = C->RKb[3], rm = C->RKbmbh[3];
-      double r1[6], eo[6], uo[6];
-      load_u(a.reg_in, i, r1);
-      load_u(a.e, i, eo);
+      double uo[6];
       const double nrm[6] = {1.0, P.err_norm_rou, P.err_norm_rou, 1.0, 1.0, 1.0};
 #pragma unroll
       for (int f = 0; f < 6; f++) {
-        uo[f] = r1[f] + rb * rhs[f];
-        const double ef = eo[f] + rm * rhs[f];
+        uo[f] = own.r1[f] + rb * rhs[f];
+        const double ef = own.eo[f] + rm * rhs[f];
         emax_loc = fmax(emax_loc, fabs(ef) * nrm[f]);
       }
       if (BND && bkind >= 0) bound_apply(P, bkind, uin_now(P, C, buin0, 5), uo);
@@ -662,7 +677,7 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
   double emax_loc = 0.0;
   if (act) {
     const Sums S{rx, ry, ux, uy, vx, vy, lu, lv, axx, ayx, axy, ayy, bxy, byy, cxx_l, cxy_l, cyy_l, q1x, q1y, q2x, q2y, q3x, q3y};
-    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S);
+    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S, load_own<FORM, STAGE>(a, nr.i));
   }
   if (STAGE == 4) {
     emax_loc = wave_max(emax_loc);
@@ -682,8 +697,13 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
 //               flight): one or two waves per SIMD, memory latency and the
 //               random LDS reads (50 clocks a link of a wave for 72 bytes a
 //               lane, 36 without bank conflicts)
-//   16k nodes   14 us (34): the chain launch -> layout -> keys -> records ->
-//               LDS -> links -> pointwise part of one wave per CU
+//   16k nodes   11.5 us (34; 14 with one wave per slice): the chain launch ->
+//               layout -> keys -> records -> LDS -> links -> pointwise part
+// Up to 32768 nodes NW wavefronts walk the links of a slice, each for its own
+// fields (flow; conformation; psi), so that every sum keeps the links' order
+// and the values do not depend on the split; more threads stage the halo, and
+// wave 0 requests the node's own values before it, for the pointwise part that
+// it does alone.
 // LDS records are the gather records as they are: 10 doubles (80 B, the last
 // one a pad) for LC, 6 for DI (48 B), read 16 bytes at a time.  Both strides
 // are odd multiples of 16 bytes, so the records' starts spread over all LDS
@@ -693,154 +713,23 @@ struct HaloL {
   static constexpr int RS = FORM == SV_FORM_LC ? SV_GS_LC : SV_GS_DI;
   static constexpr int BYTES = 8 * RS;
 };
+// sums handed to wave 0 where the fields of a slice are shared by several waves
+constexpr int PARTS_CONF = 9, PARTS_PSI = 6;
+template <int FORM>
+constexpr int stage_waves() { return FORM == SV_FORM_LC ? 3 : 2; }
 static_assert(HaloL<SV_FORM_LC>::BYTES == SV_HALO_REC, "the halo budget counts LC records");
 
-// Records a thread stages at once: a usual halo (~600 records per 256 slots,
-// ~270 per 64) in one round of requests, since a round costs two dependent
-// trips to memory (key, record).
-template <int NB>
-struct HaloC {
-  static constexpr int C = NB == SV_WAVE ? 5 : NB == 128 ? 4 : 3;
-};
 
-// The halo keys of this thread's records h, h + NB, ... of a round; past the
-// end the last key (a valid record, not stored)
-template <int NB>
-struct HaloKeys {
-  int key[HaloC<NB>::C];
-  __device__ __forceinline__ void get(const int *hx, int h, int nh) {
-#pragma unroll
-    for (int c = 0; c < HaloC<NB>::C; c++) key[c] = hx[min(h + c * NB, nh - 1)];
-  }
-};
-
-// The block's halo to LDS: load(key) reads a record, put(h, key, record)
-// stores it as record h.  keys holds the first round's keys.
-template <int NB, class Load, class Put>
-__device__ __forceinline__ void halo_stage(const int *hx, int nh, HaloKeys<NB> &keys, Load load,
-                                           Put put) {
-  constexpr int C = HaloC<NB>::C;
-  auto round = [&](int h) {
-    decltype(load(0)) r[C];
-#pragma unroll
-    for (int c = 0; c < C; c++) r[c] = load(keys.key[c] & SV_FLIP_MASK);
-#pragma unroll
-    for (int c = 0; c < C; c++)
-      if (h + c * NB < nh) put(h + c * NB, keys.key[c] >> SV_FLIP_SHIFT, r[c]);
-  };
-  // the first round apart: its requests wait for the keys only, not for the
-  // links requested after them
-  if (nh > 0) round(threadIdx.x);
-  for (int h = threadIdx.x + C * NB; h < nh; h += C * NB) {
-    keys.get(hx, h, nh);
-    round(h);
-  }
-}
-
-template <int FORM>
-__device__ __forceinline__ Rec9 halo_rec(const double *hl, int h) {
-  return load_g<FORM>(hl, h);
-}
-
-// One streamed array of a wavefront's slice (W groups of 64 values of 4 or 16
-// bytes per pair of links), read through a buffer descriptor of exactly the
-// slice's pairs: a batch costs one address addition (the pairs within it are
-// immediate offsets), and entries past them read as 0 by the hardware's range
-// check, which covers the vector and immediate offsets used here (it leaves
-// out the scalar one, kept 0), so the requests need no guards.
-template <typename T, int W, bool NT>
-struct Stream {
-  __amdgpu_buffer_rsrc_t r;
-  // n: links of the slice's longest list
-  __device__ __forceinline__ Stream(const void *base, int n)
-      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0,
-                                            (n + 1) / 2 * W * SV_WAVE * (int)sizeof(T),
-                                            0x00020000)) {}
-  // group c of the u-th pair from position p (entry_at)
-  __device__ __forceinline__ T at(int p, int u, int c) const {
-    const int vo = p * W * (int)sizeof(T) + (int)(threadIdx.x & (SV_WAVE - 1)) * (int)sizeof(T) +
-                   (u * W + c) * SV_WAVE * (int)sizeof(T);
-    constexpr int aux = NT ? 2 : 0;   // nt
-    if constexpr (sizeof(T) == 16)
-      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, vo, 0, aux));
-    else
-      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, vo, 0, aux));
-  }
-};
-
-// Position of link pair k / 2 in its slice (64 per pair), kept opaque so that
-// the pairs after it stay immediate offsets (the loop's strength reduction
-// would otherwise carry one address per pair)
-__device__ __forceinline__ int entry_at(int k) {
-  int p = k / 2 * SV_WAVE;
-  asm volatile("" : "+v"(p));
-  return p;
-}
-
-// The links of one wavefront's slice, walked in batches of U pairs with the
-// next batch's global streams in flight while a batch is consumed (two register
-// sets, no copies between them), and each link's LDS record requested before
-// the link before it is summed.  Batches that reach past the shortest list of
-// the slice send the requests of lanes past their own list out of range (no
-// memory traffic for the padding; they read record 0) and guard the sums.
-//   load(set, u, p)  requests the u-th pair from position p into entry u
-//   fetch(set, l)    the LDS record of link l of the set's 2U
-//   link(r, set, l)  adds it, with its record r
-constexpr int OUT_OF_RANGE = 1 << 22;   // past every list, in pairs times 64
-template <int U, class Rec, class Load, class Fetch, class Link>
-__device__ __forceinline__ void walk_links(int K, int KF, int KM, Load load, Fetch fetch,
-                                           Link link) {
-  constexpr int V = 2 * U;   // links of a batch
-  auto fill = [&](int s, int k0) {
-    const int p = entry_at(k0);
-#pragma unroll
-    for (int u = 0; u < U; u++) load(s, u, p);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto fill_guarded = [&](int s, int k0) {
-    const int p = entry_at(k0);
-#pragma unroll
-    for (int u = 0; u < U; u++) load(s, u, k0 + 2 * u < K ? p : OUT_OF_RANGE);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  int k = 0;
-  Rec r = fetch(0, 0);
-  for (; k + 3 * V <= KF; k += 2 * V) {
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-      fill(1 - s, k + (1 + s) * V);
-#pragma unroll
-      for (int l = 0; l < V; l++) {
-        const Rec n = l + 1 < V ? fetch(s, l + 1) : fetch(1 - s, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        link(r, s, l);
-        r = n;
-      }
-    }
-  }
-  for (; k < KM; k += 2 * V) {
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-      fill_guarded(1 - s, k + (1 + s) * V);
-#pragma unroll
-      for (int l = 0; l < V; l++) {
-        const Rec n = l + 1 < V ? fetch(s, l + 1) : fetch(1 - s, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (k + s * V + l < K) link(r, s, l);
-        r = n;
-      }
-    }
-  }
-}
-
-template <int FORM, int STAGE, bool MDIFF, bool BND, int NB, bool NT>
-__global__ __launch_bounds__(NB) void k_stage_h(StageArgs a) {
+template <int FORM, int STAGE, bool MDIFF, bool BND, int NB, bool NT, int NW>
+__global__ __launch_bounds__(NB * NW) void k_stage_h(StageArgs a) {
   extern __shared__ double hl[];
   const int bid = logical_wg<NB>(a.blist);
   // the layout's arrays cover whole blocks (no links past the last node), so
   // nothing of the streams waits for the segment
-  const int slice = __builtin_amdgcn_readfirstlane((bid * NB + (int)threadIdx.x) >> 6);
-  const int K = a.kcnt[bid * NB + (int)threadIdx.x];
+  const int slot = bid * NB + (int)threadIdx.x % NB;
+  const int slice = __builtin_amdgcn_readfirstlane(slot >> 6);
+  const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NB);
+  const int K = a.kcnt[slot];
   const int KF = a.krange[slice].x, KM = a.krange[slice].y;
   const int64_t o = a.off[slice];
   const int64_t h0 = a.hoff[bid];
@@ -856,43 +745,55 @@ __global__ __launch_bounds__(NB) void k_stage_h(StageArgs a) {
   const Stream<dbl2, 3, NT> sw(a.w3 + 3 * o, KM);
   uint32_t jc[2][U];
   dbl2 wg[2][2 * U], wl[2][U];   // d/dx and d/dy of a link; Laplacian of a pair
+  const bool laps = w == 0 || MDIFF;   // this wave's sums hold Laplacians
   auto load = [&](int s, int u, int p) {
     jc[s][u] = sc.at(p, u, 0);
-    wg[s][2 * u] = sw.at(p, u, 0); wg[s][2 * u + 1] = sw.at(p, u, 1); wl[s][u] = sw.at(p, u, 2);
+    wg[s][2 * u] = sw.at(p, u, 0); wg[s][2 * u + 1] = sw.at(p, u, 1);
+    wl[s][u] = sw.at(NW == 1 || laps ? p : OUT_OF_RANGE, u, 2);
   };
-  auto fetch = [&](int s, int l) {
-    return halo_rec<FORM>(hl, (int)(l & 1 ? jc[s][l / 2] >> 16 : jc[s][l / 2] & 0xffff));
+  auto rec = [&](int s, int l) {
+    return hl + (size_t)HaloL<FORM>::RS * (l & 1 ? jc[s][l / 2] >> 16 : jc[s][l / 2] & 0xffff);
   };
-  auto link = [&](const Rec9 &q, int s, int l) {
+  // the sums of the momentum and mass balances, of the conformation and of psi
+  auto link_flow = [&](double ro, double u, double v, int s, int l) {
     const double wx_ = wg[s][l].x, wy_ = wg[s][l].y;
     const double wl_ = l & 1 ? wl[s][l / 2].y : wl[s][l / 2].x;
-    rx += q.ro * wx_; ry += q.ro * wy_;
-    ux += q.u * wx_; uy += q.u * wy_; lu += q.u * wl_;
-    vx += q.v * wx_; vy += q.v * wy_; lv += q.v * wl_;
-    if (FORM == SV_FORM_LC) {
-      axx += q.cxx * wx_;
-      axy += q.cxy * wx_; ayy += q.cxy * wy_;
-      byy += q.cyy * wy_;
-      q1x += q.pxx * wx_; q1y += q.pxx * wy_;
-      q2x += q.pxy * wx_; q2y += q.pxy * wy_;
-      q3x += q.pyy * wx_; q3y += q.pyy * wy_;
-    } else {
-      axx += q.cxx * wx_; ayx += q.cxx * wy_;
-      axy += q.cxy * wx_; ayy += q.cxy * wy_;
-      bxy += q.cyy * wx_; byy += q.cyy * wy_;
-      if (MDIFF) { cxx_l += q.cxx * wl_; cxy_l += q.cxy * wl_; cyy_l += q.cyy * wl_; }
+    rx += ro * wx_; ry += ro * wy_;
+    ux += u * wx_; uy += u * wy_; lu += u * wl_;
+    vx += v * wx_; vy += v * wy_; lv += v * wl_;
+  };
+  auto link_conf = [&](double cxx, double cxy, double cyy, int s, int l) {
+    const double wx_ = wg[s][l].x, wy_ = wg[s][l].y;
+    axx += cxx * wx_;
+    axy += cxy * wx_; ayy += cxy * wy_;
+    byy += cyy * wy_;
+    if (FORM == SV_FORM_DI) {
+      ayx += cxx * wy_;
+      bxy += cyy * wx_;
+      if (MDIFF) {
+        const double wl_ = l & 1 ? wl[s][l / 2].y : wl[s][l / 2].x;
+        cxx_l += cxx * wl_; cxy_l += cxy * wl_; cyy_l += cyy * wl_;
+      }
     }
+  };
+  auto link_psi = [&](double pxx, double pxy, double pyy, int s, int l) {
+    const double wx_ = wg[s][l].x, wy_ = wg[s][l].y;
+    q1x += pxx * wx_; q1y += pxx * wy_;
+    q2x += pxy * wx_; q2y += pxy * wy_;
+    q3x += pyy * wx_; q3y += pyy * wy_;
   };
   // the halo's keys first, then the first batch of links, in flight while the
   // halo is staged
   const int *hx = a.hidx + h0;
-  HaloKeys<NB> keys;
+  HaloKeys<NB, NB * NW> keys;
   if (nh > 0) keys.get(hx, threadIdx.x, nh);
   __builtin_amdgcn_sched_barrier(0);
   const int p0 = entry_at(0);
 #pragma unroll
   for (int u = 0; u < U; u++) load(0, u, 2 * u < K ? p0 : OUT_OF_RANGE);
-  halo_stage<NB>(
+  Own own;
+  if (NW > 1 && w == 0) own = load_own<FORM, STAGE>(a, nr.ii);
+  halo_stage<NB, NB * NW>(
       hx, nh, keys, [&](int j) { return load_g<FORM>(a.G, j); },
       [&](int h, int fl, Rec9 r) {
         if (fl) {   // mirror ghost (reapply_mirror_bcs, mirror_boundaries.F90:285-340)
@@ -903,12 +804,61 @@ __global__ __launch_bounds__(NB) void k_stage_h(StageArgs a) {
         store_g<FORM>(hl, h, r);
       });
   __syncthreads();
-  walk_links<U, Rec9>(K, KF, KM, load, fetch, link);
+  if (NW == 1) {
+    walk_links<U, Rec9>(
+        K, KF, KM, load, [&](int s, int l) { return load_g<FORM>(rec(s, l), 0); },
+        [&](const Rec9 &q, int s, int l) {
+          link_flow(q.ro, q.u, q.v, s, l);
+          link_conf(q.cxx, q.cxy, q.cyy, s, l);
+          if (FORM == SV_FORM_LC) link_psi(q.pxx, q.pxy, q.pyy, s, l);
+        });
+    own = load_own<FORM, STAGE>(a, nr.ii);
+  } else {
+    // each wave its own fields of every link: the sums keep the links' order
+    struct Rec3 {
+      double2 a;
+      double b;
+    };
+    auto pair_first = [&](int s, int l, int q) {   // two values, aligned, then one
+      const double *r = rec(s, l) + q;
+      return Rec3{*reinterpret_cast<const double2 *>(r), r[2]};
+    };
+    auto pair_last = [&](int s, int l) {           // cxx, then cxy and cyy
+      const double *r = rec(s, l) + SV_G_CXX;
+      return Rec3{*reinterpret_cast<const double2 *>(r + 1), r[0]};
+    };
+    auto conf = [&](auto &&f) {
+      f(axx); f(axy); f(ayy); f(byy);
+      if (FORM == SV_FORM_DI) { f(ayx); f(bxy); }
+      if (MDIFF) { f(cxx_l); f(cxy_l); f(cyy_l); }
+    };
+    auto psi = [&](auto &&f) { f(q1x); f(q1y); f(q2x); f(q2y); f(q3x); f(q3y); };
+    if (w == 0)
+      walk_links<U, Rec3>(
+          K, KF, KM, load, [&](int s, int l) { return pair_first(s, l, 0); },
+          [&](const Rec3 &q, int s, int l) { link_flow(q.a.x, q.a.y, q.b, s, l); });
+    else if (w == 1)
+      walk_links<U, Rec3>(
+          K, KF, KM, load, pair_last,
+          [&](const Rec3 &q, int s, int l) { link_conf(q.b, q.a.x, q.a.y, s, l); });
+    else if (FORM == SV_FORM_LC)
+      walk_links<U, Rec3>(
+          K, KF, KM, load, [&](int s, int l) { return pair_first(s, l, SV_G_PXX); },
+          [&](const Rec3 &q, int s, int l) { link_psi(q.a.x, q.a.y, q.b, s, l); });
+    double *psums = hl + part_doubles(PARTS_CONF);
+    __syncthreads();   // the halo has been read
+    if (w == 1) give_sums(hl, conf);
+    if (FORM == SV_FORM_LC && w == 2) give_sums(psums, psi);
+    __syncthreads();
+    if (w > 0) return;
+    take_sums(hl, conf);
+    if (FORM == SV_FORM_LC) take_sums(psums, psi);
+  }
   double emax_loc = 0.0;
   if (act) {
     const Sums S{rx, ry, ux, uy, vx, vy, lu, lv, axx, ayx, axy, ayy, bxy, byy, cxx_l, cxy_l,
                  cyy_l, q1x, q1y, q2x, q2y, q3x, q3y};
-    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S);
+    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S, own);
   }
   if (STAGE == 4) {
     emax_loc = wave_max(emax_loc);
@@ -933,18 +883,28 @@ struct FilterArgs {
   const int *blist;       // launch group's logical blocks (nullable: all blocks)
 };
 
+// A node's own values in the filter
+struct OwnF {
+  double f[6], hs, vol;
+};
+
+__device__ __forceinline__ OwnF load_own(const FilterArgs &a, int i) {
+  OwnF o;
+  load_u(a.U, i, o.f);
+  o.hs = a.hsum[i];
+  o.vol = a.vol[i];
+  return o;
+}
+
 // Pointwise part of the filter for one node: the filtered record and its
 // mass-correction term.
 __device__ __forceinline__ double filter_point(const FilterArgs &a, const NodeRef &nr,
-                                               const double t[6]) {
-  const int i = nr.i;
-  const double hs = a.hsum[i];
-  double f[6], g[6];
-  load_u(a.U, i, f);
+                                               const double t[6], const OwnF &o) {
+  double g[6];
 #pragma unroll
-  for (int q = 0; q < 6; q++) g[q] = f[q] + (t[q] - f[q] * hs);
-  store_u(a.Uf, i, g);
-  return (g[0] - a.seg[nr.sg].pk.rho_char) * a.vol[i];
+  for (int q = 0; q < 6; q++) g[q] = o.f[q] + (t[q] - o.f[q] * o.hs);
+  store_u(a.Uf, nr.i, g);
+  return (g[0] - a.seg[nr.sg].pk.rho_char) * o.vol;
 }
 
 __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
@@ -981,7 +941,7 @@ __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
         for (int q = 0; q < 6; q++) t[q] += f[u][q] * w[u];
       }
   }
-  const double m = wave_sum(act ? filter_point(a, nr, t) : 0.0);
+  const double m = wave_sum(act ? filter_point(a, nr, t, load_own(a, nr.i)) : 0.0);
   if ((threadIdx.x & 63) == 0) a.partial[nr.i >> 6] = m;
 }
 
@@ -991,8 +951,9 @@ template <int NB, bool NT>
 __global__ __launch_bounds__(NB) void k_filter_h(FilterArgs a) {
   extern __shared__ double hl[];
   const int bid = logical_wg<NB>(a.blist);
-  const int slice = __builtin_amdgcn_readfirstlane((bid * NB + (int)threadIdx.x) >> 6);
-  const int K = a.kcnt[bid * NB + (int)threadIdx.x];   // as k_stage_h
+  const int slot = bid * NB + (int)threadIdx.x;   // as k_stage_h
+  const int slice = __builtin_amdgcn_readfirstlane(slot >> 6);
+  const int K = a.kcnt[slot];
   const int KF = a.krange[slice].z, KM = a.krange[slice].w;
   const int64_t o = a.off[slice];
   const int64_t h0 = a.hoff[bid];
@@ -1004,32 +965,22 @@ __global__ __launch_bounds__(NB) void k_filter_h(FilterArgs a) {
   const Stream<uint32_t, 1, NT> sc(a.lcol + o, KM);
   const Stream<dbl2, 1, NT> sw(a.wh + o, KM);
   uint32_t jc[2][U];
-  dbl2 w[2][U];
+  dbl2 wf[2][U];
   auto load = [&](int s, int u, int p) {
     jc[s][u] = sc.at(p, u, 0);
-    w[s][u] = sw.at(p, u, 0);
+    wf[s][u] = sw.at(p, u, 0);
   };
   struct Rec6 {
     double2 d0, d1, d2;
   };
-  auto fetch = [&](int s, int l) {
-    const int j = (int)(l & 1 ? jc[s][l / 2] >> 16 : jc[s][l / 2] & 0xffff);
-    const double2 *d = reinterpret_cast<const double2 *>(hl + j * 6);
-    return Rec6{d[0], d[1], d[2]};
-  };
-  auto link = [&](const Rec6 &q, int s, int l) {
-    const double w_ = l & 1 ? w[s][l / 2].y : w[s][l / 2].x;
-    t[0] += q.d0.x * w_; t[1] += q.d0.y * w_; t[2] += q.d1.x * w_;
-    t[3] += q.d1.y * w_; t[4] += q.d2.x * w_; t[5] += q.d2.y * w_;
-  };
   const int *hx = a.hidx + h0;   // keys, first links, halo: as k_stage_h
-  HaloKeys<NB> keys;
+  HaloKeys<NB, NB> keys;
   if (nh > 0) keys.get(hx, threadIdx.x, nh);
   __builtin_amdgcn_sched_barrier(0);
   const int p0 = entry_at(0);
 #pragma unroll
   for (int u = 0; u < U; u++) load(0, u, 2 * u < K ? p0 : OUT_OF_RANGE);
-  halo_stage<NB>(
+  halo_stage<NB, NB>(
       hx, nh, keys,
       [&](int j) {
         const double2 *q = reinterpret_cast<const double2 *>(a.U + (size_t)j * SV_US);
@@ -1045,8 +996,19 @@ __global__ __launch_bounds__(NB) void k_filter_h(FilterArgs a) {
         d[0] = r.d0; d[1] = r.d1; d[2] = r.d2;
       });
   __syncthreads();
-  walk_links<U, Rec6>(K, KF, KM, load, fetch, link);
-  const double m = wave_sum(act ? filter_point(a, nr, t) : 0.0);
+  walk_links<U, Rec6>(
+      K, KF, KM, load,
+      [&](int s, int l) {
+        const int j = (int)(l & 1 ? jc[s][l / 2] >> 16 : jc[s][l / 2] & 0xffff);
+        const double2 *d = reinterpret_cast<const double2 *>(hl + j * 6);
+        return Rec6{d[0], d[1], d[2]};
+      },
+      [&](const Rec6 &q, int s, int l) {
+        const double w = l & 1 ? wf[s][l / 2].y : wf[s][l / 2].x;
+        t[0] += q.d0.x * w; t[1] += q.d0.y * w; t[2] += q.d1.x * w;
+        t[3] += q.d1.y * w; t[4] += q.d2.x * w; t[5] += q.d2.y * w;
+      });
+  const double m = wave_sum(act ? filter_point(a, nr, t, load_own(a, nr.ii)) : 0.0);
   if ((threadIdx.x & 63) == 0) a.partial[nr.i >> 6] = m;
 }
 
@@ -1256,16 +1218,20 @@ void launch_sweep(sv_ctx *c, const StageArgs &a, int nb, int hmax) {
     k_stage<FORM, STAGE, MDIFF, BND><<<nb, BS, 0, c->stream>>>(a);
     return;
   }
-  const size_t shm = (size_t)hmax * HaloL<FORM>::BYTES;
+  size_t shm = (size_t)hmax * HaloL<FORM>::BYTES;
   const int hb = c->L.hb, grid = nb * (BS / hb);
-  if (hb == 64)
-    k_stage_h<FORM, STAGE, MDIFF, BND, 64, false><<<grid, 64, shm, c->stream>>>(a);
+  if (hb == 64 && c->L.split) {
+    constexpr int NW = stage_waves<FORM>();
+    shm = std::max(shm, sizeof(double) * part_doubles(PARTS_CONF + PARTS_PSI));
+    k_stage_h<FORM, STAGE, MDIFF, BND, 64, false, NW><<<grid, 64 * NW, shm, c->stream>>>(a);
+  } else if (hb == 64)
+    k_stage_h<FORM, STAGE, MDIFF, BND, 64, false, 1><<<grid, 64, shm, c->stream>>>(a);
   else if (hb == 128 && !c->L.nt)
-    k_stage_h<FORM, STAGE, MDIFF, BND, 128, false><<<grid, 128, shm, c->stream>>>(a);
+    k_stage_h<FORM, STAGE, MDIFF, BND, 128, false, 1><<<grid, 128, shm, c->stream>>>(a);
   else if (hb == 128)
-    k_stage_h<FORM, STAGE, MDIFF, BND, 128, true><<<grid, 128, shm, c->stream>>>(a);
+    k_stage_h<FORM, STAGE, MDIFF, BND, 128, true, 1><<<grid, 128, shm, c->stream>>>(a);
   else
-    k_stage_h<FORM, STAGE, MDIFF, BND, 256, true><<<grid, 256, shm, c->stream>>>(a);
+    k_stage_h<FORM, STAGE, MDIFF, BND, 256, true, 1><<<grid, 256, shm, c->stream>>>(a);
 }
 
 template <int FORM, int STAGE>

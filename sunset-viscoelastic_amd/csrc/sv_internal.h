@@ -166,6 +166,7 @@ struct sv_loopl {
   int hb = SV_BLOCK;        // slots per halo block = threads per workgroup of
                             // the sweeps: 64, 128 or 256
   bool nt = false;          // weights loaded non-temporally
+  bool split = false;       // several wavefronts per slice, by fields (hb = 64)
   int hmax = 0;             // largest halo of a block
   std::vector<int> hcnt;    // halo sizes
   int64_t *hoff = nullptr;  // [nblocks + 1]
