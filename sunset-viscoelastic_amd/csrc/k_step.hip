@@ -3,7 +3,11 @@
 // filter_variables, set_tstep and set_tstep_PID.
 //
 // One step is 8 launches, all reading their scalars from the device control
-// block so the step can be captured once and replayed as a hipGraph:
+// block so the step can be captured once and replayed as a hipGraph.  Up to
+// 32768 nodes it is 6: a launch of a single block costs 4.4 us there, a tenth of
+// the step, and the few partial results are reduced by every workgroup of the
+// kernel that needs them (k_dt's work at the head of stage 1, k_reduce's in
+// k_apply_state), in the same order:
 //   k_dt          (1 block)  set_tstep + set_tstep_PID, emax history shift,
 //                            dt-scaled RK coefficients
 //   k_stage<1..4>            ONE gather sweep per stage: every gradient and
@@ -268,6 +272,10 @@ struct StageArgs {
   const double *fx;
   const sv_ctrl *ctrl;  // [nseg]
   double *partial;      // stage 4: max error per slice
+  // stage 1 of small node sets: the limits' partial minima, and the control
+  // values made from them and ctrl (another array: other workgroups still read)
+  const double *pcfl, *pvisc;
+  sv_ctrl *ctrl_out;
   int rk1;              // STAGE 0: reference stage counter is 1
   // DI only, nullable: the stage's own gather record [ntot][SV_US] and its
   // derivative values [ntot][16] (rx ry ux uy lu vx vy lv, cxx_x cxx_y, cxy_x
@@ -294,6 +302,7 @@ __device__ __forceinline__ double uin_now(const sv_physk &P, const sv_ctrl *C, d
   if (P.u_control != 1) return uin0;
   bool set = C->uin_set != 0;
   double v = C->uin_ramp;
+#pragma unroll
   for (int q = 1; q < s; q++) {
     const double t = C->time0 + C->RKc[q - 1];
     if (t <= P.ramp_time) {
@@ -415,6 +424,116 @@ __device__ __forceinline__ void bound_rhs(const sv_physk &P, int kind, double nx
   r_rov = r_rov - v * ts - ro * L3;
 }
 
+// A control block field by field (a copy of the whole goes through scratch
+// memory where the copy lives in registers).
+__device__ __forceinline__ void copy_ctrl(const sv_ctrl &a, sv_ctrl &b) {
+  b.dt = a.dt; b.time = a.time; b.time0 = a.time0; b.dt_cfl = a.dt_cfl; b.dt_par = a.dt_par;
+  b.emax_np1 = a.emax_np1; b.emax_n = a.emax_n; b.emax_nm1 = a.emax_nm1;
+#pragma unroll
+  for (int k = 0; k < 3; k++) b.RKa[k] = a.RKa[k];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    b.RKb[k] = a.RKb[k]; b.RKbmbh[k] = a.RKbmbh[k]; b.RKc[k] = a.RKc[k];
+  }
+  b.dro = a.dro;
+  b.itime = a.itime; b.dt_mode = a.dt_mode; b.flags = a.flags;
+  b.uin_ramp = a.uin_ramp; b.uin_set = a.uin_set;
+}
+
+// set_tstep (step.F90:569-622), set_tstep_PID (:624-682) and the start of
+// step_rk3_4S_2R_EE (:239-246) from the minima of the advective and viscous
+// limits over the nodes
+__device__ __forceinline__ void next_dt(const sv_physk &P, double mc, double mv, sv_ctrl &c) {
+  c.dt_cfl = 1.0 * mc * P.L_char;
+  c.dt_par = (2.0 / 3.0) * mv * P.L_char * P.L_char;
+  if (c.dt_mode == SV_DT_PID) {
+    const double fA = SV_PID_A * log(SV_PID_TOL / c.emax_np1);
+    const double fB = SV_PID_B * log(c.emax_n / SV_PID_TOL);
+    const double fC = SV_PID_C * log(SV_PID_TOL / c.emax_nm1);
+    double f = SV_PID_K * exp(fA + fB + fC);
+    f = fmax(0.5, f);
+    f = fmin(1.02, f);
+    double dt = c.dt * f;
+    const double dmax = fmin(c.dt_cfl, c.dt_par);
+    if (dt > dmax) dt = dmax;
+    c.dt = dt;
+  } else if (c.dt_mode == SV_DT_CFL) {
+    c.dt = fmin(c.dt_par, c.dt_cfl);
+  }
+  c.emax_nm1 = c.emax_n;
+  c.emax_n = c.emax_np1;
+  const double dt = c.dt;
+  c.RKa[0] = dt * SV_RKA1; c.RKa[1] = dt * SV_RKA2; c.RKa[2] = dt * SV_RKA3;
+  const double b[4] = {SV_RKB1, SV_RKB2, SV_RKB3, SV_RKB4};
+  const double bh[4] = {SV_RKBH1, SV_RKBH2, SV_RKBH3, SV_RKBH4};
+  const double cc[4] = {0.0, SV_RKA1, SV_RKA2 + SV_RKB1, 1.0};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    c.RKb[k] = dt * b[k];
+    c.RKbmbh[k] = dt * (b[k] - bh[k]);
+    c.RKc[k] = dt * cc[k];
+  }
+  c.time0 = c.time;
+}
+
+// The end of a step: mass correction value (rhs_lc.F90:871-890), emax and the
+// counters, from the nodes' mass and largest error
+__device__ __forceinline__ void end_step(const sv_segk &S, double mass, double err, sv_ctrl &c) {
+  c.dro = mass / S.volsum;
+  c.emax_np1 = fmax(err, 1.0e-16);       // step.F90:480-485
+  if (!(err == err) || !(mass == mass)) c.flags |= 1;
+  // the step's four applies of the boundary conditions ran at
+  // time0 + RKc[0..3]; the ramped inflow velocity follows the last one at
+  // time <= ramp_time (characteristic_boundaries.F90:268-283)
+  if (S.pk.u_control == 1)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double t = c.time0 + c.RKc[q];
+      if (t <= S.pk.ramp_time) {
+        c.uin_set = 1;
+        c.uin_ramp = S.pk.u_start + (S.pk.u_end - S.pk.u_start) * t / S.pk.ramp_time;
+      }
+    }
+  c.time = c.time0 + c.RKc[3];
+  c.itime = c.itime + 1;               // sunset.F90:99
+}
+
+// One wavefront's reductions over the partial results of a segment of at most
+// 128 blocks, in the order of k_reduce and k_dt (whose trees halve 1024 entries,
+// one per block): two blocks per lane, then the lanes.
+constexpr int SMALL_BLOCKS = 128;
+struct Partials {
+  dbl2 a[2][2], b[2][2];   // two blocks of the two kinds, four slices each
+  __device__ __forceinline__ void load(const sv_segk &S, const double *pa, const double *pb,
+                                       double none_a, double none_b) {
+    const int lane = (int)threadIdx.x & (SV_WAVE - 1);
+    const dbl2 *qa = reinterpret_cast<const dbl2 *>(pa) + 2 * (size_t)S.blk0;
+    const dbl2 *qb = reinterpret_cast<const dbl2 *>(pb) + 2 * (size_t)S.blk0;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int b0 = lane + k * SV_WAVE;
+      const bool in = b0 < S.nblk;
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        a[k][h] = in ? qa[2 * b0 + h] : dbl2{none_a, none_a};
+        b[k][h] = in ? qb[2 * b0 + h] : dbl2{none_b, none_b};
+      }
+    }
+  }
+};
+__device__ __forceinline__ double sum_partials(const dbl2 p[2][2]) {
+  return wave_sum(((p[0][0].x + p[0][0].y) + (p[0][1].x + p[0][1].y)) +
+                  ((p[1][0].x + p[1][0].y) + (p[1][1].x + p[1][1].y)));
+}
+__device__ __forceinline__ double max_partials(const dbl2 p[2][2]) {
+  return wave_max(fmax(fmax(fmax(p[0][0].x, p[0][0].y), fmax(p[0][1].x, p[0][1].y)),
+                       fmax(fmax(p[1][0].x, p[1][0].y), fmax(p[1][1].x, p[1][1].y))));
+}
+__device__ __forceinline__ double min_partials(const dbl2 p[2][2]) {
+  return wave_min(fmin(fmin(fmin(p[0][0].x, p[0][0].y), fmin(p[0][1].x, p[0][1].y)),
+                       fmin(fmin(p[1][0].x, p[1][0].y), fmin(p[1][1].x, p[1][1].y))));
+}
+
 // The neighbour sums of one node in a stage: gradients and Laplacians before
 // the own-node term (sum_k w_k f_j), as named in the right-hand side.
 struct Sums {
@@ -443,7 +562,7 @@ __device__ __forceinline__ Own load_own(const StageArgs &a, int i) {
 // error norm contribution (stage 4).
 template <int FORM, int STAGE, bool MDIFF, bool BND>
 __device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef &nr, const Sums &S,
-                                              const Own &own) {
+                                              const Own &own, const sv_ctrl *C) {
   const int i = nr.i;
   double rx = S.rx, ry = S.ry, ux = S.ux, uy = S.uy, vx = S.vx, vy = S.vy, lu = S.lu, lv = S.lv;
   double axx = S.axx, ayx = S.ayx, axy = S.axy, ayy = S.ayy, bxy = S.bxy, byy = S.byy, cxx_l = S.cxx_l, cxy_l = S.cxy_l;
@@ -459,7 +578,6 @@ __device__ __forceinline__ double stage_point(const StageArgs &a, const NodeRef 
     ux = ux - u * sx; uy = uy - u * sy; lu = lu - u * sl;
     vx = vx - v * sx; vy = vy - v * sy; lv = lv - v * sl;
     const sv_physk &P = a.seg[nr.sg].pk;
-    const sv_ctrl *C = a.ctrl + nr.sg;
     // calc_rhs_ro (rhs_lc.F90:127-141)
     const double r_ro = -ro * (ux + vy + 0.0) - (u * rx + v * ry + 0.0 * 0.0);
     int bkind = -1;        // boundary node kind (BND), -1 interior
@@ -677,7 +795,8 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
   double emax_loc = 0.0;
   if (act) {
     const Sums S{rx, ry, ux, uy, vx, vy, lu, lv, axx, ayx, axy, ayy, bxy, byy, cxx_l, cxy_l, cyy_l, q1x, q1y, q2x, q2y, q3x, q3y};
-    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S, load_own<FORM, STAGE>(a, nr.i));
+    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S, load_own<FORM, STAGE>(a, nr.i),
+                                                   a.ctrl + nr.sg);
   }
   if (STAGE == 4) {
     emax_loc = wave_max(emax_loc);
@@ -793,6 +912,10 @@ __global__ __launch_bounds__(NB * NW) void k_stage_h(StageArgs a) {
   for (int u = 0; u < U; u++) load(0, u, 2 * u < K ? p0 : OUT_OF_RANGE);
   Own own;
   if (NW > 1 && w == 0) own = load_own<FORM, STAGE>(a, nr.ii);
+  // the step's control values, made here by every workgroup (small node sets)
+  constexpr bool DT = NW > 1 && STAGE == 1;
+  Partials lim;
+  if (DT && w == 0) lim.load(a.seg[nr.sg], a.pcfl, a.pvisc, 1.0e10, 1.0e10);
   halo_stage<NB, NB * NW>(
       hx, nh, keys, [&](int j) { return load_g<FORM>(a.G, j); },
       [&](int h, int fl, Rec9 r) {
@@ -854,11 +977,20 @@ __global__ __launch_bounds__(NB * NW) void k_stage_h(StageArgs a) {
     take_sums(hl, conf);
     if (FORM == SV_FORM_LC) take_sums(psums, psi);
   }
+  const sv_ctrl *C = a.ctrl + nr.sg;
+  sv_ctrl cn;
+  if (DT) {
+    const sv_segk &S = a.seg[nr.sg];
+    copy_ctrl(*C, cn);
+    next_dt(S.pk, min_partials(lim.a), min_partials(lim.b), cn);
+    if (nr.i == S.base) copy_ctrl(cn, a.ctrl_out[nr.sg]);
+    C = &cn;
+  }
   double emax_loc = 0.0;
   if (act) {
     const Sums S{rx, ry, ux, uy, vx, vy, lu, lv, axx, ayx, axy, ayy, bxy, byy, cxx_l, cxy_l,
                  cyy_l, q1x, q1y, q2x, q2y, q3x, q3y};
-    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S, own);
+    emax_loc = stage_point<FORM, STAGE, MDIFF, BND>(a, nr, S, own, C);
   }
   if (STAGE == 4) {
     emax_loc = wave_max(emax_loc);
@@ -1019,7 +1151,6 @@ __global__ __launch_bounds__(1024) void k_reduce(const sv_segk *seg, const doubl
   __shared__ double s1[1024], s2[1024];
   const sv_segk &S = seg[blockIdx.x];
   sv_ctrl *ctrl = ctrl_all + blockIdx.x;
-  const double volsum = S.volsum;
   double a = 0.0, m = 0.0;
   // a thread takes the four slices of a block at a time
   static_assert(SPB == 4, "two double2 per block");
@@ -1041,24 +1172,8 @@ __global__ __launch_bounds__(1024) void k_reduce(const sv_segk *seg, const doubl
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    ctrl->dro = s1[0] / volsum;
-    ctrl->emax_np1 = fmax(s2[0], 1.0e-16);       // step.F90:480-485
-    if (!(s2[0] == s2[0]) || !(s1[0] == s1[0])) ctrl->flags |= 1;
-    // the step's four applies of the boundary conditions ran at
-    // time0 + RKc[0..3]; the ramped inflow velocity follows the last one at
-    // time <= ramp_time (characteristic_boundaries.F90:268-283)
-    if (S.pk.u_control == 1)
-      for (int q = 0; q < 4; q++) {
-        const double t = ctrl->time0 + ctrl->RKc[q];
-        if (t <= S.pk.ramp_time) {
-          ctrl->uin_set = 1;
-          ctrl->uin_ramp = S.pk.u_start + (S.pk.u_end - S.pk.u_start) * t / S.pk.ramp_time;
-        }
-      }
-    ctrl->time = ctrl->time0 + ctrl->RKc[3];
-    ctrl->itime = ctrl->itime + 1;               // sunset.F90:99
-  }
+  if (threadIdx.x != 0) return;
+  end_step(S, s1[0], s2[0], *ctrl);
 }
 
 struct ApplyArgs {
@@ -1072,6 +1187,8 @@ struct ApplyArgs {
   double *pcfl, *pvisc;  // minima for set_tstep per slice
   const int *bidx;       // boundary nodes (nullable), as StageArgs
   const double *brec;
+  const double *pmass, *perr;   // REDUCE: partial results, control values (StageArgs)
+  sv_ctrl *ctrl_out;
 };
 
 // rho -= drho (rhs_lc.F90:887-889); the gather record: u = rou/rho
@@ -1079,14 +1196,35 @@ struct ApplyArgs {
 // (step.F90:579-602).  The record is written here as a whole (the filter
 // writing psi and c and this kernel ro, u, v made two partial writes of
 // every line).
-template <int FORM>
+// REDUCE: the end of the step as well (k_reduce's work), by every wavefront of
+// a small node set.
+template <int FORM, bool REDUCE>
 __global__ __launch_bounds__(BS) void k_apply_state(ApplyArgs a) {
   const NodeRef nr = node_ref(a.blk_seg, a.seg, sv_xcd_block());
   const int i = nr.i;
+  const sv_ctrl *C = a.ctrl ? a.ctrl + nr.sg : nullptr;
+  double dro = 0.0;
+  if (REDUCE) {
+    const sv_segk &S = a.seg[nr.sg];
+    Partials p;
+    p.load(S, a.pmass, a.perr, 0.0, 0.0);
+    const double mass = sum_partials(p.a);
+    dro = mass / S.volsum;
+    if (i - (int)threadIdx.x == S.base) {   // the segment's first block
+      const double err = max_partials(p.b);
+      if (threadIdx.x == 0) {
+        sv_ctrl n;
+        copy_ctrl(*C, n);
+        end_step(S, mass, err, n);
+        copy_ctrl(n, a.ctrl_out[nr.sg]);
+      }
+    }
+  } else if (C) {
+    dro = C->dro;
+  }
   double mc = 1.0e10, mv = 1.0e10;
   if (nr.act) {
     const sv_physk &P = a.seg[nr.sg].pk;
-    const double dro = a.ctrl ? a.ctrl[nr.sg].dro : 0.0;
     double f[6];
     load_u(a.Uf, i, f);
     f[0] = f[0] - dro;
@@ -1097,7 +1235,8 @@ __global__ __launch_bounds__(BS) void k_apply_state(ApplyArgs a) {
         const double *br = a.brec + (size_t)SV_BREC * jb;
         bk = (int)br[0];
         // the apply after filter_variables (step.F90:498)
-        if (a.ctrl) bound_apply(P, bk, uin_now(P, a.ctrl + nr.sg, br[3], 1), f);
+        // (the values of the step that has just ended)
+        if (C) bound_apply(P, bk, uin_now(P, C, br[3], REDUCE ? 5 : 1), f);
       }
     }
     store_u(a.U, i, f);
@@ -1123,15 +1262,12 @@ __global__ __launch_bounds__(BS) void k_apply_state(ApplyArgs a) {
   if ((threadIdx.x & 63) == 0) { a.pcfl[i >> 6] = mc; a.pvisc[i >> 6] = mv; }
 }
 
-// set_tstep (step.F90:569-622) + set_tstep_PID (:624-682) + the start of
-// step_rk3_4S_2R_EE (:239-246)
-// one block per segment
+// the next step's control values; one block per segment
 __global__ __launch_bounds__(1024) void k_dt(const sv_segk *seg, const double *pcfl,
                                              const double *pvisc, sv_ctrl *ctrl_all) {
   __shared__ double s1[1024], s2[1024];
   const sv_segk &S = seg[blockIdx.x];
   sv_ctrl *c = ctrl_all + blockIdx.x;
-  const double L_char = S.pk.L_char;
   double a = 1.0e10, m = 1.0e10;
   const double2 *p = reinterpret_cast<const double2 *>(pcfl) + 2 * (size_t)S.blk0;
   const double2 *q = reinterpret_cast<const double2 *>(pvisc) + 2 * (size_t)S.blk0;
@@ -1152,35 +1288,7 @@ __global__ __launch_bounds__(1024) void k_dt(const sv_segk *seg, const double *p
     __syncthreads();
   }
   if (threadIdx.x != 0) return;
-  c->dt_cfl = 1.0 * s1[0] * L_char;
-  c->dt_par = (2.0 / 3.0) * s2[0] * L_char * L_char;
-  if (c->dt_mode == SV_DT_PID) {
-    const double fA = SV_PID_A * log(SV_PID_TOL / c->emax_np1);
-    const double fB = SV_PID_B * log(c->emax_n / SV_PID_TOL);
-    const double fC = SV_PID_C * log(SV_PID_TOL / c->emax_nm1);
-    double f = SV_PID_K * exp(fA + fB + fC);
-    f = fmax(0.5, f);
-    f = fmin(1.02, f);
-    double dt = c->dt * f;
-    const double dmax = fmin(c->dt_cfl, c->dt_par);
-    if (dt > dmax) dt = dmax;
-    c->dt = dt;
-  } else if (c->dt_mode == SV_DT_CFL) {
-    c->dt = fmin(c->dt_par, c->dt_cfl);
-  }
-  c->emax_nm1 = c->emax_n;
-  c->emax_n = c->emax_np1;
-  const double dt = c->dt;
-  c->RKa[0] = dt * SV_RKA1; c->RKa[1] = dt * SV_RKA2; c->RKa[2] = dt * SV_RKA3;
-  const double b[4] = {SV_RKB1, SV_RKB2, SV_RKB3, SV_RKB4};
-  const double bh[4] = {SV_RKBH1, SV_RKBH2, SV_RKBH3, SV_RKBH4};
-  const double cc[4] = {0.0, SV_RKA1, SV_RKA2 + SV_RKB1, 1.0};
-  for (int k = 0; k < 4; k++) {
-    c->RKb[k] = dt * b[k];
-    c->RKbmbh[k] = dt * (b[k] - bh[k]);
-    c->RKc[k] = dt * cc[k];
-  }
-  c->time0 = c->time;
+  next_dt(S.pk, s1[0], s2[0], *c);
 }
 
 StageArgs stage_args(sv_ctx *c, int stage, const double *Gin, double *Gout) {
@@ -1296,12 +1404,20 @@ int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
   auto mark = [&]() {
     if (ev) (void)hipEventRecord(ev[ke++], c->stream);
   };
+  // small node sets: stage 1 makes the step's control values in the second
+  // array and the last kernel the next ones in the first
+  const bool small = c->L.halo && c->L.split && nb <= SMALL_BLOCKS;
+  sv_ctrl *cs = small ? c->ctrl + c->nseg : c->ctrl;
   mark();
-  k_dt<<<c->nseg, 1024, 0, c->stream>>>(c->segk, pc, pv, c->ctrl);
+  if (!small) k_dt<<<c->nseg, 1024, 0, c->stream>>>(c->segk, pc, pv, c->ctrl);
   mark();
   StageArgs as[4] = {stage_args(c, 1, c->GA, c->GB), stage_args(c, 2, c->GB, c->GA),
                      stage_args(c, 3, c->GA, c->GB), stage_args(c, 4, c->GB, c->GA)};
   as[3].partial = pe;
+  as[0].pcfl = pc;
+  as[0].pvisc = pv;
+  as[0].ctrl_out = cs;
+  for (int k = 1; k < 4; k++) as[k].ctrl = cs;
   if (tape)
     for (int k = 0; k < 4; k++) { as[k].tapeG = tape[2 * k]; as[k].tapeD = tape[2 * k + 1]; }
   launch_stage<FORM, 1>(c, as[0], nb);
@@ -1330,7 +1446,7 @@ int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
   f.lcol = c->L.lcol;
   launch_filter(c, f, nb);
   mark();
-  k_reduce<<<c->nseg, 1024, 0, c->stream>>>(c->segk, pm, pe, c->ctrl);
+  if (!small) k_reduce<<<c->nseg, 1024, 0, c->stream>>>(c->segk, pm, pe, c->ctrl);
   mark();
   ApplyArgs ap{};
   ap.blk_seg = c->blk_seg;
@@ -1339,12 +1455,16 @@ int step_form(sv_ctx *c, hipEvent_t *ev, double *const *tape) {
   ap.U = c->U;
   ap.G = c->GA;
   ap.s = c->L.s;
-  ap.ctrl = c->ctrl;
+  ap.ctrl = cs;
+  ap.pmass = pm;
+  ap.perr = pe;
+  ap.ctrl_out = c->ctrl;
   ap.pcfl = pc;
   ap.pvisc = pv;
   ap.bidx = c->L.bidx;
   ap.brec = c->L.brec;
-  k_apply_state<FORM><<<nb, BS, 0, c->stream>>>(ap);
+  if (small) k_apply_state<FORM, true><<<nb, BS, 0, c->stream>>>(ap);
+  else k_apply_state<FORM, false><<<nb, BS, 0, c->stream>>>(ap);
   mark();
   SV_HIP(c, hipGetLastError());
   return 0;
@@ -1368,8 +1488,8 @@ int sv_dev_init_state(sv_ctx *c) {
   ap.pvisc = c->partial + 3 * (size_t)nb * SPB;
   ap.bidx = c->L.bidx;
   ap.brec = c->L.brec;
-  if (c->cfg.form == SV_FORM_LC) k_apply_state<SV_FORM_LC><<<nb, BS, 0, c->stream>>>(ap);
-  else k_apply_state<SV_FORM_DI><<<nb, BS, 0, c->stream>>>(ap);
+  if (c->cfg.form == SV_FORM_LC) k_apply_state<SV_FORM_LC, false><<<nb, BS, 0, c->stream>>>(ap);
+  else k_apply_state<SV_FORM_DI, false><<<nb, BS, 0, c->stream>>>(ap);
   SV_HIP(c, hipGetLastError());
   SV_HIP(c, hipStreamSynchronize(c->stream));
   return 0;

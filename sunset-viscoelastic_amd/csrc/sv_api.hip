@@ -601,7 +601,7 @@ static int ensure_state_buffers(sv_ctx *c) {
   SV_HIP(c, hipMemsetAsync(c->GB, 0, ng, c->stream));
   c->npartial = 4 * c->nblk * (SV_BLOCK / SV_WAVE);   // four kinds, one per slice
   if (sv_alloc(c, (void **)&c->partial, sizeof(double) * (c->npartial + 8)) ||
-      sv_alloc(c, (void **)&c->ctrl, sizeof(sv_ctrl)) ||
+      sv_alloc(c, (void **)&c->ctrl, 2 * sizeof(sv_ctrl)) ||
       sv_alloc(c, (void **)&c->fx, sizeof(double) * c->ntot) ||
       sv_alloc(c, (void **)&c->segk, sizeof(sv_segk)) ||
       sv_alloc(c, (void **)&c->blk_seg, sizeof(int) * c->nblk))

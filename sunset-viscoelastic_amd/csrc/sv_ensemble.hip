@@ -121,7 +121,7 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
                           D * N, D * N, D * SV_US * N, D * SV_US * N, D * SV_US * N,
                           D * SV_US * N, D * E->gs * N, D * E->gs * N,
                           D * (4 * (size_t)blocks * (SV_BLOCK / SV_WAVE) + 8),
-                          sizeof(sv_ctrl) * nmembers,
+                          2 * sizeof(sv_ctrl) * nmembers,
                           sizeof(sv_segk) * nmembers, I * (size_t)blocks};
   for (size_t k = 0; k < sizeof(sizes) / sizeof(sizes[0]); k++)
     if (sv_alloc(E, bufs[k], sizes[k])) return fail(SV_E_NOMEM);

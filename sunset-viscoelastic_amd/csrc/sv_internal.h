@@ -281,7 +281,7 @@ struct sv_ctx {
   // sum of node volumes (the mass-correction denominator), of the current ones
   double volsum = 0.0;
   bool have_volsum = false;
-  sv_ctrl *ctrl = nullptr;  // [nseg]
+  sv_ctrl *ctrl = nullptr;  // [nseg], then as many within a step (small node sets)
   // segments: ntot = padded node count of the state arrays, nblk = blocks
   int nseg = 1, ntot = 0, nblk = 0;
   sv_segk *segk = nullptr;  // [nseg]
