@@ -870,10 +870,10 @@ int sv_dev_to_caller_order(sv_ctx *c, int nf, const double *in, double *out) {
   return 0;
 }
 
-int sv_dev_get_fields(sv_ctx *c, double *out) {
-  const int n = c->npfb;
-  k_get_fields<<<(n + 255) / 256, 256, 0, c->stream>>>(n, c->L.perm, c->U, c->GA, c->gs,
-                                                       c->cfg.form == SV_FORM_LC, out);
+int sv_dev_get_fields(sv_ctx *c, int base, int n, double *out) {
+  k_get_fields<<<(n + 255) / 256, 256, 0, c->stream>>>(
+      n, c->L.perm + base, c->U + (size_t)base * SV_US, c->GA + (size_t)base * c->gs, c->gs,
+      c->cfg.form == SV_FORM_LC, out);
   SV_HIP(c, hipGetLastError());
   return 0;
 }

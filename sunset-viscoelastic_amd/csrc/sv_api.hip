@@ -995,42 +995,22 @@ int sv_ensemble_get_state(sv_ctx *c, int32_t member, double *ro, double *rou, do
            c->nseg);
   if (int rc = set_device(c)) return rc;
   const sv_segk &S = c->hseg[member];
-  const double *U = c->U + (size_t)S.base * SV_US;
-  const double *GA = c->GA + (size_t)S.base * c->gs;
-  const std::vector<int> &P = c->is_ensemble ? c->member_perm[member] : c->L.hperm;
   const size_t n = (size_t)S.npfb;
-  if (!c->is_ensemble && c->L.perm) {
-    // fields picked and put in the caller's order on the device, then one
-    // copy per field (the host scatter of eleven fields cost ~50 ms at 1M)
-    if (!c->fields_buf && sv_alloc(c, (void **)&c->fields_buf, sizeof(double) * 12 * n))
-      return SV_E_NOMEM;
-    if (int rc = sv_dev_get_fields(c, c->fields_buf)) return rc;
-    SV_HIP(c, hipStreamSynchronize(c->stream));
-    double *dst[11] = {ro, rou, rov, u, v, pxx, pxy, pyy, cxx, cxy, cyy};
-    const bool lc_ = c->cfg.form == SV_FORM_LC;
-    for (int q = 0; q < 11; q++)
-      if (dst[q] && (lc_ || q < 5 || q > 7))
-        SV_HIP(c, hipMemcpy(dst[q], c->fields_buf + (size_t)q * n, sizeof(double) * n,
-                            hipMemcpyDeviceToHost));
-    return 0;
-  }
+  // fields picked and put in the caller's order on the device, then one copy
+  // per field (the host scatter of eleven fields cost ~50 ms at 1M nodes, and
+  // 9 of 29 ms for an ensemble of 566k)
+  size_t most = 0;
+  for (const sv_segk &s : c->hseg) most = std::max(most, (size_t)s.npfb);
+  if (!c->fields_buf && sv_alloc(c, (void **)&c->fields_buf, sizeof(double) * 12 * most))
+    return SV_E_NOMEM;
+  if (int rc = sv_dev_get_fields(c, S.base, S.npfb, c->fields_buf)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));
-  // two contiguous copies of the member's records, fields picked on the host
-  // (a strided copy of 8-byte rows is far slower than the whole record array)
-  std::vector<double> hu(n * SV_US), hg(n * c->gs);
-  SV_HIP(c, hipMemcpy(hu.data(), U, sizeof(double) * hu.size(), hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(hg.data(), GA, sizeof(double) * hg.size(), hipMemcpyDeviceToHost));
+  double *dst[11] = {ro, rou, rov, u, v, pxx, pxy, pyy, cxx, cxy, cyy};
   const bool lc = c->cfg.form == SV_FORM_LC;
-  struct { double *dst; const double *src; int stride; } m[] = {
-      {ro, hu.data() + 0, SV_US}, {rou, hu.data() + 1, SV_US}, {rov, hu.data() + 2, SV_US},
-      {u, hg.data() + SV_G_U, c->gs}, {v, hg.data() + SV_G_V, c->gs},
-      {pxx, lc ? hu.data() + 3 : nullptr, SV_US}, {pxy, lc ? hu.data() + 4 : nullptr, SV_US},
-      {pyy, lc ? hu.data() + 5 : nullptr, SV_US},
-      {cxx, hg.data() + SV_G_CXX, c->gs}, {cxy, hg.data() + SV_G_CXY, c->gs},
-      {cyy, hg.data() + SV_G_CYY, c->gs}};
-  for (auto &e : m)
-    if (e.dst && e.src)
-      for (size_t k = 0; k < n; k++) e.dst[P[k]] = e.src[k * e.stride];   // loop order -> caller's
+  for (int q = 0; q < 11; q++)
+    if (dst[q] && (lc || q < 5 || q > 7))
+      SV_HIP(c, hipMemcpy(dst[q], c->fields_buf + (size_t)q * n, sizeof(double) * n,
+                          hipMemcpyDeviceToHost));
   return 0;
 }
 

@@ -110,13 +110,13 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
   E->L.nnz = sell;
   const size_t N = (size_t)E->ntot, D = sizeof(double), I = sizeof(int);
   sv_loopl &EL = E->L;
-  void **bufs[] = {(void **)&EL.off, (void **)&EL.cnt, (void **)&EL.cnt_small,
+  void **bufs[] = {(void **)&EL.off, (void **)&EL.cnt, (void **)&EL.cnt_small, (void **)&EL.perm,
                    (void **)&EL.col, (void **)&EL.w3, (void **)&EL.wh, (void **)&EL.gsx, (void **)&EL.gsy, (void **)&EL.lsum,
                    (void **)&EL.hsum, (void **)&EL.vol, (void **)&EL.s, (void **)&E->fx,
                    (void **)&E->U, (void **)&E->Uf, (void **)&E->reg, (void **)&E->eacc,
                    (void **)&E->GA, (void **)&E->GB, (void **)&E->partial, (void **)&E->ctrl,
                    (void **)&E->segk, (void **)&E->blk_seg};
-  const size_t sizes[] = {sizeof(int64_t) * (EL.nslices + 1), I * N, I * N,
+  const size_t sizes[] = {sizeof(int64_t) * (EL.nslices + 1), I * N, I * N, I * N,
                           I * (size_t)sell, 3 * D * (size_t)sell, D * (size_t)sell, D * N, D * N, D * N, D * N, D * N,
                           D * N, D * N, D * SV_US * N, D * SV_US * N, D * SV_US * N,
                           D * SV_US * N, D * E->gs * N, D * E->gs * N,
@@ -163,7 +163,6 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
     const int64_t sb = sell_base[m];
     for (int k = 0; k < S.nblk; k++) bseg[S.blk0 + k] = m;
     const sv_loopl &CL = c->L;
-    E->member_perm.push_back(CL.hperm);
     int rc = copy_d2d(E, EL.off + b / SV_WAVE, CL.off, sizeof(int64_t) * (size_t)CL.nslices);
     if (!rc) rc = sv_dev_offset_i64(E, EL.off + b / SV_WAVE, CL.nslices, sb);
     if (!rc) rc = copy_d2d(E, EL.col + sb, CL.col, I * (size_t)CL.nnz);
@@ -171,6 +170,7 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
     if (!rc) rc = copy_d2d(E, EL.w3 + 3 * sb, CL.w3, 3 * D * (size_t)CL.nnz);
     if (!rc) rc = copy_d2d(E, EL.wh + sb, CL.wh, D * (size_t)CL.nnz);
     if (!rc) rc = copy_d2d(E, EL.cnt + b, CL.cnt, I * n);
+    if (!rc) rc = copy_d2d(E, EL.perm + b, CL.perm, I * n);
     if (!rc) rc = copy_d2d(E, EL.cnt_small + b, CL.cnt_small, I * n);
     const double *nsrc[7] = {CL.gsx, CL.gsy, CL.lsum, CL.hsum, CL.vol, CL.s, c->fx};
     double *ndst[7] = {EL.gsx, EL.gsy, EL.lsum, EL.hsum, EL.vol, EL.s, E->fx};

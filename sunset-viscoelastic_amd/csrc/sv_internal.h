@@ -156,7 +156,8 @@ struct sv_loopl {
   int4 *krange = nullptr;
   double *gsx = nullptr, *gsy = nullptr, *lsum = nullptr, *hsum = nullptr, *vol = nullptr;
   double *s = nullptr;
-  int *perm = nullptr, *iperm = nullptr;
+  int *perm = nullptr;      // caller's node of a slot (of the slot's ensemble member)
+  int *iperm = nullptr;
   std::vector<int> hperm;
   // Per-block neighbour halos: the distinct neighbour slots of the hb
   // slots of block b are hidx[hoff[b] .. hoff[b+1]) (ascending); lcol[sv_pair(e)]
@@ -293,8 +294,6 @@ struct sv_ctx {
   int halo_sweeps = 1;      // 1: stage neighbour halos in LDS when they fit
   int adj_lanes = 0;        // lanes per node of the adjoint's transposed gathers
                             // (1, 4; 0: by node count), read by sv_adj_setup
-  // ensemble: loop-slot -> member-node permutation of each member
-  std::vector<std::vector<int>> member_perm;
   // ensemble launch groups: the blocks of the members of one LABFM order,
   // launched together with their own LDS halo budget (blist: logical blocks,
   // device).  lgroup_mode: -1 untuned, 0 one launch over all blocks, 1 one
@@ -403,9 +402,10 @@ int sv_dev_mass_correct(sv_ctx *c, double *ro, hipStream_t st);
 // <-> loop-order records on the context's stream
 int sv_dev_gather_records(sv_ctx *c, double *dst, const double *const f[6]);
 int sv_dev_scatter_records(sv_ctx *c, const double *src, double *const f[6]);
-// the eleven fields of sv_get_state in caller order into out[11][npfb]
-// (single context; the psi rows are left untouched in DI)
-int sv_dev_get_fields(sv_ctx *c, double *out);
+// the eleven fields of sv_get_state of the n nodes from slot base on (one
+// segment), in caller order, into out[11][n] (the psi rows are left untouched
+// in DI)
+int sv_dev_get_fields(sv_ctx *c, int base, int n, double *out);
 // nf loop-order fields (in[f][npfb]) to the caller's order (out[f][npfb])
 int sv_dev_to_caller_order(sv_ctx *c, int nf, const double *in, double *out);
 // 0 if p is device memory of the context's device in this library's HIP
