@@ -202,10 +202,12 @@ int sv_get_timing(sv_ctx *ctx, const char *what, double *ms);
  *       right-hand-side sweep both ways and keeps the faster; -1 re-tunes.
  *       sv_get_timing "ensemble_groups" reports the mode,
  *       "ensemble_groups_tune_<mode>" the sample times.
- *   "adj_lanes" (0, 1, 4; read by sv_adj_setup): lanes per node of the
- *       adjoint's transposed gathers; 4 splits each node's links over a quad
- *       of lanes (node sets too small to fill the chip at one lane per node),
- *       0 (default) picks 4 below 8 waves per CU. */
+ *   "adj_lanes" (0, 1, 4; read by sv_adj_setup): 0 (default) stages the
+ *       neighbour halos of the adjoint's transposed gathers in LDS where they
+ *       fit; 1 and 4 gather from memory with that many lanes per node (4 splits
+ *       each node's links over a quad of lanes, for node sets too small to fill
+ *       the chip at one), as 0 does where they do not fit, with 4 below 8 waves
+ *       per CU. */
 int sv_set_option(sv_ctx *ctx, const char *key, double value);
 
 /* ---- derivative operators: derivatives.F90 ------------------------------ */

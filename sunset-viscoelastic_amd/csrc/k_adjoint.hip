@@ -22,12 +22,16 @@
 // inside the transposed gather of stage k (two buffer sets, ping-pong), and
 // the pointwise part of stage 4 inside the fused mass-correction + filter
 // adjoint: one step's adjoint is six launches (a per-segment sum, the filter,
-// four transposed gathers).  Rollouts keep the state every `checkpoint`
+// four transposed gathers; five of a small node set, whose filter makes the sum).  Rollouts keep the state every `checkpoint`
 // steps; the adjoint recomputes one checkpoint interval with the tape on and
-// walks it backwards.
+// walks it backwards; the last interval's tape is written by the rollout itself
+// where memory allows.
 #include <string.h>
 
+#include <algorithm>
+
 #include "sv_internal.h"
+#include "sweep.h"
 
 namespace {
 
@@ -133,19 +137,40 @@ struct PointArgs {
                              // d/d(visc_solvent), d/d(cp), d/d(lambda), d/d(eps)
 };
 
+// what the pointwise adjoint reads of a node: its tape, the sums of its weights
+// and its parameter accumulators
+struct PointOwn {
+  double g[6], sx, sy, sl;
+  double2 D[7], p0, p1;
+};
+
+__device__ __forceinline__ PointOwn load_point(const PointArgs &a, int i) {
+  PointOwn o;
+  ld6(a.tG + (size_t)i * SV_US, o.g);
+  const double2 *d = reinterpret_cast<const double2 *>(a.tD + (size_t)i * SV_TAPE_D);
+#pragma unroll
+  for (int q = 0; q < 7; q++) o.D[q] = d[q];
+  o.sx = a.gsx[i]; o.sy = a.gsy[i]; o.sl = a.lsum[i];
+  if (a.pacc) {
+    const double2 *p = reinterpret_cast<const double2 *>(a.pacc + (size_t)i * 4);
+    o.p0 = p[0];
+    o.p1 = p[1];
+  }
+  return o;
+}
+
 // the pointwise adjoint of one (active) node, Rbar given in registers
 template <bool MDIFF>
 __device__ __forceinline__ void adj_point_node(const PointArgs &a, const NodeRef &nr,
-                                               const double rb[6]) {
+                                               const double rb[6], const PointOwn &own) {
   const int i = nr.i;
   const sv_physk &P = a.seg[nr.sg].pk;
-  double g[6];
-  ld6(a.tG + (size_t)i * SV_US, g);
+  const double *g = own.g;
   const double ro = g[0], u = g[1], v = g[2], cxx = g[3], cxy = g[4], cyy = g[5];
-  const double *D = a.tD + (size_t)i * SV_TAPE_D;
-  const double rx = D[0], ry = D[1], ux = D[2], uy = D[3], vx = D[5], vy = D[6];
-  const double gxx_x = D[8], gxx_y = D[9], gxy_x = D[10], gxy_y = D[11];
-  const double gyy_x = D[12], gyy_y = D[13];
+  const double rx = own.D[0].x, ry = own.D[0].y, ux = own.D[1].x, uy = own.D[1].y;
+  const double lu = own.D[2].x, vx = own.D[2].y, vy = own.D[3].x, lv = own.D[3].y;
+  const double gxx_x = own.D[4].x, gxx_y = own.D[4].y, gxy_x = own.D[5].x, gxy_y = own.D[5].y;
+  const double gyy_x = own.D[6].x, gyy_y = own.D[6].y;
   const double Ab = rb[0], Bu = rb[1], Bv = rb[2], Xb = rb[3], Yb = rb[4], Zb = rb[5];
   // forward intermediates the adjoint needs
   const double r_ro = -ro * (ux + vy) - (u * rx + v * ry);
@@ -206,7 +231,7 @@ __device__ __forceinline__ void adj_point_node(const PointArgs &a, const NodeRef
   double blxx = 0, blxy = 0, blyy = 0;
   if (MDIFF) { blxx = P.Mdiff * Xb; blxy = P.Mdiff * Yb; blyy = P.Mdiff * Zb; }
   // D_i = sum_k w G_j - G_i * sum: own-node share
-  const double sx = a.gsx[i], sy = a.gsy[i], sl = a.lsum[i];
+  const double sx = own.sx, sy = own.sy, sl = own.sl;
   double o[6];
   o[0] = bro - (sx * brx + sy * bry);
   o[1] = bu - (sx * bux + sy * buy + sl * blu);
@@ -227,9 +252,8 @@ __device__ __forceinline__ void adj_point_node(const PointArgs &a, const NodeRef
   if (a.pacc) {
     // r_rou, r_rov hold visc_solvent*(lu, lv) and cp*(div c); the conformation
     // source fr*(c - I) holds lambda and eps through fr
-    const double lu = D[4], lv = D[7];
     double2 *Pq = reinterpret_cast<double2 *>(a.pacc + (size_t)i * 4);
-    double2 p0 = Pq[0], p1 = Pq[1];
+    double2 p0 = own.p0, p1 = own.p1;
     p0.x += Bu * lu + Bv * lv;
     p0.y += Bu * (gxx_x + gxy_y) + Bv * (gxy_x + gyy_y);
     p1.x += bfr * (-fr / P.lambda);
@@ -245,7 +269,7 @@ __global__ __launch_bounds__(AB) void k_adj_point(PointArgs a) {
   if (!nr.act) return;
   double rb[6];
   ld6(a.Rbar + (size_t)nr.i * SV_US, rb);
-  adj_point_node<MDIFF>(a, nr, rb);
+  adj_point_node<MDIFF>(a, nr, rb, load_point(a, nr.i));
 }
 
 // ---- transposed gather + G->U + RK register recurrences ------------------
@@ -254,7 +278,7 @@ struct TransArgs {
   const sv_segk *seg;
   const int64_t *toff;       // transposed SELL
   const int *tcnt, *tcol;
-  const double *twx, *twy, *twl;
+  const double *tw3;
   const double *dbar, *dbarm, *own;
   const double *tG;          // stage tape (ro, u, v of node j)
   const sv_ctrl *ctrl;       // RK coefficients (dt included)
@@ -265,23 +289,99 @@ struct TransArgs {
   double *psum;              // STAGE 1: per-sub-block sum of Ubar_ro (mass correction)
   PointArgs nxt;             // STAGE 2..4: the pointwise adjoint of stage STAGE-1,
                              // fused (its Rbar stays in registers)
+  const int4 *krange;        // halos of the transposed lists (k_adj_trans_h)
+  const int64_t *hoff;
+  const int *hidx;
+  const uint16_t *lcol;
 };
 
-// one transposed link: the stencil-adjoint record d (+ m with Mdiff) of node i
-// weighted by the link's gradient and Laplacian weights
+// a node's own values in a transposed gather
+struct TransOwn {
+  double o[6], g[6], rg[6];
+  PointOwn p;
+};
+
+template <int STAGE>
+__device__ __forceinline__ TransOwn load_own(const TransArgs &a, int j) {
+  TransOwn w;
+  ld6(a.own + (size_t)j * SV_US, w.o);
+  ld6(a.tG + (size_t)j * SV_US, w.g);
+  if (STAGE >= 1) ld6(a.regbar + (size_t)j * SV_US, w.rg);
+  if (STAGE >= 2) w.p = load_point(a.nxt, j);
+  return w;
+}
+
+// Own-node part of a transposed gather: G -> U and the RK register recurrences.
+// Returns Ubar_ro (STAGE 1).
+template <int STAGE, bool MDIFF>
+__device__ __forceinline__ double trans_point(const TransArgs &a, const NodeRef &nr,
+                                              const double acc[6], const TransOwn &w) {
+  const int j = nr.i;
+  double G[6];
+#pragma unroll
+  for (int f = 0; f < 6; f++) G[f] = w.o[f] + acc[f];
+  // G = (ro, rou/ro, rov/ro, c) -> U
+  const double ooro = 1.0 / w.g[0];
+  double Ub[6];
+  Ub[0] = G[0] - (G[1] * w.g[1] + G[2] * w.g[2]) * ooro;
+  Ub[1] = G[1] * ooro;
+  Ub[2] = G[2] * ooro;
+  Ub[3] = G[3]; Ub[4] = G[4]; Ub[5] = G[5];
+  if constexpr (STAGE == 0) {
+    st6(a.Ubar + (size_t)j * SV_US, Ub);
+  } else if constexpr (STAGE == 1) {
+#pragma unroll
+    for (int f = 0; f < 6; f++) Ub[f] += w.rg[f];
+    Ub[3] += a.seed;
+    Ub[5] += a.seed;
+    st6(a.Ubar + (size_t)j * SV_US, Ub);
+    return Ub[0];
+  } else {
+    // U_k = reg_{k-2} + a_{k-1} R_{k-1};  reg_{k-1} = reg_{k-2} + b_{k-1} R_{k-1}
+    const sv_ctrl *C = a.ctrl + nr.sg;
+    const double ra = C->RKa[STAGE - 2], rbk = C->RKb[STAGE - 2];
+    double rg[6], Rn[6];
+#pragma unroll
+    for (int f = 0; f < 6; f++) {
+      Rn[f] = ra * Ub[f] + rbk * w.rg[f];
+      rg[f] = Ub[f] + w.rg[f];
+    }
+    st6(a.regbar + (size_t)j * SV_US, rg);
+    adj_point_node<MDIFF>(a.nxt, nr, Rn, w.p);
+  }
+  return 0.0;
+}
+
+// stencil-adjoint record of a node: d0..d6, and with Mdiff m0, m1.  (Named
+// members: arrays of them end up in scratch memory.)
+struct DRec {
+  double2 d0, d1, d2, d3, d4, d5, d6, m0, m1;
+};
+template <bool MDIFF>
+__device__ __forceinline__ DRec load_rec(const double *d, const double *m) {
+  const double2 *q = reinterpret_cast<const double2 *>(d);
+  const double2 *p = reinterpret_cast<const double2 *>(m);
+  DRec r;
+  r.d0 = q[0]; r.d1 = q[1]; r.d2 = q[2]; r.d3 = q[3]; r.d4 = q[4]; r.d5 = q[5]; r.d6 = q[6];
+  if (MDIFF) { r.m0 = p[0]; r.m1 = p[1]; }
+  return r;
+}
+
+// one transposed link: the record of node i weighted by the link's gradient and
+// Laplacian weights
 template <bool MDIFF>
 __device__ __forceinline__ void trans_link(double acc[6], double wx, double wy, double wl,
-                                           const double2 d[7], const double2 m[2]) {
-  acc[0] += wx * d[0].x + wy * d[0].y;
-  acc[1] += wx * d[1].x + wy * d[1].y + wl * d[2].x;
-  acc[2] += wx * d[2].y + wy * d[3].x + wl * d[3].y;
-  acc[3] += wx * d[4].x + wy * d[4].y;
-  acc[4] += wx * d[5].x + wy * d[5].y;
-  acc[5] += wx * d[6].x + wy * d[6].y;
+                                           const DRec &r) {
+  acc[0] += wx * r.d0.x + wy * r.d0.y;
+  acc[1] += wx * r.d1.x + wy * r.d1.y + wl * r.d2.x;
+  acc[2] += wx * r.d2.y + wy * r.d3.x + wl * r.d3.y;
+  acc[3] += wx * r.d4.x + wy * r.d4.y;
+  acc[4] += wx * r.d5.x + wy * r.d5.y;
+  acc[5] += wx * r.d6.x + wy * r.d6.y;
   if (MDIFF) {
-    acc[3] += wl * m[0].x;
-    acc[4] += wl * m[0].y;
-    acc[5] += wl * m[1].x;
+    acc[3] += wl * r.m0.x;
+    acc[4] += wl * r.m0.y;
+    acc[5] += wl * r.m1.x;
   }
 }
 
@@ -311,85 +411,29 @@ __global__ __launch_bounds__(AB) void k_adj_trans(TransArgs a) {
     for (int u = 0; u < SV_ADJ_BATCH; u++) {
       const int64_t e = b + (int64_t)(k + u * LPN) * SV_WAVE;
       ix[u] = a.tcol[e];
-      wx[u] = a.twx[e];
-      wy[u] = a.twy[e];
-      wl[u] = a.twl[e];
+      wx[u] = a.tw3[sv_w3(e, 0)];
+      wy[u] = a.tw3[sv_w3(e, 1)];
+      wl[u] = a.tw3[sv_w3(e, 2)];
     }
-    double2 d[SV_ADJ_BATCH][7], m[SV_ADJ_BATCH][2];
-#pragma unroll
-    for (int u = 0; u < SV_ADJ_BATCH; u++) {
-      const double2 *r = reinterpret_cast<const double2 *>(a.dbar + (size_t)ix[u] * SV_TAPE_D);
-#pragma unroll
-      for (int q = 0; q < 7; q++) d[u][q] = r[q];
-      if (MDIFF) {
-        const double2 *rm = reinterpret_cast<const double2 *>(a.dbarm + (size_t)ix[u] * 4);
-        m[u][0] = rm[0];
-        m[u][1] = rm[1];
-      }
-    }
+    DRec d[SV_ADJ_BATCH];
 #pragma unroll
     for (int u = 0; u < SV_ADJ_BATCH; u++)
-      trans_link<MDIFF>(acc, wx[u], wy[u], wl[u], d[u], m[u]);
+      d[u] = load_rec<MDIFF>(a.dbar + (size_t)ix[u] * SV_TAPE_D, a.dbarm + (size_t)ix[u] * 4);
+#pragma unroll
+    for (int u = 0; u < SV_ADJ_BATCH; u++) trans_link<MDIFF>(acc, wx[u], wy[u], wl[u], d[u]);
   }
   for (; k < K; k += LPN) {
     const int64_t e = b + (int64_t)k * SV_WAVE;
     const int i = a.tcol[e];
-    const double2 *r = reinterpret_cast<const double2 *>(a.dbar + (size_t)i * SV_TAPE_D);
-    double2 d[7], m[2];
-#pragma unroll
-    for (int q = 0; q < 7; q++) d[q] = r[q];
-    if (MDIFF) {
-      const double2 *rm = reinterpret_cast<const double2 *>(a.dbarm + (size_t)i * 4);
-      m[0] = rm[0];
-      m[1] = rm[1];
-    }
-    trans_link<MDIFF>(acc, a.twx[e], a.twy[e], a.twl[e], d, m);
+    trans_link<MDIFF>(acc, a.tw3[sv_w3(e, 0)], a.tw3[sv_w3(e, 1)], a.tw3[sv_w3(e, 2)],
+                      load_rec<MDIFF>(a.dbar + (size_t)i * SV_TAPE_D, a.dbarm + (size_t)i * 4));
   }
   if (LPN == 4) {
 #pragma unroll
     for (int f = 0; f < 6; f++) acc[f] = quad_sum(acc[f]);
   }
   double part = 0.0;
-  if (nr.act && lr == 0) {
-    double o[6], g[6];
-    ld6(a.own + (size_t)j * SV_US, o);
-    ld6(a.tG + (size_t)j * SV_US, g);
-    double G[6];
-#pragma unroll
-    for (int f = 0; f < 6; f++) G[f] = o[f] + acc[f];
-    // G = (ro, rou/ro, rov/ro, c) -> U
-    const double ooro = 1.0 / g[0];
-    double Ub[6];
-    Ub[0] = G[0] - (G[1] * g[1] + G[2] * g[2]) * ooro;
-    Ub[1] = G[1] * ooro;
-    Ub[2] = G[2] * ooro;
-    Ub[3] = G[3]; Ub[4] = G[4]; Ub[5] = G[5];
-    const sv_ctrl *C = a.ctrl + nr.sg;
-    if (STAGE == 0) {
-      st6(a.Ubar + (size_t)j * SV_US, Ub);
-    } else if (STAGE == 1) {
-      double rg[6];
-      ld6(a.regbar + (size_t)j * SV_US, rg);
-#pragma unroll
-      for (int f = 0; f < 6; f++) Ub[f] += rg[f];
-      Ub[3] += a.seed;
-      Ub[5] += a.seed;
-      st6(a.Ubar + (size_t)j * SV_US, Ub);
-      part = Ub[0];
-    } else {
-      // U_k = reg_{k-2} + a_{k-1} R_{k-1};  reg_{k-1} = reg_{k-2} + b_{k-1} R_{k-1}
-      const double ra = C->RKa[STAGE - 2], rbk = C->RKb[STAGE - 2];
-      double rg[6], Rn[6];
-      ld6(a.regbar + (size_t)j * SV_US, rg);
-#pragma unroll
-      for (int f = 0; f < 6; f++) {
-        Rn[f] = ra * Ub[f] + rbk * rg[f];
-        rg[f] = Ub[f] + rg[f];
-      }
-      st6(a.regbar + (size_t)j * SV_US, rg);
-      adj_point_node<MDIFF>(a.nxt, nr, Rn);
-    }
-  }
+  if (nr.act && lr == 0) part = trans_point<STAGE, MDIFF>(a, nr, acc, load_own<STAGE>(a, j));
   if (STAGE == 1) {
     red[threadIdx.x] = part;
     __syncthreads();
@@ -398,6 +442,103 @@ __global__ __launch_bounds__(AB) void k_adj_trans(TransArgs a) {
       __syncthreads();
     }
     if (threadIdx.x == 0) a.psum[bid] = red[0];
+  }
+}
+
+// ---- halo-staged forms ----------------------------------------------------
+// A workgroup per 64 slots stages the records of its transposed halo (~4 per
+// node on a lattice) in LDS, as the forward sweeps do, and four wavefronts walk
+// a quarter of each list, their partial sums added in order.  The gathers
+// from memory they replace (14 doubles a link in 16-byte pieces of 64 records)
+// are bound by the CU's address rate.  A stage of 16k nodes, order 6: 30 -> 12 us;
+// filter and sum: 16.2 -> 10.1.  Records of 14 doubles (18 with polymer diffusion) and 6: odd
+// multiples of 16 bytes, which spread over the LDS banks.
+constexpr int AW = 4;
+template <bool MDIFF>
+constexpr int trans_rec() { return MDIFF ? 18 : 14; }
+
+// the six sums of the other wavefronts, added to wave 0's in their order
+__device__ __forceinline__ void add_sums(double *lds, int w, double acc[6]) {
+  const int lane = (int)threadIdx.x & (SV_WAVE - 1);
+  __syncthreads();   // the halo has been read
+  if (w > 0)
+#pragma unroll
+    for (int q = 0; q < 6; q++) lds[((w - 1) * 6 + q) * SV_WAVE + lane] = acc[q];
+  __syncthreads();
+  if (w > 0) return;
+#pragma unroll
+  for (int v = 0; v < AW - 1; v++)
+#pragma unroll
+    for (int q = 0; q < 6; q++) acc[q] += lds[(v * 6 + q) * SV_WAVE + lane];
+}
+constexpr size_t SUMS_LDS = sizeof(double) * (AW - 1) * 6 * SV_WAVE;
+
+__device__ __forceinline__ NodeRef node_ref_slice(const int *blk_seg, const sv_segk *seg, int s) {
+  NodeRef r;
+  r.sg = blk_seg[s / (BS / SV_WAVE)];
+  const sv_segk &S = seg[r.sg];
+  r.i = s * SV_WAVE + ((int)threadIdx.x & (SV_WAVE - 1));
+  r.act = r.i - S.base < S.npfb;
+  r.ii = r.act ? r.i : S.base;
+  return r;
+}
+
+template <int STAGE, bool MDIFF>
+__global__ __launch_bounds__(AW * SV_WAVE) void k_adj_trans_h(TransArgs a) {
+  extern __shared__ double hl[];
+  constexpr int RS = trans_rec<MDIFF>(), U = 3, NT = AW * SV_WAVE;
+  const int s = sv_xcd_block();
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / SV_WAVE);
+  const NodeRef nr = node_ref_slice(a.blk_seg, a.seg, s);
+  const Share<AW> sh(w, a.tcnt[nr.i], a.krange[s].x, a.krange[s].y);
+  const int64_t o = a.toff[s] + (int64_t)sh.k0 * SV_WAVE;
+  const int64_t h0 = a.hoff[s];
+  const int nh = (int)(a.hoff[s + 1] - h0);
+  const Stream<uint32_t, 1, false> sc(a.lcol + o, sh.KM);
+  const Stream<dbl2, 3, false> sw(a.tw3 + 3 * o, sh.KM);
+  uint32_t jc[2][U];
+  dbl2 wg[2][2 * U], wl[2][U];
+  auto load = [&](int b, int u, int p) {
+    jc[b][u] = sc.at(p, u, 0);
+    wg[b][2 * u] = sw.at(p, u, 0); wg[b][2 * u + 1] = sw.at(p, u, 1); wl[b][u] = sw.at(p, u, 2);
+  };
+  const int *hx = a.hidx + h0;
+  HaloKeys<SV_WAVE, NT> keys;
+  if (nh > 0) keys.get(hx, threadIdx.x, nh);
+  __builtin_amdgcn_sched_barrier(0);
+  const int p0 = entry_at(0);
+#pragma unroll
+  for (int u = 0; u < U; u++) load(0, u, 2 * u < sh.K ? p0 : OUT_OF_RANGE);
+  TransOwn own;
+  if (w == 0) own = load_own<STAGE>(a, nr.ii);
+  halo_stage<SV_WAVE, NT>(
+      hx, nh, keys,
+      [&](int j) {
+        return load_rec<MDIFF>(a.dbar + (size_t)j * SV_TAPE_D, a.dbarm + (size_t)j * 4);
+      },
+      [&](int h, int, const DRec &r) {
+        double2 *q = reinterpret_cast<double2 *>(hl + (size_t)h * RS);
+        q[0] = r.d0; q[1] = r.d1; q[2] = r.d2; q[3] = r.d3; q[4] = r.d4; q[5] = r.d5; q[6] = r.d6;
+        if (MDIFF) { q[7] = r.m0; q[8] = r.m1; }
+      });
+  __syncthreads();
+  double acc[6] = {0, 0, 0, 0, 0, 0};
+  walk_links<U, DRec>(
+      sh.K, sh.KF, sh.KM, load,
+      [&](int b, int l) {
+        const double *q = hl + (size_t)RS * (l & 1 ? jc[b][l / 2] >> 16 : jc[b][l / 2] & 0xffff);
+        return load_rec<MDIFF>(q, q + 14);
+      },
+      [&](const DRec &r, int b, int l) {
+        trans_link<MDIFF>(acc, wg[b][l].x, wg[b][l].y, l & 1 ? wl[b][l / 2].y : wl[b][l / 2].x, r);
+      });
+  add_sums(hl, w, acc);
+  if (w > 0) return;
+  double part = 0.0;
+  if (nr.act) part = trans_point<STAGE, MDIFF>(a, nr, acc, own);
+  if (STAGE == 1) {
+    part = wave_sum(part);
+    if (threadIdx.x == 0) a.psum[s] = part;
   }
 }
 
@@ -449,7 +590,44 @@ struct FiltArgs {
   const sv_ctrl *ctrl;
   double *regbar;
   PointArgs p4;
+  const int4 *krange;        // halos of the transposed lists (k_adj_filter_h)
+  const int64_t *hoff;
+  const int *hidx;
+  const uint16_t *lcol;
+  const double *psum;        // k_adj_filter_h: the npsum sums whose total it makes
+  int npsum;                 // itself instead of reading sbar (0: reads it)
 };
+
+// a node's own values in the filter's adjoint
+struct FiltOwn {
+  double f[6], vol, hs;
+  PointOwn p;
+};
+
+__device__ __forceinline__ FiltOwn load_own(const FiltArgs &a, int j) {
+  FiltOwn w;
+  ld6(a.Ubar + (size_t)j * SV_US, w.f);
+  w.vol = a.vol[j];
+  w.hs = a.hsum[j];
+  w.p = load_point(a.p4, j);
+  return w;
+}
+
+// own-node part: the filter's adjoint, then the pointwise adjoint of stage 4
+template <bool MDIFF>
+__device__ __forceinline__ void filt_point(const FiltArgs &a, const NodeRef &nr, double sv,
+                                           const double acc[6], FiltOwn &w) {
+  double out[6], rb[6];
+  w.f[0] -= w.vol * sv;
+  const double b4 = a.ctrl[nr.sg].RKb[3];
+#pragma unroll
+  for (int q = 0; q < 6; q++) {
+    out[q] = w.f[q] - w.hs * w.f[q] + acc[q];
+    rb[q] = b4 * out[q];
+  }
+  st6(a.regbar + (size_t)nr.i * SV_US, out);
+  adj_point_node<MDIFF>(a.p4, nr, rb, w.p);
+}
 
 template <bool MDIFF, int LPN>
 __global__ __launch_bounds__(AB) void k_adj_filter(FiltArgs a) {
@@ -469,7 +647,7 @@ __global__ __launch_bounds__(AB) void k_adj_filter(FiltArgs a) {
     for (int u = 0; u < SV_ADJ_BATCH; u++) {
       const int64_t e = b + (int64_t)(k + u * LPN) * SV_WAVE;
       ix[u] = a.tcol[e];
-      w[u] = a.twh[e];
+      w[u] = a.twh[sv_pair(e)];
     }
 #pragma unroll
     for (int u = 0; u < SV_ADJ_BATCH; u++) {
@@ -486,7 +664,7 @@ __global__ __launch_bounds__(AB) void k_adj_filter(FiltArgs a) {
   for (; k < K; k += LPN) {
     const int64_t e = b + (int64_t)k * SV_WAVE;
     const int i = a.tcol[e];
-    const double w = a.twh[e];
+    const double w = a.twh[sv_pair(e)];
     double f[6];
     ld6(a.Ubar + (size_t)i * SV_US, f);
     f[0] -= a.vol[i] * sv;
@@ -498,22 +676,96 @@ __global__ __launch_bounds__(AB) void k_adj_filter(FiltArgs a) {
     for (int q = 0; q < 6; q++) acc[q] = quad_sum(acc[q]);
   }
   if (!nr.act || lr != 0) return;
-  double f[6], out[6], rb[6];
-  ld6(a.Ubar + (size_t)j * SV_US, f);
-  f[0] -= a.vol[j] * sv;
-  const double hs = a.hsum[j];
-  const double b4 = a.ctrl[nr.sg].RKb[3];
-#pragma unroll
-  for (int q = 0; q < 6; q++) {
-    out[q] = f[q] - hs * f[q] + acc[q];
-    rb[q] = b4 * out[q];
-  }
-  st6(a.regbar + (size_t)j * SV_US, out);
-  adj_point_node<MDIFF>(a.p4, nr, rb);
+  FiltOwn own = load_own(a, j);
+  filt_point<MDIFF>(a, nr, sv, acc, own);
 }
 
-// trace loss of the state: per-block sums of (cxx + cyy - 2), then one block
-// per segment adds mean/T into lacc[seg]
+// the filter's adjoint with halos (see k_adj_trans_h).  Of a small node set every
+// wavefront makes the mass correction's sum itself: a launch less.
+constexpr int SMALL_SUMS = 512;
+template <bool MDIFF>
+__global__ __launch_bounds__(AW * SV_WAVE) void k_adj_filter_h(FiltArgs a) {
+  extern __shared__ double hl[];
+  constexpr int U = 4, NT = AW * SV_WAVE;
+  const int s = sv_xcd_block();
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / SV_WAVE);
+  const NodeRef nr = node_ref_slice(a.blk_seg, a.seg, s);
+  const Share<AW> sh(w, a.tcnt[nr.i], a.krange[s].z, a.krange[s].w);
+  const int64_t o = a.toff[s] + (int64_t)sh.k0 * SV_WAVE;
+  const int64_t h0 = a.hoff[s];
+  const int nh = (int)(a.hoff[s + 1] - h0);
+  const Stream<uint32_t, 1, false> sc(a.lcol + o, sh.KM);
+  const Stream<dbl2, 1, false> sw(a.twh + o, sh.KM);
+  uint32_t jc[2][U];
+  dbl2 wf[2][U];
+  auto load = [&](int b, int u, int p) {
+    jc[b][u] = sc.at(p, u, 0);
+    wf[b][u] = sw.at(p, u, 0);
+  };
+  const int *hx = a.hidx + h0;
+  HaloKeys<SV_WAVE, NT> keys;
+  if (nh > 0) keys.get(hx, threadIdx.x, nh);
+  double sv;
+  if (a.npsum > 0) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < SMALL_SUMS / SV_WAVE; k++) {
+      const int q = k * SV_WAVE + ((int)threadIdx.x & (SV_WAVE - 1));
+      v += q < a.npsum ? a.psum[q] : 0.0;
+    }
+    sv = wave_sum(v) / a.seg[nr.sg].volsum;
+  } else {
+    sv = a.sbar[nr.sg];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int p0 = entry_at(0);
+#pragma unroll
+  for (int u = 0; u < U; u++) load(0, u, 2 * u < sh.K ? p0 : OUT_OF_RANGE);
+  FiltOwn own;
+  if (w == 0) own = load_own(a, nr.ii);
+  struct Rec {
+    double2 d[3];
+    double vol;
+  };
+  halo_stage<SV_WAVE, NT>(
+      hx, nh, keys,
+      [&](int j) {
+        const double2 *q = reinterpret_cast<const double2 *>(a.Ubar + (size_t)j * SV_US);
+        return Rec{{q[0], q[1], q[2]}, a.vol[j]};
+      },
+      [&](int h, int, const Rec &r) {
+        double2 *q = reinterpret_cast<double2 *>(hl + (size_t)h * SV_US);
+        q[0] = double2{r.d[0].x - r.vol * sv, r.d[0].y};
+        q[1] = r.d[1];
+        q[2] = r.d[2];
+      });
+  __syncthreads();
+  double acc[6] = {0, 0, 0, 0, 0, 0};
+  struct Rec6 {
+    double2 d[3];
+  };
+  walk_links<U, Rec6>(
+      sh.K, sh.KF, sh.KM, load,
+      [&](int b, int l) {
+        const double2 *q = reinterpret_cast<const double2 *>(
+            hl + (size_t)SV_US * (l & 1 ? jc[b][l / 2] >> 16 : jc[b][l / 2] & 0xffff));
+        return Rec6{{q[0], q[1], q[2]}};
+      },
+      [&](const Rec6 &r, int b, int l) {
+        const double wt = l & 1 ? wf[b][l / 2].y : wf[b][l / 2].x;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          acc[2 * q] += wt * r.d[q].x;
+          acc[2 * q + 1] += wt * r.d[q].y;
+        }
+      });
+  add_sums(hl, w, acc);
+  if (w == 0 && nr.act) filt_point<MDIFF>(a, nr, sv, acc, own);
+}
+
+// trace loss of the state: per-block sums of (cxx + cyy - 2) after each step,
+// then one block per step and one thread that adds the steps' means to lacc in
+// their order
 __global__ __launch_bounds__(BS) void k_loss_part(const int *blk_seg, const sv_segk *seg,
                                                   const double *U, double *part) {
   __shared__ double red[BS];
@@ -533,19 +785,26 @@ __global__ __launch_bounds__(BS) void k_loss_part(const int *blk_seg, const sv_s
   if (threadIdx.x == 0) part[bid] = red[0];
 }
 
-__global__ __launch_bounds__(1024) void k_loss_acc(const sv_segk *seg, const double *part,
-                                                   double *lacc) {
+__global__ __launch_bounds__(1024) void k_loss_steps(const sv_segk *seg, const double *part,
+                                                     double *mean) {
   __shared__ double s1[1024];
-  const sv_segk &S = seg[blockIdx.x];
+  const sv_segk &S = seg[0];
+  const double *p = part + (size_t)blockIdx.x * S.nblk;
   double a = 0.0;
-  for (int k = threadIdx.x; k < S.nblk; k += 1024) a += part[S.blk0 + k];
+  for (int k = threadIdx.x; k < S.nblk; k += 1024) a += p[k];
   s1[threadIdx.x] = a;
   __syncthreads();
   for (int s = 512; s > 0; s >>= 1) {
     if ((int)threadIdx.x < s) s1[threadIdx.x] += s1[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) lacc[blockIdx.x] += s1[0] / S.npfb;
+  if (threadIdx.x == 0) mean[blockIdx.x] = s1[0] / S.npfb;
+}
+
+__global__ void k_loss_add(int steps, const double *mean, double *lacc) {
+  double a = *lacc;
+  for (int s = 0; s < steps; s++) a += mean[s];
+  *lacc = a;
 }
 
 // sums of the parameter-gradient accumulators over the real nodes (one block,
@@ -573,20 +832,21 @@ __global__ void k_zero(double *p, int64_t n) {
 }  // namespace
 
 // ---- host side ------------------------------------------------------------
+constexpr int LOSS_STEPS = 32;
+
 struct sv_adj {
   int every = 20;            // checkpoint interval (steps)
-  // transposed stencil (SELL-64 over j)
-  int64_t *toff = nullptr;
-  int *tcnt = nullptr, *tcol = nullptr;
-  double *twx = nullptr, *twy = nullptr, *twl = nullptr, *twh = nullptr;
-  int64_t tnnz = 0;
+  sv_loopl TL;               // transposed stencil (SELL-64 over j)
+  bool halo = false;         // its halos fit: the halo-staged sweeps
   // adjoint records [ntot][SV_US] and stencil-adjoint records
   double *Ubar = nullptr, *Rbar = nullptr, *regbar = nullptr;
   // stencil-adjoint records of two consecutive stages (ping-pong: a fused
   // kernel reads stage k's while writing stage k-1's)
   double *own[2] = {nullptr, nullptr}, *dbar[2] = {nullptr, nullptr};
   double *dbarm[2] = {nullptr, nullptr};
-  double *psum = nullptr, *sbar = nullptr, *lpart = nullptr, *lacc = nullptr;
+  double *psum = nullptr, *sbar = nullptr;
+  double *lpart = nullptr, *lmean = nullptr, *lacc = nullptr;   // loss sums of lsteps steps
+  int lsteps = 0;
   double *pacc = nullptr, *pred = nullptr;   // parameter-gradient accumulators, sums
   double pgrad[3] = {0, 0, 0};               // d/d(Wi, beta, epsPTT) of the last VJP
   // rollout: checkpoints of U records, the end state, the tape of one interval
@@ -596,6 +856,9 @@ struct sv_adj {
   double *Uend = nullptr;
   sv_ctrl ctrl_end{};
   std::vector<double *> tape;    // [every][8]
+  // the tape holds the last interval of the last rollout; tape_used: the last
+  // one that a rollout wrote was read by a reverse sweep
+  bool taped = false, tape_used = true;
   double t_fwd = 0, t_bwd = 0;   // ms of the last rollout / vjp
   int lpn = 1;                   // lanes per node of the transposed gathers (1 or 4)
 };
@@ -619,81 +882,39 @@ static int zero_dev(sv_ctx *c, double *p, int64_t n) {
   return 0;
 }
 
-// Transposed stencil of the folded SELL lists: for each j the entries (i, k)
-// with scol = j, in ascending i, stage weights zero beyond ij_count_small.
-static int build_transpose(sv_ctx *c, sv_adj *A) {
-  const sv_loopl &LP = c->L;
-  const int n = c->npfb, ns = LP.nslices;
-  std::vector<int> cnt(n), cs(n), scol(LP.nnz);
-  std::vector<int64_t> off(ns);
-  std::vector<double> w3(3 * LP.nnz), wh(LP.nnz);
-  SV_HIP(c, hipMemcpy(cnt.data(), LP.cnt, sizeof(int) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(cs.data(), LP.cnt_small, sizeof(int) * n, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(off.data(), LP.off, sizeof(int64_t) * ns, hipMemcpyDeviceToHost));
-  const size_t L = sizeof(double) * LP.nnz;
-  SV_HIP(c, hipMemcpy(scol.data(), LP.col, sizeof(int) * LP.nnz, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(w3.data(), LP.w3, 3 * L, hipMemcpyDeviceToHost));
-  SV_HIP(c, hipMemcpy(wh.data(), LP.wh, L, hipMemcpyDeviceToHost));
-  std::vector<int> tc(n, 0);
-  for (int i = 0; i < n; i++)
-    for (int k = 0; k < cnt[i]; k++) {
-      const int j = scol[off[i >> 6] + (int64_t)k * SV_WAVE + (i & 63)];
-      if (j < 0 || j >= n) return sv_fail(c, SV_E_STATE, "stencil column out of range");
-      tc[j]++;
-    }
-  const int nsl = (n + SV_WAVE - 1) / SV_WAVE;
-  std::vector<int64_t> toff(nsl + 1);
-  int64_t tot = 0;
-  for (int s = 0; s < nsl; s++) {
-    int w = 0;
-    for (int l = 0; l < SV_WAVE && s * SV_WAVE + l < n; l++) w = std::max(w, tc[s * SV_WAVE + l]);
-    toff[s] = tot;
-    tot += (int64_t)w * SV_WAVE;
+// tape of `steps` steps; what is missing in one allocation
+static int ensure_tape(sv_ctx *c, sv_adj *A, int steps) {
+  const size_t N = (size_t)c->ntot;
+  const int more = steps - (int)A->tape.size() / 8;
+  if (more <= 0) return 0;
+  double *p = nullptr;
+  if (adj_alloc(c, &p, (size_t)more * 4 * (SV_US + SV_TAPE_D) * N)) return SV_E_NOMEM;
+  for (int k = 0; k < 8 * more; k++) {
+    A->tape.push_back(p);
+    p += ((k & 1) ? SV_TAPE_D : SV_US) * N;
   }
-  toff[nsl] = tot;
-  A->tnnz = tot;
-  std::vector<int> tcol(tot);
-  std::vector<double> tx(tot, 0.0), ty(tot, 0.0), tl(tot, 0.0), th(tot, 0.0);
-  for (int s = 0; s < nsl; s++)       // padding: own node, zero weights
-    for (int64_t e = toff[s]; e < toff[s + 1]; e++)
-      tcol[e] = std::min(s * SV_WAVE + (int)((e - toff[s]) % SV_WAVE), n - 1);
-  std::vector<int> fill(n, 0);
-  for (int i = 0; i < n; i++)
-    for (int k = 0; k < cnt[i]; k++) {
-      const int64_t e = off[i >> 6] + (int64_t)k * SV_WAVE + (i & 63);
-      const int j = scol[e];
-      const int64_t d = toff[j >> 6] + (int64_t)(fill[j]++) * SV_WAVE + (j & 63);
-      tcol[d] = i;
-      const bool small = k < cs[i];
-      tx[d] = small ? w3[sv_w3(e, 0)] : 0.0;
-      ty[d] = small ? w3[sv_w3(e, 1)] : 0.0;
-      tl[d] = small ? w3[sv_w3(e, 2)] : 0.0;
-      th[d] = wh[sv_pair(e)];
-    }
-  if (sv_alloc(c, (void **)&A->toff, sizeof(int64_t) * (nsl + 1)) ||
-      sv_alloc(c, (void **)&A->tcnt, sizeof(int) * n) ||
-      sv_alloc(c, (void **)&A->tcol, sizeof(int) * (tot + 1)) || adj_alloc(c, &A->twx, tot) ||
-      adj_alloc(c, &A->twy, tot) || adj_alloc(c, &A->twl, tot) || adj_alloc(c, &A->twh, tot))
-    return SV_E_NOMEM;
-  SV_HIP(c, hipMemcpy(A->toff, toff.data(), sizeof(int64_t) * (nsl + 1), hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(A->tcnt, tc.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(A->tcol, tcol.data(), sizeof(int) * tot, hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(A->twx, tx.data(), sizeof(double) * tot, hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(A->twy, ty.data(), sizeof(double) * tot, hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(A->twl, tl.data(), sizeof(double) * tot, hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(A->twh, th.data(), sizeof(double) * tot, hipMemcpyHostToDevice));
   return 0;
 }
 
-static int ensure_tape(sv_ctx *c, sv_adj *A) {
-  const size_t N = (size_t)c->ntot;
-  while ((int)A->tape.size() < 8 * A->every) {
-    double *p = nullptr;
-    const size_t per = ((A->tape.size() & 1) ? SV_TAPE_D : SV_US) * N;
-    if (adj_alloc(c, &p, per)) return SV_E_NOMEM;
-    A->tape.push_back(p);
+// Whether a rollout writes the tape of its last interval (of `steps` steps), so
+// that the reverse sweep need not compute the interval again (75 us a step of
+// 16k nodes; writing costs 176 bytes a node and stage beside the ~2 kB read):
+// not after a rollout whose tape nothing read, nor where the tape would take
+// more than a quarter of the free memory.
+static bool want_tape(sv_ctx *c, sv_adj *A, int steps) {
+  if (!A->tape_used) return false;
+  const int more = std::max(0, steps - (int)A->tape.size() / 8);
+  if (more > 0) {
+    size_t free_b = 0, total = 0;
+    if (hipMemGetInfo(&free_b, &total) != hipSuccess) return false;
+    const size_t per = sizeof(double) * 4 * (SV_US + SV_TAPE_D) * (size_t)c->ntot;
+    if (per * more > free_b / 4) return false;
   }
-  return 0;
+  return ensure_tape(c, A, steps) == 0;
+}
+
+void sv_adj_drop_tape(sv_ctx *c) {
+  if (c->adj) c->adj->taped = false;
 }
 
 // pointwise-adjoint arguments for stage k (1..4) of a tape slot, buffer set q
@@ -721,15 +942,30 @@ static int param_grad_finish(sv_ctx *c, sv_adj *A) {
   return 0;
 }
 
+// LDS of the transposed gathers' largest halo
+static size_t trans_lds(sv_ctx *c, sv_adj *A) {
+  return sizeof(double) * (c->any_mdiff ? trans_rec<true>() : trans_rec<false>()) *
+         (size_t)A->TL.hmax;
+}
+
 // transposed gather of stage STAGE (its records in buffer set q); for STAGE
 // 2..4 fused with the pointwise adjoint of STAGE-1 into buffer set 1-q
 template <int STAGE>
 static int adj_trans(sv_ctx *c, sv_adj *A, double *const *tape, int q, double seed) {
   const int k = STAGE == 0 ? 1 : STAGE;
-  TransArgs t{c->blk_seg, c->segk, A->toff, A->tcnt, A->tcol, A->twx, A->twy, A->twl,
+  const sv_loopl &L = A->TL;
+  TransArgs t{c->blk_seg, c->segk, L.off, L.cnt, L.col, L.w3,
               A->dbar[q], A->dbarm[q], A->own[q], tape[2 * (k - 1)], c->ctrl, A->Ubar, A->Rbar,
-              A->regbar, seed, A->psum, PointArgs{}};
+              A->regbar, seed, A->psum, PointArgs{}, L.krange, L.hoff, L.hidx, L.lcol};
   if (STAGE >= 2) t.nxt = point_args(c, A, tape, STAGE - 1, 1 - q);
+  if (A->halo) {
+    const int grid = c->nblk * (BS / SV_WAVE), nt = AW * SV_WAVE;
+    const size_t shm = std::max(SUMS_LDS, trans_lds(c, A));
+    if (c->any_mdiff) k_adj_trans_h<STAGE, true><<<grid, nt, shm, c->stream>>>(t);
+    else k_adj_trans_h<STAGE, false><<<grid, nt, shm, c->stream>>>(t);
+    SV_HIP(c, hipGetLastError());
+    return 0;
+  }
   const int grid = c->nblk * subl_of(A->lpn);
   if (A->lpn == 4) {
     if (c->any_mdiff) k_adj_trans<STAGE, true, 4><<<grid, AB, 0, c->stream>>>(t);
@@ -754,11 +990,18 @@ static int adj_rhs(sv_ctx *c, sv_adj *A, double *const *tape) {
 // adjoint of one step (tape slot): Ubar (after the step, with its mass sums
 // in psum) -> Ubar (before the step) + seed on cxx, cyy.  Six launches.
 static int adj_step(sv_ctx *c, sv_adj *A, double *const *tape, double seed) {
+  const sv_loopl &L = A->TL;
   const int subl = subl_of(A->lpn), grid = c->nblk * subl;
-  k_adj_sum_reduce<<<c->nseg, 1024, 0, c->stream>>>(c->segk, A->psum, subl, A->sbar);
-  FiltArgs f{c->blk_seg, c->segk, A->toff, A->tcnt, A->tcol, A->twh, c->L.hsum, c->L.vol,
-             A->sbar, A->Ubar, c->ctrl, A->regbar, point_args(c, A, tape, 4, 0)};
-  if (A->lpn == 4) {
+  const bool small = A->halo && grid <= SMALL_SUMS;
+  if (!small) k_adj_sum_reduce<<<c->nseg, 1024, 0, c->stream>>>(c->segk, A->psum, subl, A->sbar);
+  FiltArgs f{c->blk_seg, c->segk, L.off, L.cnt, L.col, L.wh, c->L.hsum, c->L.vol,
+             A->sbar, A->Ubar, c->ctrl, A->regbar, point_args(c, A, tape, 4, 0), L.krange, L.hoff,
+             L.hidx, L.lcol, A->psum, small ? grid : 0};
+  if (A->halo) {
+    const size_t shm = std::max(SUMS_LDS, sizeof(double) * SV_US * (size_t)L.hmax);
+    if (c->any_mdiff) k_adj_filter_h<true><<<grid, AW * SV_WAVE, shm, c->stream>>>(f);
+    else k_adj_filter_h<false><<<grid, AW * SV_WAVE, shm, c->stream>>>(f);
+  } else if (A->lpn == 4) {
     if (c->any_mdiff) k_adj_filter<true, 4><<<grid, AB, 0, c->stream>>>(f);
     else k_adj_filter<false, 4><<<grid, AB, 0, c->stream>>>(f);
   } else {
@@ -772,9 +1015,16 @@ static int adj_step(sv_ctx *c, sv_adj *A, double *const *tape, double seed) {
   return adj_trans<1>(c, A, tape, 1, seed);
 }
 
-static int loss_accumulate(sv_ctx *c, sv_adj *A) {
-  k_loss_part<<<c->nblk, BS, 0, c->stream>>>(c->blk_seg, c->segk, c->U, A->lpart);
-  k_loss_acc<<<c->nseg, 1024, 0, c->stream>>>(c->segk, A->lpart, A->lacc);
+// the loss of the state after a step; the steps' sums are added up LOSS_STEPS at
+// a time, and when last
+static int loss_accumulate(sv_ctx *c, sv_adj *A, bool last) {
+  k_loss_part<<<c->nblk, BS, 0, c->stream>>>(c->blk_seg, c->segk, c->U,
+                                             A->lpart + (size_t)A->lsteps * c->nblk);
+  if (++A->lsteps == LOSS_STEPS || last) {
+    k_loss_steps<<<A->lsteps, 1024, 0, c->stream>>>(c->segk, A->lpart, A->lmean);
+    k_loss_add<<<1, 1, 0, c->stream>>>(A->lsteps, A->lmean, A->lacc);
+    A->lsteps = 0;
+  }
   SV_HIP(c, hipGetLastError());
   return 0;
 }
@@ -921,7 +1171,7 @@ int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
     sv_adj *A = new sv_adj();
     c->adj = A;
     const size_t R = (size_t)SV_US * c->ntot;
-    if (int rc = build_transpose(c, A)) return rc;
+    if (int rc = sv_dev_build_transpose(c, A->TL)) return rc;
     if (adj_alloc(c, &A->Ubar, R) || adj_alloc(c, &A->Rbar, R) || adj_alloc(c, &A->regbar, R) ||
         adj_alloc(c, &A->own[0], R) || adj_alloc(c, &A->own[1], R) ||
         adj_alloc(c, &A->dbar[0], (size_t)SV_TAPE_D * c->ntot) ||
@@ -929,11 +1179,13 @@ int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
         adj_alloc(c, &A->dbarm[0], (size_t)4 * c->ntot) ||
         adj_alloc(c, &A->dbarm[1], (size_t)4 * c->ntot) ||
         adj_alloc(c, &A->psum, (size_t)c->nblk * subl_of(4)) ||
-        adj_alloc(c, &A->sbar, c->nseg) || adj_alloc(c, &A->lpart, c->nblk) ||
+        adj_alloc(c, &A->sbar, c->nseg) || adj_alloc(c, &A->lpart, (size_t)LOSS_STEPS * c->nblk) ||
+        adj_alloc(c, &A->lmean, LOSS_STEPS) ||
         adj_alloc(c, &A->lacc, c->nseg) || adj_alloc(c, &A->Uend, R) ||
         adj_alloc(c, &A->pacc, (size_t)4 * c->ntot) || adj_alloc(c, &A->pred, 4))
       return SV_E_NOMEM;
   }
+  if (c->adj->every != checkpoint_every) c->adj->taped = false;
   c->adj->every = checkpoint_every;
   // lanes per node of the transposed gathers: 4 when one lane per node would
   // give fewer than 8 waves per CU (e.g. a 128x128 lattice: 256 waves)
@@ -943,6 +1195,11 @@ int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
     const int64_t waves = (int64_t)c->nblk * SUBS;
     c->adj->lpn = c->adj_lanes == 1 || c->adj_lanes == 4 ? c->adj_lanes
                   : (waves < 8 * (int64_t)ncu ? 4 : 1);
+    // staged halos where they fit (for either records), one slice a workgroup
+    // (adj_lanes asks for the gathers from memory)
+    c->adj->halo = c->adj_lanes == 0 && c->adj->TL.halo &&
+                   sizeof(double) * trans_rec<true>() * c->adj->TL.hmax <= (size_t)SV_HALO_LDS_MAX;
+    if (c->adj->halo) c->adj->lpn = 1;
   }
   return 0;
 }
@@ -953,7 +1210,8 @@ int sv_rhs_vjp(sv_ctx *c, const double *const rbar[6], double *const ubar[6]) {
   SV_ADJ_CHECK(c, rbar && ubar, "null argument");
   sv_adj *A = c->adj;
   SV_HIP(c, hipSetDevice(c->device));
-  if (int rc = ensure_tape(c, A)) return rc;
+  if (int rc = ensure_tape(c, A, 1)) return rc;
+  A->taped = false;
   {
     DevTmp<double> scratch;
     SV_HIP(c, scratch.alloc(6 * (size_t)c->npfb));
@@ -986,6 +1244,9 @@ int sv_rollout_forward(sv_ctx *c, int32_t nsteps, double *loss) {
     A->ckpt.push_back(p);
   }
   A->ckpt_ctrl.assign(nck, sv_ctrl{});
+  const bool tape = want_tape(c, A, nsteps - (nck - 1) * A->every);
+  A->taped = false;
+  A->lsteps = 0;
   if (int rc = zero_dev(c, A->lacc, c->nseg)) return rc;
   EventTmp e0, e1;
   SV_HIP(c, e0.create());
@@ -999,8 +1260,13 @@ int sv_rollout_forward(sv_ctx *c, int32_t nsteps, double *loss) {
       SV_HIP(c, hipMemcpyAsync(&A->ckpt_ctrl[k], c->ctrl, sizeof(sv_ctrl),
                                hipMemcpyDeviceToHost, c->stream));
     }
-    if (int rc = sv_dev_step(c, nullptr)) return rc;
-    if (int rc = loss_accumulate(c, A)) return rc;
+    const int t = s - (nck - 1) * A->every;   // step of the last interval
+    if (tape && t >= 0) {
+      if (int rc = sv_dev_step_tape(c, A->tape.data() + 8 * t)) return rc;
+    } else if (int rc = sv_dev_step(c, nullptr)) {
+      return rc;
+    }
+    if (int rc = loss_accumulate(c, A, s + 1 == nsteps)) return rc;
   }
   SV_HIP(c, hipEventRecord(e1, c->stream));
   SV_HIP(c, hipMemcpyAsync(A->Uend, c->U, sizeof(double) * R, hipMemcpyDeviceToDevice,
@@ -1014,6 +1280,8 @@ int sv_rollout_forward(sv_ctx *c, int32_t nsteps, double *loss) {
   SV_HIP(c, hipEventElapsedTime(&ms, e0, e1));
   A->t_fwd = ms;
   A->T = nsteps;
+  A->taped = tape;
+  if (tape) A->tape_used = false;
   if (loss) *loss = acc / nsteps;
   return 0;
 }
@@ -1036,8 +1304,11 @@ static int rollout_vjp(sv_ctx *c, double loss_bar, const double *const ubar_fina
   SV_ADJ_CHECK(c, grad0, "null output");
   sv_adj *A = c->adj;
   SV_HIP(c, hipSetDevice(c->device));
-  if (int rc = ensure_tape(c, A)) return rc;
   const int T = A->T, E = A->every;
+  const bool taped = A->taped;
+  if (int rc = ensure_tape(c, A, std::min(T, E))) return rc;
+  A->taped = false;
+  A->tape_used = true;
   const double seed = loss_bar / ((double)T * c->npfb);
   const size_t R = (size_t)SV_US * c->ntot;
   if (device_io) {
@@ -1062,14 +1333,19 @@ static int rollout_vjp(sv_ctx *c, double loss_bar, const double *const ubar_fina
   const int nck = (T + E - 1) / E;
   for (int k = nck - 1; k >= 0; k--) {
     const int s0 = k * E, s1 = std::min(T, s0 + E);
-    // recompute the interval from its checkpoint with the tape on
-    SV_HIP(c, hipMemcpyAsync(c->U, A->ckpt[k], sizeof(double) * R, hipMemcpyDeviceToDevice,
-                             c->stream));
-    SV_HIP(c, hipMemcpyAsync(c->ctrl, &A->ckpt_ctrl[k], sizeof(sv_ctrl), hipMemcpyHostToDevice,
-                             c->stream));
-    if (int rc = sv_dev_init_state(c)) return rc;
-    for (int s = s0; s < s1; s++)
-      if (int rc = sv_dev_step_tape(c, A->tape.data() + 8 * (s - s0))) return rc;
+    if (taped && k == nck - 1) {   // the rollout wrote its tape
+      SV_HIP(c, hipMemcpyAsync(c->ctrl, &A->ctrl_end, sizeof(sv_ctrl), hipMemcpyHostToDevice,
+                               c->stream));
+    } else {
+      // recompute the interval from its checkpoint with the tape on
+      SV_HIP(c, hipMemcpyAsync(c->U, A->ckpt[k], sizeof(double) * R, hipMemcpyDeviceToDevice,
+                               c->stream));
+      SV_HIP(c, hipMemcpyAsync(c->ctrl, &A->ckpt_ctrl[k], sizeof(sv_ctrl),
+                               hipMemcpyHostToDevice, c->stream));
+      if (int rc = sv_dev_init_state(c)) return rc;
+      for (int s = s0; s < s1; s++)
+        if (int rc = sv_dev_step_tape(c, A->tape.data() + 8 * (s - s0))) return rc;
+    }
     for (int s = s1 - 1; s >= s0; s--)
       if (int rc = adj_step(c, A, A->tape.data() + 8 * (s - s0), s >= 1 ? seed : 0.0))
         return rc;

@@ -310,6 +310,60 @@ __global__ void k_halo_compact(const int64_t *hoff, const int *list, int *hidx) 
   for (int k = threadIdx.x; k < n; k += blockDim.x) hidx[o + k] = list[(size_t)b * HC + k];
 }
 
+// ---- transposed lists -------------------------------------------------------
+// Links pointing at each slot; bad: a target outside the slots.
+constexpr int TT = 256;
+__global__ __launch_bounds__(TT) void k_t_count(int n, const int64_t *off, const int *cnt,
+                                                const int *col, int *tc, int *bad) {
+  const int lane = threadIdx.x % SV_WAVE, slot = blockIdx.x * SV_WAVE + lane;
+  if (slot >= n) return;
+  const int64_t o = off[blockIdx.x] + lane;
+  for (int k = threadIdx.x / SV_WAVE; k < cnt[slot]; k += TT / SV_WAVE) {
+    const int j = col[o + (int64_t)k * SV_WAVE];
+    if ((unsigned)j < (unsigned)n) atomicAdd(&tc[j], 1);
+    else *bad = 1;
+  }
+}
+
+// the links of each target, (source slot, position in its list), in any order
+__global__ __launch_bounds__(TT) void k_t_fill(int n, const int64_t *off, const int *cnt,
+                                               const int *col, const int64_t *start, int *fill,
+                                               uint64_t *key) {
+  const int lane = threadIdx.x % SV_WAVE, slot = blockIdx.x * SV_WAVE + lane;
+  if (slot >= n) return;
+  const int64_t o = off[blockIdx.x] + lane;
+  for (int k = threadIdx.x / SV_WAVE; k < cnt[slot]; k += TT / SV_WAVE) {
+    const int j = col[o + (int64_t)k * SV_WAVE];
+    key[start[j] + atomicAdd(&fill[j], 1)] = (uint64_t)slot << 32 | (uint64_t)k;
+  }
+}
+
+// One wavefront per target: its links ranked by source slot (each link counts
+// the smaller keys: lists are short), then written to the transposed layout.
+// Stage weights past the source's small list are zero.
+__global__ __launch_bounds__(TT) void k_t_emit(int n, const int64_t *off, const int *cnt_small,
+                                               const double *w3, const double *wh,
+                                               const int64_t *start, const int *tc,
+                                               const uint64_t *key, const int64_t *toff, int *tcol,
+                                               double *tw3, double *twh) {
+  const int j = blockIdx.x * (TT / SV_WAVE) + threadIdx.x / SV_WAVE;
+  if (j >= n) return;
+  const int K = tc[j];
+  const uint64_t *q = key + start[j];
+  for (int a = threadIdx.x % SV_WAVE; a < K; a += SV_WAVE) {
+    const uint64_t me = q[a];
+    int rank = 0;
+    for (int b = 0; b < K; b++) rank += q[b] < me;
+    const int i = (int)(me >> 32), k = (int)(me & 0xffffffffu);
+    const int64_t e = off[i >> 6] + (int64_t)k * SV_WAVE + (i & 63);
+    const int64_t d = toff[j >> 6] + (int64_t)rank * SV_WAVE + (j & 63);
+    const bool small = k < cnt_small[i];
+    tcol[d] = i;
+    for (int w = 0; w < 3; w++) tw3[sv_w3(d, w)] = small ? w3[sv_w3(e, w)] : 0.0;
+    twh[sv_pair(d)] = wh[sv_pair(e)];
+  }
+}
+
 // int -> int64 exclusive scan of n values (out[n - 1] is the sum of the first
 // n - 1)
 struct ToI64 {
@@ -428,8 +482,7 @@ int kd_order(sv_ctx *c, int *perm, int by_len) {
 
 // Halos of hb slots per block, nslot slots in all.  L.halo stays false when a
 // block's halo exceeds the LDS budget of the sweeps.
-int build_halos(sv_ctx *c, int hb, int nslot) {
-  sv_loopl &L = c->L;
+int build_halos(sv_ctx *c, sv_loopl &L, int hb, int nslot) {
   // whole node blocks, as the sweeps' grids cover them: the halo blocks past
   // the last slot are empty
   const int nb = (nslot + SV_BLOCK - 1) / SV_BLOCK * (SV_BLOCK / hb);
@@ -511,8 +564,8 @@ int sv_dev_build_halos(sv_ctx *c, int nslot) {
   const Blocks b = choose_blocks(nslot, c->L.nnz);
   c->L.nt = b.nt;
   c->L.split = b.split;
-  if (int rc = build_halos(c, b.hb, nslot)) return rc;
-  return c->L.halo || b.hb == SV_WAVE ? 0 : build_halos(c, SV_WAVE, nslot);
+  if (int rc = build_halos(c, c->L, b.hb, nslot)) return rc;
+  return c->L.halo || b.hb == SV_WAVE ? 0 : build_halos(c, c->L, SV_WAVE, nslot);
 }
 
 static int build_layout(sv_ctx *c, int hb) {
@@ -578,7 +631,7 @@ static int build_layout(sv_ctx *c, int hb) {
     SV_HIP(c, hipGetLastError());
   }
   if (c->halo_sweeps)
-    if (int rc = build_halos(c, hb, n)) return rc;
+    if (int rc = build_halos(c, L, hb, n)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));
   L.valid = true;
   return 0;
@@ -593,5 +646,64 @@ int sv_dev_build_loop(sv_ctx *c) {
   }
   c->L.nt = b.nt && c->L.hb != SV_WAVE;
   c->L.split = b.split;
+  return 0;
+}
+
+// The transposed lists of the loop layout: for each slot j the links (i, k) that
+// point at it, by ascending i, with the halos of 64-slot blocks.  (On the host
+// this was 30 ms of a 16k-node gradient's first 48.)
+int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
+  const sv_loopl &L = c->L;
+  const int n = c->npfb, ns = L.nslices;
+  const int nslot = (n + SV_BLOCK - 1) / SV_BLOCK * SV_BLOCK;
+  T.nslices = ns;
+  if (sv_alloc(c, (void **)&T.off, sizeof(int64_t) * (nslot / SV_WAVE + 1)) ||
+      sv_alloc(c, (void **)&T.cnt, sizeof(int) * nslot))
+    return SV_E_NOMEM;
+  T.cnt_small = T.cnt;
+  DevTmp<int> fill, bad;
+  DevTmp<int64_t> start, w;
+  SV_HIP(c, fill.alloc(n));
+  SV_HIP(c, bad.alloc(1));
+  SV_HIP(c, start.alloc((size_t)n + 1));
+  SV_HIP(c, w.alloc((size_t)ns + 1));
+  SV_HIP(c, hipMemsetAsync(T.off, 0, sizeof(int64_t) * (nslot / SV_WAVE + 1), c->stream));
+  SV_HIP(c, hipMemsetAsync(T.cnt, 0, sizeof(int) * nslot, c->stream));
+  SV_HIP(c, hipMemsetAsync(fill, 0, sizeof(int) * n, c->stream));
+  SV_HIP(c, hipMemsetAsync(bad, 0, sizeof(int), c->stream));
+  SV_HIP(c, hipMemsetAsync(w.p + ns, 0, sizeof(int64_t), c->stream));
+  k_t_count<<<ns, TT, 0, c->stream>>>(n, L.off, L.cnt, L.col, T.cnt, bad);
+  k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, T.cnt, w);
+  SV_HIP(c, hipGetLastError());
+  if (int rc = scan_i64(c, (const int64_t *)w.p, T.off, ns + 1)) return rc;
+  int64_t links = 0;
+  {
+    DevTmp<int> one;   // the counts and a last zero, for an exclusive scan of n + 1
+    SV_HIP(c, one.alloc((size_t)n + 1));
+    SV_HIP(c, hipMemcpyAsync(one, T.cnt, sizeof(int) * n, hipMemcpyDeviceToDevice, c->stream));
+    SV_HIP(c, hipMemsetAsync(one.p + n, 0, sizeof(int), c->stream));
+    hipcub::TransformInputIterator<int64_t, ToI64, const int *> in(one.p, ToI64());
+    if (int rc = scan_i64(c, in, start, n + 1)) return rc;   // synchronises
+  }
+  int hbad = 0;
+  SV_HIP(c, hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  SV_HIP(c, hipMemcpyAsync(&links, start.p + n, sizeof(int64_t), hipMemcpyDeviceToHost,
+                           c->stream));
+  SV_HIP(c, hipMemcpyAsync(&T.nnz, T.off + ns, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+  SV_HIP(c, hipStreamSynchronize(c->stream));
+  if (hbad) return sv_fail(c, SV_E_STATE, "stencil column out of range");
+  const size_t E = (size_t)T.nnz + 1;
+  DevTmp<uint64_t> key;
+  SV_HIP(c, key.alloc((size_t)links));
+  if (sv_alloc(c, (void **)&T.col, sizeof(int) * E) ||
+      sv_alloc(c, (void **)&T.w3, 3 * sizeof(double) * E) ||
+      sv_alloc(c, (void **)&T.wh, sizeof(double) * E))
+    return SV_E_NOMEM;
+  k_t_fill<<<ns, TT, 0, c->stream>>>(n, L.off, L.cnt, L.col, start, fill, key);
+  k_t_emit<<<(n + TT / SV_WAVE - 1) / (TT / SV_WAVE), TT, 0, c->stream>>>(
+      n, L.off, L.cnt_small, L.w3, L.wh, start, T.cnt, key, T.off, T.col, T.w3, T.wh);
+  SV_HIP(c, hipGetLastError());
+  if (int rc = build_halos(c, T, SV_WAVE, n)) return rc;
+  SV_HIP(c, hipStreamSynchronize(c->stream));   // the temporaries go out of scope
   return 0;
 }

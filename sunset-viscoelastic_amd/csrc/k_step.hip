@@ -97,25 +97,6 @@ __device__ __forceinline__ int logical_wg(const int *blist) {
   return blist ? blist[b / SUB] * SUB + b % SUB : b;
 }
 
-// Reductions over a wavefront in a fixed order (every lane ends with the
-// result).  The partial results of the node kernels are per 64-slot slice, so
-// they do not depend on the workgroup size a sweep runs with.
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-  return v;
-}
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmin(v, __shfl_xor(v, o));
-  return v;
-}
-
 // ---- conformation algebra (conf_transforms.F90) -------------------------
 // 2D eigens (:399-444); R column-major R[0]=R11 R[1]=R21 R[2]=R12 R[3]=R22
 __device__ __forceinline__ void eigens2(double a, double b, double d, double &l1, double &l2,

@@ -637,6 +637,7 @@ int sv_set_phys(sv_ctx *c, const sv_phys *p) {
                                  "sv_ensemble_create");
   c->phys = *p;
   derive_phys(c);
+  sv_adj_drop_tape(c);   // a reverse sweep computes its intervals with the new values
   c->have_phys = true;
   c->graph_valid = false;
   if (c->have_state) {

@@ -102,6 +102,7 @@ struct sv_physk {
 struct sv_adj;   // adjoint work space (k_adjoint.hip)
 struct sv_ctx;
 void sv_adj_free(sv_ctx *c);
+void sv_adj_drop_tape(sv_ctx *c);   // a rollout's tape no longer holds
 #define SV_G_RO 0
 #define SV_G_U 1
 #define SV_G_V 2
@@ -374,6 +375,7 @@ int sv_dev_build_sell(sv_ctx *c);
 int sv_dev_build_loop(sv_ctx *c);
 // the halos of the layout in c->L over nslot slots (a context's own, or an
 // ensemble's concatenated one)
+int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T);
 int sv_dev_build_halos(sv_ctx *c, int nslot);
 int sv_ensure_loop(sv_ctx *c);
 // ---- kernels: weights (k_weights.hip) ----

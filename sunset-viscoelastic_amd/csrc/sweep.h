@@ -10,6 +10,25 @@ namespace {
 
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 
+// Reductions over a wavefront in a fixed order (every lane ends with the
+// result).  The partial results of the node kernels are per 64-slot slice, so
+// they do not depend on the workgroup size a sweep runs with.
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+  return v;
+}
+__device__ __forceinline__ double wave_min(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+  return v;
+}
+
 // Records a thread stages at once: a usual halo (~600 records per 256 slots,
 // ~270 per 64) in one round of requests, since a round costs two dependent
 // trips to memory (key, record).
@@ -98,6 +117,21 @@ __device__ __forceinline__ int entry_at(int k) {
 //   load(set, u, p)  requests the u-th pair from position p into entry u
 //   fetch(set, l)    the LDS record of link l of the set's 2U
 //   link(r, set, l)  adds it, with its record r
+// The share of a slice's links that one of NW wavefronts walks: whole pairs,
+// the same for all lanes; k0 its first link.
+template <int NW>
+struct Share {
+  int k0, K, KF, KM;   // first link; this lane's, fewest and most links of the share
+  __device__ __forceinline__ Share(int w, int k, int kf, int km) {
+    const int n = 2 * (((km + 1) / 2 + NW - 1) / NW);
+    k0 = w * n;
+    auto part = [&](int v) { return min(max(v - k0, 0), n); };
+    K = part(k);
+    KF = part(kf);
+    KM = part(km);
+  }
+};
+
 constexpr int OUT_OF_RANGE = 1 << 22;   // past every list, in pairs times 64
 template <int U, class Rec, class Load, class Fetch, class Link>
 __device__ __forceinline__ void walk_links(int K, int KF, int KM, Load load, Fetch fetch,
