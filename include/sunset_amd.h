@@ -279,8 +279,9 @@ int sv_calc_all_rhs(sv_ctx *ctx, int32_t iRKstep, double *rhs_ro, double *rhs_ro
                     double *rhs_rov, double *rhs_xx, double *rhs_xy, double *rhs_yy);
 /* nsteps of the main loop (sunset.F90:75-106): set_tstep, set_tstep_PID
  * (PID mode), step_rk3_4S_2R_EE (step.F90:218-512), itime += 1.  State stays
- * on the device; dt lives on the device.  use_graph != 0 replays one captured
- * step as a hipGraph. */
+ * on the device; dt lives on the device.  use_graph != 0 captures the steps of
+ * the call (up to 16) as a hipGraph and replays it; steps that do not fill one
+ * are launched singly. */
 int sv_run(sv_ctx *ctx, int32_t nsteps, int32_t use_graph);
 /* As sv_run (eager launches) with HIP events recorded on the context's stream
  * between the launches of every step.  kernel_ms[8]: mean device time per step

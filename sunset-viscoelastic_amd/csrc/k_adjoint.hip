@@ -1151,6 +1151,13 @@ int sv_dev_scatter_records(sv_ctx *c, const double *src, double *const f[6]) {
     if (!(cond)) return sv_fail((c), SV_E_ARG, __VA_ARGS__);  \
   } while (0)
 
+// the control block after the work queued on the context's stream
+static int read_ctrl(sv_ctx *c, sv_ctrl *h) {
+  SV_HIP(c, hipMemcpyAsync(h, c->ctrl, sizeof(*h), hipMemcpyDeviceToHost, c->stream));
+  SV_HIP(c, hipStreamSynchronize(c->stream));
+  return 0;
+}
+
 extern "C" {
 
 int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
@@ -1164,7 +1171,7 @@ int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
                "checkpoint interval must be in [1, 1000]");
   SV_HIP(c, hipSetDevice(c->device));
   sv_ctrl h{};
-  SV_HIP(c, hipMemcpy(&h, c->ctrl, sizeof(h), hipMemcpyDeviceToHost));
+  if (int rc = read_ctrl(c, &h)) return rc;
   SV_ADJ_CHECK(c, h.dt_mode == SV_DT_FIXED,
                "the adjoint needs a fixed time step (sv_set_control with SV_DT_FIXED)");
   if (!c->adj) {
@@ -1233,7 +1240,7 @@ int sv_rollout_forward(sv_ctx *c, int32_t nsteps, double *loss) {
   SV_HIP(c, hipSetDevice(c->device));
   {
     sv_ctrl h{};
-    SV_HIP(c, hipMemcpy(&h, c->ctrl, sizeof(h), hipMemcpyDeviceToHost));
+    if (int rc = read_ctrl(c, &h)) return rc;
     SV_ADJ_CHECK(c, h.dt_mode == SV_DT_FIXED, "the adjoint needs a fixed time step");
   }
   const int nck = (nsteps + A->every - 1) / A->every;

@@ -74,7 +74,22 @@ __global__ __launch_bounds__(1024) void k_total(int n, const double *v, double *
   if (threadIdx.x == 0) *out = s[0];
 }
 
+// (two copies of the block across the bus, each waited for, cost 30 us)
+__global__ void k_set_control(sv_ctrl *c, double dt, double time, int itime, double e1, double e2,
+                              double e3, int dt_mode) {
+  c->dt = dt; c->time = time; c->itime = itime;
+  c->emax_np1 = e1; c->emax_n = e2; c->emax_nm1 = e3;
+  c->dt_mode = dt_mode;
+}
+
 }  // namespace
+
+int sv_dev_set_control(sv_ctx *c, double dt, double time, int itime, double e1, double e2,
+                       double e3, int dt_mode) {
+  k_set_control<<<1, 1, 0, c->stream>>>(c->ctrl, dt, time, itime, e1, e2, e3, dt_mode);
+  SV_HIP(c, hipGetLastError());
+  return 0;
+}
 
 int sv_dev_init_records(sv_ctx *c, const double *fields) {
   const int n = c->npfb;

@@ -721,8 +721,8 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
   h.dt = 1.0e-6;                         // setup_flow.F90:149-151
   h.emax_np1 = h.emax_n = h.emax_nm1 = SV_PID_TOL;
   h.dt_mode = SV_DT_PID;
-  SV_HIP(c, hipMemcpy(c->ctrl, &h, sizeof(h), hipMemcpyHostToDevice));
-  if (int rc = sv_dev_init_state(c)) return rc;
+  SV_HIP(c, hipMemcpyAsync(c->ctrl, &h, sizeof(h), hipMemcpyHostToDevice, c->stream));
+  if (int rc = sv_dev_init_state(c)) return rc;   // synchronises
   c->have_state = true;
   c->graph_valid = false;
   return 0;
@@ -837,13 +837,7 @@ int sv_set_control(sv_ctx *c, double dt, double time, int32_t itime, double e1, 
   SV_CHECK(c, dt_mode == SV_DT_PID || dt_mode == SV_DT_FIXED || dt_mode == SV_DT_CFL,
            "bad dt mode %d (0 PID, 1 fixed, 2 CFL-limited)", dt_mode);
   if (int rc = set_device(c)) return rc;
-  sv_ctrl h{};
-  SV_HIP(c, hipMemcpy(&h, c->ctrl, sizeof(h), hipMemcpyDeviceToHost));
-  h.dt = dt; h.time = time; h.itime = itime;
-  h.emax_np1 = e1; h.emax_n = e2; h.emax_nm1 = e3;
-  h.dt_mode = dt_mode;
-  SV_HIP(c, hipMemcpy(c->ctrl, &h, sizeof(h), hipMemcpyHostToDevice));
-  return 0;
+  return sv_dev_set_control(c, dt, time, itime, e1, e2, e3, dt_mode);
 }
 
 int sv_ensemble_get_control(sv_ctx *c, int32_t member, double *dt, double *time,
@@ -894,6 +888,8 @@ int sv_calc_all_rhs(sv_ctx *c, int32_t iRKstep, double *r0, double *r1, double *
   return 0;
 }
 
+constexpr int GRAPH_STEPS = 16;
+
 int sv_run(sv_ctx *c, int32_t nsteps, int32_t use_graph) {
   SV_CHECK(c, c && c->have_state, "sv_set_initial must come first");
   SV_CHECK(c, nsteps >= 0, "nsteps must be >= 0");
@@ -902,24 +898,33 @@ int sv_run(sv_ctx *c, int32_t nsteps, int32_t use_graph) {
   SV_HIP(c, e0.create());
   SV_HIP(c, e1.create());
   SV_HIP(c, hipEventRecord(e0, c->stream));
+  int s = 0;
   if (use_graph && nsteps > 0) {
-    if (!c->graph_valid) {
+    // Consecutive graph launches leave the GPU idle for ~8 us, so a graph holds
+    // the steps of a call, GRAPH_STEPS at most; it is captured again for calls
+    // of at least twice as many as it holds.  Steps that do not fill a graph
+    // are launched one by one.
+    const int want = std::min(nsteps, GRAPH_STEPS);
+    if (!c->graph_valid || want >= 2 * c->graph_steps) {
+      c->graph_valid = false;
       if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
       hipGraph_t g;
       SV_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int rc = sv_dev_step(c, nullptr);
+      int rc = 0;
+      for (int k = 0; k < want && !rc; k++) rc = sv_dev_step(c, nullptr);
       hipError_t ce = hipStreamEndCapture(c->stream, &g);
       if (rc) return rc;
       SV_HIP(c, ce);
       SV_HIP(c, hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0));
       SV_HIP(c, hipGraphDestroy(g));
+      c->graph_steps = want;
       c->graph_valid = true;
     }
-    for (int s = 0; s < nsteps; s++) SV_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
-  } else {
-    for (int s = 0; s < nsteps; s++)
-      if (int rc = sv_dev_step(c, nullptr)) return rc;
+    for (; s + c->graph_steps <= nsteps; s += c->graph_steps)
+      SV_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
   }
+  for (; s < nsteps; s++)
+    if (int rc = sv_dev_step(c, nullptr)) return rc;
   SV_HIP(c, hipEventRecord(e1, c->stream));
   SV_HIP(c, hipEventSynchronize(e1));
   float ms = 0;

@@ -310,6 +310,7 @@ struct sv_ctx {
   double *tmp_phi = nullptr, *tmp_out = nullptr; int tmp_cap = 0;
   // graph
   hipGraphExec_t graph_exec = nullptr;
+  int graph_steps = 0;      // steps the captured graph holds
   bool graph_valid = false;
   // timings (ms)
   double t_neigh = 0, t_weights = 0, t_weights_tune = 0, t_step = 0;
@@ -417,7 +418,10 @@ int sv_check_device_ptr(sv_ctx *c, const void *p, const char *what);
 // state records in U from six caller-order device arrays (ro, u, v, c),
 // fields[6][npfb]
 int sv_dev_init_records(sv_ctx *c, const double *fields);
-int sv_dev_forcing(sv_ctx *c);                       // fx from the physics constants
+int sv_dev_forcing(sv_ctx *c);
+// sv_set_control's values, in the order of the context's stream
+int sv_dev_set_control(sv_ctx *c, double dt, double time, int itime, double e1, double e2,
+                       double e3, int dt_mode);                       // fx from the physics constants
 int sv_dev_volume_sum(sv_ctx *c, double *sum);       // of the real nodes
 // ---- kernels: time stepping (k_step.hip) ----
 // gather records and set_tstep minima of the state in U (no correction)
