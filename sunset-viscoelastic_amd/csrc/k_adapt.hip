@@ -21,8 +21,8 @@
 // amplification sums use the device's cos/sin and a wave reduction: they are
 // compared with 1.0001 and 0, not with rounding-level thresholds.
 //
-// One block (one wavefront) per real node; LDS holds the node's SVD (U, V,
-// the original matrix), a batch of monomial/ABF rows and per-neighbour data.
+// One block (one wavefront) per real node; LDS holds the node's SVD (U, V) and
+// per-neighbour data.
 #pragma clang fp contract(off)
 
 #include <math.h>
@@ -277,14 +277,24 @@ __device__ bool svd_gr(double *U, double *W, double *V, double *rv1) {
       g = gr_pythag(f, 1.0);
       f = ((x - z) * (x + z) + h * ((y / (f + f_sign(g, f))) - h)) / x;
       c = 1.0; s = 1.0;
+      // The chase: column j of U and V stays in registers from the rotation
+      // before, and what the next rotation reads (nothing that this one writes)
+      // is requested before this one's chain of divisions and roots.
+      const int lr = ln < n ? ln : n - 1;
+      double vj = VM(lr, l), uj = UM(lr, l);
+      double g_n = rv1[l + 1], y_n = W[l + 1], vi_n = VM(lr, l + 1), ui_n = UM(lr, l + 1);
       for (int j = l; j <= nm; j++) {
         const int i = j + 1;
-        g = rv1[i];
-        y = W[i];
+        const double vi = vi_n, ui = ui_n;
+        g = g_n;
+        y = y_n;
+        {
+          const int q = i < k ? i + 1 : i;
+          g_n = rv1[q]; y_n = W[q]; vi_n = VM(lr, q); ui_n = UM(lr, q);
+        }
         h = s * g;
         g = c * g;
         z = gr_pythag(f, h);
-        __syncthreads();
         if (ln == 0) rv1[j] = z;
         c = f / z;
         s = h / z;
@@ -292,11 +302,8 @@ __device__ bool svd_gr(double *U, double *W, double *V, double *rv1) {
         g = -(x * s) + (g * c);
         h = y * s;
         y = y * c;
-        if (ln < n) {
-          const double xv = VM(ln, j), zv = VM(ln, i);
-          VM(ln, j) = (xv * c) + (zv * s);
-          VM(ln, i) = -(xv * s) + (zv * c);
-        }
+        if (ln < n) VM(ln, j) = (vj * c) + (vi * s);
+        vj = -(vj * s) + (vi * c);
         z = gr_pythag(f, h);
         if (ln == 0) W[j] = z;
         if (z != 0.0) {
@@ -306,13 +313,14 @@ __device__ bool svd_gr(double *U, double *W, double *V, double *rv1) {
         }
         f = (c * g) + (s * y);
         x = -(s * g) + (c * y);
-        if (ln < n) {
-          const double yv = UM(ln, j), zv = UM(ln, i);
-          UM(ln, j) = (yv * c) + (zv * s);
-          UM(ln, i) = -(yv * s) + (zv * c);
-        }
-        __syncthreads();
+        if (ln < n) UM(ln, j) = (uj * c) + (ui * s);
+        uj = -(uj * s) + (ui * c);
       }
+      if (ln < n) {
+        VM(ln, k) = vj;
+        UM(ln, k) = uj;
+      }
+      __syncthreads();
       if (ln == 0) {
         rv1[l] = 0.0;
         rv1[k] = f;
@@ -364,11 +372,29 @@ struct AdaptArgs {
   int kcap;                     // longest list
 };
 
-// LDS of one node (doubles): U, V, M [NG*NG]; rows X, G [RB][NG]; W, rv1,
-// tmp, bL, bX, bY, xv [NG]; per neighbour x, y, dL, dX, dY [kcap]; list ints
+// LDS of one node (doubles): the SVD's U and V [NG*NG each]; W, rv1, tmp, bL, bX,
+// bY, xv [NG]; per neighbour x, y [kcap]; list ints.  Before the SVD U and V hold
+// the rows X, G [RB][NG] of the matrix build, after it the matrix again (kept in
+// registers meanwhile) and then the weights dL, dX, dY [kcap].  What bounds the
+// kernel is the chain of divisions and roots of each rotation (~750 rotations
+// an SVD of order 6), so what counts is nodes in flight: with an area for each
+// of these 6 fitted a CU at order 6, 10 do so (9216 nodes: 42.0 -> 30.3 ms with
+// the chase's requests ahead of its chain).
 template <int MF>
-constexpr int lds_doubles_fixed() {
-  return 3 * nsz(MF) * nsz(MF) + 2 * RB * nsz(MF) + 7 * nsz(MF);
+constexpr int svd_doubles(int kcap) {
+  const int uv = 2 * nsz(MF) * nsz(MF), rows = 2 * RB * nsz(MF), w = 3 * kcap;
+  return uv > rows ? (uv > w ? uv : w) : (rows > w ? rows : w);
+}
+template <int MF>
+constexpr size_t lds_bytes(int kcap) {
+  return sizeof(double) * ((size_t)svd_doubles<MF>(kcap) + 7 * nsz(MF) + 2 * (size_t)kcap) +
+         sizeof(int) * (size_t)kcap + 64;
+}
+// longest list taken
+template <int MF>
+constexpr int list_max() {
+  constexpr int fixed = 3 * nsz(MF) * nsz(MF) + 2 * RB * nsz(MF) + 7 * nsz(MF);
+  return (64 * 1024 - 64 - 8 * fixed) / 44;
 }
 
 // One pass over node i: returns the accepted reductions, or -1 (no SVD
@@ -379,13 +405,13 @@ __device__ int adapt_pass(const AdaptArgs &a, int i, int pass, double *lds) {
   constexpr int NG = nsz(MF), n = nsz(M);
   constexpr int NE = (n * n + WV - 1) / WV;
   const int ln = threadIdx.x;
-  double *U = lds, *V = U + NG * NG, *Mx = V + NG * NG;
-  double *RX = Mx + NG * NG, *RG = RX + RB * NG;
-  double *Wv = RG + RB * NG, *rv1 = Wv + NG, *tmp = rv1 + NG, *bL = tmp + NG, *bX = bL + NG,
-         *bY = bX + NG, *xv = bY + NG;
-  double *kx = xv + NG, *ky = kx + a.kcap, *dL = ky + a.kcap, *dX = dL + a.kcap,
-         *dY = dX + a.kcap;
-  int *list = reinterpret_cast<int *>(dY + a.kcap);
+  double *U = lds, *V = U + NG * NG, *Mx = lds;
+  double *RX = lds, *RG = RX + RB * NG;
+  double *dL = lds, *dX = dL + a.kcap, *dY = dX + a.kcap;
+  double *Wv = lds + svd_doubles<MF>(a.kcap), *rv1 = Wv + NG, *tmp = rv1 + NG, *bL = tmp + NG,
+         *bX = bL + NG, *bY = bX + NG, *xv = bY + NG;
+  double *kx = xv + NG, *ky = kx + a.kcap;
+  int *list = reinterpret_cast<int *>(ky + a.kcap);
   const double xi = a.x[i], yi = a.y[i];
   const int64_t base = a.row_ptr[i];
   const double rtol = a.rtol[pass - 1], amp_tol = 1.0001;
@@ -439,7 +465,7 @@ __device__ int adapt_pass(const AdaptArgs &a, int i, int pass, double *lds) {
 #pragma unroll
     for (int m = 0; m < NE; m++) {
       const int e = ln + m * WV;
-      if (e < n * n) { U[e] = acc[m]; Mx[e] = acc[m]; }
+      if (e < n * n) U[e] = acc[m];
     }
     if (ln < n) {
       bL[ln] = (ln == 2 || ln == 4) ? 1.0 / hh / hh : 0.0;
@@ -451,6 +477,12 @@ __device__ int adapt_pass(const AdaptArgs &a, int i, int pass, double *lds) {
     svd_backsub<n>(U, Wv, V, bL, tmp);
     svd_backsub<n>(U, Wv, V, bX, tmp);
     svd_backsub<n>(U, Wv, V, bY, tmp);
+#pragma unroll
+    for (int m = 0; m < NE; m++) {   // the matrix, for the residual
+      const int e = ln + m * WV;
+      if (e < n * n) Mx[e] = acc[m];
+    }
+    __syncthreads();
     // residual of the Laplacian solution: row r by lane r, then the sum of
     // squares in row order
     if (ln < n) {
@@ -554,11 +586,10 @@ __global__ __launch_bounds__(WV) void k_adapt(AdaptArgs a) {
 
 template <int MF, int MD>
 int launch_adapt(sv_ctx *c, const AdaptArgs &a) {
-  const size_t shm = sizeof(double) * ((size_t)lds_doubles_fixed<MF>() + 5 * (size_t)a.kcap) +
-                     sizeof(int) * (size_t)a.kcap + 64;
-  if (shm > 64 * 1024)
-    return sv_fail(c, SV_E_ARG, "adapt_stencils: %d-entry lists need %zu bytes of LDS (> 64 KiB)",
-                   a.kcap, shm);
+  if (a.kcap > list_max<MF>())
+    return sv_fail(c, SV_E_ARG, "adapt_stencils: %d-entry lists are longer than the LDS area for "
+                   "them (%d entries at this order)", a.kcap, list_max<MF>());
+  const size_t shm = lds_bytes<MF>(a.kcap);
   k_adapt<MF, MD><<<a.npfb, WV, shm, c->stream>>>(a);
   SV_HIP(c, hipGetLastError());
   return 0;
