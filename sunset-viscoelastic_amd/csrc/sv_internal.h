@@ -206,6 +206,12 @@ __host__ __device__ __forceinline__ int64_t sv_w3(int64_t e, int c) {
 #define SV_FLIP_SHIFT 29
 #define SV_FLIP_MASK ((1 << SV_FLIP_SHIFT) - 1)
 
+// a block of device memory
+struct sv_blk {
+  void *p;
+  size_t bytes;
+};
+
 struct sv_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -315,7 +321,8 @@ struct sv_ctx {
   // timings (ms)
   double t_neigh = 0, t_weights = 0, t_weights_tune = 0, t_step = 0;
   // device buffer registry for cleanup
-  std::vector<void *> allocs;
+  std::vector<sv_blk> allocs;   // device memory in use
+  std::vector<sv_blk> spare;    // of the node set before, not yet taken over
 };
 
 // ---- helpers (sv_api.cpp) ----
@@ -365,6 +372,7 @@ struct EventTmp {
 };
 int sv_ensure_sell(sv_ctx *c);
 void sv_free(sv_ctx *c, void *p);
+void sv_release_spare(sv_ctx *c);
 
 // ---- kernels: nodes/neighbours (k_nodes.hip) ----
 int sv_dev_create_ghosts(sv_ctx *c);

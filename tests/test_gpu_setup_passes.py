@@ -100,3 +100,33 @@ def test_initial_records_round_trip():
             for k in ic if form == "di" else ("ro", "u", "v"):
                 assert np.abs(g[k] - ic[k]).max() <= tol, (form, k)
             s.close()
+
+
+def test_node_sets_one_after_another():
+    """A context's node sets of growing, equal and shrinking sizes and other orders'
+    lists, each set up in the memory of the one before: fields and operators
+    equal, bit for bit, those of a context that holds that set alone."""
+    sets = [jittered_lattice(nx, ny, seed=nx, h_over_s=h)
+            for nx, ny, h in ((24, 23, 1.8), (24, 23, 1.8), (26, 24, 1.8), (25, 23, 2.4),
+                              (60, 50, 1.8), (24, 23, 1.8))]
+    sets.append(wall_channel(16, 16, order=4, seed=1))
+    one = sunset_amd.Solver(morder=4, form="lc")
+
+    def passes(s, ns):
+        s.setup(ns)
+        s.set_phys(Re=10.0, Wi=1.0, beta=0.5, Ma=0.1)
+        n = ns.npfb
+        phi = np.sin(2 * np.pi * ns.x) * np.cos(2 * np.pi * ns.y)
+        # s.np values: the ghosts' are their parents'
+        op = s.laplacian(np.concatenate([phi, np.zeros(s.np - n)]))
+        s.set_initial(dict(ro=np.ones(n), u=0.1 * phi, v=0.1 * phi, cxx=1 + 0.1 * phi ** 2,
+                           cxy=0.05 * phi, cyy=np.ones(n)), dt=1e-6)
+        s.run(2)
+        f = s.fields()
+        return [op] + [f[k] for k in ("ro", "rou", "rov", "cxx", "cxy", "cyy")]
+    for k, ns in enumerate(sets):
+        alone = sunset_amd.Solver(morder=4, form="lc")
+        for a, b in zip(passes(one, ns), passes(alone, ns)):
+            assert np.isfinite(a).all() and np.array_equal(a, b), k
+        alone.close()
+    one.close()
