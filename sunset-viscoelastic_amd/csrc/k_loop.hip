@@ -177,12 +177,12 @@ __global__ void k_kd_split(int nseg, const int *start, const int *left, const in
 
 // ---- SELL offsets -------------------------------------------------------------
 // entries of slice s: 64 times its longest list, made even
-__global__ void k_slice_width(int n, const int *cnt, int64_t *w) {
+__global__ void k_slice_width(int n, const int *cnt, int even, int64_t *w) {
   const int s = blockIdx.x, slot = s * SV_WAVE + (int)threadIdx.x;
   int m = slot < n ? cnt[slot] : 0;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o));
-  if (threadIdx.x == 0) w[s] = (int64_t)((m + 1) & ~1) * SV_WAVE;
+  if (threadIdx.x == 0) w[s] = (int64_t)(even ? (m + 1) & ~1 : m) * SV_WAVE;
 }
 
 // fewest and most links of the slice's nodes, small and full lists
@@ -214,7 +214,9 @@ static_assert(HT == 1 << 12, "halo_hash gives 12 bits");
 // Distinct link targets of halo block b (slots [b * hb, (b + 1) * hb)), sorted,
 // into list[b * HC ..), their number into hcnt[b] (HC + 1 when there are more
 // than HC: such a layout has no halo sweeps), and every link's rank into lcol.
-// Latency-bound LDS work: 28 KB per workgroup, five workgroups per CU.
+// Latency-bound LDS work: 28 KB per workgroup, five workgroups per CU.  PAIRS:
+// lcol and the padding by pairs of links (the loop layout), else entry by entry.
+template <bool PAIRS>
 __global__ __launch_bounds__(HTHREADS) void k_halo(int hb, int nslot, const int64_t *off,
                                                    const int *cnt, const int *col,
                                                    const uint8_t *flip, int *hcnt, int *list,
@@ -288,17 +290,17 @@ __global__ __launch_bounds__(HTHREADS) void k_halo(int hb, int nslot, const int6
     int W = K;   // the slice's padded length: padding entries get rank 0
 #pragma unroll
     for (int o2 = 32; o2 >= 1; o2 >>= 1) W = max(W, __shfl_xor(W, o2));
-    W = (W + 1) & ~1;
+    if (PAIRS) W = (W + 1) & ~1;
     for (int k = wave; k < W; k += HTHREADS / SV_WAVE) {
       const int64_t e = o + (int64_t)k * SV_WAVE + lane;
       if (k >= K) {
-        lcol[sv_pair(e)] = 0;
+        lcol[PAIRS ? sv_pair(e) : e] = 0;
         continue;
       }
       const int key = flip ? col[e] | (int)flip[e] << SV_FLIP_SHIFT : col[e];
       int h = halo_hash(key);
       while (tab[h] != key) h = (h + 1) & (HT - 1);
-      lcol[sv_pair(e)] = rank[h];
+      lcol[PAIRS ? sv_pair(e) : e] = rank[h];
     }
   }
 }
@@ -497,7 +499,7 @@ int build_halos(sv_ctx *c, sv_loopl &L, int hb, int nslot) {
     k_slice_range<<<nsl, SV_WAVE, 0, c->stream>>>(L.cnt_small, L.cnt, L.krange);
     SV_HIP(c, hipGetLastError());
   }
-  k_halo<<<nb, HTHREADS, 0, c->stream>>>(hb, nslot, L.off, L.cnt, L.col, L.lflip, hcnt, list,
+  k_halo<true><<<nb, HTHREADS, 0, c->stream>>>(hb, nslot, L.off, L.cnt, L.col, L.lflip, hcnt, list,
                                          L.lcol);
   SV_HIP(c, hipGetLastError());
   L.hcnt.resize(nb);
@@ -613,7 +615,7 @@ static int build_layout(sv_ctx *c, int hb) {
     DevTmp<int64_t> w;
     SV_HIP(c, w.alloc((size_t)ns + 1));
     SV_HIP(c, hipMemsetAsync(w.p + ns, 0, sizeof(int64_t), c->stream));
-    k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, L.cnt, w);
+    k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, L.cnt, 1, w);
     SV_HIP(c, hipGetLastError());
     if (int rc = scan_i64(c, (const int64_t *)w.p, L.off, ns + 1)) return rc;
   }
@@ -673,7 +675,7 @@ int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
   SV_HIP(c, hipMemsetAsync(bad, 0, sizeof(int), c->stream));
   SV_HIP(c, hipMemsetAsync(w.p + ns, 0, sizeof(int64_t), c->stream));
   k_t_count<<<ns, TT, 0, c->stream>>>(n, L.off, L.cnt, L.col, T.cnt, bad);
-  k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, T.cnt, w);
+  k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, T.cnt, 1, w);
   SV_HIP(c, hipGetLastError());
   if (int rc = scan_i64(c, (const int64_t *)w.p, T.off, ns + 1)) return rc;
   int64_t links = 0;
@@ -705,5 +707,68 @@ int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
   SV_HIP(c, hipGetLastError());
   if (int rc = build_halos(c, T, SV_WAVE, n)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));   // the temporaries go out of scope
+  return 0;
+}
+
+// Slice offsets of lists of cnt[n] links (exact widths), on the device
+int sv_dev_slice_offsets(sv_ctx *c, int n, const int *cnt, int64_t *off, int64_t *total) {
+  const int ns = (n + SV_WAVE - 1) / SV_WAVE;
+  DevTmp<int64_t> w;
+  SV_HIP(c, w.alloc((size_t)ns + 1));
+  SV_HIP(c, hipMemsetAsync(w.p + ns, 0, sizeof(int64_t), c->stream));
+  k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, cnt, 0, w);
+  SV_HIP(c, hipGetLastError());
+  if (int rc = scan_i64(c, (const int64_t *)w.p, off, ns + 1)) return rc;
+  SV_HIP(c, hipMemcpyAsync(total, off + ns, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+  SV_HIP(c, hipStreamSynchronize(c->stream));
+  return 0;
+}
+
+// Halos of the drop-in layout's slices (folded columns), for the operators.
+// shmax 0: none (a slice has more than HC distinct neighbours, or no memory).
+int sv_dev_sell_halos(sv_ctx *c) {
+  const int n = c->npfb, ns = c->nslices;
+  c->shmax = 0;
+  DevTmp<int> hcnt, list;
+  SV_HIP(c, hcnt.alloc((size_t)ns + 1));
+  if (list.alloc((size_t)ns * HC) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if ((!c->slcol && sv_alloc(c, (void **)&c->slcol, sizeof(uint16_t) * ((size_t)c->sell_nnz + 1))) ||
+      (!c->shoff && sv_alloc(c, (void **)&c->shoff, sizeof(int64_t) * ((size_t)ns + 1)))) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  k_halo<false><<<ns, HTHREADS, 0, c->stream>>>(SV_WAVE, n, c->sell_off, c->cnt, c->scol, nullptr,
+                                                hcnt, list, c->slcol);
+  SV_HIP(c, hipGetLastError());
+  std::vector<int> hc(ns);
+  SV_HIP(c, hipMemcpyAsync(hc.data(), hcnt.p, sizeof(int) * ns, hipMemcpyDeviceToHost, c->stream));
+  SV_HIP(c, hipStreamSynchronize(c->stream));
+  int most = 0;
+  int64_t tot = 0;
+  for (int v : hc) {
+    most = std::max(most, v);
+    tot += v;
+  }
+  if (most > HC) return 0;
+  if (tot > c->shcap) {
+    sv_free(c, c->shidx);
+    c->shidx = nullptr;
+    c->shcap = 0;
+    if (sv_alloc(c, (void **)&c->shidx, sizeof(int) * ((size_t)tot + 1))) {
+      (void)hipGetLastError();
+      return 0;
+    }
+    c->shcap = tot;
+  }
+  SV_HIP(c, hipMemsetAsync(hcnt.p + ns, 0, sizeof(int), c->stream));
+  hipcub::TransformInputIterator<int64_t, ToI64, const int *> in(hcnt.p, ToI64());
+  if (int rc = scan_i64(c, in, c->shoff, ns + 1)) return rc;
+  k_halo_compact<<<ns, HTHREADS, 0, c->stream>>>(c->shoff, list, c->shidx);
+  SV_HIP(c, hipGetLastError());
+  SV_HIP(c, hipStreamSynchronize(c->stream));
+  c->shmax = most;
   return 0;
 }

@@ -428,47 +428,51 @@ int sv_dev_find_neighbours(sv_ctx *c) {
   return 0;
 }
 
+// links per slice, padding included
+static __global__ void k_slice_links(int ns, const int64_t *off, int *w) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s < ns) w[s] = (int)((off[s + 1] - off[s]) / SV_WAVE);
+}
+
 int sv_dev_build_sell(sv_ctx *c) {
   const int npfb = c->npfb;
   const int ns = (npfb + SV_WAVE - 1) / SV_WAVE;
-  std::vector<int> hc(npfb);
-  SV_HIP(c, hipMemcpy(hc.data(), c->cnt, sizeof(int) * npfb, hipMemcpyDeviceToHost));
-  std::vector<int> w(ns);
-  std::vector<int64_t> off(ns + 1);
-  off[0] = 0;
-  int wmax = 0;
-  for (int s = 0; s < ns; s++) {
-    int m = 0;
-    for (int l = 0; l < SV_WAVE && s * SV_WAVE + l < npfb; l++)
-      m = hc[s * SV_WAVE + l] > m ? hc[s * SV_WAVE + l] : m;
-    w[s] = m;
-    wmax = m > wmax ? m : wmax;
-    off[s + 1] = off[s] + (int64_t)m * SV_WAVE;
-  }
-  if (c->nslices != ns || c->sell_nnz != off[ns]) {
-    void *bufs[] = {c->sell_off, c->sell_w, c->scol, c->scol_raw, c->swx, c->swy, c->swl, c->swh};
-    for (void *b : bufs)
-      if (b) sv_free(c, b);
-    c->nslices = ns;
-    c->sell_nnz = off[ns];
-    const size_t L = (size_t)c->sell_nnz + 1;
+  if (c->nslices != ns) {
+    for (void *b : {(void *)c->sell_off, (void *)c->sell_w, (void *)c->shoff}) sv_free(c, b);
+    c->sell_off = c->shoff = nullptr;
+    c->sell_w = nullptr;
     if (sv_alloc(c, (void **)&c->sell_off, sizeof(int64_t) * (ns + 1)) ||
-        sv_alloc(c, (void **)&c->sell_w, sizeof(int) * (ns + 1)) ||
-        sv_alloc(c, (void **)&c->scol, sizeof(int) * L) ||
+        sv_alloc(c, (void **)&c->sell_w, sizeof(int) * (ns + 1)))
+      return SV_E_NOMEM;
+  }
+  int64_t nnz = 0;
+  if (int rc = sv_dev_slice_offsets(c, npfb, c->cnt, c->sell_off, &nnz)) return rc;
+  if (c->nslices != ns || c->sell_nnz != nnz) {
+    for (void *b : {(void *)c->scol, (void *)c->scol_raw, (void *)c->swx, (void *)c->swy,
+                    (void *)c->swl, (void *)c->swh, (void *)c->slcol})
+      sv_free(c, b);
+    c->scol = c->scol_raw = nullptr;
+    c->slcol = nullptr;
+    c->swx = c->swy = c->swl = c->swh = nullptr;
+    c->nslices = ns;
+    c->sell_nnz = nnz;
+    const size_t L = (size_t)c->sell_nnz + 1;
+    if (sv_alloc(c, (void **)&c->scol, sizeof(int) * L) ||
         sv_alloc(c, (void **)&c->scol_raw, sizeof(int) * L) ||
         sv_alloc(c, (void **)&c->swx, sizeof(double) * L) ||
         sv_alloc(c, (void **)&c->swy, sizeof(double) * L) ||
         sv_alloc(c, (void **)&c->swl, sizeof(double) * L) ||
-        sv_alloc(c, (void **)&c->swh, sizeof(double) * L))
+        sv_alloc(c, (void **)&c->swh, sizeof(double) * L)) {
+      c->nslices = 0;
       return SV_E_NOMEM;
+    }
   }
-  SV_HIP(c, hipMemcpy(c->sell_off, off.data(), sizeof(int64_t) * (ns + 1),
-                      hipMemcpyHostToDevice));
-  SV_HIP(c, hipMemcpy(c->sell_w, w.data(), sizeof(int) * ns, hipMemcpyHostToDevice));
+  k_slice_links<<<(ns + 255) / 256, 256, 0, c->stream>>>(ns, c->sell_off, c->sell_w);
   k_sell_pack<<<ns, SP_T, 0, c->stream>>>(npfb, c->sell_off, c->sell_w, c->row_ptr, c->cnt,
                                           c->col_raw, c->irel, c->wx, c->wy, c->wl, c->wh,
                                           c->scol, c->scol_raw, c->swx, c->swy, c->swl, c->swh);
   SV_HIP(c, hipGetLastError());
+  if (int rc = sv_dev_sell_halos(c)) return rc;
   SV_HIP(c, hipStreamSynchronize(c->stream));
   c->sell_dirty = false;
   return 0;

@@ -26,6 +26,10 @@ struct ApplyArgs {
   const double *s0, *s1;    // weight sums
   const double *phi[AP_NF];
   double *o0[AP_NF], *o1[AP_NF];
+  const uint16_t *lcol;     // halos (k_apply_h)
+  const int64_t *hoff;
+  const int *hidx;
+  int hmax;
 };
 
 // One lane per node, one wavefront per workgroup, links in batches of AP_U:
@@ -34,7 +38,7 @@ struct ApplyArgs {
 // padding (or its last link again) and leaves it out of the sums.
 // 511x513 order 6, three fields: gradients 315 us in three launches of one field
 // each, 152 so, Laplacians 200 and 122, filters 195 and 115 (the scattered reads
-// of phi, up to 64 lines a wave, are what is left).
+// of phi, up to 64 lines a wave, are what is left: see k_apply_h).
 constexpr int AP_U = 4;
 template <int OP, int NF>
 __global__ __launch_bounds__(SV_WAVE) void k_apply(ApplyArgs a) {
@@ -83,8 +87,74 @@ __global__ __launch_bounds__(SV_WAVE) void k_apply(ApplyArgs a) {
   }
 }
 
+// k_apply with the slice's distinct neighbour values staged in LDS first (11 per
+// node in row order, order 6): a wavefront per field stages and walks its own
+// field, so every sum is k_apply's.  k_apply's scattered reads find little in the
+// L1 and take ~100 clocks each.  511x513 order 6, three fields, gradients 152 ->
+// 124 us, Laplacians 122 -> 73, filters 115 -> 71; what is left is the requests'
+// latency at 24 wavefronts a CU.  Taken where no slice has more than 1024 distinct
+// neighbours (not on the cylinder channel's order of nodes), on folded columns.
+constexpr int AH_U = 8;     // values a lane stages, and links it reads, at once (12, 16: the
+                            // same, 24: 8% slower)
+template <int OP>
+__global__ __launch_bounds__(SV_WAVE *AP_NF) void k_apply_h(ApplyArgs a) {
+  extern __shared__ double hl[];
+  constexpr bool GRAD = OP == SV_OP_GRAD;
+  const int s = sv_xcd_block();
+  const int lane = (int)threadIdx.x & (SV_WAVE - 1);
+  const int f = __builtin_amdgcn_readfirstlane((int)threadIdx.x / SV_WAVE);
+  const int i = s * SV_WAVE + lane;
+  const bool act = i < a.npfb;
+  const int64_t b = a.off[s] + lane;
+  const int K = act ? a.kcnt[i] : 0, W = a.width[s];
+  const int64_t h0 = a.hoff[s];
+  const int nh = (int)(a.hoff[s + 1] - h0);
+  const double *phi = a.phi[f];
+  double *hf = hl + (size_t)f * a.hmax;
+  for (int h = lane; h < nh; h += AH_U * SV_WAVE) {
+    int j[AH_U];
+#pragma unroll
+    for (int u = 0; u < AH_U; u++) j[u] = a.hidx[h0 + min(h + u * SV_WAVE, nh - 1)];
+    double v[AH_U];
+#pragma unroll
+    for (int u = 0; u < AH_U; u++) v[u] = phi[j[u]];
+#pragma unroll
+    for (int u = 0; u < AH_U; u++)
+      if (h + u * SV_WAVE < nh) hf[h + u * SV_WAVE] = v[u];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // its own wavefront reads it
+  double t0 = 0.0, t1 = 0.0;
+  for (int k = 0; k < W; k += AH_U) {
+    int j[AH_U];
+    double w0[AH_U], w1[AH_U];
+#pragma unroll
+    for (int u = 0; u < AH_U; u++) {
+      const int64_t e = b + (int64_t)min(k + u, W - 1) * SV_WAVE;
+      j[u] = a.lcol[e];
+      w0[u] = a.w0[e];
+      if (GRAD) w1[u] = a.w1[e];
+    }
+#pragma unroll
+    for (int u = 0; u < AH_U; u++)
+      if (k + u < K) {
+        const double p = hf[j[u]];
+        t0 = t0 + p * w0[u];
+        if (GRAD) t1 = t1 + p * w1[u];
+      }
+  }
+  if (!act) return;
+  const double pi = phi[i], s0 = a.s0[i];
+  if (OP == SV_OP_FILTER) a.o0[f][i] = pi + (t0 - pi * s0);
+  else a.o0[f][i] = t0 - pi * s0;
+  if (GRAD) a.o1[f][i] = t1 - pi * a.s1[i];
+}
+
 template <int OP>
 void launch_apply(const ApplyArgs &a, int nf, int ns, hipStream_t st) {
+  if (a.hmax > 0) {
+    k_apply_h<OP><<<ns, SV_WAVE * nf, sizeof(double) * (size_t)nf * a.hmax, st>>>(a);
+    return;
+  }
   switch (nf) {
   case 1: k_apply<OP, 1><<<ns, SV_WAVE, 0, st>>>(a); break;
   case 2: k_apply<OP, 2><<<ns, SV_WAVE, 0, st>>>(a); break;
@@ -153,6 +223,12 @@ int sv_dev_apply(sv_ctx *c, int op, int nfields, const double *const *phi, doubl
   a.off = c->sell_off;
   a.width = c->sell_w;
   a.col = raw_cols ? c->scol_raw : c->scol;
+  if (!raw_cols) {   // the halos are of the folded columns
+    a.lcol = c->slcol;
+    a.hoff = c->shoff;
+    a.hidx = c->shidx;
+    a.hmax = c->shmax;
+  }
   switch (op) {
   case SV_OP_GRAD: a.kcnt = c->cnt_small; a.w0 = c->swx; a.w1 = c->swy; a.s0 = c->gsx; a.s1 = c->gsy; break;
   case SV_OP_LAP:

@@ -199,6 +199,7 @@ int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, cons
   c->wx = c->wy = c->wl = c->wh = nullptr;
   c->gsx = c->gsy = c->lsum = c->hsum = c->vol = nullptr;
   c->sell_off = nullptr; c->sell_w = nullptr; c->scol = c->scol_raw = nullptr;
+  c->slcol = nullptr; c->shoff = nullptr; c->shidx = nullptr; c->shmax = 0; c->shcap = 0;
   c->swx = c->swy = c->swl = c->swh = nullptr; c->nslices = 0; c->sell_nnz = 0;
   c->singular = nullptr; c->fx = nullptr; c->partial = nullptr; c->ctrl = nullptr;
   c->U = c->Uf = c->reg = c->eacc = nullptr;

@@ -263,6 +263,13 @@ struct sv_ctx {
   int *sell_w = nullptr;
   int *scol = nullptr, *scol_raw = nullptr;
   double *swx = nullptr, *swy = nullptr, *swl = nullptr, *swh = nullptr;
+  // halos of its slices, for the operators (shmax 0: none): the distinct folded
+  // columns of slice s shidx[shoff[s] .. shoff[s + 1]), links' ranks slcol
+  uint16_t *slcol = nullptr;
+  int64_t *shoff = nullptr;
+  int *shidx = nullptr;
+  int shmax = 0;
+  int64_t shcap = 0;        // entries shidx has room for
   bool sell_dirty = true;
   int *singular = nullptr;  // count of zero pivots in the last solve
   int n_singular = 0, n_systems = 0;
@@ -385,6 +392,8 @@ int sv_dev_build_loop(sv_ctx *c);
 // the halos of the layout in c->L over nslot slots (a context's own, or an
 // ensemble's concatenated one)
 int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T);
+int sv_dev_slice_offsets(sv_ctx *c, int n, const int *cnt, int64_t *off, int64_t *total);
+int sv_dev_sell_halos(sv_ctx *c);
 int sv_dev_build_halos(sv_ctx *c, int nslot);
 int sv_ensure_loop(sv_ctx *c);
 // ---- kernels: weights (k_weights.hip) ----
