@@ -88,6 +88,7 @@ int sv_dev_set_control(sv_ctx *c, double dt, double time, int itime, double e1, 
                        double e3, int dt_mode) {
   k_set_control<<<1, 1, 0, c->stream>>>(c->ctrl, dt, time, itime, e1, e2, e3, dt_mode);
   SV_HIP(c, hipGetLastError());
+  SV_HIP(c, hipStreamSynchronize(c->stream));   // diagnostics read it on other streams
   return 0;
 }
 

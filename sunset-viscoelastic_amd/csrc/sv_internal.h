@@ -436,7 +436,7 @@ int sv_check_device_ptr(sv_ctx *c, const void *p, const char *what);
 // fields[6][npfb]
 int sv_dev_init_records(sv_ctx *c, const double *fields);
 int sv_dev_forcing(sv_ctx *c);
-// sv_set_control's values, in the order of the context's stream
+// sv_set_control's values (waits for them)
 int sv_dev_set_control(sv_ctx *c, double dt, double time, int itime, double e1, double e2,
                        double e3, int dt_mode);                       // fx from the physics constants
 int sv_dev_volume_sum(sv_ctx *c, double *sum);       // of the real nodes
