@@ -167,7 +167,10 @@ int sv_get_weights(sv_ctx *ctx, int32_t nplink, double *ij_w_grad, double *ij_w_
  * sv_calc_labf_weights; "weights_variant_m4|6|8" the launch variant used for
  * that order (bit 0: persistent grid, else one block per system; bit 1:
  * 32-neighbour assembly tiles, else 16; -1 none);
- * "weights_tune_m<order>_<variant>" the autotuning sample time of a variant. */
+ * "weights_tune_m<order>_<variant>" the autotuning sample time of a variant;
+ * "spare_bytes" the device memory that the context still holds of the node set
+ * before (given back by the first operator, sv_set_initial, sv_get_weights,
+ * sv_adapt_stencils, or an allocation that fails without it). */
 int sv_get_timing(sv_ctx *ctx, const char *what, double *ms);
 /* Tuning switches:
  *   "weights_autotune" (default 1): for an order with >= 409600 systems, the

@@ -616,8 +616,8 @@ int sv_dev_adapt(sv_ctx *c, int *reductions_host) {
     return sv_fail(c, SV_E_ARG, "adapt_stencils: LABFM order %d is not supported on the device "
                                 "(its SVD takes a lane per column, at most 64)", mf);
   DevTmp<int> red, fail;
-  SV_HIP(c, red.alloc(2 * (size_t)n));
-  SV_HIP(c, fail.alloc(1));
+  SV_HIP(c, red.alloc(c, 2 * (size_t)n));
+  SV_HIP(c, fail.alloc(c, 1));
   SV_HIP(c, hipMemsetAsync(fail, 0, sizeof(int), c->stream));
   AdaptArgs a{};
   a.npfb = n;

@@ -1221,7 +1221,7 @@ int sv_rhs_vjp(sv_ctx *c, const double *const rbar[6], double *const ubar[6]) {
   A->taped = false;
   {
     DevTmp<double> scratch;
-    SV_HIP(c, scratch.alloc(6 * (size_t)c->npfb));
+    SV_HIP(c, scratch.alloc(c, 6 * (size_t)c->npfb));
     if (int rc = sv_dev_rhs(c, 1, scratch, A->tape[0], A->tape[1])) return rc;
   }
   if (int r2 = upload_records(c, A->Rbar, rbar)) return r2;

@@ -377,7 +377,7 @@ int scan_i64(sv_ctx *c, In in, int64_t *out, int n) {
   size_t tb = 0;
   SV_HIP(c, hipcub::DeviceScan::ExclusiveSum(nullptr, tb, in, out, n, c->stream));
   DevTmp<char> tmp;
-  SV_HIP(c, tmp.alloc(tb > 0 ? tb : 16));
+  SV_HIP(c, tmp.alloc(c, tb > 0 ? tb : 16));
   SV_HIP(c, hipcub::DeviceScan::ExclusiveSum((void *)tmp, tb, in, out, n, c->stream));
   SV_HIP(c, hipStreamSynchronize(c->stream));
   return 0;
@@ -435,14 +435,14 @@ int kd_order(sv_ctx *c, int *perm, int by_len) {
   DevTmp<char> tmp;
   const size_t P = starts.size();
   size_t tb = 0;
-  SV_HIP(c, plan.alloc(3 * P));
-  SV_HIP(c, alt.alloc(n));
-  SV_HIP(c, key.alloc(2 * (size_t)n));
-  SV_HIP(c, boxes.alloc(2 * most));
+  SV_HIP(c, plan.alloc(c, 3 * P));
+  SV_HIP(c, alt.alloc(c, n));
+  SV_HIP(c, key.alloc(c, 2 * (size_t)n));
+  SV_HIP(c, boxes.alloc(c, 2 * most));
   hipcub::DoubleBuffer<uint64_t> kb(key.p, key.p + n);
   hipcub::DoubleBuffer<int> vb(perm, alt.p);
   SV_HIP(c, hipcub::DeviceRadixSort::SortPairs(nullptr, tb, kb, vb, n, 0, 64, c->stream));
-  SV_HIP(c, tmp.alloc(tb > 0 ? tb : 16));
+  SV_HIP(c, tmp.alloc(c, tb > 0 ? tb : 16));
   const KdBox dom{c->xmin, c->xmax, c->ymin, c->ymax};
   std::vector<int> h(3 * P);
   std::copy(starts.begin(), starts.end(), h.begin());
@@ -489,8 +489,8 @@ int build_halos(sv_ctx *c, sv_loopl &L, int hb, int nslot) {
   // the last slot are empty
   const int nb = (nslot + SV_BLOCK - 1) / SV_BLOCK * (SV_BLOCK / hb);
   DevTmp<int> hcnt, list;
-  SV_HIP(c, hcnt.alloc((size_t)nb + 1));
-  SV_HIP(c, list.alloc((size_t)nb * HC));
+  SV_HIP(c, hcnt.alloc(c, (size_t)nb + 1));
+  SV_HIP(c, list.alloc(c, (size_t)nb * HC));
   if (!L.lcol) {
     const int nsl = (nslot + SV_BLOCK - 1) / SV_BLOCK * (SV_BLOCK / SV_WAVE);
     if (sv_alloc(c, (void **)&L.lcol, sizeof(uint16_t) * (L.nnz + 1)) ||
@@ -613,7 +613,7 @@ static int build_layout(sv_ctx *c, int hb) {
   SV_HIP(c, hipGetLastError());
   {
     DevTmp<int64_t> w;
-    SV_HIP(c, w.alloc((size_t)ns + 1));
+    SV_HIP(c, w.alloc(c, (size_t)ns + 1));
     SV_HIP(c, hipMemsetAsync(w.p + ns, 0, sizeof(int64_t), c->stream));
     k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, L.cnt, 1, w);
     SV_HIP(c, hipGetLastError());
@@ -665,10 +665,10 @@ int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
   T.cnt_small = T.cnt;
   DevTmp<int> fill, bad;
   DevTmp<int64_t> start, w;
-  SV_HIP(c, fill.alloc(n));
-  SV_HIP(c, bad.alloc(1));
-  SV_HIP(c, start.alloc((size_t)n + 1));
-  SV_HIP(c, w.alloc((size_t)ns + 1));
+  SV_HIP(c, fill.alloc(c, n));
+  SV_HIP(c, bad.alloc(c, 1));
+  SV_HIP(c, start.alloc(c, (size_t)n + 1));
+  SV_HIP(c, w.alloc(c, (size_t)ns + 1));
   SV_HIP(c, hipMemsetAsync(T.off, 0, sizeof(int64_t) * (nslot / SV_WAVE + 1), c->stream));
   SV_HIP(c, hipMemsetAsync(T.cnt, 0, sizeof(int) * nslot, c->stream));
   SV_HIP(c, hipMemsetAsync(fill, 0, sizeof(int) * n, c->stream));
@@ -681,7 +681,7 @@ int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
   int64_t links = 0;
   {
     DevTmp<int> one;   // the counts and a last zero, for an exclusive scan of n + 1
-    SV_HIP(c, one.alloc((size_t)n + 1));
+    SV_HIP(c, one.alloc(c, (size_t)n + 1));
     SV_HIP(c, hipMemcpyAsync(one, T.cnt, sizeof(int) * n, hipMemcpyDeviceToDevice, c->stream));
     SV_HIP(c, hipMemsetAsync(one.p + n, 0, sizeof(int), c->stream));
     hipcub::TransformInputIterator<int64_t, ToI64, const int *> in(one.p, ToI64());
@@ -696,7 +696,7 @@ int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
   if (hbad) return sv_fail(c, SV_E_STATE, "stencil column out of range");
   const size_t E = (size_t)T.nnz + 1;
   DevTmp<uint64_t> key;
-  SV_HIP(c, key.alloc((size_t)links));
+  SV_HIP(c, key.alloc(c, (size_t)links));
   if (sv_alloc(c, (void **)&T.col, sizeof(int) * E) ||
       sv_alloc(c, (void **)&T.w3, 3 * sizeof(double) * E) ||
       sv_alloc(c, (void **)&T.wh, sizeof(double) * E))
@@ -714,7 +714,7 @@ int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T) {
 int sv_dev_slice_offsets(sv_ctx *c, int n, const int *cnt, int64_t *off, int64_t *total) {
   const int ns = (n + SV_WAVE - 1) / SV_WAVE;
   DevTmp<int64_t> w;
-  SV_HIP(c, w.alloc((size_t)ns + 1));
+  SV_HIP(c, w.alloc(c, (size_t)ns + 1));
   SV_HIP(c, hipMemsetAsync(w.p + ns, 0, sizeof(int64_t), c->stream));
   k_slice_width<<<ns, SV_WAVE, 0, c->stream>>>(n, cnt, 0, w);
   SV_HIP(c, hipGetLastError());
@@ -730,8 +730,8 @@ int sv_dev_sell_halos(sv_ctx *c) {
   const int n = c->npfb, ns = c->nslices;
   c->shmax = 0;
   DevTmp<int> hcnt, list;
-  SV_HIP(c, hcnt.alloc((size_t)ns + 1));
-  if (list.alloc((size_t)ns * HC) != hipSuccess) {
+  SV_HIP(c, hcnt.alloc(c, (size_t)ns + 1));
+  if (list.alloc(c, (size_t)ns * HC) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }

@@ -314,7 +314,7 @@ static int scan_int(sv_ctx *c, const int *in, int *out, int n) {
   size_t tb = 0;
   SV_HIP(c, hipcub::DeviceScan::ExclusiveSum(nullptr, tb, in, out, n, c->stream));
   DevTmp<char> tmp;
-  SV_HIP(c, tmp.alloc(tb > 0 ? tb : 16));
+  SV_HIP(c, tmp.alloc(c, tb > 0 ? tb : 16));
   SV_HIP(c, hipcub::DeviceScan::ExclusiveSum((void *)tmp, tb, in, out, n, c->stream));
   SV_HIP(c, hipStreamSynchronize(c->stream));
   return 0;
@@ -324,8 +324,8 @@ int sv_dev_create_ghosts(sv_ctx *c) {
   const int n = c->npfb;
   GhostDom g{c->xmin, c->xmax, c->ymin, c->ymax, c->bc[0], c->bc[1], c->bc[2], c->bc[3]};
   DevTmp<int> gcount, goff;
-  SV_HIP(c, gcount.alloc(n + 1));
-  SV_HIP(c, goff.alloc(n + 1));
+  SV_HIP(c, gcount.alloc(c, n + 1));
+  SV_HIP(c, goff.alloc(c, n + 1));
   SV_HIP(c, hipMemsetAsync(gcount, 0, sizeof(int) * (n + 1), c->stream));
   const int B = 256, nb = (n + B - 1) / B;
   k_ghost_count<<<nb, B, 0, c->stream>>>(n, g, c->x, c->y, c->h, gcount);
@@ -370,10 +370,10 @@ int sv_dev_find_neighbours(sv_ctx *c) {
   G.h0 = c->h0;
   const int nct = G.ncx * G.ncy;
   DevTmp<int> cellof, ccount, cstart, ip;
-  SV_HIP(c, cellof.alloc(np));
-  SV_HIP(c, ccount.alloc(nct + 1));
-  SV_HIP(c, cstart.alloc(nct + 1));
-  SV_HIP(c, ip.alloc(np));
+  SV_HIP(c, cellof.alloc(c, np));
+  SV_HIP(c, ccount.alloc(c, nct + 1));
+  SV_HIP(c, cstart.alloc(c, nct + 1));
+  SV_HIP(c, ip.alloc(c, np));
   SV_HIP(c, hipMemsetAsync(ccount, 0, sizeof(int) * (nct + 1), c->stream));
   const int B = 256;
   k_cell_count<<<(np + B - 1) / B, B, 0, c->stream>>>(np, G, c->x, c->y, cellof, ccount);

@@ -1509,7 +1509,7 @@ int sv_dev_rhs(sv_ctx *c, int iRKstep, double *out6, double *tapeG, double *tape
 int sv_dev_tune_groups(sv_ctx *c, int reps) {
   if (c->lgroups.size() < 2) { c->lgroup_mode = 0; return 0; }
   DevTmp<double> out;
-  SV_HIP(c, out.alloc(6 * (size_t)c->ntot));
+  SV_HIP(c, out.alloc(c, 6 * (size_t)c->ntot));
   EventTmp e0, e1;
   SV_HIP(c, e0.create());
   SV_HIP(c, e1.create());

@@ -1346,17 +1346,17 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   DevTmp<uint32_t> keys, vals;
   DevTmp<char> tmp;
   const size_t N2 = 2 * (size_t)n;
-  SV_HIP(c, dn.alloc(N2 + 1));
-  SV_HIP(c, dk.alloc(N2 + 1));
-  SV_HIP(c, dq.alloc(8));
-  SV_HIP(c, num.alloc((size_t)n + 1));
-  SV_HIP(c, first.alloc((size_t)n + 1));
-  SV_HIP(c, keys.alloc(2 * N2));
-  SV_HIP(c, vals.alloc(2 * N2));
+  SV_HIP(c, dn.alloc(c, N2 + 1));
+  SV_HIP(c, dk.alloc(c, N2 + 1));
+  SV_HIP(c, dq.alloc(c, 8));
+  SV_HIP(c, num.alloc(c, (size_t)n + 1));
+  SV_HIP(c, first.alloc(c, (size_t)n + 1));
+  SV_HIP(c, keys.alloc(c, 2 * N2));
+  SV_HIP(c, vals.alloc(c, 2 * N2));
   SysList sl_{n, c->cfg.morder, c->cfg.forder, c->nb, c->maxK, nullptr, c->cnt, c->cnt_small,
               c->node_type, c->h, c->hs};
   if (order_map_host) {
-    SV_HIP(c, dmap.alloc(n));
+    SV_HIP(c, dmap.alloc(c, n));
     SV_HIP(c, hipMemcpyAsync(dmap.p, order_map_host, sizeof(int) * n, hipMemcpyHostToDevice,
                              c->stream));
     sl_.order_map = dmap.p;
@@ -1368,7 +1368,7 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   SV_HIP(c, hipcub::DeviceScan::ExclusiveSum(nullptr, tb1, num.p, first.p, n + 1, c->stream));
   SV_HIP(c, hipcub::DeviceRadixSort::SortPairs(nullptr, tb2, kb, vb, (int)N2, 0, bits, c->stream));
   size_t tb = std::max(tb1, tb2);
-  SV_HIP(c, tmp.alloc(tb > 0 ? tb : 16));
+  SV_HIP(c, tmp.alloc(c, tb > 0 ? tb : 16));
   const int TB = 256;
   SV_HIP(c, hipMemsetAsync(dq.p, 0xff, sizeof(int) * 8, c->stream));
   k_sys_count<<<(n + TB) / TB, TB, 0, c->stream>>>(sl_, num);
@@ -1459,8 +1459,8 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
     if (!c->weights_autotune || sl.count < SV_TUNE_MIN || c->wtune[mi] >= 0) continue;
     const int stride = sl.count / S;
     DevTmp<int> tn, tk;
-    SV_HIP(c, tn.alloc(S));
-    SV_HIP(c, tk.alloc(S));
+    SV_HIP(c, tn.alloc(c, S));
+    SV_HIP(c, tk.alloc(c, S));
     k_sys_sample<<<(S + TB - 1) / TB, TB, 0, c->stream>>>(S, stride, dn.p + sl.first,
                                                           dk.p + sl.first, tn, tk);
     SV_HIP(c, hipGetLastError());
@@ -1491,8 +1491,8 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
   DevTmp<int> mn, mk;            // its nodes and kinds
   // the queue: the orders' slices, highest order first
   auto make_queue = [&]() -> int {
-    SV_HIP(c, mn.alloc(nsys));
-    SV_HIP(c, mk.alloc(nsys));
+    SV_HIP(c, mn.alloc(c, nsys));
+    SV_HIP(c, mk.alloc(c, nsys));
     int at = 0;
     for (auto it = slices.rbegin(); it != slices.rend(); ++it) {
       const size_t b = sizeof(int) * it->count;
@@ -1518,10 +1518,10 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
       for (int q = 0; q < S; q++) sm[q] = qm[q * stride];
       const std::vector<int> su = units_of(sm);
       DevTmp<int> tn, tk, tm, tu;
-      SV_HIP(c, tn.alloc(S));
-      SV_HIP(c, tk.alloc(S));
-      SV_HIP(c, tm.alloc(S));
-      SV_HIP(c, tu.alloc(su.size()));
+      SV_HIP(c, tn.alloc(c, S));
+      SV_HIP(c, tk.alloc(c, S));
+      SV_HIP(c, tm.alloc(c, S));
+      SV_HIP(c, tu.alloc(c, su.size()));
       k_sys_sample<<<(S + TB - 1) / TB, TB, 0, c->stream>>>(S, stride, mn, mk, tn, tk);
       SV_HIP(c, hipGetLastError());
       SV_HIP(c, hipMemcpy(tm, sm.data(), sizeof(int) * S, hipMemcpyHostToDevice));
@@ -1579,8 +1579,8 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
     const int total = nsys;
     const std::vector<int> qu = units_of(qm);
     DevTmp<int> mm, mu;
-    SV_HIP(c, mm.alloc(total));
-    SV_HIP(c, mu.alloc(qu.size()));
+    SV_HIP(c, mm.alloc(c, total));
+    SV_HIP(c, mu.alloc(c, qu.size()));
     SV_HIP(c, hipMemcpy(mm, qm.data(), sizeof(int) * total, hipMemcpyHostToDevice));
     SV_HIP(c, hipMemcpy(mu, qu.data(), sizeof(int) * qu.size(), hipMemcpyHostToDevice));
     SysArgs am = a;

@@ -26,56 +26,6 @@ int sv_fail(sv_ctx *c, int code, const char *fmt, ...) {
   return code;
 }
 
-// Device memory of a context.  A new node set takes over the blocks of the one
-// before it that fit (spare, at most a quarter larger than asked for): hipFree
-// and hipMalloc of ~60 blocks were 14 of the 24 ms of a 262k-node start-up.
-// What is left of them is given back once the set-up is complete (a first state
-// or operator), when memory runs out, with the next node set, and with the
-// context; more than SPARE_MAX is given back at once (a set-up of that size
-// takes 0.1 s).
-constexpr size_t SPARE_MAX = (size_t)4 << 30;
-int sv_alloc(sv_ctx *c, void **p, size_t bytes) {
-  if (bytes == 0) bytes = 16;
-  size_t best = c->spare.size();
-  for (size_t k = 0; k < c->spare.size(); k++) {
-    const size_t have = c->spare[k].bytes;
-    if (have >= bytes && have - bytes <= bytes / 4 &&
-        (best == c->spare.size() || have < c->spare[best].bytes))
-      best = k;
-  }
-  if (best < c->spare.size()) {
-    c->allocs.push_back(c->spare[best]);
-    c->spare.erase(c->spare.begin() + best);
-    *p = c->allocs.back().p;
-    return 0;
-  }
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && !c->spare.empty()) {
-    (void)hipGetLastError();
-    sv_release_spare(c);
-    e = hipMalloc(p, bytes);
-  }
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return sv_fail(c, SV_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
-  }
-  c->allocs.push_back(sv_blk{*p, bytes});
-  return 0;
-}
-
-void sv_release_spare(sv_ctx *c) {
-  for (const sv_blk &b : c->spare) (void)hipFree(b.p);
-  c->spare.clear();
-}
-
-void sv_free(sv_ctx *c, void *p) {
-  if (!p) return;
-  auto it = std::find_if(c->allocs.begin(), c->allocs.end(),
-                         [p](const sv_blk &b) { return b.p == p; });
-  if (it != c->allocs.end()) c->allocs.erase(it);
-  (void)hipFree(p);
-}
-
 #define SV_CHECK(c, cond, ...)                        \
   do {                                                \
     if (!(cond)) return sv_fail((c), SV_E_ARG, __VA_ARGS__); \
@@ -189,9 +139,7 @@ int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, cons
   SV_HIP(c, hipDeviceSynchronize());
   sv_release_spare(c);
   c->spare.swap(c->allocs);
-  size_t spare = 0;
-  for (const sv_blk &b : c->spare) spare += b.bytes;
-  if (spare > SPARE_MAX) sv_release_spare(c);
+  if (sv_spare_bytes(c) > SV_SPARE_MAX) sv_release_spare(c);
   sv_adj_free(c);
   c->x = c->y = c->h = c->hs = c->s = nullptr;
   c->node_type = c->irel = c->vrel = nullptr;
@@ -379,6 +327,7 @@ int sv_adapt_stencils(sv_ctx *c, double *h, double *h_small, int32_t *reductions
   if (h) SV_HIP(c, hipMemcpy(h, c->h, sizeof(double) * c->npfb, hipMemcpyDeviceToHost));
   if (h_small)
     SV_HIP(c, hipMemcpy(h_small, c->hs, sizeof(double) * c->npfb, hipMemcpyDeviceToHost));
+  sv_release_spare(c);   // a caller may have wanted the stencils alone
   return 0;
 }
 
@@ -453,6 +402,7 @@ int sv_get_weights(sv_ctx *c, int32_t nplink, double *w_grad, double *w_lap, dou
   if (lsum) SV_HIP(c, hipMemcpy(lsum, c->lsum, sizeof(double) * n, hipMemcpyDeviceToHost));
   if (hsum) SV_HIP(c, hipMemcpy(hsum, c->hsum, sizeof(double) * n, hipMemcpyDeviceToHost));
   if (vol) SV_HIP(c, hipMemcpy(vol, c->vol, sizeof(double) * n, hipMemcpyDeviceToHost));
+  sv_release_spare(c);   // a caller may have wanted the weights alone
   return 0;
 }
 
@@ -463,6 +413,7 @@ int sv_get_timing(sv_ctx *c, const char *what, double *ms) {
   else if (!strcmp(what, "weights_tune")) *ms = c->t_weights_tune;
   else if (!strcmp(what, "step")) *ms = c->t_step;
   else if (!strcmp(what, "systems")) *ms = c->n_systems;
+  else if (!strcmp(what, "spare_bytes")) *ms = (double)sv_spare_bytes(c);
   else if (!strncmp(what, "weights_variant_m", 17) && (what[17] == '4' || what[17] == '6' ||
                                                         what[17] == '8'))
     *ms = c->wvariant[(what[17] - '0') / 2 - 2];
@@ -850,8 +801,8 @@ int sv_filter_variables(sv_ctx *c, double *ro, double *rou, double *rov, double 
   if (int rc = ensure_sell(c)) return rc;
   const int np = c->np, n = c->npfb;
   DevTmp<double> in, out;
-  SV_HIP(c, in.alloc(6 * (size_t)np));
-  SV_HIP(c, out.alloc(6 * (size_t)n));
+  SV_HIP(c, in.alloc(c, 6 * (size_t)np));
+  SV_HIP(c, out.alloc(c, 6 * (size_t)n));
   double *f[6] = {ro, rou, rov, xx, xy, yy};
   const double *fin[6];
   double *fout[6];

@@ -348,7 +348,15 @@ static inline bool sv_order_supported(int m) { return m == 4 || m == 6 || m == 8
       return sv_fail((c), SV_E_HIP, "%s failed: %s (%s:%d)", #call,            \
                      hipGetErrorString(e_), __FILE__, __LINE__);               \
   } while (0)
+// ---- device memory (sv_mem.hip) ----
+// most that a context keeps of the node set before, bytes
+constexpr size_t SV_SPARE_MAX = (size_t)4 << 30;
 int sv_alloc(sv_ctx *c, void **p, size_t bytes);
+void sv_free(sv_ctx *c, void *p);
+// hipMalloc; where that fails, once more with the context's spare blocks given back
+hipError_t sv_dev_malloc(sv_ctx *c, void **p, size_t bytes);
+size_t sv_spare_bytes(const sv_ctx *c);
+void sv_release_spare(sv_ctx *c);
 
 // A temporary device buffer owned by the enclosing scope: freed on every exit
 // path, error returns included (hipFree waits for work that still uses it).
@@ -361,7 +369,9 @@ struct DevTmp {
   ~DevTmp() {
     if (p) (void)hipFree(p);
   }
-  hipError_t alloc(size_t count) { return hipMalloc((void **)&p, sizeof(T) * (count ? count : 1)); }
+  hipError_t alloc(sv_ctx *c, size_t count) {
+    return sv_dev_malloc(c, (void **)&p, sizeof(T) * (count ? count : 1));
+  }
   operator T *() const { return p; }
 };
 
@@ -378,8 +388,6 @@ struct EventTmp {
   operator hipEvent_t() const { return e; }
 };
 int sv_ensure_sell(sv_ctx *c);
-void sv_free(sv_ctx *c, void *p);
-void sv_release_spare(sv_ctx *c);
 
 // ---- kernels: nodes/neighbours (k_nodes.hip) ----
 int sv_dev_create_ghosts(sv_ctx *c);
