@@ -210,7 +210,16 @@ int sv_get_timing(sv_ctx *ctx, const char *what, double *ms);
  *       fit; 1 and 4 gather from memory with that many lanes per node (4 splits
  *       each node's links over a quad of lanes, for node sets too small to fill
  *       the chip at one), as 0 does where they do not fit, with 4 below 8 waves
- *       per CU. */
+ *       per CU.
+ *   "rollout_tape" (-1, 0, 1): whether sv_rollout_forward keeps what the reverse
+ *       sweep of its last checkpoint interval reads (704 bytes a node and step),
+ *       which sv_rollout_vjp otherwise computes again; the gradient is the same.
+ *       1: yes, where it takes at most a quarter of the free device memory;
+ *       0: no; -1 (default): in memory that an earlier sv_rollout_vjp took,
+ *       unless nothing read the tape of the rollout before.  sv_get_timing
+ *       "tape_steps" gives the steps there is memory for, "tape_written" 1 while
+ *       the last rollout's tape holds, "vjp_recomputed" the steps that the last
+ *       sv_rollout_vjp computed again. */
 int sv_set_option(sv_ctx *ctx, const char *key, double value);
 
 /* ---- derivative operators: derivatives.F90 ------------------------------ */

@@ -22,10 +22,10 @@
 // inside the transposed gather of stage k (two buffer sets, ping-pong), and
 // the pointwise part of stage 4 inside the fused mass-correction + filter
 // adjoint: one step's adjoint is six launches (a per-segment sum, the filter,
-// four transposed gathers; five of a small node set, whose filter makes the sum).  Rollouts keep the state every `checkpoint`
-// steps; the adjoint recomputes one checkpoint interval with the tape on and
-// walks it backwards; the last interval's tape is written by the rollout itself
-// where memory allows.
+// four transposed gathers; five of a small node set, whose filter makes the sum).
+// Rollouts keep the state every `checkpoint` steps; the adjoint recomputes one
+// checkpoint interval with the tape on and walks it backwards; the last
+// interval's tape is written by the rollout itself where it is wanted (want_tape).
 #include <string.h>
 
 #include <algorithm>
@@ -856,10 +856,11 @@ struct sv_adj {
   double *Uend = nullptr;
   sv_ctrl ctrl_end{};
   std::vector<double *> tape;    // [every][8]
-  // the tape holds the last interval of the last rollout; tape_used: the last
-  // one that a rollout wrote was read by a reverse sweep
+  // the tape holds the last interval of the last rollout; tape_used: a reverse
+  // sweep has followed the last rollout that wrote one
   bool taped = false, tape_used = true;
   double t_fwd = 0, t_bwd = 0;   // ms of the last rollout / vjp
+  int recomputed = 0;            // steps that the last vjp computed again
   int lpn = 1;                   // lanes per node of the transposed gathers (1 or 4)
 };
 
@@ -898,12 +899,14 @@ static int ensure_tape(sv_ctx *c, sv_adj *A, int steps) {
 
 // Whether a rollout writes the tape of its last interval (of `steps` steps), so
 // that the reverse sweep need not compute the interval again (75 us a step of
-// 16k nodes; writing costs 176 bytes a node and stage beside the ~2 kB read):
-// not after a rollout whose tape nothing read, nor where the tape would take
-// more than a quarter of the free memory.
+// 16k nodes; writing costs 176 bytes a node and stage beside the ~2 kB read).
+// Asked for ("rollout_tape" 1): where the tape takes at most a quarter of the
+// free memory.  Left to the library (-1): into the memory of an earlier reverse
+// sweep only, since whether this rollout will have one is not known (20 steps of
+// 1M nodes take 14 GB), and not after a rollout whose tape nothing read.
 static bool want_tape(sv_ctx *c, sv_adj *A, int steps) {
-  if (!A->tape_used) return false;
   const int more = std::max(0, steps - (int)A->tape.size() / 8);
+  if (c->rollout_tape <= 0) return c->rollout_tape < 0 && A->tape_used && more == 0;
   if (more > 0) {
     size_t free_b = 0, total = 0;
     if (hipMemGetInfo(&free_b, &total) != hipSuccess) return false;
@@ -911,6 +914,15 @@ static bool want_tape(sv_ctx *c, sv_adj *A, int steps) {
     if (per * more > free_b / 4) return false;
   }
   return ensure_tape(c, A, steps) == 0;
+}
+
+bool sv_adj_stat(sv_ctx *c, const char *what, double *v) {
+  const sv_adj *A = c->adj;
+  if (!strcmp(what, "tape_steps")) *v = A ? (double)(A->tape.size() / 8) : 0.0;
+  else if (!strcmp(what, "tape_written")) *v = A && A->taped;
+  else if (!strcmp(what, "vjp_recomputed")) *v = A ? A->recomputed : 0;
+  else return false;
+  return true;
 }
 
 void sv_adj_drop_tape(sv_ctx *c) {
@@ -1338,6 +1350,7 @@ static int rollout_vjp(sv_ctx *c, double loss_bar, const double *const ubar_fina
     k_adj_sum<1><<<c->nblk * SUBS, AB, 0, c->stream>>>(c->blk_seg, c->segk, A->Ubar, A->psum);
   SV_HIP(c, hipGetLastError());
   const int nck = (T + E - 1) / E;
+  A->recomputed = 0;
   for (int k = nck - 1; k >= 0; k--) {
     const int s0 = k * E, s1 = std::min(T, s0 + E);
     if (taped && k == nck - 1) {   // the rollout wrote its tape
@@ -1350,6 +1363,7 @@ static int rollout_vjp(sv_ctx *c, double loss_bar, const double *const ubar_fina
       SV_HIP(c, hipMemcpyAsync(c->ctrl, &A->ckpt_ctrl[k], sizeof(sv_ctrl),
                                hipMemcpyHostToDevice, c->stream));
       if (int rc = sv_dev_init_state(c)) return rc;
+      A->recomputed += s1 - s0;
       for (int s = s0; s < s1; s++)
         if (int rc = sv_dev_step_tape(c, A->tape.data() + 8 * (s - s0))) return rc;
     }

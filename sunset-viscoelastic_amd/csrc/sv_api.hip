@@ -428,7 +428,7 @@ int sv_get_timing(sv_ctx *c, const char *what, double *ms) {
            (what[14] == '4' || what[14] == '6' || what[14] == '8') && what[16] >= '0' &&
            what[16] <= '3')
     *ms = c->wtune_ms[(what[14] - '0') / 2 - 2][what[16] - '0'];
-  else return sv_fail(c, SV_E_ARG, "unknown timing '%s'", what);
+  else if (!sv_adj_stat(c, what, ms)) return sv_fail(c, SV_E_ARG, "unknown timing '%s'", what);
   return 0;
 }
 
@@ -465,6 +465,10 @@ int sv_set_option(sv_ctx *c, const char *key, double value) {
     SV_CHECK(c, value == 0.0 || value == 1.0 || value == 4.0,
              "adj_lanes must be 0 (by node count), 1 or 4");
     c->adj_lanes = (int)value;
+  } else if (!strcmp(key, "rollout_tape")) {
+    SV_CHECK(c, value == -1.0 || value == 0.0 || value == 1.0,
+             "rollout_tape must be -1 (as memory is there), 0 or 1");
+    c->rollout_tape = (int)value;
   } else if (!strcmp(key, "halo_sweeps")) {
     SV_CHECK(c, !c->have_state, "halo_sweeps must be set before sv_set_initial");
     c->halo_sweeps = value != 0.0 ? 1 : 0;

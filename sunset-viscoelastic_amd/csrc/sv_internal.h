@@ -103,6 +103,7 @@ struct sv_adj;   // adjoint work space (k_adjoint.hip)
 struct sv_ctx;
 void sv_adj_free(sv_ctx *c);
 void sv_adj_drop_tape(sv_ctx *c);   // a rollout's tape no longer holds
+bool sv_adj_stat(sv_ctx *c, const char *what, double *v);   // sv_get_timing's, of the adjoint
 #define SV_G_RO 0
 #define SV_G_U 1
 #define SV_G_V 2
@@ -308,6 +309,8 @@ struct sv_ctx {
   int halo_sweeps = 1;      // 1: stage neighbour halos in LDS when they fit
   int adj_lanes = 0;        // lanes per node of the adjoint's transposed gathers
                             // (1, 4; 0: by node count), read by sv_adj_setup
+  int rollout_tape = -1;    // rollouts write a tape: 0 no, 1 yes, -1 into memory that
+                            // an earlier reverse sweep took
   // ensemble launch groups: the blocks of the members of one LABFM order,
   // launched together with their own LDS halo budget (blist: logical blocks,
   // device).  lgroup_mode: -1 untuned, 0 one launch over all blocks, 1 one

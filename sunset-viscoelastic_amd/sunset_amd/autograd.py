@@ -38,7 +38,7 @@ def _set_params(solver, Wi, beta, eps):
 
 class RolloutLoss(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, U0, Wi, beta, eps, solver, nsteps, dt, checkpoint_every):
+    def forward(ctx, U0, Wi, beta, eps, solver, nsteps, dt, checkpoint_every, tape=None):
         _set_params(solver, Wi, beta, eps)
         if U0.is_cuda:
             U = U0.detach().to(torch.float64).contiguous()
@@ -58,7 +58,7 @@ class RolloutLoss(torch.autograd.Function):
             solver.set_state({k: u[q] for q, k in enumerate(KEYS)}, dt=dt)
             solver._has_state = True
         solver.adj_setup(checkpoint_every)
-        L = solver.rollout_forward(nsteps)
+        L = solver.rollout_forward(nsteps, tape)
         ctx.solver = solver
         ctx.device = U0.device
         ctx.cuda = U0.is_cuda
@@ -80,9 +80,13 @@ class RolloutLoss(torch.autograd.Function):
         out = []
         for has, key in zip(ctx.has, ("Wi", "beta", "eps")):
             out.append(torch.tensor(pg[key], dtype=torch.float64) if has else None)
-        return (G, *out, None, None, None, None)
+        return (G, *out, None, None, None, None, None)
 
 
 def rollout_loss(solver, U0, nsteps: int, dt: float, checkpoint_every: int = 20, Wi=None,
                  beta=None, eps=None):
-    return RolloutLoss.apply(U0, Wi, beta, eps, solver, nsteps, dt, checkpoint_every)
+    # a rollout that is differentiated keeps what its reverse sweep reads; an
+    # evaluation takes no memory for it
+    wanted = torch.is_grad_enabled() and any(
+        isinstance(t, torch.Tensor) and t.requires_grad for t in (U0, Wi, beta, eps))
+    return RolloutLoss.apply(U0, Wi, beta, eps, solver, nsteps, dt, checkpoint_every, wanted)

@@ -172,6 +172,7 @@ class Solver:
         self.h = h
         self.npfb = 0
         self.np = 0
+        self._tape = -1
 
     def close(self):
         if getattr(self, "h", None):
@@ -286,6 +287,8 @@ class Solver:
     def set_option(self, key: str, value: float):
         """sv_set_option (e.g. "halo_sweeps" 0/1 before set_initial)."""
         self._ck(lib().sv_set_option(self.h, key.encode(), float(value)))
+        if key == "rollout_tape":
+            self._tape = value
 
     def timing(self, what: str) -> float:
         v = C.c_double()
@@ -405,9 +408,17 @@ class Solver:
         self._ck(lib().sv_rhs_vjp(self.h, pin, pout))
         return dict(zip(self.STATE_KEYS, out))
 
-    def rollout_forward(self, nsteps: int) -> float:
+    def rollout_forward(self, nsteps: int, tape: Optional[bool] = None) -> float:
+        """tape: whether a rollout_vjp follows, for this rollout ("rollout_tape")."""
         L = C.c_double()
-        self._ck(lib().sv_rollout_forward(self.h, nsteps, C.byref(L)))
+        before = self._tape
+        if tape is not None:
+            self.set_option("rollout_tape", 1 if tape else 0)
+        try:
+            self._ck(lib().sv_rollout_forward(self.h, nsteps, C.byref(L)))
+        finally:
+            if tape is not None:
+                self.set_option("rollout_tape", before)
         return L.value
 
     def rollout_vjp(self, loss_bar: float = 1.0, ubar_final=None):
