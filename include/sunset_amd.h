@@ -168,6 +168,7 @@ int sv_get_weights(sv_ctx *ctx, int32_t nplink, double *ij_w_grad, double *ij_w_
  * that order (bit 0: persistent grid, else one block per system; bit 1:
  * 32-neighbour assembly tiles, else 16; -1 none);
  * "weights_tune_m<order>_<variant>" the autotuning sample time of a variant;
+ * "graph_steps" the steps of the last sv_run that hipGraphs ran;
  * "spare_bytes" the device memory that the context still holds of the node set
  * before (given back by the first operator, sv_set_initial, sv_get_weights,
  * sv_adapt_stencils, or an allocation that fails without it). */
@@ -291,9 +292,10 @@ int sv_calc_all_rhs(sv_ctx *ctx, int32_t iRKstep, double *rhs_ro, double *rhs_ro
                     double *rhs_rov, double *rhs_xx, double *rhs_xy, double *rhs_yy);
 /* nsteps of the main loop (sunset.F90:75-106): set_tstep, set_tstep_PID
  * (PID mode), step_rk3_4S_2R_EE (step.F90:218-512), itime += 1.  State stays
- * on the device; dt lives on the device.  use_graph != 0 captures the steps of
- * the call (up to 16) as a hipGraph and replays it; steps that do not fill one
- * are launched singly. */
+ * on the device; dt lives on the device.  use_graph != 0 replays hipGraphs: a
+ * call of up to 16 steps is one graph, captured by the first call of that many;
+ * a longer call replays graphs of 16, and the steps past the last of them are
+ * launched singly behind it.  New physics drop the graphs. */
 int sv_run(sv_ctx *ctx, int32_t nsteps, int32_t use_graph);
 /* As sv_run (eager launches) with HIP events recorded on the context's stream
  * between the launches of every step.  kernel_ms[8]: mean device time per step

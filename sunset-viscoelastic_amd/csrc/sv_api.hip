@@ -83,11 +83,21 @@ int sv_create(const sv_config *cfg, sv_ctx **out) {
   return 0;
 }
 
+// the captured steps hold the physics, the layout and the launch mode they were
+// captured with
+static void sv_drop_graphs(sv_ctx *c) {
+  for (hipGraphExec_t &g : c->graph_exec)
+    if (g) {
+      (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
+}
+
 void sv_destroy(sv_ctx *c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
+  sv_drop_graphs(c);
   for (const sv_blk &b : c->allocs) (void)hipFree(b.p);
   sv_release_spare(c);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -155,8 +165,7 @@ int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, cons
   c->segk = nullptr; c->blk_seg = nullptr; c->hseg.clear();
   c->L = sv_loopl{};
   c->tmp_phi = c->tmp_out = nullptr; c->tmp_cap = 0;
-  if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
-  c->graph_valid = false;
+  sv_drop_graphs(c);
   c->have_lists = c->have_weights = c->have_sums = c->have_filter = false;
   c->have_state = c->have_volsum = false;
   c->blist = nullptr; c->rnx = c->rny = nullptr; c->ooR = nullptr;
@@ -243,7 +252,7 @@ int sv_set_inflow(sv_ctx *c, int32_t inflow_type, int32_t velocity_control, doub
   c->ramp_time = ramp_time;
   if (c->have_phys) {
     derive_phys(c);
-    c->graph_valid = false;
+    sv_drop_graphs(c);
     if (c->have_state) {
       if (int rc = set_device(c)) return rc;
       return upload_segment(c);
@@ -413,6 +422,7 @@ int sv_get_timing(sv_ctx *c, const char *what, double *ms) {
   else if (!strcmp(what, "weights_tune")) *ms = c->t_weights_tune;
   else if (!strcmp(what, "step")) *ms = c->t_step;
   else if (!strcmp(what, "systems")) *ms = c->n_systems;
+  else if (!strcmp(what, "graph_steps")) *ms = c->graph_steps;
   else if (!strcmp(what, "spare_bytes")) *ms = (double)sv_spare_bytes(c);
   else if (!strncmp(what, "weights_variant_m", 17) && (what[17] == '4' || what[17] == '6' ||
                                                         what[17] == '8'))
@@ -439,7 +449,7 @@ int sv_set_option(sv_ctx *c, const char *key, double value) {
     SV_CHECK(c, value == -1.0 || value == 0.0 || value == 1.0,
              "ensemble_groups: -1 (retune), 0 (one launch) or 1 (one launch per group)");
     if (int rc = set_device(c)) return rc;
-    c->graph_valid = false;
+    sv_drop_graphs(c);
     if (value < 0.0) return sv_dev_tune_groups(c, 5);
     c->lgroup_mode = (value > 0.0 && c->lgroups.size() >= 2) ? 1 : 0;
     return 0;
@@ -635,7 +645,7 @@ int sv_set_phys(sv_ctx *c, const sv_phys *p) {
   derive_phys(c);
   sv_adj_drop_tape(c);   // a reverse sweep computes its intervals with the new values
   c->have_phys = true;
-  c->graph_valid = false;
+  sv_drop_graphs(c);
   if (c->have_state) {
     if (int rc = set_device(c)) return rc;
     return upload_segment(c);
@@ -721,7 +731,7 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
   if (int rc = sv_dev_init_state(c)) return rc;   // synchronises
   sv_release_spare(c);
   c->have_state = true;
-  c->graph_valid = false;
+  sv_drop_graphs(c);
   return 0;
 }
 
@@ -885,7 +895,22 @@ int sv_calc_all_rhs(sv_ctx *c, int32_t iRKstep, double *r0, double *r1, double *
   return 0;
 }
 
-constexpr int GRAPH_STEPS = 16;
+// The graph of `steps` steps: one for each length that a call asked for, so that
+// calls of mixed lengths replay theirs, whatever came before.
+static int step_graph(sv_ctx *c, int steps) {
+  if (c->graph_exec[steps]) return 0;
+  SV_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  int rc = 0;
+  for (int k = 0; k < steps && !rc; k++) rc = sv_dev_step(c, nullptr);
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamEndCapture(c->stream, &g);
+  if (!rc && e == hipSuccess) e = hipGraphInstantiate(&c->graph_exec[steps], g, nullptr, nullptr, 0);
+  if (g) (void)hipGraphDestroy(g);
+  if (rc) return rc;
+  if (e != hipSuccess) c->graph_exec[steps] = nullptr;
+  SV_HIP(c, e);
+  return 0;
+}
 
 int sv_run(sv_ctx *c, int32_t nsteps, int32_t use_graph) {
   SV_CHECK(c, c && c->have_state, "sv_set_initial must come first");
@@ -897,29 +922,16 @@ int sv_run(sv_ctx *c, int32_t nsteps, int32_t use_graph) {
   SV_HIP(c, hipEventRecord(e0, c->stream));
   int s = 0;
   if (use_graph && nsteps > 0) {
-    // Consecutive graph launches leave the GPU idle for ~8 us, so a graph holds
-    // the steps of a call, GRAPH_STEPS at most; it is captured again for calls
-    // of at least twice as many as it holds.  Steps that do not fill a graph
-    // are launched one by one.
-    const int want = std::min(nsteps, GRAPH_STEPS);
-    if (!c->graph_valid || want >= 2 * c->graph_steps) {
-      c->graph_valid = false;
-      if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
-      hipGraph_t g;
-      SV_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int rc = 0;
-      for (int k = 0; k < want && !rc; k++) rc = sv_dev_step(c, nullptr);
-      hipError_t ce = hipStreamEndCapture(c->stream, &g);
-      if (rc) return rc;
-      SV_HIP(c, ce);
-      SV_HIP(c, hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0));
-      SV_HIP(c, hipGraphDestroy(g));
-      c->graph_steps = want;
-      c->graph_valid = true;
-    }
-    for (; s + c->graph_steps <= nsteps; s += c->graph_steps)
-      SV_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
+    // Consecutive graph launches leave the GPU idle for ~8 us, so a call of up to
+    // SV_GRAPH_STEPS steps is one graph and a longer one graphs of that many; the
+    // steps past the last of these are launched singly, while the graphs run (a
+    // graph of their own would cost a new context's first call its capture, 11 us
+    // a step and 55 more).
+    const int want = std::min(nsteps, SV_GRAPH_STEPS);
+    if (int rc = step_graph(c, want)) return rc;
+    for (; s + want <= nsteps; s += want) SV_HIP(c, hipGraphLaunch(c->graph_exec[want], c->stream));
   }
+  c->graph_steps = s;
   for (; s < nsteps; s++)
     if (int rc = sv_dev_step(c, nullptr)) return rc;
   SV_HIP(c, hipEventRecord(e1, c->stream));

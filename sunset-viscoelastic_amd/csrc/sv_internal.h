@@ -207,6 +207,9 @@ __host__ __device__ __forceinline__ int64_t sv_w3(int64_t e, int c) {
 #define SV_FLIP_SHIFT 29
 #define SV_FLIP_MASK ((1 << SV_FLIP_SHIFT) - 1)
 
+// steps that one hipGraph holds at most
+#define SV_GRAPH_STEPS 16
+
 // a block of device memory
 struct sv_blk {
   void *p;
@@ -325,9 +328,8 @@ struct sv_ctx {
   // scratch for drop-in ops
   double *tmp_phi = nullptr, *tmp_out = nullptr; int tmp_cap = 0;
   // graph
-  hipGraphExec_t graph_exec = nullptr;
-  int graph_steps = 0;      // steps the captured graph holds
-  bool graph_valid = false;
+  hipGraphExec_t graph_exec[SV_GRAPH_STEPS + 1] = {};   // of 1 .. SV_GRAPH_STEPS steps
+  int graph_steps = 0;      // steps of the last sv_run that graphs ran
   // timings (ms)
   double t_neigh = 0, t_weights = 0, t_weights_tune = 0, t_step = 0;
   // device buffer registry for cleanup
