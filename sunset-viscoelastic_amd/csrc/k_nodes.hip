@@ -409,9 +409,11 @@ int sv_dev_find_neighbours(sv_ctx *c) {
                            hipMemcpyHostToDevice, c->stream));
   if (c->col_raw) sv_free(c, c->col_raw);
   if (sv_alloc(c, (void **)&c->col_raw, sizeof(int) * (c->nnz + 1))) return SV_E_NOMEM;
+  static_assert(NW * SV_LIST_MAX * (sizeof(double) + sizeof(int)) <= 64 * 1024,
+                "the longest lists of a block's nodes fit LDS");
   const int cap = maxk > 0 ? maxk : 1;
   const size_t shm = (size_t)NW * cap * (sizeof(double) + sizeof(int));
-  if (shm > 64 * 1024)
+  if (maxk > SV_LIST_MAX)
     return sv_fail(c, SV_E_OVERFLOW, "neighbour list of %d entries too long for the search", maxk);
   k_neigh<1><<<nb, NW * SV_WAVE, shm, c->stream>>>(npfb, G, c->x, c->y, c->h, c->hs, cstart, ip,
                                                    c->cnt, c->cnt_small, c->row_ptr, c->col_raw,

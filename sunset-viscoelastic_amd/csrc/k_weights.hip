@@ -1006,12 +1006,12 @@ __global__ __launch_bounds__(320, 1) void k_weights_big(SysArgs S_) {
 // 1581 -> 194 us on the 126k-node cylinder channel.)
 constexpr int SUM_B = 256;      // threads per block
 constexpr int SUM_E = 1024;     // CSR entries per block: sums, four arrays
-constexpr int FIL_E = 2048;     // filter coefficients, two arrays; no list is longer: the
-                                // neighbour search sorts at most 1365 candidates in LDS
+constexpr int FIL_E = 2048;     // filter coefficients, two arrays
 constexpr int SUM_R = 64;       // most rows per block
+static_assert(SV_LIST_MAX <= FIL_E, "k_filter_coeffs stages a block's rows at once, one at least");
 
-// rows per block for lists of at most maxk links (SUM_E / maxk, at least 1;
-// longer lists than that are walked in pieces)
+// rows per block for lists of at most maxk links: whole lists of `entries`, and
+// one at least (k_sums walks a longer one in pieces)
 inline int sum_rows(int maxk, int entries) {
   return std::max(1, std::min(SUM_R, entries / std::max(maxk, 1)));
 }
@@ -1633,6 +1633,9 @@ int sv_dev_sums(sv_ctx *c) {
 
 int sv_dev_filter_coeffs(sv_ctx *c) {
   const int n = c->npfb, R = sum_rows(c->maxK, FIL_E);
+  if ((int64_t)R * c->maxK > FIL_E)
+    return sv_fail(c, SV_E_OVERFLOW, "filter coefficients of %d-entry lists (%d at most)", c->maxK,
+                   FIL_E);
   k_filter_coeffs<<<(n + R - 1) / R, SUM_B, 0, c->stream>>>(n, R, c->row_ptr, c->cnt, c->col_raw,
                                                             c->x, c->y, c->h, c->s, c->node_type,
                                                             c->nb, c->wh, c->hsum);

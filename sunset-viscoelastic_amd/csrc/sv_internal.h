@@ -207,6 +207,10 @@ __host__ __device__ __forceinline__ int64_t sv_w3(int64_t e, int c) {
 #define SV_FLIP_SHIFT 29
 #define SV_FLIP_MASK ((1 << SV_FLIP_SHIFT) - 1)
 
+// Links a list has at most: the neighbour search sorts its candidates in LDS
+// (k_neigh), and the filter coefficients stage whole lists there.
+#define SV_LIST_MAX 1365
+
 // steps that one hipGraph holds at most
 #define SV_GRAPH_STEPS 16
 
