@@ -512,7 +512,7 @@ int build_halos(sv_ctx *c, sv_loopl &L, int hb, int nslot) {
     L.hmax = std::max(L.hmax, v);
     tot += v;
   }
-  L.halo = L.hmax <= SV_HALO_MAX && (size_t)L.hmax * SV_HALO_REC <= SV_HALO_LDS_MAX;
+  L.halo = L.hmax <= (hb == SV_WAVE ? SV_HALO_MAX : SV_HALO_LDS_MAX / SV_HALO_REC);
   if (!L.halo) return 0;
   L.hb = hb;
   SV_HIP(c, hipMemsetAsync(hcnt.p + nb, 0, sizeof(int), c->stream));

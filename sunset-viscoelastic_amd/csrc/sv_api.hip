@@ -663,7 +663,7 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
   if (int rc = sv_ensure_loop(c)) return rc;
   SV_CHECK(c, !c->has_mirror || c->L.halo,
            "symmetric/no-slip mirror ghosts need the LDS halo sweeps (halo_sweeps = 1 and "
-           "block halos within %d records)", SV_HALO_MAX);
+           "the halos of 64 nodes within %d records)", SV_HALO_MAX);
   if (int rc = ensure_state_buffers(c)) return rc;
   const int n = c->npfb;
   const bool lc = c->cfg.form == SV_FORM_LC;

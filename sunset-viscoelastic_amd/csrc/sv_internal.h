@@ -119,12 +119,12 @@ bool sv_adj_stat(sv_ctx *c, const char *what, double *v);   // sv_get_timing's, 
 // SV_BLOCK nodes, so every block of the node kernels lies in one member and
 // per-block partial reductions are per-member partial reductions.
 #define SV_BLOCK 256
-// LDS budget of a block's staged halo records (bytes)
-#define SV_HALO_LDS_MAX (64 * 1024)
 // LDS bytes of a staged halo record (log-conformation form; the direct form's
-// are smaller)
+// are smaller), and the budget of a block's: two workgroups a CU and more
 #define SV_HALO_REC 80
-// Halo records a block may have for the halo sweeps to be used at all
+#define SV_HALO_LDS_MAX (64 * 1024)
+// Halo records that a block of 64 slots, the smallest, may have (67 KB of the
+// CU's 160): mirror ghosts have no other way than the halo sweeps
 #define SV_HALO_MAX 853
 struct sv_segk {
   int base;      // first node (concatenated numbering), a multiple of SV_BLOCK
