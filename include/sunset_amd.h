@@ -168,6 +168,9 @@ int sv_get_weights(sv_ctx *ctx, int32_t nplink, double *ij_w_grad, double *ij_w_
  * that order (bit 0: persistent grid, else one block per system; bit 1:
  * 32-neighbour assembly tiles, else 16; -1 none);
  * "weights_tune_m<order>_<variant>" the autotuning sample time of a variant;
+ * "sweep_slots" the nodes per workgroup of the RK sweeps (0: gathers from memory),
+ * "sweep_fields" 1 where a slice's fields are shared by several wavefronts,
+ * "sweep_stream" 1 where the weights are loaded past the caches;
  * "graph_steps" the steps of the last sv_run that hipGraphs ran;
  * "spare_bytes" the device memory that the context still holds of the node set
  * before (given back by the first operator, sv_set_initial, sv_get_weights,

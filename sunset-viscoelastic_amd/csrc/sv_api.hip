@@ -422,6 +422,9 @@ int sv_get_timing(sv_ctx *c, const char *what, double *ms) {
   else if (!strcmp(what, "weights_tune")) *ms = c->t_weights_tune;
   else if (!strcmp(what, "step")) *ms = c->t_step;
   else if (!strcmp(what, "systems")) *ms = c->n_systems;
+  else if (!strcmp(what, "sweep_slots")) *ms = c->L.valid && c->L.halo ? c->L.hb : 0;
+  else if (!strcmp(what, "sweep_fields")) *ms = c->L.valid && c->L.halo && c->L.split;
+  else if (!strcmp(what, "sweep_stream")) *ms = c->L.valid && c->L.halo && c->L.nt;
   else if (!strcmp(what, "graph_steps")) *ms = c->graph_steps;
   else if (!strcmp(what, "spare_bytes")) *ms = (double)sv_spare_bytes(c);
   else if (!strncmp(what, "weights_variant_m", 17) && (what[17] == '4' || what[17] == '6' ||
