@@ -39,16 +39,6 @@ namespace {
 constexpr int BS = SV_BLOCK;   // threads per block of the node kernels
 constexpr int SPB = BS / SV_WAVE;   // slices (and partial results) per block
 
-// Gather-loop tuning (compile time): links processed per iteration, and
-// whether the streamed stencil arrays (columns, weights; read once per sweep)
-// are loaded non-temporally so they do not displace the gathered records in
-// the caches.
-#ifndef SV_GATHER_UNROLL
-#define SV_GATHER_UNROLL 2
-#endif
-#ifndef SV_STREAM_NT
-#define SV_STREAM_NT 1
-#endif
 // Pairs of links per batch in the halo-staged sweeps (the global streams are
 // prefetched one batch ahead), by threads per workgroup: a small node set has
 // one wave per SIMD at most and needs many requests per wave (128^2 order 6,
@@ -59,13 +49,11 @@ struct HaloU {
   static constexpr int U = NB == 64 ? 3 : NB == 128 ? 2 : 1;   // stage sweeps
   static constexpr int UF = NB == 64 ? 4 : 2;                  // the filter
 };
+// the stencil arrays of the sweeps that gather from memory: read once per sweep,
+// loaded non-temporally so that they do not displace the gathered records
 template <typename T>
 __device__ __forceinline__ T ld_stream(const T *p) {
-#if SV_STREAM_NT
   return __builtin_nontemporal_load(p);
-#else
-  return *p;
-#endif
 }
 
 // The node handled by this thread: segment of the block, concatenated index i,
@@ -745,25 +733,24 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
       if (MDIFF) { cxx_l += r.cxx * wlk; cxy_l += r.cxy * wlk; cyy_l += r.cyy * wlk; }
     }
   };
-  // Links in pairs, the column indices of the next pair loaded before the
-  // current pair is consumed, so each lane keeps two record gathers and the
-  // next index loads in flight.  Summation stays sequential in k.
-  constexpr int U = SV_GATHER_UNROLL;
+  // Links in pairs, as their weights lie (sv_w3): three 16-byte loads a pair (six
+  // of 8 bytes at 16-byte strides: 863 us a step of 400x400 order 6 LC, 670 so),
+  // the column indices of the next pair loaded before the current pair is
+  // consumed, so each lane keeps two record gathers and the next index loads in
+  // flight.  The pair at an odd list's end reads padding.  Summation stays
+  // sequential in k.
+  constexpr int U = 2;
   int jn[U];
 #pragma unroll
   for (int u = 0; u < U; u++) jn[u] = (u < K) ? ld_stream(a.col + b + (int64_t)u * SV_WAVE) : ii;
   for (int k = 0; k < K; k += U) {
     Rec9 r[U];
-    double wxk[U], wyk[U], wlk[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (k + u < K) {
-        const int64_t e = b + (int64_t)(k + u) * SV_WAVE;
-        r[u] = load_g<FORM>(a.G, jn[u]);
-        wxk[u] = ld_stream(a.w3 + sv_w3(e, 0)); wyk[u] = ld_stream(a.w3 + sv_w3(e, 1));
-        wlk[u] = ld_stream(a.w3 + sv_w3(e, 2));
-      }
-    }
+    for (int u = 0; u < U; u++)
+      if (k + u < K) r[u] = load_g<FORM>(a.G, jn[u]);
+    const dbl2 *w = reinterpret_cast<const dbl2 *>(a.w3 + sv_w3(b + (int64_t)k * SV_WAVE, 0));
+    const dbl2 wg[U] = {ld_stream(w), ld_stream(w + SV_WAVE)};
+    const dbl2 wl = ld_stream(w + 2 * SV_WAVE);
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int kn = k + U + u;
@@ -771,7 +758,7 @@ __global__ __launch_bounds__(BS) void k_stage(StageArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (k + u < K) accum(r[u], wxk[u], wyk[u], wlk[u]);
+      if (k + u < K) accum(r[u], wg[u].x, wg[u].y, u ? wl.y : wl.x);
   }
   double emax_loc = 0.0;
   if (act) {
@@ -1029,19 +1016,17 @@ __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
   const int K = act ? a.kcnt[ii] : 0;
   double t[6] = {0, 0, 0, 0, 0, 0};
   // pairs of links with the next pair's column indices prefetched, as k_stage
-  constexpr int U = SV_GATHER_UNROLL;
+  constexpr int U = 2;
   int jn[U];
 #pragma unroll
   for (int u = 0; u < U; u++) jn[u] = (u < K) ? ld_stream(a.col + b + (int64_t)u * SV_WAVE) : ii;
   for (int k = 0; k < K; k += U) {
-    double f[U][6], w[U];
+    double f[U][6];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (k + u < K) {
-        load_u(a.U, jn[u], f[u]);
-        w[u] = ld_stream(a.wh + sv_pair(b + (int64_t)(k + u) * SV_WAVE));
-      }
-    }
+    for (int u = 0; u < U; u++)
+      if (k + u < K) load_u(a.U, jn[u], f[u]);
+    const dbl2 w = ld_stream(
+        reinterpret_cast<const dbl2 *>(a.wh + sv_pair(b + (int64_t)k * SV_WAVE)));
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int kn = k + U + u;
@@ -1051,7 +1036,7 @@ __global__ __launch_bounds__(BS) void k_filter(FilterArgs a) {
     for (int u = 0; u < U; u++)
       if (k + u < K) {
 #pragma unroll
-        for (int q = 0; q < 6; q++) t[q] += f[u][q] * w[u];
+        for (int q = 0; q < 6; q++) t[q] += f[u][q] * (u ? w.y : w.x);
       }
   }
   const double m = wave_sum(act ? filter_point(a, nr, t, load_own(a, nr.i)) : 0.0);
