@@ -8,6 +8,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
+#include <new>
 
 #include "sv_internal.h"
 
@@ -1016,7 +1018,11 @@ int sv_ensemble_get_state(sv_ctx *c, int32_t member, double *ro, double *rou, do
   const size_t n = (size_t)S.npfb;
   // fields picked and put in the caller's order on the device, then one copy
   // per field (the host scatter of eleven fields cost ~50 ms at 1M nodes, and
-  // 9 of 29 ms for an ensemble of 566k)
+  // 9 of 29 ms for an ensemble of 566k).  A copy costs ~10 us however short, so
+  // the fields of few nodes come down together: 1600 nodes 237 -> 119 us, 16640
+  // 223 -> 185 (LC) and 180 -> 176 (DI), 32220 283 -> 299 and 232 -> 273; of an
+  // ensemble's member of 552 nodes 185 -> 64.
+  constexpr size_t TOGETHER = 16384;
   size_t most = 0;
   for (const sv_segk &s : c->hseg) most = std::max(most, (size_t)s.npfb);
   if (!c->fields_buf && sv_alloc(c, (void **)&c->fields_buf, sizeof(double) * 12 * most))
@@ -1025,8 +1031,21 @@ int sv_ensemble_get_state(sv_ctx *c, int32_t member, double *ro, double *rou, do
   SV_HIP(c, hipStreamSynchronize(c->stream));
   double *dst[11] = {ro, rou, rov, u, v, pxx, pxy, pyy, cxx, cxy, cyy};
   const bool lc = c->cfg.form == SV_FORM_LC;
+  int want = 0;
+  for (int q = 0; q < 11; q++) {
+    if (!lc && q >= 5 && q <= 7) dst[q] = nullptr;   // no psi
+    want += dst[q] != nullptr;
+  }
+  std::unique_ptr<double[]> h(want > 2 && n <= TOGETHER ? new (std::nothrow) double[11 * n]
+                                                        : nullptr);
+  if (h) {
+    SV_HIP(c, hipMemcpy(h.get(), c->fields_buf, sizeof(double) * 11 * n, hipMemcpyDeviceToHost));
+    for (int q = 0; q < 11; q++)
+      if (dst[q]) memcpy(dst[q], h.get() + (size_t)q * n, sizeof(double) * n);
+    return 0;
+  }
   for (int q = 0; q < 11; q++)
-    if (dst[q] && (lc || q < 5 || q > 7))
+    if (dst[q])
       SV_HIP(c, hipMemcpy(dst[q], c->fields_buf + (size_t)q * n, sizeof(double) * n,
                           hipMemcpyDeviceToHost));
   return 0;
