@@ -390,7 +390,9 @@ constexpr size_t lds_bytes(int kcap) {
   return sizeof(double) * ((size_t)svd_doubles<MF>(kcap) + 7 * nsz(MF) + 2 * (size_t)kcap) +
          sizeof(int) * (size_t)kcap + 64;
 }
-// longest list taken
+// Longest list taken: the limit of a layout with an area of its own for each of
+// these (U, V, the matrix, the rows, five arrays per neighbour) in 64 KB.  Longer
+// lists would fit today's; what is refused has stayed as it was.
 template <int MF>
 constexpr int list_max() {
   constexpr int fixed = 3 * nsz(MF) * nsz(MF) + 2 * RB * nsz(MF) + 7 * nsz(MF);

@@ -6,10 +6,9 @@
 // so every 64-node slice and every 256-node block is a compact rectangle of
 // the domain whatever the node counts along its sides.  A Morton order of the
 // positions does the same only on 2^k lattices: on a 301x283 order-8 lattice
-// its 256-node halos reached 947 records (mean 787) and no longer fitted the
-// 60 KB budget of the sweeps; split, they are 694 at most (mean 667); on
-// 260x260 at order 6, 829 -> 617 records, three resident blocks per CU
-// instead of two.
+// its 256-node halos reached 947 records (mean 787), more than the 819 that the
+// sweeps' LDS budget holds; split, they are 694 at most (mean 667); on 260x260
+// at order 6, 829 -> 617 records.
 // One level of the split is a stable radix sort of (segment, coordinate)
 // keys, 14 levels at 1M nodes.
 //
@@ -483,7 +482,7 @@ int kd_order(sv_ctx *c, int *perm, int by_len) {
 }
 
 // Halos of hb slots per block, nslot slots in all.  L.halo stays false when a
-// block's halo exceeds the LDS budget of the sweeps.
+// block's halo exceeds the LDS budget of the sweeps (of 64 slots: SV_HALO_MAX).
 int build_halos(sv_ctx *c, sv_loopl &L, int hb, int nslot) {
   // whole node blocks, as the sweeps' grids cover them: the halo blocks past
   // the last slot are empty

@@ -341,7 +341,7 @@ struct sv_ctx {
   std::vector<sv_blk> spare;    // of the node set before, not yet taken over
 };
 
-// ---- helpers (sv_api.cpp) ----
+// ---- helpers (sv_api.hip) ----
 // Sets the context's message (or, for c == NULL, the calling thread's
 // context-free message that sv_last_error(NULL) returns) and returns code.
 int sv_fail(sv_ctx *c, int code, const char *fmt, ...);
@@ -408,10 +408,13 @@ int sv_dev_build_sell(sv_ctx *c);
 int sv_dev_build_loop(sv_ctx *c);
 // the halos of the layout in c->L over nslot slots (a context's own, or an
 // ensemble's concatenated one)
-int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T);
-int sv_dev_slice_offsets(sv_ctx *c, int n, const int *cnt, int64_t *off, int64_t *total);
-int sv_dev_sell_halos(sv_ctx *c);
 int sv_dev_build_halos(sv_ctx *c, int nslot);
+// the lists of c->L by their targets, with their halos
+int sv_dev_build_transpose(sv_ctx *c, sv_loopl &T);
+// SELL-64 offsets of lists of cnt[n] links, and the entries in all
+int sv_dev_slice_offsets(sv_ctx *c, int n, const int *cnt, int64_t *off, int64_t *total);
+// the halos of the drop-in layout's slices
+int sv_dev_sell_halos(sv_ctx *c);
 int sv_ensure_loop(sv_ctx *c);
 // ---- kernels: weights (k_weights.hip) ----
 int sv_dev_weights(sv_ctx *c, const int *order_map_host);
@@ -452,10 +455,10 @@ int sv_check_device_ptr(sv_ctx *c, const void *p, const char *what);
 // state records in U from six caller-order device arrays (ro, u, v, c),
 // fields[6][npfb]
 int sv_dev_init_records(sv_ctx *c, const double *fields);
-int sv_dev_forcing(sv_ctx *c);
+int sv_dev_forcing(sv_ctx *c);                       // fx from the physics constants
 // sv_set_control's values (waits for them)
 int sv_dev_set_control(sv_ctx *c, double dt, double time, int itime, double e1, double e2,
-                       double e3, int dt_mode);                       // fx from the physics constants
+                       double e3, int dt_mode);
 int sv_dev_volume_sum(sv_ctx *c, double *sum);       // of the real nodes
 // ---- kernels: time stepping (k_step.hip) ----
 // gather records and set_tstep minima of the state in U (no correction)
