@@ -29,6 +29,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 
 #include "sv_internal.h"
 #include "sweep.h"
@@ -1170,6 +1171,24 @@ static int read_ctrl(sv_ctx *c, sv_ctrl *h) {
   return 0;
 }
 
+// how the reverse sweeps gather
+static int choose_gathers(sv_ctx *c) {
+  sv_adj *A = c->adj;
+  // lanes per node of the transposed gathers: 4 when one lane per node would
+  // give fewer than 8 waves per CU (e.g. a 128x128 lattice: 256 waves)
+  int ncu = 0;
+  SV_HIP(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+  const int64_t waves = (int64_t)c->nblk * SUBS;
+  A->lpn = c->adj_lanes == 1 || c->adj_lanes == 4 ? c->adj_lanes
+           : (waves < 8 * (int64_t)ncu ? 4 : 1);
+  // staged halos where they fit (for either records), one slice a workgroup
+  // (adj_lanes asks for the gathers from memory)
+  A->halo = c->adj_lanes == 0 && A->TL.halo &&
+            sizeof(double) * trans_rec<true>() * A->TL.hmax <= (size_t)SV_HALO_LDS_MAX;
+  if (A->halo) A->lpn = 1;
+  return 0;
+}
+
 extern "C" {
 
 int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
@@ -1186,41 +1205,28 @@ int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {
   if (int rc = read_ctrl(c, &h)) return rc;
   SV_ADJ_CHECK(c, h.dt_mode == SV_DT_FIXED,
                "the adjoint needs a fixed time step (sv_set_control with SV_DT_FIXED)");
-  if (!c->adj) {
-    sv_adj *A = new sv_adj();
-    c->adj = A;
-    const size_t R = (size_t)SV_US * c->ntot;
-    if (int rc = sv_dev_build_transpose(c, A->TL)) return rc;
-    if (adj_alloc(c, &A->Ubar, R) || adj_alloc(c, &A->Rbar, R) || adj_alloc(c, &A->regbar, R) ||
-        adj_alloc(c, &A->own[0], R) || adj_alloc(c, &A->own[1], R) ||
-        adj_alloc(c, &A->dbar[0], (size_t)SV_TAPE_D * c->ntot) ||
-        adj_alloc(c, &A->dbar[1], (size_t)SV_TAPE_D * c->ntot) ||
-        adj_alloc(c, &A->dbarm[0], (size_t)4 * c->ntot) ||
-        adj_alloc(c, &A->dbarm[1], (size_t)4 * c->ntot) ||
-        adj_alloc(c, &A->psum, (size_t)c->nblk * subl_of(4)) ||
-        adj_alloc(c, &A->sbar, c->nseg) || adj_alloc(c, &A->lpart, (size_t)LOSS_STEPS * c->nblk) ||
-        adj_alloc(c, &A->lmean, LOSS_STEPS) ||
-        adj_alloc(c, &A->lacc, c->nseg) || adj_alloc(c, &A->Uend, R) ||
-        adj_alloc(c, &A->pacc, (size_t)4 * c->ntot) || adj_alloc(c, &A->pred, 4))
-      return SV_E_NOMEM;
+  if (!c->adj) {   // whole or not at all
+    std::unique_ptr<sv_adj> A(new sv_adj());
+    const size_t R = (size_t)SV_US * c->ntot, N = c->ntot;
+    int rc = sv_dev_build_transpose(c, A->TL);
+    if (!rc)
+      rc = sv_alloc_all(
+          c, {sv_want(&A->Ubar, R), sv_want(&A->Rbar, R), sv_want(&A->regbar, R),
+              sv_want(&A->own[0], R), sv_want(&A->own[1], R), sv_want(&A->dbar[0], SV_TAPE_D * N),
+              sv_want(&A->dbar[1], SV_TAPE_D * N), sv_want(&A->dbarm[0], 4 * N),
+              sv_want(&A->dbarm[1], 4 * N), sv_want(&A->psum, (size_t)c->nblk * subl_of(4)),
+              sv_want(&A->sbar, c->nseg), sv_want(&A->lpart, (size_t)LOSS_STEPS * c->nblk),
+              sv_want(&A->lmean, LOSS_STEPS), sv_want(&A->lacc, c->nseg), sv_want(&A->Uend, R),
+              sv_want(&A->pacc, 4 * N), sv_want(&A->pred, 4)});
+    if (rc) {
+      sv_free_layout(c, A->TL);
+      return rc;
+    }
+    c->adj = A.release();
   }
   if (c->adj->every != checkpoint_every) c->adj->taped = false;
   c->adj->every = checkpoint_every;
-  // lanes per node of the transposed gathers: 4 when one lane per node would
-  // give fewer than 8 waves per CU (e.g. a 128x128 lattice: 256 waves)
-  {
-    int ncu = 0;
-    SV_HIP(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
-    const int64_t waves = (int64_t)c->nblk * SUBS;
-    c->adj->lpn = c->adj_lanes == 1 || c->adj_lanes == 4 ? c->adj_lanes
-                  : (waves < 8 * (int64_t)ncu ? 4 : 1);
-    // staged halos where they fit (for either records), one slice a workgroup
-    // (adj_lanes asks for the gathers from memory)
-    c->adj->halo = c->adj_lanes == 0 && c->adj->TL.halo &&
-                   sizeof(double) * trans_rec<true>() * c->adj->TL.hmax <= (size_t)SV_HALO_LDS_MAX;
-    if (c->adj->halo) c->adj->lpn = 1;
-  }
-  return 0;
+  return choose_gathers(c);
 }
 
 // calc_all_rhs vector-Jacobian product at the current state: ubar = J^T rbar

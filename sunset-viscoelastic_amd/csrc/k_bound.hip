@@ -357,11 +357,8 @@ int sv_dev_boundary_normals(sv_ctx *c, const double *rnx_host, const double *rny
       return sv_fail(c, SV_E_ARG, "boundary node %d: normal (%g, %g) is not a unit vector", i,
                      nx[i], ny[i]);
   }
-  if (!c->rnx) {
-    if (sv_alloc(c, (void **)&c->rnx, sizeof(double) * c->cap) ||
-        sv_alloc(c, (void **)&c->rny, sizeof(double) * c->cap))
-      return SV_E_NOMEM;
-  }
+  if (!c->rnx)
+    if (int rc = sv_alloc_all(c, {sv_want(&c->rnx, c->cap), sv_want(&c->rny, c->cap)})) return rc;
   SV_HIP(c, hipMemcpy(c->rnx, nx.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   SV_HIP(c, hipMemcpy(c->rny, ny.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   const int ng = c->np - n;

@@ -569,16 +569,19 @@ int sv_dev_build_halos(sv_ctx *c, int nslot) {
   return c->L.halo || b.hb == SV_WAVE ? 0 : build_halos(c, c->L, SV_WAVE, nslot);
 }
 
-static int build_layout(sv_ctx *c, int hb) {
-  const int n = c->npfb;
-  sv_loopl &L = c->L;
-  // (re)allocate
+void sv_free_layout(sv_ctx *c, sv_loopl &L) {
+  if (L.cnt_small == L.cnt) L.cnt_small = nullptr;   // transposed lists have the one
   void *old[] = {L.off, L.col, L.w3, L.wh, L.cnt, L.cnt_small, L.gsx, L.gsy,
                  L.lsum, L.hsum, L.vol, L.s, L.perm, L.iperm, L.hoff, L.hidx, L.lcol,
                  L.bidx, L.brec, L.lflip, L.krange};
-  for (void *b : old)
-    if (b) sv_free(c, b);
+  for (void *b : old) sv_free(c, b);
   L = sv_loopl{};
+}
+
+static int build_layout(sv_ctx *c, int hb) {
+  const int n = c->npfb;
+  sv_loopl &L = c->L;
+  sv_free_layout(c, L);
   const int ns = (n + SV_WAVE - 1) / SV_WAVE;
   L.nslices = ns;
   const size_t D = sizeof(double), I = sizeof(int);

@@ -383,11 +383,10 @@ int sv_dev_find_neighbours(sv_ctx *c) {
   k_cell_fill<<<(np + B - 1) / B, B, 0, c->stream>>>(np, cellof, cstart, ccount, ip);
   SV_HIP(c, hipGetLastError());
   // counts
-  if (!c->cnt) {
-    if (sv_alloc(c, (void **)&c->cnt, sizeof(int) * npfb)) return SV_E_NOMEM;
-    if (sv_alloc(c, (void **)&c->cnt_small, sizeof(int) * npfb)) return SV_E_NOMEM;
-    if (sv_alloc(c, (void **)&c->row_ptr, sizeof(int64_t) * (npfb + 1))) return SV_E_NOMEM;
-  }
+  if (!c->cnt)
+    if (int rc = sv_alloc_all(c, {sv_want(&c->cnt, npfb), sv_want(&c->cnt_small, npfb),
+                                  sv_want(&c->row_ptr, (size_t)npfb + 1)}))
+      return rc;
   const int nb = (npfb + NW - 1) / NW;
   k_neigh<0><<<nb, NW * SV_WAVE, 0, c->stream>>>(npfb, G, c->x, c->y, c->h, c->hs, cstart, ip,
                                                  c->cnt, c->cnt_small, nullptr, nullptr, 0);
@@ -407,7 +406,8 @@ int sv_dev_find_neighbours(sv_ctx *c) {
   c->nnz = rp[npfb];
   SV_HIP(c, hipMemcpyAsync(c->row_ptr, rp.data(), sizeof(int64_t) * (npfb + 1),
                            hipMemcpyHostToDevice, c->stream));
-  if (c->col_raw) sv_free(c, c->col_raw);
+  sv_free(c, c->col_raw);
+  c->col_raw = nullptr;
   if (sv_alloc(c, (void **)&c->col_raw, sizeof(int) * (c->nnz + 1))) return SV_E_NOMEM;
   static_assert(NW * SV_LIST_MAX * (sizeof(double) + sizeof(int)) <= 64 * 1024,
                 "the longest lists of a block's nodes fit LDS");

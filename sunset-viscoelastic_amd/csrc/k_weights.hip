@@ -1390,19 +1390,12 @@ int sv_dev_weights(sv_ctx *c, const int *order_map_host) {
     SV_HIP(c, hipStreamSynchronize(c->stream));
   }
   const size_t L = (size_t)c->nnz + 1;
-  if (!c->wx) {
-    if (sv_alloc(c, (void **)&c->wx, sizeof(double) * L) ||
-        sv_alloc(c, (void **)&c->wy, sizeof(double) * L) ||
-        sv_alloc(c, (void **)&c->wl, sizeof(double) * L) ||
-        sv_alloc(c, (void **)&c->wh, sizeof(double) * L) ||
-        sv_alloc(c, (void **)&c->vol, sizeof(double) * n) ||
-        sv_alloc(c, (void **)&c->gsx, sizeof(double) * n) ||
-        sv_alloc(c, (void **)&c->gsy, sizeof(double) * n) ||
-        sv_alloc(c, (void **)&c->lsum, sizeof(double) * n) ||
-        sv_alloc(c, (void **)&c->hsum, sizeof(double) * n) ||
-        sv_alloc(c, (void **)&c->singular, sizeof(int) * 4))
-      return SV_E_NOMEM;
-  }
+  if (!c->wx)
+    if (int rc = sv_alloc_all(
+            c, {sv_want(&c->wx, L), sv_want(&c->wy, L), sv_want(&c->wl, L), sv_want(&c->wh, L),
+                sv_want(&c->vol, n), sv_want(&c->gsx, n), sv_want(&c->gsy, n),
+                sv_want(&c->lsum, n), sv_want(&c->hsum, n), sv_want(&c->singular, 4)}))
+      return rc;
   SV_HIP(c, hipMemsetAsync(c->wx, 0, sizeof(double) * L, c->stream));
   SV_HIP(c, hipMemsetAsync(c->wy, 0, sizeof(double) * L, c->stream));
   SV_HIP(c, hipMemsetAsync(c->wl, 0, sizeof(double) * L, c->stream));

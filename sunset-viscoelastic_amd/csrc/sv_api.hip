@@ -40,6 +40,16 @@ int sv_ensure_sell(sv_ctx *c) {
   return 0;
 }
 
+// the captured steps hold the physics, the layout and the launch mode they were
+// captured with
+static void sv_drop_graphs(sv_ctx *c) {
+  for (hipGraphExec_t &g : c->graph_exec)
+    if (g) {
+      (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
+}
+
 int sv_ensure_loop(sv_ctx *c) {
   if (c->L.valid) return 0;
   return sv_dev_build_loop(c);
@@ -83,16 +93,6 @@ int sv_create(const sv_config *cfg, sv_ctx **out) {
   sv_diag_scratch_init(c->device);
   *out = c;
   return 0;
-}
-
-// the captured steps hold the physics, the layout and the launch mode they were
-// captured with
-static void sv_drop_graphs(sv_ctx *c) {
-  for (hipGraphExec_t &g : c->graph_exec)
-    if (g) {
-      (void)hipGraphExecDestroy(g);
-      g = nullptr;
-    }
 }
 
 void sv_destroy(sv_ctx *c) {
@@ -197,12 +197,11 @@ int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, cons
   c->nb = (int)c->hblist.size();
   c->npfb = npfb;
   c->cap = 9 * npfb + 64;      // at most 8 ghosts per node
-  const size_t D = sizeof(double) * c->cap, I = sizeof(int) * c->cap;
-  if (sv_alloc(c, (void **)&c->x, D) || sv_alloc(c, (void **)&c->y, D) ||
-      sv_alloc(c, (void **)&c->h, D) || sv_alloc(c, (void **)&c->hs, D) ||
-      sv_alloc(c, (void **)&c->s, D) || sv_alloc(c, (void **)&c->node_type, I) ||
-      sv_alloc(c, (void **)&c->irel, I) || sv_alloc(c, (void **)&c->vrel, I))
-    return SV_E_NOMEM;
+  const size_t N = c->cap;
+  if (int rc = sv_alloc_all(c, {sv_want(&c->x, N), sv_want(&c->y, N), sv_want(&c->h, N),
+                                sv_want(&c->hs, N), sv_want(&c->s, N), sv_want(&c->node_type, N),
+                                sv_want(&c->irel, N), sv_want(&c->vrel, N)}))
+    return rc;
   const size_t n8 = sizeof(double) * npfb;
   SV_HIP(c, hipMemcpy(c->x, x, n8, hipMemcpyHostToDevice));
   SV_HIP(c, hipMemcpy(c->y, y, n8, hipMemcpyHostToDevice));
@@ -500,11 +499,11 @@ int sv_set_option(sv_ctx *c, const char *key, double value) {
 static int ensure_tmp(sv_ctx *c) {
   const int need = c->np > 2 * c->npfb ? c->np : 2 * c->npfb;
   if (c->tmp_cap >= need) return 0;
-  if (c->tmp_phi) sv_free(c, c->tmp_phi);
-  if (c->tmp_out) sv_free(c, c->tmp_out);
-  if (sv_alloc(c, (void **)&c->tmp_phi, sizeof(double) * need) ||
-      sv_alloc(c, (void **)&c->tmp_out, sizeof(double) * need))
-    return SV_E_NOMEM;
+  sv_free(c, c->tmp_phi);
+  sv_free(c, c->tmp_out);
+  c->tmp_cap = 0;
+  if (int rc = sv_alloc_all(c, {sv_want(&c->tmp_phi, need), sv_want(&c->tmp_out, need)}))
+    return rc;
   c->tmp_cap = need;
   return 0;
 }
@@ -602,21 +601,16 @@ static int ensure_state_buffers(sv_ctx *c) {
   c->nseg = 1;
   c->nblk = (c->npfb + SV_BLOCK - 1) / SV_BLOCK;
   c->ntot = c->nblk * SV_BLOCK;
-  const size_t nu = sizeof(double) * SV_US * (size_t)c->ntot;
-  const size_t ng = sizeof(double) * c->gs * (size_t)c->ntot;
-  if (sv_alloc(c, (void **)&c->U, nu) || sv_alloc(c, (void **)&c->Uf, nu) ||
-      sv_alloc(c, (void **)&c->reg, nu) || sv_alloc(c, (void **)&c->eacc, nu) ||
-      sv_alloc(c, (void **)&c->GA, ng) || sv_alloc(c, (void **)&c->GB, ng))
-    return SV_E_NOMEM;
-  SV_HIP(c, hipMemsetAsync(c->GA, 0, ng, c->stream));
-  SV_HIP(c, hipMemsetAsync(c->GB, 0, ng, c->stream));
   c->npartial = 4 * c->nblk * (SV_BLOCK / SV_WAVE);   // four kinds, one per slice
-  if (sv_alloc(c, (void **)&c->partial, sizeof(double) * (c->npartial + 8)) ||
-      sv_alloc(c, (void **)&c->ctrl, 2 * sizeof(sv_ctrl)) ||
-      sv_alloc(c, (void **)&c->fx, sizeof(double) * c->ntot) ||
-      sv_alloc(c, (void **)&c->segk, sizeof(sv_segk)) ||
-      sv_alloc(c, (void **)&c->blk_seg, sizeof(int) * c->nblk))
-    return SV_E_NOMEM;
+  const size_t N = c->ntot, nu = SV_US * N, ng = c->gs * N;
+  if (int rc = sv_alloc_all(
+          c, {sv_want(&c->U, nu), sv_want(&c->Uf, nu), sv_want(&c->reg, nu),
+              sv_want(&c->eacc, nu), sv_want(&c->GA, ng), sv_want(&c->GB, ng),
+              sv_want(&c->partial, (size_t)c->npartial + 8), sv_want(&c->ctrl, 2),
+              sv_want(&c->fx, N), sv_want(&c->segk, 1), sv_want(&c->blk_seg, c->nblk)}))
+    return rc;
+  SV_HIP(c, hipMemsetAsync(c->GA, 0, sizeof(double) * ng, c->stream));
+  SV_HIP(c, hipMemsetAsync(c->GB, 0, sizeof(double) * ng, c->stream));
   SV_HIP(c, hipMemsetAsync(c->fx, 0, sizeof(double) * c->ntot, c->stream));
   SV_HIP(c, hipMemsetAsync(c->blk_seg, 0, sizeof(int) * c->nblk, c->stream));
   return 0;
@@ -681,6 +675,7 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
   // the six arrays to the device as they are, the records made there
   if (!c->fields_buf && sv_alloc(c, (void **)&c->fields_buf, sizeof(double) * 12 * (size_t)n))
     return SV_E_NOMEM;
+  c->have_state = false;   // until the new one is whole
   const double *src[6] = {ro, u, v, cxx, cxy, cyy};
   for (int q = 0; q < 6; q++)
     SV_HIP(c, hipMemcpyAsync(c->fields_buf + (size_t)q * n, src[q], sizeof(double) * n,
@@ -717,11 +712,8 @@ int sv_set_initial(sv_ctx *c, const double *ro, const double *u, const double *v
     for (int k = 0; k < n; k++) bidx[k] = jbof[P[k]];
     sv_free(c, c->L.bidx);
     sv_free(c, c->L.brec);
-    c->L.bidx = nullptr;
-    c->L.brec = nullptr;
-    if (sv_alloc(c, (void **)&c->L.bidx, sizeof(int) * c->ntot) ||
-        sv_alloc(c, (void **)&c->L.brec, sizeof(double) * br.size()))
-      return SV_E_NOMEM;
+    if (int rc = sv_alloc_all(c, {sv_want(&c->L.bidx, c->ntot), sv_want(&c->L.brec, br.size())}))
+      return rc;
     SV_HIP(c, hipMemset(c->L.bidx, 0xff, sizeof(int) * c->ntot));
     SV_HIP(c, hipMemcpy(c->L.bidx, bidx.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     SV_HIP(c, hipMemcpy(c->L.brec, br.data(), sizeof(double) * br.size(),

@@ -47,6 +47,19 @@ int sv_alloc(sv_ctx *c, void **p, size_t bytes) {
   return 0;
 }
 
+int sv_alloc_all(sv_ctx *c, std::initializer_list<sv_req> reqs) {
+  for (const sv_req &r : reqs) *r.p = nullptr;
+  for (const sv_req &r : reqs)
+    if (int rc = sv_alloc(c, r.p, r.bytes)) {
+      for (const sv_req &q : reqs) {
+        sv_free(c, *q.p);
+        *q.p = nullptr;
+      }
+      return rc;
+    }
+  return 0;
+}
+
 size_t sv_spare_bytes(const sv_ctx *c) {
   size_t n = 0;
   for (const sv_blk &b : c->spare) n += b.bytes;
