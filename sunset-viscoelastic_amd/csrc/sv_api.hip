@@ -136,44 +136,8 @@ int sv_set_domain(sv_ctx *c, double xmin, double xmax, double ymin, double ymax,
   return 0;
 }
 
-int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, const double *s,
-                 const double *h, const double *h_small, const int32_t *node_type) {
-  SV_CHECK(c, c && x && y && s && h && h_small, "null argument");
-  SV_CHECK(c, c->have_domain, "sv_set_domain must come first");
-  SV_CHECK(c, !c->is_ensemble, "not available on an ensemble context");
-  SV_CHECK(c, npfb > 0, "npfb must be positive");
-  if (int rc = set_device(c)) return rc;
-  for (int i = 0; i < npfb; i++)
-    SV_CHECK(c, h[i] > 0 && h_small[i] > 0 && h_small[i] <= h[i] && s[i] > 0,
-             "node %d: need 0 < h_small <= h and s > 0", i);
-  // drop everything derived from an earlier node set; no work of any stream on
-  // its memory is left
-  SV_HIP(c, hipDeviceSynchronize());
-  sv_release_spare(c);
-  c->spare.swap(c->allocs);
-  if (sv_spare_bytes(c) > SV_SPARE_MAX) sv_release_spare(c);
-  sv_adj_free(c);
-  c->x = c->y = c->h = c->hs = c->s = nullptr;
-  c->node_type = c->irel = c->vrel = nullptr;
-  c->cnt = c->cnt_small = nullptr; c->row_ptr = nullptr; c->col_raw = nullptr;
-  c->wx = c->wy = c->wl = c->wh = nullptr;
-  c->gsx = c->gsy = c->lsum = c->hsum = c->vol = nullptr;
-  c->sell_off = nullptr; c->sell_w = nullptr; c->scol = c->scol_raw = nullptr;
-  c->slcol = nullptr; c->shoff = nullptr; c->shidx = nullptr; c->shmax = 0; c->shcap = 0;
-  c->swx = c->swy = c->swl = c->swh = nullptr; c->nslices = 0; c->sell_nnz = 0;
-  c->singular = nullptr; c->fx = nullptr; c->partial = nullptr; c->ctrl = nullptr;
-  c->U = c->Uf = c->reg = c->eacc = nullptr;
-  c->GA = c->GB = nullptr;
-  c->segk = nullptr; c->blk_seg = nullptr; c->hseg.clear();
-  c->L = sv_loopl{};
-  c->tmp_phi = c->tmp_out = nullptr; c->tmp_cap = 0;
-  sv_drop_graphs(c);
-  c->have_lists = c->have_weights = c->have_sums = c->have_filter = false;
-  c->have_state = c->have_volsum = false;
-  c->blist = nullptr; c->rnx = c->rny = nullptr; c->ooR = nullptr;
-  c->wtt = c->wtt_sum = nullptr; c->wtt_ld = 0;
-  c->fields_buf = nullptr;
-  c->have_normals = c->have_bweights = false;
+static int take_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, const double *s,
+                      const double *h, const double *h_small, const int32_t *node_type) {
   // boundary nodes and their FD rows (setup_domain.F90:179-193, :314-326)
   c->hnt.assign(npfb, 999);
   if (node_type) c->hnt.assign(node_type, node_type + npfb);
@@ -227,6 +191,51 @@ int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, cons
                         hipMemcpyHostToDevice));
   }
   return sv_dev_create_ghosts(c);
+}
+
+int sv_set_nodes(sv_ctx *c, int32_t npfb, const double *x, const double *y, const double *s,
+                 const double *h, const double *h_small, const int32_t *node_type) {
+  SV_CHECK(c, c && x && y && s && h && h_small, "null argument");
+  SV_CHECK(c, c->have_domain, "sv_set_domain must come first");
+  SV_CHECK(c, !c->is_ensemble, "not available on an ensemble context");
+  SV_CHECK(c, npfb > 0, "npfb must be positive");
+  if (int rc = set_device(c)) return rc;
+  for (int i = 0; i < npfb; i++)
+    SV_CHECK(c, h[i] > 0 && h_small[i] > 0 && h_small[i] <= h[i] && s[i] > 0,
+             "node %d: need 0 < h_small <= h and s > 0", i);
+  // drop everything derived from an earlier node set; no work of any stream on
+  // its memory is left
+  SV_HIP(c, hipDeviceSynchronize());
+  sv_release_spare(c);
+  c->spare.swap(c->allocs);
+  if (sv_spare_bytes(c) > SV_SPARE_MAX) sv_release_spare(c);
+  sv_adj_free(c);
+  c->x = c->y = c->h = c->hs = c->s = nullptr;
+  c->node_type = c->irel = c->vrel = nullptr;
+  c->cnt = c->cnt_small = nullptr; c->row_ptr = nullptr; c->col_raw = nullptr;
+  c->wx = c->wy = c->wl = c->wh = nullptr;
+  c->gsx = c->gsy = c->lsum = c->hsum = c->vol = nullptr;
+  c->sell_off = nullptr; c->sell_w = nullptr; c->scol = c->scol_raw = nullptr;
+  c->slcol = nullptr; c->shoff = nullptr; c->shidx = nullptr; c->shmax = 0; c->shcap = 0;
+  c->swx = c->swy = c->swl = c->swh = nullptr; c->nslices = 0; c->sell_nnz = 0;
+  c->singular = nullptr; c->fx = nullptr; c->partial = nullptr; c->ctrl = nullptr;
+  c->U = c->Uf = c->reg = c->eacc = nullptr;
+  c->GA = c->GB = nullptr;
+  c->segk = nullptr; c->blk_seg = nullptr; c->hseg.clear();
+  c->L = sv_loopl{};
+  c->tmp_phi = c->tmp_out = nullptr; c->tmp_cap = 0;
+  sv_drop_graphs(c);
+  c->have_lists = c->have_weights = c->have_sums = c->have_filter = false;
+  c->have_state = c->have_volsum = false;
+  c->blist = nullptr; c->rnx = c->rny = nullptr; c->ooR = nullptr;
+  c->wtt = c->wtt_sum = nullptr; c->wtt_ld = 0;
+  c->fields_buf = nullptr;
+  c->have_normals = c->have_bweights = false;
+  // a set that is refused leaves none
+  c->npfb = c->np = c->nb = 0;
+  const int rc = take_nodes(c, npfb, x, y, s, h, h_small, node_type);
+  if (rc) c->npfb = c->np = c->nb = 0;
+  return rc;
 }
 
 int sv_set_boundaries(sv_ctx *c, const double *rnx, const double *rny) {
@@ -298,7 +307,10 @@ int sv_find_neighbours(sv_ctx *c, int32_t nplink, int32_t *ij_count, int32_t *ij
                        int32_t *ij_link) {
   SV_CHECK(c, c && c->npfb > 0, "sv_set_nodes must come first");
   if (int rc = set_device(c)) return rc;
-  if (int rc = sv_dev_find_neighbours(c)) return rc;
+  if (int rc = sv_dev_find_neighbours(c)) {   // no lists: nothing that reads them
+    c->have_lists = c->have_weights = c->have_sums = c->have_filter = false;
+    return rc;
+  }
   c->nplink = nplink;
   if (ij_count)
     SV_HIP(c, hipMemcpy(ij_count, c->cnt, sizeof(int) * c->npfb, hipMemcpyDeviceToHost));
