@@ -1189,6 +1189,22 @@ static int choose_gathers(sv_ctx *c) {
   return 0;
 }
 
+// Where the lists cannot be made the adjoint goes (its buffers with the node
+// set), so that no reverse sweep runs on lists of the old layout.
+int sv_adj_new_layout(sv_ctx *c) {
+  sv_adj *A = c->adj;
+  if (!A) return 0;
+  A->taped = false;
+  sv_free_layout(c, A->TL);
+  int rc = sv_dev_build_transpose(c, A->TL);
+  if (!rc) rc = choose_gathers(c);
+  if (rc) {
+    sv_free_layout(c, A->TL);
+    sv_adj_free(c);
+  }
+  return rc;
+}
+
 extern "C" {
 
 int sv_adj_setup(sv_ctx *c, int32_t checkpoint_every) {

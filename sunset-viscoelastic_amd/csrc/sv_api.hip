@@ -52,7 +52,19 @@ static void sv_drop_graphs(sv_ctx *c) {
 
 int sv_ensure_loop(sv_ctx *c) {
   if (c->L.valid) return 0;
-  return sv_dev_build_loop(c);
+  // What holds the old layout goes with it: captured steps, the transposed lists,
+  // and boundary records, without which a state is none.  (The node order follows
+  // from positions and list lengths, which change with a new node set alone, but
+  // for the pruned lists of boundary nodes.)
+  sv_drop_graphs(c);
+  const bool state = c->have_state;
+  c->have_state = false;
+  if (int rc = sv_dev_build_loop(c)) {
+    sv_adj_free(c);
+    return rc;
+  }
+  c->have_state = state && c->nb == 0;
+  return sv_adj_new_layout(c);
 }
 
 static int set_device(sv_ctx *c) {

@@ -79,6 +79,9 @@ int sv_ensemble_create(sv_ctx *const *members, int32_t nmembers, sv_ctx **out) {
     sv_ctx *c = members[m];
     if (hipSetDevice(c->device) != hipSuccess) return fail(SV_E_HIP);
     if (int rc = sv_ensure_loop(c)) return fail_msg(rc, c->err.c_str());
+    if (!c->have_state)
+      return fail_msg(SV_E_STATE, "a member with boundary nodes had its stencils made again "
+                                  "after sv_set_initial, which must follow them");
     if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(SV_E_HIP);
     sv_segk &S = E->hseg[m];
     S.base = (int)nodes;

@@ -105,6 +105,7 @@ struct sv_adj;   // adjoint work space (k_adjoint.hip)
 struct sv_ctx;
 void sv_adj_free(sv_ctx *c);
 void sv_adj_drop_tape(sv_ctx *c);   // a rollout's tape no longer holds
+int sv_adj_new_layout(sv_ctx *c);   // the transposed lists of a layout made again
 bool sv_adj_stat(sv_ctx *c, const char *what, double *v);   // sv_get_timing's, of the adjoint
 #define SV_G_RO 0
 #define SV_G_U 1
